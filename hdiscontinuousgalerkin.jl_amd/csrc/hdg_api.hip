@@ -16,7 +16,7 @@
 #include "../../include/hdg.h"
 #include "hdg_arena.h"
 #include "hdg_host.h"
-#include "hdg_internal.h"
+#include "hdg_quad.h"
 #include "hdg_tables.h"
 
 using namespace hdg;
@@ -33,12 +33,9 @@ struct hdg_ctx {
   hdg_arena* arena = nullptr;  // serving loop's arena, or null
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // second stream for the multigrid set-up beside the Lanczos steps
+  // second stream for the vertex-level set-up beside the Lanczos steps
   hipStream_t aux = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_fill = nullptr, ev_join = nullptr;
-  // hdg_run queued the multigrid set-up on aux beside the assembly; the
-  // solve joins it instead of queueing it
-  bool mg_forked = false;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::string err;
 
   // mesh
@@ -85,10 +82,14 @@ struct hdg_ctx {
   double* d_scal = nullptr; // [0] errornorm, [1] true residual^2
   double* d_part2 = nullptr;
 
-  // mixed precision (HDG_MIXED): the multigrid preconditioner's trace-level
-  // data in float: trace matrix, Jacobi blocks, S P0, e0, res0
-  float *f_vals = nullptr, *f_blk = nullptr, *f_Dinv = nullptr, *f_sp = nullptr;
-  float *f_e0 = nullptr, *f_res0 = nullptr;
+  // multigrid contexts: the reduced trace system (hdg_quad.h)
+  QuadSys qs;
+  QuadInst qi;
+  QuadLaunch ql;
+  int* d_plain = nullptr;
+  // the assembled trace matrix and rhs (T) hold the current operators (a
+  // multigrid context's hdg_run does not need them)
+  bool filled = false;
 
   // captured chunks of CG iterations, one per read-back slot (valid until
   // the next hdg_setup / hdg_set_mesh); solves since the set-up
@@ -212,18 +213,29 @@ void free_problem(hdg_ctx* c) {
   dfree(c, c->cg.part);
   dfree(c, c->d_uhat);
   dfree(c, c->d_part2);
-  dfree(c, c->mg.cellA);
-  dfree(c, c->mg.e0);
-  dfree(c, c->mg.res0);
-  dfree(c, c->mg.fc);
-  dfree(c, c->mg.sp);
+  QuadSys& q = c->qs;
+  dfree(c, q.blk);
+  dfree(c, q.D);
+  dfree(c, q.Dinv);
+  dfree(c, q.tp);
+  dfree(c, q.bq);
+  dfree(c, q.cq);
+  dfree(c, q.fblk);
+  dfree(c, q.fDinv);
+  dfree(c, q.ftp);
+  dfree(c, q.mask);
+  dfree(c, q.x);
+  dfree(c, q.r0);
+  dfree(c, q.r1);
+  dfree(c, q.z);
+  dfree(c, q.p);
+  dfree(c, q.q);
+  dfree(c, q.res);
+  dfree(c, q.part);
+  dfree(c, c->d_plain);
+  q = QuadSys{};
+  c->filled = false;
   dfree(c, c->d_mg);
-  dfree(c, c->f_vals);
-  dfree(c, c->f_blk);
-  dfree(c, c->f_Dinv);
-  dfree(c, c->f_sp);
-  dfree(c, c->f_e0);
-  dfree(c, c->f_res0);
   c->has_setup = c->assembled = c->solved = c->recovered = false;
   c->csched = CondenseSched{};
   c->tuned = false;
@@ -241,11 +253,6 @@ void free_mesh(hdg_ctx* c) {
   dfree(c, c->pat.self);
   dfree(c, c->pat.tslot);
   dfree(c, c->pat.nbr);
-  dfree(c, c->mg.fv);
-  dfree(c, c->mg.vf_ptr);
-  dfree(c, c->mg.vf_idx);
-  dfree(c, c->mg.vf2);
-  dfree(c, c->mg.fq4);
   dfree(c, c->mg.tailpack);
   dfree(c, c->mg.cinv);
   for (int l = 0; l < kMaxLevels; ++l) {
@@ -288,47 +295,6 @@ bool detect_structured(int64_t nn, int64_t nc, const int64_t* cells, int* nx_out
 
 namespace hdg {
 
-bool face_vertex_maps(int64_t nn, int64_t nf, const int64_t* faces, const int64_t* cells, std::vector<int>& fv,
-                      std::vector<int>& vf_ptr, std::vector<int>& vf_idx, std::vector<int>* fq4) {
-  fv.assign(2 * nf, 0);
-  vf_ptr.assign(nn + 1, 0);
-  for (int64_t f = 0; f < nf; ++f) {
-    const int a = (int)faces[f] - 1, b = (int)faces[f + nf] - 1;
-    fv[2 * f] = std::min(a, b);
-    fv[2 * f + 1] = std::max(a, b);
-    vf_ptr[a + 1]++;
-    vf_ptr[b + 1]++;
-  }
-  for (int64_t v = 0; v < nn; ++v) vf_ptr[v + 1] += vf_ptr[v];
-  vf_idx.assign(vf_ptr[nn], 0);
-  std::vector<int> pos(vf_ptr.begin(), vf_ptr.end() - 1);
-  for (int64_t f = 0; f < nf; ++f) {
-    vf_idx[pos[fv[2 * f]]++] = (int)f;
-    vf_idx[pos[fv[2 * f + 1]]++] = (int)f;
-  }
-  if (!fq4) return true;
-  fq4->assign(4 * nf, 0);
-  for (int64_t f = 0; f < nf; ++f) {
-    const int a = fv[2 * f], b = fv[2 * f + 1];
-    int opp[2];
-    for (int side = 0; side < 2; ++side) {
-      const int64_t cc = faces[f + (2 + side) * nf] - 1;
-      opp[side] = -1;
-      if (cc < 0) continue;
-      for (int w = 0; w < 3; ++w) {
-        const int nw = (int)cells[6 * cc + w] - 1;
-        if (nw != a && nw != b) opp[side] = nw;
-      }
-    }
-    if (opp[0] < 0) return false;
-    (*fq4)[4 * f] = a;
-    (*fq4)[4 * f + 1] = b;
-    (*fq4)[4 * f + 2] = opp[0];
-    (*fq4)[4 * f + 3] = opp[1] < 0 ? opp[0] : opp[1];
-  }
-  return true;
-}
-
 void mg_plan_levels(int nx, int ny, MgData& M) {
   M.nx = nx;
   M.ny = ny;
@@ -338,8 +304,6 @@ void mg_plan_levels(int nx, int ny, MgData& M) {
     L.nx = lx;
     L.ny = ly;
     L.n = (int64_t)(lx + 1) * (ly + 1);
-    // RAP across a one-cell-wide coarse column or row adds the (+1,+1) pair
-    L.npts = l == 1 ? 7 : ((M.lev[l - 1].npts > 7 || M.lev[l - 1].nx % 2 || M.lev[l - 1].ny % 2) ? kStencil : 7);
     ++l;
     if (std::max(lx, ly) <= 2 || l >= kMaxLevels) break;
     lx = (lx + 1) / 2;  // coarsening with a ragged end on odd sides
@@ -360,29 +324,9 @@ void mg_plan_levels(int nx, int ny, MgData& M) {
 
 namespace {
 
-// face end points and the vertex -> face lists (any mesh), and the vertex
-// grid hierarchy when the mesh is structured
-int build_vertex_structures(hdg_ctx* c, int64_t nn, int64_t nf, const int64_t* faces, const int64_t* cells,
-                            int64_t nc) {
-  std::vector<int> fv, cnt, idx, fq4;
-  int nx = 0, ny = 0;
-  c->structured = detect_structured(nn, nc, cells, &nx, &ny);
-  if (!face_vertex_maps(nn, nf, faces, cells, fv, cnt, idx, c->structured ? &fq4 : nullptr))
-    return fail(c, HDG_ERR_ARG, "a face has no first cell");
+// the vertex grid hierarchy of a structured mesh of nx x ny cells
+int build_vertex_levels(hdg_ctx* c, int nx, int ny) {
   MgData& M = c->mg;
-  TRY(dalloc(c, &M.fv, 2 * nf));
-  TRY(dalloc(c, &M.vf_ptr, nn + 1));
-  TRY(dalloc(c, &M.vf_idx, idx.size()));
-  TRY(dalloc(c, &M.vf2, idx.size()));
-  HIPCHK(c, hipMemcpyAsync(M.fv, fv.data(), sizeof(int) * fv.size(), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(M.vf_ptr, cnt.data(), sizeof(int) * cnt.size(), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(M.vf_idx, idx.data(), sizeof(int) * idx.size(), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  M.nv = nn;
-  if (!c->structured) return HDG_OK;
-  TRY(dalloc(c, &M.fq4, 4 * nf));
-  HIPCHK(c, hipMemcpyAsync(M.fq4, fq4.data(), sizeof(int) * fq4.size(), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   mg_plan_levels(nx, ny, M);
   for (int l = 1; l < M.nlev; ++l) {
     MgLevel& L = M.lev[l];
@@ -483,40 +427,47 @@ int ensure_aux(hdg_ctx* c) {
   if (c->aux) return HDG_OK;
   HIPCHK(c, hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking));
   HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-  HIPCHK(c, hipEventCreateWithFlags(&c->ev_fill, hipEventDisableTiming));
   HIPCHK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
   return HDG_OK;
 }
 
-// Condensation, trace matrix and Jacobi blocks.  With mg_early (hdg_run on
-// a multigrid context with its own streams), the multigrid set-up goes to
-// the second stream as soon as its inputs exist: the per-cell coarse blocks
-// after the condensation (beside the fill and the Jacobi blocks), S P0 and
-// the vertex levels after the fill; the solve joins it.
-int assemble_impl(hdg_ctx* c, bool mg_early = false) {
+// Storage of the assembled trace matrix: symmetric blocks at four modes per
+// face, else the face-ELL (the exports expand the blocks on demand).
+int alloc_system(hdg_ctx* c) {
+  const int64_t N = c->T.N;
+  if (sym_blocks(c->nt)) {
+    if (!c->T.blk) TRY(dalloc(c, &c->T.blk, sym_blk_count(c->nt, c->mesh.nf)));
+  } else if (!c->T.vals) {
+    TRY(dalloc(c, &c->T.vals, (size_t)kSlots * c->nt * N));
+  }
+  if (!c->T.rhs) TRY(dalloc(c, &c->T.rhs, N));
+  return HDG_OK;
+}
+
+// The assembled trace matrix and rhs of the current condensed blocks.
+int ensure_system(hdg_ctx* c) {
+  if (c->filled) return HDG_OK;
+  TRY(alloc_system(c));
+  LAUNCHCHK(c, launch_fill(c->mesh, c->pat, c->d_Ate, c->d_bte, c->T, c->stream));
+  c->filled = true;
+  return HDG_OK;
+}
+
+// Condensation and trace matrix; on a block-Jacobi context its Jacobi blocks.
+// run: the solve follows at once, and a multigrid context builds its reduced
+// system from the condensed blocks, so the assembled matrix is left to the
+// exports (ensure_system).
+int assemble_impl(hdg_ctx* c, bool run = false) {
   if (!c->has_setup) return fail(c, HDG_ERR_STATE, "hdg_setup has not been called");
   if ((c->opt.schedule & HDG_SCHEDULE_AUTOTUNE) && !c->tuned) TRY(autotune_impl(c));
-  c->mg_forked = false;
-  const bool early = mg_early && use_mg(c) && c->arena == nullptr;
+  c->filled = false;
   HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
   LAUNCHCHK(c, launch_condense_cells(c, condense_args(c)));
-  if (early) {
-    TRY(ensure_aux(c));
-    HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
-    HIPCHK(c, hipStreamWaitEvent(c->aux, c->ev_fork, 0));
-    LAUNCHCHK(c, mg_setup_cells(c->mesh, c->mg, c->T, c->d_Ate, c->aux));
+  if (!use_mg(c) || !run) TRY(ensure_system(c));
+  if (!use_mg(c)) {
+    LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
+    c->jacobi_dirty = false;
   }
-  LAUNCHCHK(c, launch_fill(c->mesh, c->pat, c->d_Ate, c->d_bte, c->T, c->stream));
-  if (early) {
-    HIPCHK(c, hipEventRecord(c->ev_fill, c->stream));
-    HIPCHK(c, hipStreamWaitEvent(c->aux, c->ev_fill, 0));
-    LAUNCHCHK(c, mg_setup_sp(c->mg, c->T, c->pat, mixed(c) ? c->f_sp : nullptr, c->aux));
-    LAUNCHCHK(c, mg_setup_levels(c->mg, c->d_mg, c->aux));
-    HIPCHK(c, hipEventRecord(c->ev_join, c->aux));
-    c->mg_forked = true;
-  }
-  LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
-  c->jacobi_dirty = false;
   c->assembled = true;
   c->solved = c->recovered = false;
   return HDG_OK;
@@ -531,15 +482,59 @@ bool mixed(const hdg_ctx* c) { return use_mg(c) && c->opt.precision == HDG_MIXED
 TraceOp<double> op64(const hdg_ctx* c) {
   return TraceOp<double>{c->T.nt, c->T.nf, c->T.N, c->T.vals, c->T.Dinv, c->T.dmask, c->T.blk};
 }
-TraceOp<float> op32(const hdg_ctx* c) {
-  return TraceOp<float>{c->T.nt, c->T.nf, c->T.N, c->f_vals, c->f_Dinv, c->T.dmask, c->f_blk};
-}
 Krylov<double> kv64(const hdg_ctx* c) {
   const CgVectors& v = c->cg;
   return Krylov<double>{v.r, v.z, v.p0, v.p1, v.q, v.x, v.part, v.st, v.nblocks};
 }
-MgVecs<double> mv64(const hdg_ctx* c) { return MgVecs<double>{c->mg.e0, c->mg.res0, c->mg.sp}; }
-MgVecs<float> mv32(const hdg_ctx* c) { return MgVecs<float>{c->f_e0, c->f_res0, c->f_sp}; }
+// The reduced system's arrays and launch plan (multigrid contexts).
+int setup_quad(hdg_ctx* c) {
+  QuadSys& q = c->qs;
+  QuadInst& I = c->qi;
+  q = QuadSys{};
+  I = QuadInst{};
+  quad_plan(c->mg.nx, c->mg.ny, c->nt, I);
+  const int nt = c->nt;
+  const size_t pts = (size_t)I.ntiles * 64;
+  TRY(dalloc(c, &q.blk, pts * quad_blk_vals(nt)));
+  // the couplings of the quads that do not exist stay zero
+  HIPCHK(c, hipMemsetAsync(q.blk, 0, sizeof(double) * pts * quad_blk_vals(nt), c->stream));
+  TRY(dalloc(c, &q.D, pts * quad_diag_vals(nt)));
+  TRY(dalloc(c, &q.Dinv, pts * quad_diag_vals(nt)));
+  TRY(dalloc(c, &q.tp, pts * quad_tp_vals(nt)));
+  TRY(dalloc(c, &q.bq, pts * quad_bq_vals(nt)));
+  TRY(dalloc(c, &q.cq, pts * kQuadCq));
+  TRY(dalloc(c, &q.mask, pts));
+  for (double** v : {&q.x, &q.r0, &q.r1, &q.z, &q.p, &q.q, &q.res}) TRY(dalloc(c, v, pts * 2 * nt));
+  q.nbt = std::max(I.nbM, I.nbE);
+  TRY(dalloc(c, &q.part, (size_t)kQuadPartials * q.nbt));
+  if (mixed(c)) {
+    TRY(dalloc(c, &q.fblk, pts * quad_blk_vals(nt)));
+    TRY(dalloc(c, &q.fDinv, pts * quad_diag_vals(nt)));
+    TRY(dalloc(c, &q.ftp, pts * quad_tp_vals(nt)));
+  }
+  TRY(dalloc(c, &c->d_plain, 1));
+  TRY(dalloc(c, &c->d_mg, 1));
+  HIPCHK(c, hipMemcpyAsync(c->d_mg, &c->mg, sizeof(MgData), hipMemcpyHostToDevice, c->stream));
+  q.nt = nt;
+  q.tiles = I.ntiles;
+  q.shift = c->opt.tau == 1.0 ? 1 : 0;
+  q.cf = c->mesh.cf;
+  q.dmask = c->d_dmask;
+  q.uD = c->d_uD;
+  q.Ate = c->d_Ate;
+  q.bte = c->d_bte;
+  q.P = c->pat;
+  I.st = c->cg.st;
+  I.plain = c->d_plain;
+  const MgLevel& L = c->mg.lev[1];
+  I.r1 = L.r;
+  I.e1 = L.e;
+  I.l1a = L.a;
+  I.l1dinv = L.dinv;
+  I.vmask = L.mask;
+  c->ql = quad_launch_one(I, nt);
+  return HDG_OK;
+}
 
 // PCG iterations enqueued between convergence checks
 int chunk_of(const hdg_ctx* c) { return use_mg(c) ? 4 : 64; }
@@ -549,16 +544,14 @@ int chunk_of(const hdg_ctx* c) { return use_mg(c) ? 4 : 64; }
 int enqueue_chunk(hdg_ctx* c, double rtol2, int maxit) {
   const int n = chunk_of(c);
   for (int it = 0; it < n; ++it) {
-    LAUNCHCHK(c, launch_cg_spmv(c->pat, op64(c), kv64(c), 0, rtol2, maxit, 0, c->stream));
-    if (mixed(c)) {
-      LAUNCHCHK(c, launch_mg_update(op32(c), kv64(c), mv32(c), c->stream));
-      LAUNCHCHK(c, launch_cg_check(kv64(c), c->T.N, rtol2, maxit, c->stream));
-      LAUNCHCHK(c, launch_mg_precond(c->pat, op32(c), kv64(c), c->mg, c->d_mg, mv32(c), c->stream));
-    } else if (use_mg(c)) {
-      LAUNCHCHK(c, launch_mg_update(op64(c), kv64(c), mv64(c), c->stream));
-      LAUNCHCHK(c, launch_cg_check(kv64(c), c->T.N, rtol2, maxit, c->stream));
-      LAUNCHCHK(c, launch_mg_precond(c->pat, op64(c), kv64(c), c->mg, c->d_mg, mv64(c), c->stream));
+    if (use_mg(c)) {
+      LAUNCHCHK(c, launch_quad_product(c->qs, c->ql, rtol2, maxit, c->stream));
+      LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));
+      LAUNCHCHK(c, launch_quad_check(c->qs, c->ql, rtol2, maxit, c->stream));
+      LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, c->stream));
+      LAUNCHCHK(c, launch_quad_smooth(c->qs, c->ql, mixed(c), c->stream));
     } else {
+      LAUNCHCHK(c, launch_cg_spmv(c->pat, op64(c), kv64(c), 0, rtol2, maxit, 0, c->stream));
       LAUNCHCHK(c, launch_cg_update(c->T, c->cg, 0, 0, c->stream));
     }
   }
@@ -604,53 +597,44 @@ int finish_solve(hdg_ctx* c, hdg_solve_info* info, int maxit, int* err_flag);
 // for hdg_run); the recovery counts only if the solve converged.
 int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
-  if (c->jacobi_dirty) {
-    LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
-    c->jacobi_dirty = false;
+  if (!use_mg(c)) {
+    TRY(ensure_system(c));
+    if (c->jacobi_dirty) {
+      LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
+      c->jacobi_dirty = false;
+    }
   }
   const double rtol = c->opt.rtol > 0 ? c->opt.rtol : 1e-12;
   const int maxit = c->opt.maxit > 0 ? c->opt.maxit : 200000;
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   if (use_mg(c)) {
-    const bool mx = mixed(c);
-    if (mx) {
-      const int64_t N = c->T.N;
-      if (c->T.blk)
-        LAUNCHCHK(c, launch_to_float(c->T.blk, c->f_blk, (int64_t)sym_blk_count(c->nt, c->mesh.nf), c->stream));
-      else
-        LAUNCHCHK(c, launch_to_float(c->T.vals, c->f_vals, (int64_t)kSlots * c->nt * N, c->stream));
-      LAUNCHCHK(c, launch_to_float(c->T.Dinv, c->f_Dinv, (int64_t)dinv_count(c->nt, c->mesh.nf), c->stream));
-    }
-    // The multigrid set-up (small, latency-bound kernels writing the level
-    // arrays and S P0) and the Lanczos estimate of the smoothing weight
-    // (bandwidth-bound, writing the CG vectors, which serve as its scratch,
-    // and the CG state) only read the trace system in common: the set-up
-    // runs on the second stream beside the estimate.
-    // A serving slot (a context on the server's arena) stays on one stream:
-    // the other slots keep the device busy, and a second stream per slot
-    // would outnumber the hardware queues.
+    c->qs.uD = c->T.uD;
+    HIPCHK(c, hipMemsetAsync(c->d_plain, 0, sizeof(int), c->stream));
+    LAUNCHCHK(c, launch_quad_build(c->qs, c->ql, c->stream));
+    // T P and the vertex levels (small, latency-bound kernels) and the Lanczos
+    // estimate of the smoothing weight (bandwidth-bound, on the CG vectors)
+    // only read the system in common: they run side by side.  A serving slot
+    // (a context on the server's arena) stays on one stream: the other slots
+    // keep the device busy, and a second stream per slot would outnumber the
+    // hardware queues.
     const bool fork = c->arena == nullptr;
-    if (!c->mg_forked) {
-      if (fork) TRY(ensure_aux(c));
-      hipStream_t ss = fork ? c->aux : c->stream;
-      if (fork) {
-        HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
-        HIPCHK(c, hipStreamWaitEvent(c->aux, c->ev_fork, 0));
-      }
-      LAUNCHCHK(c, mg_setup_numeric(c->mesh, c->mg, c->d_mg, c->T, c->pat, c->d_Ate, mx ? c->f_sp : nullptr, ss));
-      if (fork) HIPCHK(c, hipEventRecord(c->ev_join, c->aux));
+    if (fork) {
+      TRY(ensure_aux(c));
+      HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
+      HIPCHK(c, hipStreamWaitEvent(c->aux, c->ev_fork, 0));
     }
-    c->mg_forked = false;
-    LAUNCHCHK(c, launch_lanczos_omega(c->pat, c->T, c->cg, Whole{c->T.N, c->cg.st}, c->cg.nblocks, nullptr, 1,
-                                      c->mg.omega_factor, c->mg.lanczos_steps, c->stream));
+    hipStream_t ss = fork ? c->aux : c->stream;
+    LAUNCHCHK(c, launch_quad_l1(c->qs, c->ql, ss));
+    LAUNCHCHK(c, mg_setup_levels(c->mg, c->d_mg, ss));
+    LAUNCHCHK(c, launch_quad_tp(c->qs, c->ql, ss));
+    if (mixed(c)) LAUNCHCHK(c, launch_quad_float(c->qs, ss));
+    if (fork) HIPCHK(c, hipEventRecord(c->ev_join, c->aux));
+    LAUNCHCHK(c, launch_quad_omega(c->qs, c->ql, quad_omega_factor(c->k), kQuadLanczos, c->stream));
+    LAUNCHCHK(c, launch_quad_init(c->qs, c->ql, c->stream));
     if (fork) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
-    if (mx) {
-      LAUNCHCHK(c, launch_mg_init(c->pat, c->T, op32(c), kv64(c), mv32(c), c->stream));
-      LAUNCHCHK(c, launch_mg_precond(c->pat, op32(c), kv64(c), c->mg, c->d_mg, mv32(c), c->stream));
-    } else {
-      LAUNCHCHK(c, launch_mg_init(c->pat, c->T, op64(c), kv64(c), mv64(c), c->stream));
-      LAUNCHCHK(c, launch_mg_precond(c->pat, op64(c), kv64(c), c->mg, c->d_mg, mv64(c), c->stream));
-    }
+    LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));
+    LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, c->stream));
+    LAUNCHCHK(c, launch_quad_smooth(c->qs, c->ql, mixed(c), c->stream));
   } else {
     LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
   }
@@ -695,9 +679,14 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
 
 // uhat = x (+ Dirichlet values), the FP64 residual, the solve record
 int finish_solve(hdg_ctx* c, hdg_solve_info* info, int maxit, int* err_flag) {
-  LAUNCHCHK(c, launch_cg_finish(c->T, c->cg, c->d_uhat, c->stream));
-  HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-  LAUNCHCHK(c, launch_true_residual(c->pat, c->T, c->d_uhat, c->d_scal + 1, c->cg, c->stream));
+  if (use_mg(c)) {
+    LAUNCHCHK(c, launch_quad_finish(c->qs, c->ql, c->d_uhat, c->d_scal + 1, c->stream));
+    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+  } else {
+    LAUNCHCHK(c, launch_cg_finish(c->T, c->cg, c->d_uhat, c->stream));
+    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+    LAUNCHCHK(c, launch_true_residual(c->pat, c->T, c->d_uhat, c->d_scal + 1, c->cg, c->stream));
+  }
   if (err_flag) {
     LAUNCHCHK(c, launch_recover_cells(c));
     HIPCHK(c, hipMemcpyAsync(err_flag, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
@@ -798,7 +787,6 @@ void hdg_destroy(hdg_ctx* c) {
     (void)hipStreamDestroy(c->aux);
   }
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
-  if (c->ev_fill) (void)hipEventDestroy(c->ev_fill);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->stream) {
     (void)hipStreamSynchronize(c->stream);
@@ -874,7 +862,9 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->h_cf.swap(cf);
   c->nblock_cols = nblk;
-  TRY(build_vertex_structures(c, nn, nf, faces, cells, nc));
+  int nx = 0, ny = 0;
+  c->structured = detect_structured(nn, nc, cells, &nx, &ny);
+  if (c->structured) TRY(build_vertex_levels(c, nx, ny));
   c->has_mesh = true;
   return HDG_OK;
 }
@@ -900,12 +890,6 @@ int hdg_set_rectangle_mesh(hdg_ctx* c, int64_t nx, int64_t ny, double x0, double
   TRY(dalloc(c, &dcn, 3 * nc));
   TRY(dalloc(c, &dcf, 3 * nc));
   TRY(dalloc(c, &dfc, 2 * nf));
-  MgData& M = c->mg;
-  TRY(dalloc(c, &M.fv, 2 * nf));
-  TRY(dalloc(c, &M.vf_ptr, nn + 1));
-  TRY(dalloc(c, &M.vf_idx, 2 * nf));
-  TRY(dalloc(c, &M.vf2, 2 * nf));
-  TRY(dalloc(c, &M.fq4, 4 * nf));
   HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
   RectMeshArgs a;
   a.nx = nx;
@@ -921,10 +905,6 @@ int hdg_set_rectangle_mesh(hdg_ctx* c, int64_t nx, int64_t ny, double x0, double
   a.cn = dcn;
   a.cf = dcf;
   a.fcell = dfc;
-  a.fv = M.fv;
-  a.vf_ptr = M.vf_ptr;
-  a.vf_idx = M.vf_idx;
-  a.fq4 = M.fq4;
   a.err = c->d_err;
   LAUNCHCHK(c, launch_rect_mesh(a, c->stream));
   c->mesh.nn = nn;
@@ -952,23 +932,7 @@ int hdg_set_rectangle_mesh(hdg_ctx* c, int64_t nx, int64_t ny, double x0, double
   const int64_t nbdry = 2 * nx + 2 * ny;
   c->nblock_cols = 5 * (nf - nbdry) + 3 * nbdry;
   c->structured = true;
-  M.nv = nn;
-  mg_plan_levels((int)nx, (int)ny, M);
-  for (int l = 1; l < M.nlev; ++l) {
-    MgLevel& L = M.lev[l];
-    TRY(dalloc(c, &L.a, kStencil * L.n));
-    TRY(dalloc(c, &L.dinv, L.n));
-    TRY(dalloc(c, &L.mask, L.n));
-    TRY(dalloc(c, &L.r, L.n));
-    TRY(dalloc(c, &L.e, L.n));
-    TRY(dalloc(c, &L.t, L.n));
-  }
-  TRY(dalloc(c, &M.cinv, (size_t)kCoarseDirect * kCoarseDirect));
-  if (M.tail < M.nlev) {
-    int64_t tn = 0;
-    for (int t = M.tail; t < M.nlev; ++t) tn += M.lev[t].n;
-    TRY(dalloc(c, &M.tailpack, (kStencil + 1) * tn));
-  }
+  TRY(build_vertex_levels(c, (int)nx, (int)ny));
   c->has_mesh = true;
   return HDG_OK;
 }
@@ -1030,48 +994,28 @@ int hdg_setup(hdg_ctx* c, const hdg_options* opt) {
   c->T.nt = c->nt;
   c->T.nf = nf;
   c->T.N = N;
-  // the trace operator: symmetric blocks at four modes per face, else the
-  // face-ELL (the exports expand the blocks into a face-ELL on demand)
-  if (sym_blocks(c->nt))
-    TRY(dalloc(c, &c->T.blk, sym_blk_count(c->nt, c->mesh.nf)));
-  else
-    TRY(dalloc(c, &c->T.vals, (size_t)kSlots * c->nt * N));
-  TRY(dalloc(c, &c->T.rhs, N));
-  TRY(dalloc(c, &c->T.Dinv, dinv_count(c->nt, c->mesh.nf)));
   TRY(dalloc(c, &c->d_dmask, N));
   TRY(dalloc(c, &c->d_uD, N));
   HIPCHK(c, hipMemsetAsync(c->d_dmask, 0, N, c->stream));
   HIPCHK(c, hipMemsetAsync(c->d_uD, 0, sizeof(double) * N, c->stream));
   c->T.dmask = c->d_dmask;
   c->T.uD = c->d_uD;
-  c->cg.nblocks = cg_blocks(N, c->nt);
-  TRY(dalloc(c, &c->cg.x, N));
-  TRY(dalloc(c, &c->cg.r, N));
-  TRY(dalloc(c, &c->cg.z, N));
-  TRY(dalloc(c, &c->cg.p0, N));
-  TRY(dalloc(c, &c->cg.p1, N));
-  TRY(dalloc(c, &c->cg.q, N));
-  TRY(dalloc(c, &c->cg.part, 4 * (size_t)c->cg.nblocks + 64));
   TRY(dalloc(c, &c->d_uhat, N));
   TRY(dalloc(c, &c->d_part2, 4096));
-  if (c->structured) {
-    TRY(dalloc(c, &c->mg.cellA, 9 * nc));
-    TRY(dalloc(c, &c->mg.e0, N));
-    TRY(dalloc(c, &c->mg.res0, N));
-    TRY(dalloc(c, &c->mg.fc, 2 * c->mesh.nf));
-    TRY(dalloc(c, &c->mg.sp, 4 * N));
-    TRY(dalloc(c, &c->d_mg, 1));
-    HIPCHK(c, hipMemcpyAsync(c->d_mg, &c->mg, sizeof(MgData), hipMemcpyHostToDevice, c->stream));
-  }
-  if (c->structured && o.precision == HDG_MIXED) {
-    if (c->T.blk)
-      TRY(dalloc(c, &c->f_blk, sym_blk_count(c->nt, c->mesh.nf)));
-    else
-      TRY(dalloc(c, &c->f_vals, (size_t)kSlots * c->nt * N));
-    TRY(dalloc(c, &c->f_Dinv, dinv_count(c->nt, c->mesh.nf)));
-    TRY(dalloc(c, &c->f_sp, 4 * N));
-    TRY(dalloc(c, &c->f_e0, N));
-    TRY(dalloc(c, &c->f_res0, N));
+  if (use_mg(c)) {
+    TRY(setup_quad(c));
+  } else {
+    // block-Jacobi CG on the assembled matrix
+    TRY(alloc_system(c));
+    TRY(dalloc(c, &c->T.Dinv, dinv_count(c->nt, c->mesh.nf)));
+    c->cg.nblocks = cg_blocks(N, c->nt);
+    TRY(dalloc(c, &c->cg.x, N));
+    TRY(dalloc(c, &c->cg.r, N));
+    TRY(dalloc(c, &c->cg.z, N));
+    TRY(dalloc(c, &c->cg.p0, N));
+    TRY(dalloc(c, &c->cg.p1, N));
+    TRY(dalloc(c, &c->cg.q, N));
+    TRY(dalloc(c, &c->cg.part, 4 * (size_t)c->cg.nblocks + 64));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->src = SrcParams{};
@@ -1185,7 +1129,7 @@ int hdg_query_sizes(const hdg_ctx* c, hdg_sizes* s) {
   s->nfq = c->nfq;
   // rows of a face with two cells hold 5 block columns, with one cell 3
   s->nnz = c->nblock_cols * (int64_t)c->nt * c->nt;
-  s->sym_blocks = c->T.blk ? 1 : 0;
+  s->sym_blocks = sym_blocks(c->nt) ? 1 : 0;
   return HDG_OK;
 }
 
@@ -1336,6 +1280,7 @@ int hdg_get_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double* nzval, 
   if (!c) return HDG_ERR_ARG;
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
   TRY(select_device(c));
+  TRY(ensure_system(c));
   if (!c->T.blk || !nzval) return export_csc(c, c->T.vals, c->T.rhs, colptr, rowval, nzval, rhs);
   double* vals = nullptr;
   TRY(dalloc(c, &vals, (size_t)kSlots * c->nt * c->T.N));
@@ -1353,6 +1298,7 @@ int hdg_get_applied_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double*
   if (!c) return HDG_ERR_ARG;
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
   TRY(select_device(c));
+  TRY(ensure_system(c));
   const int64_t N = c->T.N;
   double *vals = nullptr, *b = nullptr, *part = nullptr;
   int r = dalloc(c, &vals, (size_t)kSlots * c->nt * N);
@@ -1521,7 +1467,17 @@ int hdg_time_kernel(hdg_ctx* c, int which, int reps, double* avg_us) {
   TRY(select_device(c));
   // make sure the solver state exists (pq, rz) so the kernels divide by
   // finite numbers; timing runs leave x and r untouched
-  if (!c->solved) LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
+  const bool mg = use_mg(c);
+  if (!c->solved) {
+    if (mg) {
+      HIPCHK(c, hipMemsetAsync(c->d_plain, 0, sizeof(int), c->stream));
+      LAUNCHCHK(c, launch_quad_build(c->qs, c->ql, c->stream));
+      LAUNCHCHK(c, launch_quad_omega(c->qs, c->ql, quad_omega_factor(c->k), 1, c->stream));
+      LAUNCHCHK(c, launch_quad_init(c->qs, c->ql, c->stream));
+    } else {
+      LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
+    }
+  }
   const CondenseArgs a = condense_args(c);
   double* scratch = nullptr;
   const int64_t ncopy = (int64_t)kSlots * c->nt * c->T.N;  // the size of the face-ELL values
@@ -1535,6 +1491,7 @@ int hdg_time_kernel(hdg_ctx* c, int which, int reps, double* avg_us) {
     }
   }
   auto once = [&]() -> int {
+    if (mg && which < 2) return launch_quad_time(c->qs, c->ql, which, c->stream);
     if (which == 0) return launch_cg_spmv(c->pat, op64(c), kv64(c), 2, 0.0, 0, 1, c->stream);
     if (which == 1) return launch_cg_update(c->T, c->cg, 2, 1, c->stream);
     if (which == 3) return launch_copy(csrc, scratch, ncopy, c->stream);
@@ -1559,6 +1516,8 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   if (!c || !relres || outer < 0 || outer > 64 || !(inner_rtol >= 0.0)) return HDG_ERR_ARG;
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
   TRY(select_device(c));
+  TRY(ensure_system(c));
+  const bool mg = use_mg(c);
   for (int j = 0; j <= outer; ++j) relres[j] = std::nan("");
   if (inner_iters)
     for (int j = 0; j < outer; ++j) inner_iters[j] = 0;
@@ -1573,6 +1532,7 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   drop_graphs(c);
   const TraceSystem saved = c->T;
   const hdg_options opt = c->opt;
+  const int saved_shift = c->qs.shift;
   c->opt.schedule |= HDG_SCHEDULE_EAGER;
   if (inner_rtol > 0.0) c->opt.rtol = inner_rtol;
   auto step = [&]() -> int {
@@ -1595,8 +1555,16 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
       if (nb) c->T.blk = vb;
       c->T.rhs = res;
       c->T.uD = zero;
-      LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
-      c->jacobi_dirty = false;
+      if (mg) {
+        // the reduced system of the rounded matrix, which no longer
+        // annihilates constants
+        c->qs.from_k = 1;
+        c->qs.shift = 0;
+        c->qs.K = c->T;
+      } else {
+        LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
+        c->jacobi_dirty = false;
+      }
       hdg_solve_info info{};
       const int e = solve_impl(c, &info);
       if (inner_iters) inner_iters[j] = info.iters;
@@ -1607,9 +1575,11 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   if (rc == HDG_OK) rc = step();
   // the assembled system as it was, u_outer as the trace
   c->T = saved;
+  c->qs.from_k = 0;
+  c->qs.shift = saved_shift;
   c->opt = opt;
   drop_graphs(c);
-  int rc2 = launch_jacobi(c->pat, c->T, c->stream);
+  int rc2 = mg ? 0 : launch_jacobi(c->pat, c->T, c->stream);
   if (rc == HDG_OK && u) {
     if (rc2 == 0) rc2 = (int)hipMemcpyAsync(c->d_uhat, u, sizeof(double) * N, hipMemcpyDeviceToDevice, c->stream);
     if (rc2 == 0) rc2 = (int)hipStreamSynchronize(c->stream);
@@ -1623,7 +1593,7 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   dfree(c, res);
   dfree(c, zero);
   dfree(c, part);
-  c->jacobi_dirty = false;
+  if (!mg) c->jacobi_dirty = false;
   c->solved = rc == HDG_OK;
   c->recovered = false;
   return rc;

@@ -25,7 +25,7 @@
 #include "../../include/hdg.h"
 #include "hdg_arena.h"
 #include "hdg_host.h"
-#include "hdg_internal.h"
+#include "hdg_quad.h"
 #include "hdg_tables.h"
 
 using namespace hdg;
@@ -73,7 +73,6 @@ struct Group {
   int* err = nullptr;  // [ninst] condensation error flags
   SrcParams* srcs = nullptr;
   int* cell_inst = nullptr;
-  int *fv = nullptr, *vf_ptr = nullptr, *vf_idx = nullptr, *vf2 = nullptr, *fq4 = nullptr;  // face end points, vertex -> faces
   // launch tables
   CgState* st = nullptr;
   Seg *segs = nullptr, *csegs = nullptr;
@@ -82,14 +81,14 @@ struct Group {
   double* part2 = nullptr;  // error-norm partials
   double* res = nullptr;    // [ninst] ||K uhat - rhs||^2, [ninst] squared L2 error
   // multigrid
-  MgData Mu;                // the packed mesh's view (level 1 spans every vertex)
+  QuadSys qs;               // the instances' reduced systems, packed by tiles
+  QuadLaunch ql;
   std::vector<MgData> Mi;   // per-instance hierarchies (views into the level buffers)
   MgData* dMi = nullptr;
   LevelBuf lev[kMaxLevels];
   MgGroup G;
   MgSetupGroup S;
   CondenseSched csched;  // condensation schedule (autotuned at create with HDG_SCHEDULE_AUTOTUNE)
-  float *f_vals = nullptr, *f_blk = nullptr, *f_Dinv = nullptr, *f_sp = nullptr, *f_e0 = nullptr, *f_res0 = nullptr;
   // read-back
   CgState* h_st = nullptr;  // pinned, 2 x ninst (chunk slots) + ninst (final)
   double* h_res = nullptr;  // pinned, 2 x ninst, then ninst error flags (ints)
@@ -255,6 +254,84 @@ int tune_group(hdg_batch* b, Group& g) {
   return HDG_OK;
 }
 
+// The reduced systems of a multigrid group's instances, packed tile by tile,
+// and the block maps of their launches: instance j gets the blocks it would
+// get alone.
+int build_quad_group(hdg_batch* b, Group& g) {
+  const int n = (int)g.in.size(), nt = g.nt, qb = quad_build_quads(nt);
+  QuadSys& q = g.qs;
+  std::vector<QuadInst> inst(n);
+  std::vector<BlockMap> mM, mE, mQ;
+  int64_t tiles = 0;
+  int* plain;
+  BTRY(galloc(b, g, &plain, n));
+  // no instance prescribes dofs of a diagonal face
+  BHIP(b, hipMemsetAsync(plain, 0, sizeof(int) * n, g.s));
+  for (int j = 0; j < n; ++j) {
+    QuadInst& I = inst[j];
+    quad_plan((int)g.in[j].nx, (int)g.in[j].ny, nt, I);
+    I.tile0 = tiles;
+    tiles += I.ntiles;
+    I.cell0 = g.in[j].cell0;
+    I.pM = (int)mM.size();
+    I.pE = (int)mE.size();
+    I.st = g.st + j;
+    I.plain = plain + j;
+    const MgLevel& L = g.Mi[j].lev[1];
+    I.r1 = L.r;
+    I.e1 = L.e;
+    I.l1a = L.a;
+    I.l1dinv = L.dinv;
+    I.vmask = L.mask;
+    for (int u = 0; u < I.nbM; ++u) mM.push_back(BlockMap{j, u});
+    for (int u = 0; u < I.nbE; ++u) mE.push_back(BlockMap{j, u});
+    const int64_t nq = ((int64_t)I.nx * I.ny + qb - 1) / qb;
+    for (int64_t u = 0; u < nq; ++u) mQ.push_back(BlockMap{j, (int)u});
+  }
+  const size_t pts = (size_t)tiles * 64;
+  BTRY(galloc(b, g, &q.blk, pts * quad_blk_vals(nt)));
+  BHIP(b, hipMemsetAsync(q.blk, 0, sizeof(double) * pts * quad_blk_vals(nt), g.s));
+  BTRY(galloc(b, g, &q.D, pts * quad_diag_vals(nt)));
+  BTRY(galloc(b, g, &q.Dinv, pts * quad_diag_vals(nt)));
+  BTRY(galloc(b, g, &q.tp, pts * quad_tp_vals(nt)));
+  BTRY(galloc(b, g, &q.bq, pts * quad_bq_vals(nt)));
+  BTRY(galloc(b, g, &q.cq, pts * kQuadCq));
+  BTRY(galloc(b, g, &q.mask, pts));
+  for (double** v : {&q.x, &q.r0, &q.r1, &q.z, &q.p, &q.q, &q.res}) BTRY(galloc(b, g, v, pts * 2 * nt));
+  q.nbt = (int)std::max(mM.size(), mE.size());
+  BTRY(galloc(b, g, &q.part, (size_t)kQuadPartials * q.nbt));
+  if (g.mixed) {
+    BTRY(galloc(b, g, &q.fblk, pts * quad_blk_vals(nt)));
+    BTRY(galloc(b, g, &q.fDinv, pts * quad_diag_vals(nt)));
+    BTRY(galloc(b, g, &q.ftp, pts * quad_tp_vals(nt)));
+  }
+  q.nt = nt;
+  q.tiles = tiles;
+  q.shift = g.opt.tau == 1.0 ? 1 : 0;
+  q.cf = g.mesh.cf;
+  q.dmask = g.dmask;
+  q.uD = g.uD;
+  q.Ate = g.Ate;
+  q.bte = g.bte;
+  q.P = g.pat;
+  QuadLaunch& L = g.ql;
+  QuadInst* di;
+  BlockMap *dM, *dE, *dQ;
+  BTRY(upload(b, g, &di, inst));
+  BTRY(upload(b, g, &dM, mM));
+  BTRY(upload(b, g, &dE, mE));
+  BTRY(upload(b, g, &dQ, mQ));
+  L.inst = di;
+  L.mapM = dM;
+  L.mapE = dE;
+  L.mapQ = dQ;
+  L.gM = (int)mM.size();
+  L.gE = (int)mE.size();
+  L.gQ = (int)mQ.size();
+  L.ninst = n;
+  return HDG_OK;
+}
+
 // Lays out one group: offsets, levels, host packing, device arrays, tables.
 int build_group(hdg_batch* b, Group& g) {
   const int n = (int)g.in.size();
@@ -300,11 +377,6 @@ int build_group(hdg_batch* b, Group& g) {
   BTRY(galloc(b, g, &dfc, 2 * g.nf));
   BTRY(galloc(b, g, &g.cell_inst, g.nc));
   BTRY(galloc(b, g, &g.dmask, g.N));
-  BTRY(galloc(b, g, &g.fv, 2 * g.nf));
-  BTRY(galloc(b, g, &g.vf_ptr, g.nn + 1));
-  BTRY(galloc(b, g, &g.vf_idx, 2 * g.nf));
-  BTRY(galloc(b, g, &g.vf2, 2 * g.nf));
-  if (g.mg) BTRY(galloc(b, g, &g.fq4, 4 * g.nf));
   BTRY(galloc(b, g, &merr, 1));
   BHIP(b, hipMemsetAsync(merr, 0, sizeof(int), g.s));
   for (int j = 0; j < n; ++j) {
@@ -320,15 +392,10 @@ int build_group(hdg_batch* b, Group& g) {
     a.cell0 = I.cell0;
     a.face0 = I.face0;
     a.inst = j;
-    a.last = j + 1 == n;
     a.xy = dxy;
     a.cn = dcn;
     a.cf = dcf;
     a.fcell = dfc;
-    a.fv = g.fv;
-    a.vf_ptr = g.vf_ptr;
-    a.vf_idx = g.vf_idx;
-    a.fq4 = g.fq4;
     a.cell_inst = g.cell_inst;
     a.err = merr;
     BLAUNCH(b, launch_rect_mesh(a, g.s));
@@ -379,12 +446,14 @@ int build_group(hdg_batch* b, Group& g) {
   g.T.nt = g.nt;
   g.T.nf = g.nf;
   g.T.N = N;
-  if (sym_blocks(g.nt))
-    BTRY(galloc(b, g, &g.T.blk, sym_blk_count(g.nt, g.nf)));
-  else
-    BTRY(galloc(b, g, &g.T.vals, (size_t)kSlots * g.nt * N));
-  BTRY(galloc(b, g, &g.T.rhs, N));
-  BTRY(galloc(b, g, &g.T.Dinv, dinv_count(g.nt, g.nf)));
+  if (!g.mg) {
+    if (sym_blocks(g.nt))
+      BTRY(galloc(b, g, &g.T.blk, sym_blk_count(g.nt, g.nf)));
+    else
+      BTRY(galloc(b, g, &g.T.vals, (size_t)kSlots * g.nt * N));
+    BTRY(galloc(b, g, &g.T.rhs, N));
+    BTRY(galloc(b, g, &g.T.Dinv, dinv_count(g.nt, g.nf)));
+  }
   g.T.dmask = g.dmask;
   g.T.uD = g.uD;
 
@@ -412,14 +481,14 @@ int build_group(hdg_batch* b, Group& g) {
   CgVectors& v = g.cg;
   v.nblocks = g.nbt;
   v.st = g.st;
-  BTRY(galloc(b, g, &v.x, N));
-  BTRY(galloc(b, g, &v.r, N));
-  BTRY(galloc(b, g, &v.z, N));
-  BTRY(galloc(b, g, &v.p0, N));
-  BTRY(galloc(b, g, &v.p1, N));
-  BTRY(galloc(b, g, &v.q, N));
-  BTRY(galloc(b, g, &v.part, 4 * (size_t)g.nbt + 64));
   if (!g.mg) {
+    BTRY(galloc(b, g, &v.x, N));
+    BTRY(galloc(b, g, &v.r, N));
+    BTRY(galloc(b, g, &v.z, N));
+    BTRY(galloc(b, g, &v.p0, N));
+    BTRY(galloc(b, g, &v.p1, N));
+    BTRY(galloc(b, g, &v.q, N));
+    BTRY(galloc(b, g, &v.part, 4 * (size_t)g.nbt + 64));
     BTRY(tune_group(b, g));
     BHIP(b, hipStreamSynchronize(g.s));
     return HDG_OK;
@@ -454,44 +523,9 @@ int build_group(hdg_batch* b, Group& g) {
     I.tail_off = tailn;
     for (int t = I.plan.tail; t < I.plan.nlev; ++t) tailn += (kStencil + 1) * I.plan.lev[t].n;
   }
-  double *cellA, *cinv, *tailpack;
-  BTRY(galloc(b, g, &cellA, 9 * nc));
+  double *cinv, *tailpack;
   BTRY(galloc(b, g, &cinv, (size_t)n * kCoarseDirect * kCoarseDirect));
   BTRY(galloc(b, g, &tailpack, tailn));
-  MgData& U = g.Mu;
-  U.nlev = 2;
-  U.nv = g.nn;
-  U.fv = g.fv;
-  U.vf_ptr = g.vf_ptr;
-  U.vf_idx = g.vf_idx;
-  U.vf2 = g.vf2;
-  U.fq4 = g.fq4;
-  U.cellA = cellA;
-  {
-    MgLevel& L1 = U.lev[1];
-    const LevelBuf& B = g.lev[1];
-    L1.n = g.nn;
-    L1.a = B.a;
-    L1.dinv = B.dinv;
-    L1.mask = B.mask;
-    L1.r = B.r;
-    L1.e = B.e;
-    L1.t = B.t;
-  }
-  BTRY(galloc(b, g, &U.e0, N));
-  BTRY(galloc(b, g, &U.res0, N));
-  BTRY(galloc(b, g, &U.fc, 2 * g.nf));
-  BTRY(galloc(b, g, &U.sp, 4 * N));
-  if (g.mixed) {
-    if (g.T.blk)
-      BTRY(galloc(b, g, &g.f_blk, sym_blk_count(g.nt, g.nf)));
-    else
-      BTRY(galloc(b, g, &g.f_vals, (size_t)kSlots * g.nt * N));
-    BTRY(galloc(b, g, &g.f_Dinv, dinv_count(g.nt, g.nf)));
-    BTRY(galloc(b, g, &g.f_sp, 4 * N));
-    BTRY(galloc(b, g, &g.f_e0, N));
-    BTRY(galloc(b, g, &g.f_res0, N));
-  }
   MgData choice;
   mg_order_choices(g.k, choice);  // as hdg_setup chooses for a single problem
   g.Mi.assign(n, MgData{});
@@ -499,9 +533,7 @@ int build_group(hdg_batch* b, Group& g) {
     const Inst& I = g.in[j];
     MgData& M = g.Mi[j];
     M = I.plan;
-    M.nv = I.nn;
     M.vsweeps = choice.vsweeps;
-    M.cellA = cellA + 9 * I.cell0;
     M.cinv = cinv + (size_t)j * kCoarseDirect * kCoarseDirect;
     M.tailpack = tailpack + I.tail_off;
     for (int l = 1; l < M.nlev; ++l) {
@@ -515,7 +547,6 @@ int build_group(hdg_batch* b, Group& g) {
       V.e = B.e + o;
       V.t = B.t + o;
     }
-    if (I.lev_off[1] != I.node0) return fail(b, HDG_ERR_HIP, "level-1 layout differs from the node numbering");
   }
   BTRY(upload(b, g, &g.dMi, g.Mi));
   MgGroup& G = g.G;
@@ -547,20 +578,12 @@ int build_group(hdg_batch* b, Group& g) {
     G.gnode[d] = (int)node.size();
     G.gres[d] = (int)res.size();
   }
+  BTRY(build_quad_group(b, g));
   BTRY(tune_group(b, g));
-  // set-up tables: level-1 assembly, then cmask / RAP for every level pair
+  // set-up tables: cmask / RAP for every level pair
   MgSetupGroup& S = g.S;
   S.ninst = n;
   S.dM = g.dMi;
-  {
-    std::vector<BlockMap> l1;
-    for (int j = 0; j < n; ++j)
-      for (int64_t u = 0; u < (g.Mi[j].lev[1].n + 255) / 256; ++u) l1.push_back(BlockMap{j, (int)u});
-    BlockMap* dl1;
-    BTRY(upload(b, g, &dl1, l1));
-    S.l1map = dl1;
-    S.gl1 = (int)l1.size();
-  }
   S.ndepth = maxlev - 1;
   for (int d = 1; d < S.ndepth; ++d) {
     std::vector<VRec> rec;
@@ -592,16 +615,10 @@ Grouped rows(const Group& g) { return Grouped{g.segs, g.binst}; }
 TraceOp<double> op64(const Group& g) {
   return TraceOp<double>{g.nt, g.nf, g.N, g.T.vals, g.T.Dinv, g.dmask, g.T.blk};
 }
-TraceOp<float> op32(const Group& g) {
-  return TraceOp<float>{g.nt, g.nf, g.N, g.f_vals, g.f_Dinv, g.dmask, g.f_blk};
-}
 Krylov<double> kv(const Group& g) {
   const CgVectors& v = g.cg;
   return Krylov<double>{v.r, v.z, v.p0, v.p1, v.q, v.x, v.part, v.st, v.nblocks};
 }
-MgVecs<double> mv64(const Group& g) { return MgVecs<double>{g.Mu.e0, g.Mu.res0, g.Mu.sp}; }
-MgVecs<float> mv32(const Group& g) { return MgVecs<float>{g.f_e0, g.f_res0, g.f_sp}; }
-
 double rtol2_of(const Group& g) {
   const double rtol = g.opt.rtol > 0 ? g.opt.rtol : 1e-12;
   return rtol * rtol;
@@ -612,34 +629,23 @@ int maxit_of(const Group& g) { return g.opt.maxit > 0 ? g.opt.maxit : 200000; }
 int enqueue_setup(hdg_batch* b, Group& g) {
   BHIP(b, hipMemsetAsync(g.err, 0, sizeof(int) * g.in.size(), g.s));
   BLAUNCH(b, launch_group_condense(g, group_condense_args(g)));
-  BLAUNCH(b, launch_fill(g.mesh, g.pat, g.Ate, g.bte, g.T, g.s));
-  BLAUNCH(b, launch_jacobi(g.pat, g.T, g.s));
-  const Grouped gr = rows(g);
-  const int n = (int)g.in.size();
   if (!g.mg) {
-    BLAUNCH(b, launch_cg_init_t(g.pat, g.T, g.cg, gr, g.nbt, g.s));
+    BLAUNCH(b, launch_fill(g.mesh, g.pat, g.Ate, g.bte, g.T, g.s));
+    BLAUNCH(b, launch_jacobi(g.pat, g.T, g.s));
+    BLAUNCH(b, launch_cg_init_t(g.pat, g.T, g.cg, rows(g), g.nbt, g.s));
     return HDG_OK;
   }
-  const double factor = g.Mi[0].omega_factor;
-  if (g.mixed) {
-    if (g.T.blk)
-      BLAUNCH(b, launch_to_float(g.T.blk, g.f_blk, (int64_t)sym_blk_count(g.nt, g.nf), g.s));
-    else
-      BLAUNCH(b, launch_to_float(g.T.vals, g.f_vals, (int64_t)kSlots * g.nt * g.N, g.s));
-    BLAUNCH(b, launch_to_float(g.T.Dinv, g.f_Dinv, (int64_t)dinv_count(g.nt, g.nf), g.s));
-    BLAUNCH(b, mg_setup_mesh(g.mesh, g.Mu, g.T, g.pat, g.Ate, g.f_sp, g.s));
-    BLAUNCH(b, mg_setup_levels_group(g.S, g.s));
-    BLAUNCH(b, launch_lanczos_omega(g.pat, g.T, g.cg, gr, g.nbt, g.segs, n, factor, g.Mi[0].lanczos_steps, g.s));
-    BLAUNCH(b, launch_mg_init_group(g.pat, g.T, op32(g), kv(g), mv32(g), gr, g.nbt, g.s));
-    BLAUNCH(b, launch_mg_precond_group(g.pat, op32(g), kv(g), g.Mu, g.G, mv32(g), gr, g.nbt, g.s));
-  } else {
-    BLAUNCH(b, mg_setup_mesh(g.mesh, g.Mu, g.T, g.pat, g.Ate, nullptr, g.s));
-    BLAUNCH(b, mg_setup_levels_group(g.S, g.s));
-    // the CG vectors serve as scratch before the solve initialises them
-    BLAUNCH(b, launch_lanczos_omega(g.pat, g.T, g.cg, gr, g.nbt, g.segs, n, factor, g.Mi[0].lanczos_steps, g.s));
-    BLAUNCH(b, launch_mg_init_group(g.pat, g.T, op64(g), kv(g), mv64(g), gr, g.nbt, g.s));
-    BLAUNCH(b, launch_mg_precond_group(g.pat, op64(g), kv(g), g.Mu, g.G, mv64(g), gr, g.nbt, g.s));
-  }
+  BLAUNCH(b, launch_quad_build(g.qs, g.ql, g.s));
+  BLAUNCH(b, launch_quad_l1(g.qs, g.ql, g.s));
+  BLAUNCH(b, mg_setup_levels_group(g.S, g.s));
+  BLAUNCH(b, launch_quad_tp(g.qs, g.ql, g.s));
+  if (g.mixed) BLAUNCH(b, launch_quad_float(g.qs, g.s));
+  // the CG vectors serve as scratch before the solve initialises them
+  BLAUNCH(b, launch_quad_omega(g.qs, g.ql, quad_omega_factor(g.k), kQuadLanczos, g.s));
+  BLAUNCH(b, launch_quad_init(g.qs, g.ql, g.s));
+  BLAUNCH(b, launch_quad_residual(g.qs, g.ql, g.mixed, g.s));
+  BLAUNCH(b, launch_vcycle_group(g.G, g.s));
+  BLAUNCH(b, launch_quad_smooth(g.qs, g.ql, g.mixed, g.s));
   return HDG_OK;
 }
 
@@ -650,16 +656,14 @@ int enqueue_chunk(hdg_batch* b, Group& g) {
   const int iters = chunk_iters(g);
   const Grouped gr = rows(g);
   for (int it = 0; it < iters; ++it) {
-    BLAUNCH(b, launch_cg_spmv_t(g.pat, op64(g), kv(g), gr, g.nbt, 0, rtol2_of(g), maxit_of(g), 0, g.s));
-    if (g.mixed) {
-      BLAUNCH(b, launch_mg_update_group(op32(g), kv(g), mv32(g), gr, g.nbt, g.s));
-      BLAUNCH(b, launch_cg_check_group(kv(g), gr, (int)g.in.size(), rtol2_of(g), maxit_of(g), g.s));
-      BLAUNCH(b, launch_mg_precond_group(g.pat, op32(g), kv(g), g.Mu, g.G, mv32(g), gr, g.nbt, g.s));
-    } else if (g.mg) {
-      BLAUNCH(b, launch_mg_update_group(op64(g), kv(g), mv64(g), gr, g.nbt, g.s));
-      BLAUNCH(b, launch_cg_check_group(kv(g), gr, (int)g.in.size(), rtol2_of(g), maxit_of(g), g.s));
-      BLAUNCH(b, launch_mg_precond_group(g.pat, op64(g), kv(g), g.Mu, g.G, mv64(g), gr, g.nbt, g.s));
+    if (g.mg) {
+      BLAUNCH(b, launch_quad_product(g.qs, g.ql, rtol2_of(g), maxit_of(g), g.s));
+      BLAUNCH(b, launch_quad_residual(g.qs, g.ql, g.mixed, g.s));
+      BLAUNCH(b, launch_quad_check(g.qs, g.ql, rtol2_of(g), maxit_of(g), g.s));
+      BLAUNCH(b, launch_vcycle_group(g.G, g.s));
+      BLAUNCH(b, launch_quad_smooth(g.qs, g.ql, g.mixed, g.s));
     } else {
+      BLAUNCH(b, launch_cg_spmv_t(g.pat, op64(g), kv(g), gr, g.nbt, 0, rtol2_of(g), maxit_of(g), 0, g.s));
       BLAUNCH(b, launch_cg_update_t(g.T, g.cg, gr, g.nbt, 0, 0, g.s));
     }
   }
@@ -711,9 +715,13 @@ bool all_done(const Group& g, int slot) {
 int enqueue_finish(hdg_batch* b, Group& g) {
   const int n = (int)g.in.size();
   const Grouped gr = rows(g);
-  BLAUNCH(b, launch_cg_finish(g.T, g.cg, g.uhat, g.s));
-  BLAUNCH(b, launch_true_residual_t(g.pat, g.T, g.uhat, g.cg.part, gr, g.nbt, g.s));
-  BLAUNCH(b, launch_reduce_segs(g.cg.part, g.segs, n, g.res, g.s));
+  if (g.mg) {
+    BLAUNCH(b, launch_quad_finish(g.qs, g.ql, g.uhat, g.res, g.s));
+  } else {
+    BLAUNCH(b, launch_cg_finish(g.T, g.cg, g.uhat, g.s));
+    BLAUNCH(b, launch_true_residual_t(g.pat, g.T, g.uhat, g.cg.part, rows(g), g.nbt, g.s));
+    BLAUNCH(b, launch_reduce_segs(g.cg.part, g.segs, n, g.res, g.s));
+  }
   // a group on the Schur form holds only the u rows of K_e and b_e
   if (g.d_spd)
     BLAUNCH(b, launch_recover_spd(g.k, g.mesh, g.d_spd, g.Ke, g.be, g.uhat, g.qu, g.s));

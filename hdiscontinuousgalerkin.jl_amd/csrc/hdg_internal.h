@@ -384,18 +384,10 @@ struct Krylov {
   CgState* st;
   int nblocks;
 };
-template <class W>
-struct MgVecs {
-  W* e0;           // trace-level correction
-  W* res0;         // trace-level residual
-  const W* sp;     // S P0 rows (4 per row)
-};
-
 // Multigrid hierarchy on the vertex grids of a structured mesh (level 0 is
-// the trace space, levels 1.. are vertex grids with 7-point stencils).
+// the reduced trace space, levels 1.. are vertex grids with 9-point stencils).
 struct MgLevel {
   int nx = 0, ny = 0;
-  int npts = 7;                  // 7, or kStencil once a ragged coarsening is above this level
   int64_t n = 0;                 // (nx+1)(ny+1) nodes
   double* a = nullptr;           // stencils, a[s*n + v], s < kStencil
   double* dinv = nullptr;        // 1 / a[0], 0 on fixed nodes
@@ -418,36 +410,14 @@ constexpr int kCoarseDirect = 16;
 struct MgData {
   int nlev = 0;                  // levels 1..nlev-1 are vertex grids
   int nx = 0, ny = 0;
-  int64_t nv = 0;
   MgLevel lev[kMaxLevels];
-  int* fv = nullptr;             // [2*nf] lower, higher node id of each face
-  int* vf_ptr = nullptr;         // vertex -> incident faces (CSR)
-  int* vf_idx = nullptr;
-  int* vf2 = nullptr;            // [2*nf] the same entries as 2 f + (1 where the vertex is f's higher end)
-  double* fc = nullptr;          // [2*nf] per face: P0^T res0 restricted to the face, at its lower and
-                                 // higher end (even nt: written by the level-0 residual)
-  double* cellA = nullptr;       // [9*nc] per-cell P^T (-Ate) P
-  double* e0 = nullptr;          // trace-level correction
-  double* res0 = nullptr;        // trace-level residual
-  int* fq4 = nullptr;            // [4*nf] the 4 vertices of the two cells of a face:
-                                 // lower, higher end point, opposite vertex of cell 1, of cell 2
-                                 // (= that of cell 1 on boundary faces)
-  double* sp = nullptr;          // [4*N] S P0 restricted to the rows: sp[j*N + r] couples
-                                 // row r with vertex fq4[4*face(r) + j]
   int tail = kMaxLevels;         // levels tail..nlev-1 run in one workgroup (LDS)
   double* cinv = nullptr;        // [kCoarseDirect^2] inverse of the coarsest operator (row-major)
-  double* tailpack = nullptr;    // stencils (7 n) and dinv (n) of levels tail.. back to back,
+  double* tailpack = nullptr;    // stencils (9 n) and dinv (n) of levels tail.. back to back,
                                  // the LDS image the tail kernel loads
-  // vertex-level Jacobi weight: 0.6-0.7 take one CG iteration fewer than
-  // 0.8 at 512^2 P2 (37 vs 38), 0.9 four more; 1024^2 P3 stays at 29
-  double omega_v = 0.7;
-  double omega_factor = 1.6;     // trace-level weight = factor / lambda_max(Dinv S) (Lanczos estimate)
+  double omega_v = 0.7;          // vertex-level Jacobi weight
   int coarse_sweeps = 20;
   int vsweeps = 2;               // pre- and post-smoothing sweeps on the vertex levels (1 or 2)
-  // block-Jacobi PCG (Lanczos) steps behind omega: 6 estimate lambda_max
-  // a little lower than 8, which lands omega * lambda_max between 1.6 and
-  // 1.7, still short of the 1.8 where iterations grow
-  int lanczos_steps = 6;
 };
 // per-order choices of the V-cycle, shared by single problems and batches:
 // V(1,1) on the vertex levels for k <= 3, V(2,2) at k = 4 (fewest CG
@@ -563,10 +533,6 @@ int launch_apply(const DevPattern& P, const TraceSystem& T, double* part, double
 // grid = blocks of the launch; the Whole forms above call these).
 template <class G>
 int launch_cg_init_t(const DevPattern& P, const TraceSystem& T, CgVectors& v, G g, int grid, hipStream_t s);
-// the next product's convergence test right after the multigrid update (one
-// instance, or one block per instance of a group)
-int launch_cg_check(const Krylov<double>& v, int64_t N, double rtol2, int maxit, hipStream_t s);
-int launch_cg_check_group(const Krylov<double>& v, Grouped g, int ninst, double rtol2, int maxit, hipStream_t s);
 template <class G>
 int launch_cg_spmv_t(const DevPattern& P, const TraceOp<double>& T, const Krylov<double>& v, G g, int grid,
                      int i_fixed, double rtol2, int maxit, int force, hipStream_t s);
@@ -583,39 +549,9 @@ int launch_errornorm_t(const DevMesh& m, const double* tables, const TabLayoutDe
 // out[j] = sum of part over the blocks of segment j
 int launch_reduce_segs(const double* part, const Seg* seg, int nseg, double* out, hipStream_t s);
 
-// vertex hierarchy and S P0 (FP64, and a float copy of S P0 when sp32 is set)
-int mg_setup_numeric(const DevMesh& mesh, MgData& M, const MgData* dM, TraceSystem& T, const DevPattern& P,
-                     const double* Ate, float* sp32, hipStream_t s);
-// the two halves of mg_setup_numeric: the parts that run over the whole
-// (possibly packed) mesh -- vertex masks, per-cell coarse blocks, S P0 --
-// and the vertex levels of one structured instance (M describes it, with
-// its arrays at its own offsets; dM is its device copy)
-int mg_setup_mesh(const DevMesh& mesh, const MgData& M, const TraceSystem& T, const DevPattern& P,
-                  const double* Ate, float* sp32, hipStream_t s);
-// mg_setup_mesh in two parts: what needs only the condensed blocks (vertex
-// masks, per-cell coarse blocks) and what reads the assembled trace matrix
-// (S P0), so that the first can run beside the assembly
-int mg_setup_cells(const DevMesh& mesh, const MgData& M, const TraceSystem& T, const double* Ate, hipStream_t s);
-int mg_setup_sp(const MgData& M, const TraceSystem& T, const DevPattern& P, float* sp32, hipStream_t s);
+// the vertex levels below level 1 of one structured problem (M describes it,
+// dM is its device copy), after level 1 is assembled (launch_quad_l1)
 int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s);
-// omega = factor / lambda_max(Dinv S), lambda_max the largest Ritz value of
-// `steps` block-Jacobi PCG iterations from a random right-hand side (the
-// Lanczos tridiagonal matrix of Dinv S built from their coefficients); uses
-// the CG vectors as scratch.  Whole: one problem (st); Grouped: one estimate
-// per instance (seg[0 .. ninst)).
-template <class G>
-int launch_lanczos_omega(const DevPattern& P, const TraceSystem& T, CgVectors& v, G g, int grid, const Seg* seg,
-                         int ninst, double factor, int steps, hipStream_t s);
-// r = b~, x = p = 0, e0 = omega Dinv r (preconditioner storage W)
-template <class W>
-int launch_mg_init(const DevPattern& P, const TraceSystem& T64, const TraceOp<W>& T, const Krylov<double>& v,
-                   const MgVecs<W>& mv, hipStream_t s);
-template <class W>
-int launch_mg_update(const TraceOp<W>& T, const Krylov<double>& v, const MgVecs<W>& mv, hipStream_t s);
-// dM: a device copy of M (read by the one-workgroup tail kernel)
-template <class W>
-int launch_mg_precond(const DevPattern& P, const TraceOp<W>& T, const Krylov<double>& v, const MgData& M,
-                      const MgData* dM, const MgVecs<W>& mv, hipStream_t s);
 
 // Launch tables of the multigrid preconditioner of a group of instances:
 // per vertex depth d (1 <= d < ndepth), the instances whose level d lies
@@ -634,14 +570,12 @@ struct MgGroup {
   int vsweeps = 2;
   double omega_v = 0.7;
 };
-// Set-up tables of a group's vertex hierarchies: level-1 assembly blocks
-// (instance, block) and, per depth d, the instances with a level d+1, with
-// block maps over the coarse nodes (cmask) and 8 lanes per coarse node (RAP).
+// Set-up tables of a group's vertex hierarchies: per depth d, the instances
+// with a level d+1, with block maps over the coarse nodes (cmask) and 8 lanes
+// per coarse node (RAP).
 struct MgSetupGroup {
   int ninst = 0;
   const MgData* dM = nullptr;
-  const BlockMap* l1map = nullptr;
-  int gl1 = 0;
   int ndepth = 1;
   VGroup cmask[kMaxLevels];
   int gcmask[kMaxLevels];
@@ -650,18 +584,6 @@ struct MgSetupGroup {
 };
 int mg_setup_levels_group(const MgSetupGroup& S, hipStream_t s);
 
-// grouped forms: rows of each instance from the Grouped selector (grid
-// blocks); Mu describes the packed mesh (its level 1 spans every
-// instance's vertices)
-template <class W>
-int launch_mg_init_group(const DevPattern& P, const TraceSystem& T64, const TraceOp<W>& T, const Krylov<double>& v,
-                         const MgVecs<W>& mv, Grouped g, int grid, hipStream_t s);
-template <class W>
-int launch_mg_update_group(const TraceOp<W>& T, const Krylov<double>& v, const MgVecs<W>& mv, Grouped g, int grid,
-                           hipStream_t s);
-template <class W>
-int launch_mg_precond_group(const DevPattern& P, const TraceOp<W>& T, const Krylov<double>& v, const MgData& Mu,
-                            const MgGroup& G, const MgVecs<W>& mv, Grouped g, int grid, hipStream_t s);
 // float copy of n doubles
 int launch_to_float(const double* src, float* dst, int64_t n, hipStream_t s);
 
@@ -676,18 +598,16 @@ int launch_add(double* u, const double* d, int64_t n, hipStream_t s);
 
 // rectangle_mesh generated on the device into (possibly packed) arrays:
 // nodes, cells and faces land at node0 / cell0 / face0; ids written are
-// global (shifted); cell_inst (optional) receives inst for every cell;
-// vf_ptr / vf_idx / fq4 optional; err bit 4: a one-cell face off the box.
+// global (shifted); cell_inst (optional) receives inst for every cell; err
+// bit 4: a one-cell face off the box.
 struct RectMeshArgs {
   int64_t nx = 0, ny = 0, nf = 0;
   double x0 = 0, y0 = 0, x1 = 1, y1 = 1, jitter = 0;
   uint64_t seed = 0;
   int64_t node0 = 0, cell0 = 0, face0 = 0;
   int inst = 0;
-  bool last = true;  // writes the closing entry of vf_ptr
   double* xy = nullptr;
-  int *cn = nullptr, *cf = nullptr, *fcell = nullptr, *fv = nullptr;
-  int *vf_ptr = nullptr, *vf_idx = nullptr, *fq4 = nullptr, *cell_inst = nullptr;
+  int *cn = nullptr, *cf = nullptr, *fcell = nullptr, *cell_inst = nullptr;
   int* err = nullptr;
 };
 int launch_rect_mesh(const RectMeshArgs& a, hipStream_t s);

@@ -1,35 +1,29 @@
-// Multigrid preconditioner for the HDG trace system on structured meshes.
+// The vertex levels of the multigrid preconditioner on structured meshes.
 //
-// Level 0 is the trace space (N dofs) with damped block-Jacobi smoothing.
-// Level 1 is the continuous P1 space on the mesh vertices: the prolongation
-// maps vertex values to the Legendre modes 0 and 1 of the trace of the
-// piecewise-linear function on every face (mode 0 = mean, mode 1 =
-// (v_hi - v_lo) / (2 sqrt 3), the face parameter running from the lower to
-// the higher node id), and the coarse operator is the Galerkin product
-// P^T S P, assembled cell by cell from the condensed blocks.  Levels 2.. are
-// the vertex grids of a rectangle_mesh coarsened by two (a side with n
-// cells gets (n + 1) / 2: coarse node I sits on fine node min(2I, n), so an
-// odd side keeps its last fine column as a one-cell-wide coarse column),
-// with linear interpolation on the nested triangulation and Galerkin (RAP)
-// operators; every level is a 7-point stencil.  One symmetric V-cycle (damped Jacobi,
-// fixed sweep counts, Jacobi sweeps on the coarsest grid) is a fixed SPD
-// operator, so it preconditions CG.
+// Level 0 is the reduced trace space (hdg_quad.hip).  Level 1 is the vertex
+// space: the prolongation maps vertex values to the Legendre modes 0 and 1 of
+// the trace of the linear function on every axis face (mode 0 = mean, mode 1
+// = (v_hi - v_lo) / (2 sqrt 3), the face parameter running from the lower to
+// the higher node id), and the operator is the Galerkin product P^T T P,
+// assembled quad by quad (q_build_kernel, q_l1_kernel).  Levels 2.. are the
+// vertex grids coarsened by two (a side with n cells gets (n + 1) / 2: coarse
+// node I sits on fine node min(2I, n), so an odd side keeps its last fine
+// column as a one-cell-wide coarse column), with bilinear interpolation and
+// Galerkin (RAP) operators; every level is a 9-point stencil.  One symmetric
+// V-cycle (damped Jacobi, fixed sweep counts, the coarsest grid exactly or by
+// Jacobi sweeps) is a fixed SPD operator, so it preconditions CG.
 //
 // Stencil slots: 0 (0,0), 1 (+1,0), 2 (-1,0), 3 (0,+1), 4 (0,-1), 5 (+1,-1),
 // 6 (-1,+1), 7 (+1,+1), 8 (-1,-1); node (i, j) of a level with nx cells per
-// row is i + j (nx+1).  The vertex operator of the mesh and the Galerkin
-// operators of even coarsening use slots 0-6; a one-cell-wide coarse column
-// or row is not nested in the coarse triangulation, and RAP across it also
-// couples the (+1,+1) neighbours (9 points close under RAP).
+// row is i + j (nx+1).
 #include <hip/hip_runtime.h>
 
-#include "hdg_internal.h"
+#include "hdg_quad.h"
 
 namespace hdg {
 
 namespace {
 
-constexpr double kS3 = 0.28867513459481288225;  // 1 / (2 sqrt 3)
 __constant__ int kOffX[kStencil] = {0, 1, -1, 0, 0, 1, -1, 1, -1};
 __constant__ int kOffY[kStencil] = {0, 0, 0, 1, -1, -1, 1, 1, -1};
 
@@ -57,191 +51,32 @@ __device__ inline Par1 parents1(int x, int n) {
 // fine index of coarse index I on a side of n fine cells
 __device__ inline int fine_of(int I, int n) { return min(2 * I, n); }
 
-// Linear interpolation of the coarse vector ec (row length cnx + 1) at fine
-// node (x, y) of a level with fnx x fny cells: along x, along y, or along the
-// cell diagonal ((x+1)/2, (y-1)/2) -- ((x-1)/2, (y+1)/2) when both are odd.
+// Bilinear interpolation of the coarse vector ec (row length cnx + 1) at fine
+// node (x, y) of a level with fnx x fny cells.  (The level-1 operator couples
+// the four vertices of a grid cell alike; interpolating along one diagonal
+// only costs 3-5 CG iterations: P3 160^2 18 instead of 15.)
 __device__ inline double prolong_at(int fnx, int fny, int cnx, const double* ec, int x, int y) {
   const Par1 px = parents1(x, fnx), py = parents1(y, fny);
   const int64_t cs = cnx + 1;
-  if (px.a == px.b && py.a == py.b) return ec[py.a * cs + px.a];
-  if (py.a == py.b) return 0.5 * (ec[py.a * cs + px.a] + ec[py.a * cs + px.b]);
-  if (px.a == px.b) return 0.5 * (ec[py.a * cs + px.a] + ec[py.b * cs + px.a]);
-  return 0.5 * (ec[py.a * cs + px.b] + ec[py.b * cs + px.a]);
+  const double lo = px.a == px.b ? ec[py.a * cs + px.a] : 0.5 * (ec[py.a * cs + px.a] + ec[py.a * cs + px.b]);
+  if (py.a == py.b) return lo;
+  const double hi = px.a == px.b ? ec[py.b * cs + px.a] : 0.5 * (ec[py.b * cs + px.a] + ec[py.b * cs + px.b]);
+  return 0.5 * (lo + hi);
 }
 
 // weight of coarse node (I, J) in prolong_at at fine node (x, y)
 __device__ inline double pweight(int fnx, int fny, int x, int y, int I, int J) {
   const Par1 px = parents1(x, fnx), py = parents1(y, fny);
-  const bool sx = px.a == px.b, sy = py.a == py.b;
-  if (sx && sy) return (px.a == I && py.a == J) ? 1.0 : 0.0;
-  if (sy) return (py.a == J && (px.a == I || px.b == I)) ? 0.5 : 0.0;
-  if (sx) return (px.a == I && (py.a == J || py.b == J)) ? 0.5 : 0.0;
-  return ((px.b == I && py.a == J) || (px.a == I && py.b == J)) ? 0.5 : 0.0;
-}
-
-__device__ inline double wave_sum_mg(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
-}
-
-template <int NW>
-__device__ inline double block_sum_mg(double v, double* sh) {
-  v = wave_sum_mg(v);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  if (l == 0) sh[w] = v;
-  __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < NW; ++i) s += sh[i];
-  __syncthreads();
-  return s;
-}
-
-template <int NW>
-__device__ inline double sum_partials_mg(const double* p, int n, double* sh) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) s += p[i];
-  s = wave_sum_mg(s);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  if (l == 0) sh[w] = s;
-  __syncthreads();
-  double t = 0.0;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) t += sh[i];
-  __syncthreads();
-  return t;
-}
-
-// (S x)_row for S = -K on free rows, from the matrix stored as V: the
-// symmetric blocks at four modes per face, else the face-ELL values
-// (accumulated in FP64; values read once per product by nontemporal loads,
-// as in the CG product).
-template <int NT, class V>
-__device__ inline double s_row(const DevPattern& P, const TraceOp<V>& T, const V* x, int64_t r) {
-  const int64_t f = r / NT;
-  double acc = 0.0;
-  if constexpr (kSymBlocks<NT>) {
-    acc = sym_row<NT>(P.nbr, T.blk, T.nf, f, (int)(r - f * NT), [&](int64_t g, int b) { return (double)x[g * NT + b]; });
-  } else {
-#pragma unroll
-    for (int s = 0; s < kSlots; ++s) {
-      const int64_t g = (int64_t)__ldg(P.bcol + f * kSlots + s) * NT;
-#pragma unroll
-      for (int b = 0; b < NT; ++b)
-        acc = fma((double)__builtin_nontemporal_load(T.vals + (int64_t)(s * NT + b) * T.N + r), (double)x[g + b],
-                  acc);
-    }
-  }
-  return T.dmask[r] ? 0.0 : -acc;
+  const double wx = px.a == px.b ? (px.a == I ? 1.0 : 0.0) : (px.a == I || px.b == I ? 0.5 : 0.0);
+  const double wy = py.a == py.b ? (py.a == J ? 1.0 : 0.0) : (py.a == J || py.b == J ? 0.5 : 0.0);
+  return wx * wy;
 }
 
 // ------------------------------------------------------------ set-up
-// vertex mask: a vertex is fixed when a face through it has a Dirichlet
-// mode-0 dof.
-__global__ void mg_vmask_kernel(MgData M, TraceSystem T) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= M.nv) return;
-  unsigned char m = 0;
-  for (int k = M.vf_ptr[v]; k < M.vf_ptr[v + 1]; ++k) m |= T.dmask[(int64_t)M.vf_idx[k] * T.nt];
-  M.lev[1].mask[v] = m;
-}
-
-// A1_c = P_c^T (-Ate_c) P_c for every cell, masked.
-template <int NT>
-__global__ void mg_cell_coarse_kernel(DevMesh mesh, MgData M, TraceSystem T, const double* __restrict__ Ate) {
-  constexpr int NTR = 3 * NT;
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= mesh.nc) return;
-  int vg[3];
-  unsigned char vm[3];
-#pragma unroll
-  for (int v = 0; v < 3; ++v) {
-    vg[v] = mesh.cn[3 * c + v];
-    vm[v] = M.lev[1].mask[vg[v]];
-  }
-  // P_c rows of modes 0 and 1 of each local face: weights on local vertices
-  // local face lf joins local vertices (lf+1)%3, (lf+2)%3
-  double Pw[3][2][3];
-#pragma unroll
-  for (int lf = 0; lf < 3; ++lf) {
-    const int a = (lf + 1) % 3, b = (lf + 2) % 3;
-    const int lo = vg[a] < vg[b] ? a : b, hi = vg[a] < vg[b] ? b : a;
-    const int64_t f = mesh.cf[3 * c + lf];
-    const bool d0 = T.dmask[f * NT] != 0, d1 = T.dmask[f * NT + 1] != 0;
-#pragma unroll
-    for (int w = 0; w < 3; ++w) {
-      const double keep = vm[w] ? 0.0 : 1.0;
-      Pw[lf][0][w] = d0 ? 0.0 : keep * ((w == a || w == b) ? 0.5 : 0.0);
-      Pw[lf][1][w] = d1 ? 0.0 : keep * (w == hi ? kS3 : (w == lo ? -kS3 : 0.0));
-    }
-  }
-  const double* at = Ate + c * NTR * NTR;
-  // Q = (-Ate) P_c  (NTR x 3), then A = P_c^T Q
-  double A[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll
-  for (int lf = 0; lf < 3; ++lf)
-#pragma unroll
-    for (int md = 0; md < 2; ++md) {
-      const int row = lf * NT + md;
-      double q[3] = {0, 0, 0};
-#pragma unroll
-      for (int lg = 0; lg < 3; ++lg)
-#pragma unroll
-        for (int me = 0; me < 2; ++me) {
-          const double s = -at[row * NTR + lg * NT + me];
-#pragma unroll
-          for (int w = 0; w < 3; ++w) q[w] = fma(s, Pw[lg][me][w], q[w]);
-        }
-#pragma unroll
-      for (int u = 0; u < 3; ++u)
-#pragma unroll
-        for (int w = 0; w < 3; ++w) A[u][w] = fma(Pw[lf][md][u], q[w], A[u][w]);
-    }
-#pragma unroll
-  for (int u = 0; u < 3; ++u)
-#pragma unroll
-    for (int w = 0; w < 3; ++w) M.cellA[c * 9 + u * 3 + w] = A[u][w];
-}
-
-// Level-1 stencils gathered from the (up to) six cells around each vertex.
-// One hierarchy (map null: Ms[0] over the grid) or one per block via map.
-__global__ void mg_assemble_l1_kernel(const MgData* __restrict__ Ms, const BlockMap* __restrict__ map) {
-  const BlockMap bm = map ? map[blockIdx.x] : BlockMap{0, (int)blockIdx.x};
-  const MgData& M = Ms[bm.inst];
-  const int64_t v = (int64_t)bm.lb * blockDim.x + threadIdx.x;
-  const MgLevel& L = M.lev[1];
-  if (v >= L.n) return;
-  const int nx = M.nx, ny = M.ny;
-  const int i = (int)(v % (nx + 1)), j = (int)(v / (nx + 1));
-  double st[kStencil] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  if (!L.mask[v]) {
-    // (cell grid position, upper?, local index of v)
-    const int ca[6] = {i, i - 1, i, i - 1, i - 1, i};
-    const int cb[6] = {j, j, j - 1, j, j - 1, j - 1};
-    const int up[6] = {0, 0, 0, 1, 1, 1};
-    const int lv[6] = {0, 1, 2, 0, 1, 2};
-    for (int t = 0; t < 6; ++t) {
-      const int a = ca[t], b = cb[t];
-      if (a < 0 || a >= nx || b < 0 || b >= ny) continue;
-      const int64_t c = 2 * ((int64_t)b * nx + a) + up[t];
-      // local vertex grid positions of the cell
-      int px[3], py[3];
-      if (!up[t]) { px[0] = a; py[0] = b; px[1] = a + 1; py[1] = b; px[2] = a; py[2] = b + 1; }
-      else { px[0] = a + 1; py[0] = b; px[1] = a + 1; py[1] = b + 1; px[2] = a; py[2] = b + 1; }
-      for (int w = 0; w < 3; ++w) {
-        const int s = slot_of(px[w] - i, py[w] - j);
-        if (s >= 0) st[s] += M.cellA[c * 9 + lv[t] * 3 + w];
-      }
-    }
-  }
-  for (int s = 0; s < kStencil; ++s) L.a[s * L.n + v] = L.mask[v] ? (s == 0 ? 1.0 : 0.0) : st[s];
-  L.dinv[v] = L.mask[v] ? 0.0 : 1.0 / st[0];
-}
-
 // Galerkin coarse stencil R A P on the next level: R = P^T with the weights
-// of prolong_at.  Eight lanes per coarse node: lane t < 7 takes the fine
-// node at support offset t, and a fixed shuffle tree sums the lanes' stencils.
+// of prolong_at.  Eight lanes per coarse node: lane t takes the fine node at
+// support offset t (lane 0 the ninth too), and a fixed shuffle tree sums the
+// lanes' stencils.
 template <class VS>
 __global__ __launch_bounds__(256) void mg_rap_kernel(VS sel) {
   int lb;
@@ -256,35 +91,31 @@ __global__ __launch_bounds__(256) void mg_rap_kernel(VS sel) {
   const int I = live ? (int)(C % (cnx + 1)) : 0, J = live ? (int)(C / (cnx + 1)) : 0;
   const unsigned char cm = live ? Cc.mask[C] : 1;  // written by mg_cmask_kernel
   double st[kStencil] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  if (!cm && t < 7) {
-    const int fx = fine_of(I, fnx) + (t == 1 || t == 5 ? 1 : (t == 2 || t == 6 ? -1 : 0));
-    const int fy = fine_of(J, fny) + (t == 3 || t == 6 ? 1 : (t == 4 || t == 5 ? -1 : 0));
+  for (int o = t; !cm && o < kStencil; o += 8) {
+    const int fx = fine_of(I, fnx) + kOffX[o], fy = fine_of(J, fny) + kOffY[o];
     const int64_t fi = (int64_t)fy * (fnx + 1) + fx;
     const bool in = fx >= 0 && fx <= fnx && fy >= 0 && fy <= fny && !F.mask[fi];
     const double w1 = in ? pweight(fnx, fny, fx, fy, I, J) : 0.0;
-    if (w1 != 0.0) {
-      for (int s = 0; s < F.npts; ++s) {
-        const double av = F.a[s * F.n + fi];
-        if (av == 0.0) continue;
-        const int gx = fx + kOffX[s], gy = fy + kOffY[s];
-        if (gx < 0 || gx > fnx || gy < 0 || gy > fny) continue;
-        if (F.mask[(int64_t)gy * (fnx + 1) + gx]) continue;
-        // coarse parents of fine node g, as prolong_at weighs them
-        const Par1 px = parents1(gx, fnx), py = parents1(gy, fny);
-        int qx[2], qy[2], np = 2;
-        double w2 = 0.5;
-        if (px.a == px.b && py.a == py.b) { qx[0] = px.a; qy[0] = py.a; np = 1; w2 = 1.0; }
-        else if (py.a == py.b) { qx[0] = px.a; qx[1] = px.b; qy[0] = qy[1] = py.a; }
-        else if (px.a == px.b) { qx[0] = qx[1] = px.a; qy[0] = py.a; qy[1] = py.b; }
-        else { qx[0] = px.b; qy[0] = py.a; qx[1] = px.a; qy[1] = py.b; }
-        for (int q = 0; q < np; ++q) {
-          if (Cc.mask[(int64_t)qy[q] * (cnx + 1) + qx[q]]) continue;  // zero column of P
-          const int sl = slot_of(qx[q] - I, qy[q] - J);
+    if (w1 == 0.0) continue;
+    for (int s = 0; s < kStencil; ++s) {
+      const double av = F.a[s * F.n + fi];
+      if (av == 0.0) continue;
+      const int gx = fx + kOffX[s], gy = fy + kOffY[s];
+      if (gx < 0 || gx > fnx || gy < 0 || gy > fny) continue;
+      if (F.mask[(int64_t)gy * (fnx + 1) + gx]) continue;
+      // coarse parents of fine node g, as prolong_at weighs them
+      const Par1 px = parents1(gx, fnx), py = parents1(gy, fny);
+      const int mx = px.a == px.b ? 1 : 2, my = py.a == py.b ? 1 : 2;
+      const double w2 = (mx == 1 ? 1.0 : 0.5) * (my == 1 ? 1.0 : 0.5);
+      for (int v = 0; v < my; ++v)
+        for (int u = 0; u < mx; ++u) {
+          const int qx = u ? px.b : px.a, qy = v ? py.b : py.a;
+          if (Cc.mask[(int64_t)qy * (cnx + 1) + qx]) continue;  // zero column of P
+          const int sl = slot_of(qx - I, qy - J);
 #pragma unroll
-          for (int u = 0; u < kStencil; ++u)
-            if (u == sl) st[u] = fma(w1 * av, w2, st[u]);
+          for (int k = 0; k < kStencil; ++k)
+            if (k == sl) st[k] = fma(w1 * av, w2, st[k]);
         }
-      }
     }
   }
 #pragma unroll
@@ -317,7 +148,7 @@ __global__ __launch_bounds__(1024) void mg_coarse_inverse_kernel(const MgData* _
   for (int v = threadIdx.x; v < n; v += blockDim.x) {
     const int i = v % (L.nx + 1), j = v / (L.nx + 1);
     m[v * W + n + v] = 1.0;
-    for (int s = 0; s < L.npts; ++s) {
+    for (int s = 0; s < kStencil; ++s) {
       const int gx = i + kOffX[s], gy = j + kOffY[s];
       if (gx < 0 || gx > L.nx || gy < 0 || gy > L.ny) continue;
       m[v * W + gy * (L.nx + 1) + gx] += L.a[s * L.n + v];
@@ -383,291 +214,6 @@ __global__ void mg_cmask_kernel(VS sel) {
   Cc.mask[C] = F.mask[(int64_t)fine_of(J, F.ny) * (F.nx + 1) + fine_of(I, F.nx)];
 }
 
-// S P0 restricted to each row: sp[j N + r] = sum over the free gathered
-// columns (g, b < 2) of S[r, (g, b)] P0[(g, b), fq4[4 f + j]], where
-// P0[(g, 0), lo] = P0[(g, 0), hi] = 1/2 and P0[(g, 1), hi] = -P0[(g, 1), lo]
-// = 1/(2 sqrt 3).  Every face of the two cells of face f has its end points
-// among fq4[4f .. 4f+3].
-template <int NT>
-__global__ __launch_bounds__(256) void mg_sp_kernel(DevPattern P, TraceSystem T, MgData M, float* sp32) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= T.N) return;
-  const int64_t f = r / NT;
-  int q[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) q[j] = M.fq4[4 * f + j];
-  double w[4] = {0.0, 0.0, 0.0, 0.0};
-  // entry S[r, (g, b)] = -kv of a mode b < 2 column
-  auto add = [&](int64_t g, int b, double kv) {
-    if (b >= 2 || T.dmask[g * NT + b]) return;
-    const int lo = M.fv[2 * g], hi = M.fv[2 * g + 1];
-    const double sv = -kv;
-    const double cl = b == 0 ? 0.5 : -kS3, ch = b == 0 ? 0.5 : kS3;
-    bool dl = false, dh = false;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool ml = !dl && q[j] == lo, mh = !dh && q[j] == hi;
-      w[j] = ml ? fma(sv, cl, w[j]) : w[j];
-      w[j] = mh ? fma(sv, ch, w[j]) : w[j];
-      dl = dl || ml;
-      dh = dh || mh;
-    }
-  };
-  if (!T.dmask[r]) {
-    if constexpr (kSymBlocks<NT>) {
-      sym_row_entries<NT>(P.nbr, T.blk, T.nf, f, (int)(r - f * NT), add);
-    } else {
-      for (int sl = 0; sl < kSlots; ++sl) {
-        const int64_t g = P.bcol[f * kSlots + sl];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) add(g, b, T.vals[(int64_t)(sl * NT + b) * T.N + r]);
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    M.sp[(int64_t)j * T.N + r] = w[j];
-    if (sp32) sp32[(int64_t)j * T.N + r] = (float)w[j];
-  }
-}
-
-// ------------------------------------------------------- level 0 (trace)
-// update(i) with the multigrid preconditioner: x += alpha p; r -= alpha q;
-// e0 = omega Dinv r (first smoothing step, preconditioner storage W);
-// partial (r, r).
-template <int NT, class W, class G>
-__global__ __launch_bounds__(64 * NT) void mg_update_kernel(TraceOp<W> T, Krylov<double> v, MgVecs<W> mv, G gsel) {
-  constexpr int NTH = 64 * NT;
-  __shared__ double rs[NTH];
-  __shared__ double sh[NT];
-  const Seg S = seg_of(gsel);
-  CgState* st = S.st;
-  if (st->done) return;
-  const int i = st->i_upd;
-  const int lb = blockIdx.x - S.b0;
-  if (lb == 0 && threadIdx.x == 0) st->i_pre = i;
-  const size_t nbt = (size_t)v.nblocks;
-  const double pq = sum_partials_mg<NT>(v.part + S.b0, S.nb, sh);
-  const double rz = st->rz[i & 1];
-  if (!(pq > 0.0)) {
-    if (lb == 0 && threadIdx.x == 0) {
-      st->done = 3;
-      st->it = i - 1;
-    }
-    return;
-  }
-  const double alpha = rz / pq, om = st->omega;
-  const double* __restrict__ p = (i & 1) ? v.p1 : v.p0;
-  double prr = 0.0;
-  for (int64_t r0 = S.lo + (int64_t)lb * NTH; r0 < S.hi; r0 += (int64_t)S.nb * NTH) {
-    const int64_t r = r0 + threadIdx.x;
-    double rn = 0.0;
-    if (r < S.hi) {
-      v.x[r] = fma(alpha, p[r], v.x[r]);
-      rn = fma(-alpha, v.q[r], v.r[r]);
-      v.r[r] = rn;
-      prr = fma(rn, rn, prr);
-    }
-    jacobi_apply<NT>(T.Dinv, T.nf, rs, rn, r, r < S.hi, [&](double z) { mv.e0[r] = (W)(om * z); });
-  }
-  const double b = block_sum_mg<NT>(prr, sh);
-  if (threadIdx.x == 0) v.part[nbt * 3 + blockIdx.x] = b;
-}
-
-// init (update(0)) for the multigrid path: r0 = b~ = -(rhs - K uD), x = p = 0,
-// e0 = omega Dinv r0.  uD is zero off the Dirichlet dofs, so the lift reads
-// only the matrix columns of Dirichlet dofs (the mask decides per column).
-template <int NT, class W, class G>
-__global__ __launch_bounds__(64 * NT) void mg_init_kernel(DevPattern P, TraceSystem T64, TraceOp<W> T,
-                                                          Krylov<double> v, MgVecs<W> mv, G gsel) {
-  constexpr int NTH = 64 * NT;
-  __shared__ double rs[NTH];
-  __shared__ double sh[NT];
-  const Seg S = seg_of(gsel);
-  const int lb = blockIdx.x - S.b0;
-  const double om = S.st->omega;
-  double prr = 0.0;
-  for (int64_t r0 = S.lo + (int64_t)lb * NTH; r0 < S.hi; r0 += (int64_t)S.nb * NTH) {
-    const int64_t r = r0 + threadIdx.x;
-    double b = 0.0;
-    if (r < S.hi) {
-      if (!T64.dmask[r]) {
-        const int64_t f = r / NT;
-        double s = T64.rhs[r];
-        if constexpr (kSymBlocks<NT>) {
-          s -= sym_row_lift<NT>(P.nbr, T64.blk, T64.nf, T64.dmask, T64.uD, f, (int)(r - f * NT));
-        } else {
-#pragma unroll
-          for (int sl = 0; sl < kSlots; ++sl) {
-            const int64_t g = (int64_t)P.bcol[f * kSlots + sl] * NT;
-#pragma unroll
-            for (int c = 0; c < NT; ++c)
-              if (T64.dmask[g + c]) s -= T64.vals[(int64_t)(sl * NT + c) * T64.N + r] * T64.uD[g + c];
-          }
-        }
-        b = -s;
-      }
-      v.r[r] = b;
-      v.x[r] = 0.0;
-      v.p0[r] = 0.0;
-      v.p1[r] = 0.0;
-      prr = fma(b, b, prr);
-    }
-    jacobi_apply<NT>(T.Dinv, T.nf, rs, b, r, r < S.hi, [&](double z) { mv.e0[r] = (W)(om * z); });
-  }
-  const double bb = block_sum_mg<NT>(prr, sh);
-  if (threadIdx.x == 0) v.part[(size_t)v.nblocks * 3 + blockIdx.x] = bb;
-  if (lb == 0 && threadIdx.x == 0) {
-    S.st->done = 0;
-    S.st->it = 0;
-    S.st->pq = 0.0;
-    S.st->i_pre = 0;  // the first smoother call completes update(0)
-  }
-}
-
-// res0 = r - S e0 over all rows (of every instance when packed; v.st null:
-// no convergence check).  For even nt the lane of mode 0 of a face also
-// writes the face's restriction weights fc (P0^T res0 at its lower and
-// higher end: 0.5 res0_0 -+ res0_1 / (2 sqrt 3)), with mode 1 taken from the
-// next lane (a face's rows are consecutive lanes of one wavefront).
-template <int NT, class W>
-__global__ __launch_bounds__(256) void mg_resid0_kernel(DevPattern P, TraceOp<W> T, Krylov<double> v,
-                                                        MgVecs<W> mv, double* __restrict__ fc) {
-  if (v.st && v.st->done) return;
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < T.N; r += (int64_t)gridDim.x * blockDim.x) {
-    // every row's product, the Dirichlet rows masked afterwards: the loads
-    // do not wait for the mask
-    const double sr = s_row<NT, W>(P, T, mv.e0, r);
-    const W res = T.dmask[r] ? (W)0 : (W)(v.r[r] - sr);
-    mv.res0[r] = res;
-    if constexpr (NT % 2 == 0) {
-      // the grid is a multiple of 64 threads and N of NT: lane r + 1 of a
-      // mode-0 lane r is in the same wavefront and active
-      const double r1 = (double)__shfl_down((double)res, 1, 64);
-      if (r % NT == 0) {
-        const double r0 = (double)res;
-        fc[2 * (r / NT)] = 0.5 * r0 + (-kS3) * r1;
-        fc[2 * (r / NT) + 1] = 0.5 * r0 + kS3 * r1;
-      }
-    }
-  }
-}
-
-// vf2: the vertex -> face entries with the side of the vertex on the face.
-__global__ void mg_vf2_kernel(MgData M) {
-  const int64_t vv = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (vv >= M.nv) return;
-  for (int k = M.vf_ptr[vv]; k < M.vf_ptr[vv + 1]; ++k) {
-    const int f = M.vf_idx[k];
-    M.vf2[k] = 2 * f + (M.fv[2 * f] == vv ? 0 : 1);
-  }
-}
-
-// r1 = P0^T res0, vertex by vertex over the incident faces.
-template <int NT, class W>
-__global__ __launch_bounds__(256) void mg_restrict0_kernel(Krylov<double> v, MgData M, MgVecs<W> mv) {
-  if (v.st && v.st->done) return;
-  const MgLevel L = M.lev[1];
-  const int64_t vv = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (vv >= L.n) return;
-  double s = 0.0;
-  if (!L.mask[vv]) {
-    if constexpr (NT % 2 == 0) {
-      // the weights the residual kernel wrote per face end, summed in the
-      // vertex's face order; the first 8 indices are loaded before any
-      // weight, so that the gathers are in flight together
-      const int k0 = M.vf_ptr[vv], k1 = M.vf_ptr[vv + 1];
-      int id[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) id[u] = k0 + u < k1 ? M.vf2[k0 + u] : -1;
-      double w[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) w[u] = id[u] >= 0 ? M.fc[id[u]] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (id[u] >= 0) s += w[u];
-      for (int k = k0 + 8; k < k1; ++k) s += M.fc[M.vf2[k]];
-    } else {
-      // modes 0 and 1 of the incident faces, in the vertex's face order,
-      // the first 8 faces' loads issued together
-      const int k0 = M.vf_ptr[vv], k1 = M.vf_ptr[vv + 1];
-      int64_t fa[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) fa[u] = k0 + u < k1 ? (int64_t)M.vf_idx[k0 + u] : -1;
-      double t[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        t[u] = 0.0;
-        if (fa[u] >= 0) {
-          const int64_t f = fa[u];
-          const bool lo = M.fv[2 * f] == vv;
-          t[u] = 0.5 * (double)mv.res0[f * NT] + (lo ? -kS3 : kS3) * (double)mv.res0[f * NT + 1];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (fa[u] >= 0) s += t[u];
-      for (int k = k0 + 8; k < k1; ++k) {
-        const int64_t f = M.vf_idx[k];
-        const bool lo = M.fv[2 * f] == vv;
-        s += 0.5 * (double)mv.res0[f * NT] + (lo ? -kS3 : kS3) * (double)mv.res0[f * NT + 1];
-      }
-    }
-  }
-  L.r[vv] = s;
-}
-
-// z = e0 + P0 e1 + omega Dinv (res0 - (S P0) e1): the post-smoothing step.
-// S (e0 + P0 e1) = S e0 + (S P0) e1 and res0 = r - S e0, so the trace matrix
-// is not read again; and e0 = omega Dinv r, so z = P0 e1 + omega Dinv (r +
-// res0 - (S P0) e1) and e0 is not read either (r is, for the partial (r, z)
-// of the next iteration).
-template <int NT, class W, class G>
-__global__ __launch_bounds__(64 * NT) void mg_smooth0_kernel(TraceOp<W> T, Krylov<double> v, MgData M,
-                                                             MgVecs<W> mv, G gsel) {
-  constexpr int NTH = 64 * NT;
-  __shared__ double rs[NTH];
-  __shared__ double sh[NT];
-  const Seg S = seg_of(gsel);
-  CgState* st = S.st;
-  if (st->done) return;
-  const int i = st->i_pre;
-  const int lb = blockIdx.x - S.b0;
-  if (lb == 0 && threadIdx.x == 0) st->i_spmv = i + 1;
-  const double om = st->omega;
-  const double* __restrict__ e1 = M.lev[1].e;
-  double prz = 0.0;
-  for (int64_t r0 = S.lo + (int64_t)lb * NTH; r0 < S.hi; r0 += (int64_t)S.nb * NTH) {
-    const int64_t r = r0 + threadIdx.x;
-    double rv = 0.0, rr = 0.0, pe = 0.0;
-    if (r < S.hi) {
-      // every row formed, the Dirichlet rows masked afterwards (the loads do
-      // not wait for the mask)
-      rv = v.r[r];
-      const int64_t f = r / NT;
-      double s = rv + (double)mv.res0[r];
-      // the face's 4 vertices, its lower and higher end point first
-      const int4 q = *reinterpret_cast<const int4*>(M.fq4 + 4 * f);
-      const double ev[4] = {e1[q.x], e1[q.y], e1[q.z], e1[q.w]};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s = fma(-(double)mv.sp[(int64_t)j * T.N + r], ev[j], s);
-      const int a = (int)(r - f * NT);
-      const double pc = a == 0 ? 0.5 * (ev[0] + ev[1]) : (a == 1 ? kS3 * (ev[1] - ev[0]) : 0.0);
-      if (!T.dmask[r]) {
-        rr = s;
-        pe = pc;
-      }
-    }
-    jacobi_apply<NT>(T.Dinv, T.nf, rs, rr, r, r < S.hi, [&](double z) {
-      const double zv = fma(om, z, pe);
-      v.z[r] = zv;
-      prz = fma(rv, zv, prz);
-    });
-  }
-  const double b = block_sum_mg<NT>(prz, sh);
-  if (threadIdx.x == 0) v.part[(size_t)v.nblocks * (1 + ((i + 1) & 1)) + blockIdx.x] = b;
-}
-
 // ------------------------------------------------------- vertex levels
 // (A x)_v on a level, with x given as a function of (index, i, j), so that
 // fused kernels can form x on the fly.
@@ -681,10 +227,8 @@ __device__ inline double stencil_apply(const MgLevel& L, int64_t v, int i, int j
   if (j > 0) s = fma(L.a[4 * L.n + v], xv(v - row, i, j - 1), s);
   if (i < L.nx && j > 0) s = fma(L.a[5 * L.n + v], xv(v + 1 - row, i + 1, j - 1), s);
   if (i > 0 && j < L.ny) s = fma(L.a[6 * L.n + v], xv(v - 1 + row, i - 1, j + 1), s);
-  if (L.npts > 7) {
-    if (i < L.nx && j < L.ny) s = fma(L.a[7 * L.n + v], xv(v + 1 + row, i + 1, j + 1), s);
-    if (i > 0 && j > 0) s = fma(L.a[8 * L.n + v], xv(v - 1 - row, i - 1, j - 1), s);
-  }
+  if (i < L.nx && j < L.ny) s = fma(L.a[7 * L.n + v], xv(v + 1 + row, i + 1, j + 1), s);
+  if (i > 0 && j > 0) s = fma(L.a[8 * L.n + v], xv(v - 1 - row, i - 1, j - 1), s);
   return s;
 }
 
@@ -736,10 +280,10 @@ __device__ inline double fine_res(const MgLevel& F, int fx, int fy, bool one_swe
   return F.r[fi] - stencil_apply(F, fi, fx, fy, ev);
 }
 
-// coarse r = R (r - A e), R = P^T: the fine node of C and its six stencil
+// coarse r = R (r - A e), R = P^T: the fine node of C and its eight stencil
 // neighbours, weighted as prolong_at weighs C there.  Eight lanes per
-// coarse node: lane t < 7 forms the fine residual at stencil offset t, and a
-// fixed shuffle tree sums them.
+// coarse node: lane t forms the fine residual at stencil offset t (lane 0
+// the ninth too), and a fixed shuffle tree sums them.
 template <class VS>
 __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, int one_sweep, double om) {
   int lb;
@@ -751,12 +295,13 @@ __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, int one_sweep, 
   const int64_t C = g >> 3;
   const int t = (int)(g & 7);
   double val = 0.0;
-  if (C < Cc.n && t < 7 && !Cc.mask[C]) {
+  if (C < Cc.n && !Cc.mask[C]) {
     const int I = (int)(C % (Cc.nx + 1)), J = (int)(C / (Cc.nx + 1));
-    const int x = fine_of(I, F.nx) + (t == 1 || t == 5 ? 1 : (t == 2 || t == 6 ? -1 : 0));
-    const int y = fine_of(J, F.ny) + (t == 3 || t == 6 ? 1 : (t == 4 || t == 5 ? -1 : 0));
-    const double w = (x < 0 || x > F.nx || y < 0 || y > F.ny) ? 0.0 : pweight(F.nx, F.ny, x, y, I, J);
-    if (w != 0.0) val = w * fine_res(F, x, y, one_sweep != 0, om);
+    for (int o = t; o < kStencil; o += 8) {
+      const int x = fine_of(I, F.nx) + kOffX[o], y = fine_of(J, F.ny) + kOffY[o];
+      const double w = (x < 0 || x > F.nx || y < 0 || y > F.ny) ? 0.0 : pweight(F.nx, F.ny, x, y, I, J);
+      if (w != 0.0) val = fma(w, fine_res(F, x, y, one_sweep != 0, om), val);
+    }
   }
   val += __shfl_xor(val, 1, 8);
   val += __shfl_xor(val, 2, 8);
@@ -813,7 +358,7 @@ __global__ __launch_bounds__(1024) void v_coarsest_kernel(MgLevel L, double om, 
 // Level of the one-workgroup tail: stencils, diagonal inverse and vectors
 // all in LDS.  A fixed node has dinv = 0 (its stencil row is the identity).
 struct TailLevel {
-  int nx, ny, n, npts;
+  int nx, ny, n;
   const double* a;     // a[s*n + v]
   const double* dinv;
 };
@@ -827,10 +372,8 @@ __device__ inline double tail_apply(const TailLevel& L, const double* x, int v, 
   if (j > 0) s = fma(L.a[4 * L.n + v], x[v - row], s);
   if (i < L.nx && j > 0) s = fma(L.a[5 * L.n + v], x[v + 1 - row], s);
   if (i > 0 && j < L.ny) s = fma(L.a[6 * L.n + v], x[v - 1 + row], s);
-  if (L.npts > 7) {
-    if (i < L.nx && j < L.ny) s = fma(L.a[7 * L.n + v], x[v + 1 + row], s);
-    if (i > 0 && j > 0) s = fma(L.a[8 * L.n + v], x[v - 1 - row], s);
-  }
+  if (i < L.nx && j < L.ny) s = fma(L.a[7 * L.n + v], x[v + 1 + row], s);
+  if (i > 0 && j > 0) s = fma(L.a[8 * L.n + v], x[v - 1 - row], s);
   return s;
 }
 
@@ -878,7 +421,6 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
     L.nx = M.lev[l].nx;
     L.ny = M.lev[l].ny;
     L.n = (int)M.lev[l].n;
-    L.npts = M.lev[l].npts;
     L.a = SA + (kStencil + 1) * o;
     L.dinv = SA + (kStencil + 1) * o + kStencil * L.n;
     return L;
@@ -913,7 +455,7 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
                      : pweight(L.nx, L.ny, fx, fy, I, J) * e[fy * (L.nx + 1) + fx];
         };
         s = res(x, y) + res(x + 1, y) + res(x - 1, y) + res(x, y + 1) + res(x, y - 1) + res(x + 1, y - 1) +
-            res(x - 1, y + 1);
+            res(x - 1, y + 1) + res(x + 1, y + 1) + res(x - 1, y - 1);
       }
       rc[C] = s;
     }
@@ -984,15 +526,6 @@ int grid1(int64_t n, int t = 256) {
   return (int)g;
 }
 
-#define MG_NT_DISPATCH(nt, CALL) \
-  switch (nt) {                  \
-    case 2: CALL(2); break;      \
-    case 3: CALL(3); break;      \
-    case 4: CALL(4); break;      \
-    case 5: CALL(5); break;      \
-    default: return (int)hipErrorInvalidValue; \
-  }
-
 // V-cycle from level l down; the result is left in lev[l].e.  dM is the
 // device copy of M that the tail kernel reads.
 int vcycle(const MgData& M, const MgData* dM, int l, const CgState* st, hipStream_t s) {
@@ -1039,32 +572,7 @@ int vcycle_group(const MgGroup& G, hipStream_t s) {
 
 }  // namespace
 
-int mg_setup_cells(const DevMesh& mesh, const MgData& M, const TraceSystem& T, const double* Ate, hipStream_t s) {
-  hipLaunchKernelGGL(mg_vmask_kernel, dim3(grid1(M.nv)), dim3(256), 0, s, M, T);
-  if (T.nt % 2 == 0) hipLaunchKernelGGL(mg_vf2_kernel, dim3(grid1(M.nv)), dim3(256), 0, s, M);
-#define CELL(NT) hipLaunchKernelGGL(mg_cell_coarse_kernel<NT>, dim3(grid1(mesh.nc)), dim3(256), 0, s, mesh, M, T, Ate);
-  MG_NT_DISPATCH(T.nt, CELL)
-#undef CELL
-  return (int)hipGetLastError();
-}
-
-int mg_setup_sp(const MgData& M, const TraceSystem& T, const DevPattern& P, float* sp32, hipStream_t s) {
-  if (!trace_op_ready(P, T)) return (int)hipErrorInvalidValue;
-#define SPK(NT) hipLaunchKernelGGL(mg_sp_kernel<NT>, dim3(grid1(T.N)), dim3(256), 0, s, P, T, M, sp32);
-  MG_NT_DISPATCH(T.nt, SPK)
-#undef SPK
-  return (int)hipGetLastError();
-}
-
-int mg_setup_mesh(const DevMesh& mesh, const MgData& M, const TraceSystem& T, const DevPattern& P,
-                  const double* Ate, float* sp32, hipStream_t s) {
-  const int e = mg_setup_cells(mesh, M, T, Ate, s);
-  if (e) return e;
-  return mg_setup_sp(M, T, P, sp32, s);
-}
-
 int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
-  hipLaunchKernelGGL(mg_assemble_l1_kernel, dim3(grid1(M.lev[1].n)), dim3(256), 0, s, dM, (const BlockMap*)nullptr);
   for (int l = 1; l + 1 < M.nlev; ++l) {
     const VOne rec{VRec{M.lev[l], M.lev[l + 1], nullptr}};
     hipLaunchKernelGGL(mg_cmask_kernel<VOne>, dim3(grid1(M.lev[l + 1].n)), dim3(256), 0, s, rec);
@@ -1076,7 +584,6 @@ int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
 }
 
 int mg_setup_levels_group(const MgSetupGroup& S, hipStream_t s) {
-  hipLaunchKernelGGL(mg_assemble_l1_kernel, dim3(S.gl1), dim3(256), 0, s, S.dM, S.l1map);
   for (int d = 1; d < S.ndepth; ++d) {
     hipLaunchKernelGGL(mg_cmask_kernel<VGroup>, dim3(S.gcmask[d]), dim3(256), 0, s, S.cmask[d]);
     hipLaunchKernelGGL(mg_rap_kernel<VGroup>, dim3(S.grap[d]), dim3(256), 0, s, S.rap[d]);
@@ -1086,122 +593,9 @@ int mg_setup_levels_group(const MgSetupGroup& S, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-int mg_setup_numeric(const DevMesh& mesh, MgData& M, const MgData* dM, TraceSystem& T, const DevPattern& P,
-                     const double* Ate, float* sp32, hipStream_t s) {
-  const int e = mg_setup_mesh(mesh, M, T, P, Ate, sp32, s);
-  if (e) return e;
-  return mg_setup_levels(M, dM, s);
+int launch_vcycle(const MgData& M, const MgData* dM, const CgState* st, hipStream_t s) {
+  return vcycle(M, dM, 1, st, s);
 }
-
-template <class W, class G>
-int mg_init_t(const DevPattern& P, const TraceSystem& T64, const TraceOp<W>& T, const Krylov<double>& v,
-              const MgVecs<W>& mv, G g, int grid, hipStream_t s) {
-  if (!trace_op_ready(P, T64)) return (int)hipErrorInvalidValue;
-#define INIT(NT) \
-  hipLaunchKernelGGL((mg_init_kernel<NT, W, G>), dim3(grid), dim3(64 * NT), 0, s, P, T64, T, v, mv, g);
-  MG_NT_DISPATCH(T.nt, INIT)
-#undef INIT
-  return (int)hipGetLastError();
-}
-
-template <class W, class G>
-int mg_update_t(const TraceOp<W>& T, const Krylov<double>& v, const MgVecs<W>& mv, G g, int grid, hipStream_t s) {
-#define UPD(NT) hipLaunchKernelGGL((mg_update_kernel<NT, W, G>), dim3(grid), dim3(64 * NT), 0, s, T, v, mv, g);
-  MG_NT_DISPATCH(T.nt, UPD)
-#undef UPD
-  return (int)hipGetLastError();
-}
-
-template <class W>
-int launch_mg_init(const DevPattern& P, const TraceSystem& T64, const TraceOp<W>& T, const Krylov<double>& v,
-                   const MgVecs<W>& mv, hipStream_t s) {
-  return mg_init_t(P, T64, T, v, mv, Whole{T.N, v.st}, v.nblocks, s);
-}
-
-template <class W>
-int launch_mg_init_group(const DevPattern& P, const TraceSystem& T64, const TraceOp<W>& T, const Krylov<double>& v,
-                         const MgVecs<W>& mv, Grouped g, int grid, hipStream_t s) {
-  return mg_init_t(P, T64, T, v, mv, g, grid, s);
-}
-
-template <class W>
-int launch_mg_update(const TraceOp<W>& T, const Krylov<double>& v, const MgVecs<W>& mv, hipStream_t s) {
-  return mg_update_t(T, v, mv, Whole{T.N, v.st}, v.nblocks, s);
-}
-
-template <class W>
-int launch_mg_update_group(const TraceOp<W>& T, const Krylov<double>& v, const MgVecs<W>& mv, Grouped g, int grid,
-                           hipStream_t s) {
-  return mg_update_t(T, v, mv, g, grid, s);
-}
-
-// z = V-cycle(r), starting from e0 = omega Dinv r already in mv.e0; writes
-// the (r, z) partials of the next iteration.
-template <class W>
-int launch_mg_precond(const DevPattern& P, const TraceOp<W>& T, const Krylov<double>& v, const MgData& M,
-                      const MgData* dM, const MgVecs<W>& mv, hipStream_t s) {
-  const int gr = grid1(T.N, 256);
-  const int grows = gr > 16384 ? 16384 : gr;
-  if (!trace_op_ready(P, T)) return (int)hipErrorInvalidValue;
-#define RES(NT) hipLaunchKernelGGL((mg_resid0_kernel<NT, W>), dim3(grows), dim3(256), 0, s, P, T, v, mv, M.fc);
-  MG_NT_DISPATCH(T.nt, RES)
-#undef RES
-#define RST(NT) \
-  hipLaunchKernelGGL((mg_restrict0_kernel<NT, W>), dim3(grid1(M.lev[1].n)), dim3(256), 0, s, v, M, mv);
-  MG_NT_DISPATCH(T.nt, RST)
-#undef RST
-  int e = vcycle(M, dM, 1, v.st, s);
-  if (e) return e;
-#define SMO(NT) \
-  hipLaunchKernelGGL((mg_smooth0_kernel<NT, W, Whole>), dim3(v.nblocks), dim3(64 * NT), 0, s, T, v, M, mv, \
-                     Whole{T.N, v.st});
-  MG_NT_DISPATCH(T.nt, SMO)
-#undef SMO
-  return (int)hipGetLastError();
-}
-
-// Grouped: the residual and the restriction to level 1 run over the packed
-// mesh (every instance, no convergence check), the vertex levels through
-// the group's tables, the smoother per instance.
-template <class W>
-int launch_mg_precond_group(const DevPattern& P, const TraceOp<W>& T, const Krylov<double>& v, const MgData& Mu,
-                            const MgGroup& G, const MgVecs<W>& mv, Grouped g, int grid, hipStream_t s) {
-  Krylov<double> vu = v;
-  vu.st = nullptr;
-  const int gr = grid1(T.N, 256);
-  const int grows = gr > 8192 ? 8192 : gr;
-  if (!trace_op_ready(P, T)) return (int)hipErrorInvalidValue;
-#define RES(NT) hipLaunchKernelGGL((mg_resid0_kernel<NT, W>), dim3(grows), dim3(256), 0, s, P, T, vu, mv, Mu.fc);
-  MG_NT_DISPATCH(T.nt, RES)
-#undef RES
-#define RST(NT) \
-  hipLaunchKernelGGL((mg_restrict0_kernel<NT, W>), dim3(grid1(Mu.lev[1].n)), dim3(256), 0, s, vu, Mu, mv);
-  MG_NT_DISPATCH(T.nt, RST)
-#undef RST
-  int e = vcycle_group(G, s);
-  if (e) return e;
-#define SMO(NT) \
-  hipLaunchKernelGGL((mg_smooth0_kernel<NT, W, Grouped>), dim3(grid), dim3(64 * NT), 0, s, T, v, Mu, mv, g);
-  MG_NT_DISPATCH(T.nt, SMO)
-#undef SMO
-  return (int)hipGetLastError();
-}
-
-#define MG_INSTANTIATE(W)                                                                                      \
-  template int launch_mg_init<W>(const DevPattern&, const TraceSystem&, const TraceOp<W>&, const Krylov<double>&, \
-                                 const MgVecs<W>&, hipStream_t);                                                \
-  template int launch_mg_init_group<W>(const DevPattern&, const TraceSystem&, const TraceOp<W>&,                 \
-                                       const Krylov<double>&, const MgVecs<W>&, Grouped, int, hipStream_t);      \
-  template int launch_mg_update<W>(const TraceOp<W>&, const Krylov<double>&, const MgVecs<W>&, hipStream_t);   \
-  template int launch_mg_update_group<W>(const TraceOp<W>&, const Krylov<double>&, const MgVecs<W>&, Grouped,  \
-                                         int, hipStream_t);                                                     \
-  template int launch_mg_precond<W>(const DevPattern&, const TraceOp<W>&, const Krylov<double>&, const MgData&,  \
-                                    const MgData*, const MgVecs<W>&, hipStream_t);                              \
-  template int launch_mg_precond_group<W>(const DevPattern&, const TraceOp<W>&, const Krylov<double>&,           \
-                                          const MgData&, const MgGroup&, const MgVecs<W>&, Grouped, int,        \
-                                          hipStream_t);
-MG_INSTANTIATE(double)
-MG_INSTANTIATE(float)
-#undef MG_INSTANTIATE
+int launch_vcycle_group(const MgGroup& G, hipStream_t s) { return vcycle_group(G, s); }
 
 }  // namespace hdg

@@ -103,96 +103,34 @@ __global__ void rm_cells_kernel(RectMeshArgs a) {
     a.cell_inst[cl] = a.inst;
     a.cell_inst[cu] = a.inst;
   }
-  // face f (1-based, local): end points v1, v2, cells c1, c2 (0-based, global; -1 none)
-  auto setf = [&](int64_t f, int64_t v1, int64_t v2, int64_t c1, int64_t c2) {
+  // cells c1, c2 (0-based, global; -1 none) of face f (1-based, local)
+  auto setf = [&](int64_t f, int64_t c1, int64_t c2) {
     const int64_t F = a.face0 + f - 1;
     a.fcell[2 * F] = (int)c1;
     a.fcell[2 * F + 1] = (int)c2;
-    a.fv[2 * F] = (int)min(v1, v2);
-    a.fv[2 * F + 1] = (int)max(v1, v2);
   };
-  setf(fD, node(i + 1, j), node(i, j + 1), cl, cu);
-  if (i == 1) setf(fL, node(i, j + 1), node(i, j), cl, -1);
-  if (j == 1) setf(fB, node(i, j), node(i + 1, j), cl, -1);
-  setf(fT, node(i + 1, j + 1), node(i, j + 1), cu, j < a.ny ? a.cell0 + 2 * (j * a.nx + (i - 1)) : -1);
-  setf(fR, node(i + 1, j), node(i + 1, j + 1), cu, i < a.nx ? a.cell0 + 2 * ((j - 1) * a.nx + i) : -1);
+  setf(fD, cl, cu);
+  if (i == 1) setf(fL, cl, -1);
+  if (j == 1) setf(fB, cl, -1);
+  setf(fT, cu, j < a.ny ? a.cell0 + 2 * (j * a.nx + (i - 1)) : -1);
+  setf(fR, cu, i < a.nx ? a.cell0 + 2 * ((j - 1) * a.nx + i) : -1);
 }
 
 // A face with one cell must lie on a side of the box: both end points on
 // the bottom, right, top or left side, by exact coordinate equality
 // (_get_rectangular_boundary_sets, generate_mesh.jl:60-89); else bit 4 of
-// the error flag (HDG_ERR_BOUNDARY on the host).  Also the four vertices
-// around every face (lower, higher end point, opposite vertex of cell 1, of
-// cell 2 or cell 1 again).
+// the error flag (HDG_ERR_BOUNDARY on the host).
 __global__ void rm_faces_kernel(RectMeshArgs a) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= a.nf) return;
   const int64_t F = a.face0 + f;
-  const int lo = a.fv[2 * F], hi = a.fv[2 * F + 1];
-  const int c1 = a.fcell[2 * F], c2 = a.fcell[2 * F + 1];
-  if (c2 < 0) {
-    const double *p = a.xy + 2 * (int64_t)lo, *q = a.xy + 2 * (int64_t)hi;
-    const bool ok = (p[1] == a.y0 && q[1] == a.y0) || (p[0] == a.x1 && q[0] == a.x1) ||
-                    (p[1] == a.y1 && q[1] == a.y1) || (p[0] == a.x0 && q[0] == a.x0);
-    if (!ok) atomicOr(a.err, 4);
-  }
-  if (!a.fq4) return;
-  auto opp = [&](int c) {
-    int o = -1;
-    for (int w = 0; w < 3; ++w) {
-      const int nw = a.cn[3 * (int64_t)c + w];
-      if (nw != lo && nw != hi) o = nw;
-    }
-    return o;
-  };
-  const int o1 = opp(c1);
-  a.fq4[4 * F] = lo;
-  a.fq4[4 * F + 1] = hi;
-  a.fq4[4 * F + 2] = o1;
-  a.fq4[4 * F + 3] = c2 < 0 ? o1 : opp(c2);
-}
-
-// Vertex -> face lists: node (i, j) (0-based column, row) meets the faces
-// to its right, left, top and bottom neighbours and the two diagonal ones
-// that exist; listed in ascending face order, as the host builds them.
-__global__ void rm_vertex_faces_kernel(RectMeshArgs a) {
-  const int64_t nnx = a.nx + 1, nny = a.ny + 1;
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= nnx * nny) return;
-  const int64_t i0 = v % nnx, j0 = v / nnx;
-  const int64_t i = i0 + 1, j = j0 + 1;  // 1-based grid position
-  const SweepD S{a.nx, a.ny};
-  int64_t f[6];
-  int d = 0;
-  // edge along x from node (i, j) to (i + 1, j): bottom edge of cell (i, j)
-  // or, on the top row, top edge of cell (i, ny)
-  auto hedge = [&](int64_t ii) { return j <= a.ny ? S.B(ii, j) : S.T(ii, a.ny); };
-  // edge along y from (i, j) to (i, j + 1): left edge of cell (i, j) or, on
-  // the last column, right edge of cell (nx, j)
-  auto vedge = [&](int64_t jj) { return i <= a.nx ? S.L(i, jj) : S.R(a.nx, jj); };
-  if (i0 < a.nx) f[d++] = hedge(i);
-  if (i0 > 0) f[d++] = hedge(i - 1);
-  if (j0 < a.ny) f[d++] = vedge(j);
-  if (j0 > 0) f[d++] = vedge(j - 1);
-  if (i0 > 0 && j0 < a.ny) f[d++] = S.D(i - 1, j);
-  if (i0 < a.nx && j0 > 0) f[d++] = S.D(i, j - 1);
-  // ascending (insertion sort of at most 6)
-  for (int p = 1; p < d; ++p)
-    for (int q = p; q > 0 && f[q - 1] > f[q]; --q) {
-      const int64_t t = f[q];
-      f[q] = f[q - 1];
-      f[q - 1] = t;
-    }
-  // entries before node v: whole rows 0..j0-1, then columns 0..i0-1 of row j0
-  const int64_t nx = a.nx, ny = a.ny;
-  const int64_t rows = 2 * nx * j0 + (2 * nx + 1) * (min(j0, ny) + max(j0 - 1, (int64_t)0));
-  const int64_t top = j0 < ny, bot = j0 > 0;
-  const int64_t cols = min(i0, nx) + max(i0 - 1, (int64_t)0) + i0 * top + i0 * bot +
-                       max(i0 - 1, (int64_t)0) * top + min(i0, nx) * bot;
-  const int64_t p0 = 2 * a.face0 + rows + cols;
-  a.vf_ptr[a.node0 + v] = (int)p0;
-  for (int k = 0; k < d; ++k) a.vf_idx[p0 + k] = (int)(a.face0 + f[k] - 1);
-  if (a.last && v == nnx * nny - 1) a.vf_ptr[a.node0 + v + 1] = (int)(p0 + d);
+  if (a.fcell[2 * F + 1] >= 0) return;
+  const int64_t c = a.fcell[2 * F];
+  const int l = a.cf[3 * c] == F ? 0 : (a.cf[3 * c + 1] == F ? 1 : 2);
+  const double *p = a.xy + 2 * (int64_t)a.cn[3 * c + (l + 1) % 3], *q = a.xy + 2 * (int64_t)a.cn[3 * c + (l + 2) % 3];
+  const bool ok = (p[1] == a.y0 && q[1] == a.y0) || (p[0] == a.x1 && q[0] == a.x1) ||
+                  (p[1] == a.y1 && q[1] == a.y1) || (p[0] == a.x0 && q[0] == a.x0);
+  if (!ok) atomicOr(a.err, 4);
 }
 
 // Every dof of every face with one cell is prescribed, the others are free.
@@ -218,7 +156,6 @@ int launch_rect_mesh(const RectMeshArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(rm_nodes_kernel, dim3(blocks_for(nn)), dim3(256), 0, s, a);
   hipLaunchKernelGGL(rm_cells_kernel, dim3(blocks_for(a.nx * a.ny)), dim3(256), 0, s, a);
   hipLaunchKernelGGL(rm_faces_kernel, dim3(blocks_for(a.nf)), dim3(256), 0, s, a);
-  if (a.vf_ptr) hipLaunchKernelGGL(rm_vertex_faces_kernel, dim3(blocks_for(nn)), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -324,16 +324,23 @@ size_t hdg_server_footprint(const hdg_request* q) {
   const double nn = (nx + 1) * (ny + 1), nc = 2 * nx * ny, nf = nx + ny + 3 * nx * ny;
   const int k = q->opt.k, nu = (k + 1) * (k + 2) / 2, m = 3 * nu, nt = k + 1, ntr = 3 * nt;
   const double N = nf * nt;
-  // mesh, face pattern, vertex structures
-  double b = 16 * nn + 24 * nc + 8 * nf + 67 * nf + 32 * nf + 4 * nn;
+  // mesh, face pattern
+  double b = 16 * nn + 24 * nc + 8 * nf + 67 * nf;
+  // per-cell operators, trace solution and Dirichlet data
+  b += 8 * nc * ((double)ntr * ntr + ntr + (double)m * ntr + 2 * m) + N * (1 + 8 + 8);
+  if (q->opt.precond == HDG_PC_BLOCK_JACOBI) {
+    // assembled trace matrix (face-ELL at most) and rhs, Jacobi blocks, CG vectors
+    b += N * (8 * 5 * nt + 8 + 8 * nt + 6 * 8);
+  }
   // vertex hierarchy over ~4/3 nn nodes: 9-point stencil, inverse, three
   // vectors (13 doubles) and a mask byte per node
   b += (13.0 * 8 + 1) * nn * 4.0 / 3.0;
-  // per-cell operators, trace system, solver and multigrid trace-level data
-  b += 8 * nc * ((double)ntr * ntr + ntr + (double)m * ntr + 2 * m + 9);
-  b += N * (1 + 8 + 8 * 5 * nt + 8 + 8 * nt + 6 * 8 + 8 + 2 * 8 + 4 * 8);
+  if (q->opt.precond != HDG_PC_BLOCK_JACOBI) {
+    // the reduced trace system per grid point (hdg_quad.h)
+    b += nn * (8 * (8.0 * nt * nt + 37 * nt + 10) + 2);
+    if (q->opt.precision == HDG_MIXED) b += nn * 4 * (7.0 * nt * nt + 13 * nt);
+  }
   if (q->src.kind == HDG_SRC_VALUES) b += 8 * nc * 16;
-  if (q->opt.precision == HDG_MIXED) b += N * (4 * 5 * nt + 4 * nt + 4 * 4 + 4 * 4);
   // allocation granularity and small buffers
   return (size_t)(b * 1.05) + (8u << 20);
 }
