@@ -253,7 +253,6 @@ void free_mesh(hdg_ctx* c) {
   dfree(c, c->pat.self);
   dfree(c, c->pat.tslot);
   dfree(c, c->pat.nbr);
-  dfree(c, c->mg.tailpack);
   dfree(c, c->mg.cinv);
   for (int l = 0; l < kMaxLevels; ++l) {
     MgLevel& L = c->mg.lev[l];
@@ -262,7 +261,6 @@ void free_mesh(hdg_ctx* c) {
     dfree(c, L.mask);
     dfree(c, L.r);
     dfree(c, L.e);
-    dfree(c, L.t);
   }
   c->mg = MgData{};
   c->structured = false;
@@ -305,7 +303,7 @@ void mg_plan_levels(int nx, int ny, MgData& M) {
     L.ny = ly;
     L.n = (int64_t)(lx + 1) * (ly + 1);
     ++l;
-    if (std::max(lx, ly) <= 2 || l >= kMaxLevels) break;
+    if (L.n <= kCoarseDirect || l >= kMaxLevels) break;
     lx = (lx + 1) / 2;  // coarsening with a ragged end on odd sides
     ly = (ly + 1) / 2;
   }
@@ -335,14 +333,8 @@ int build_vertex_levels(hdg_ctx* c, int nx, int ny) {
     TRY(dalloc(c, &L.mask, L.n));
     TRY(dalloc(c, &L.r, L.n));
     TRY(dalloc(c, &L.e, L.n));
-    TRY(dalloc(c, &L.t, L.n));
   }
   TRY(dalloc(c, &M.cinv, (size_t)kCoarseDirect * kCoarseDirect));
-  if (M.tail < M.nlev) {
-    int64_t tn = 0;
-    for (int t = M.tail; t < M.nlev; ++t) tn += M.lev[t].n;
-    TRY(dalloc(c, &M.tailpack, (kStencil + 1) * tn));
-  }
   return HDG_OK;
 }
 
@@ -513,6 +505,8 @@ int setup_quad(hdg_ctx* c) {
     TRY(dalloc(c, &q.ftp, pts * quad_tp_vals(nt)));
   }
   TRY(dalloc(c, &c->d_plain, 1));
+  c->mg.part = q.part + 3 * (size_t)q.nbt;
+  c->mg.npart = I.nbM;
   TRY(dalloc(c, &c->d_mg, 1));
   HIPCHK(c, hipMemcpyAsync(c->d_mg, &c->mg, sizeof(MgData), hipMemcpyHostToDevice, c->stream));
   q.nt = nt;
@@ -547,8 +541,7 @@ int enqueue_chunk(hdg_ctx* c, double rtol2, int maxit) {
     if (use_mg(c)) {
       LAUNCHCHK(c, launch_quad_product(c->qs, c->ql, rtol2, maxit, c->stream));
       LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));
-      LAUNCHCHK(c, launch_quad_check(c->qs, c->ql, rtol2, maxit, c->stream));
-      LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, c->stream));
+      LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, rtol2, maxit, c->stream));
       LAUNCHCHK(c, launch_quad_smooth(c->qs, c->ql, mixed(c), c->stream));
     } else {
       LAUNCHCHK(c, launch_cg_spmv(c->pat, op64(c), kv64(c), 0, rtol2, maxit, 0, c->stream));
@@ -633,7 +626,7 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
     LAUNCHCHK(c, launch_quad_init(c->qs, c->ql, c->stream));
     if (fork) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
     LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));
-    LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, c->stream));
+    LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, 0.0, -1, c->stream));
     LAUNCHCHK(c, launch_quad_smooth(c->qs, c->ql, mixed(c), c->stream));
   } else {
     LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
@@ -653,7 +646,7 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
   bool behind = false;
   for (;;) {
     const int nxt = slot ^ 1;
-    behind = nread < 2 || !chunk_converges(prev, last, chunk_of(c) + (use_mg(c) ? 1 : 0), rtol2);
+    behind = nread < 2 || !chunk_converges(prev, last, chunk_of(c), rtol2);
     if (behind) {
       TRY(launch_chunk(c, nxt, rtol2, maxit));
       HIPCHK(c, hipEventRecord(evs[nxt], c->stream));
@@ -959,7 +952,6 @@ int hdg_setup(hdg_ctx* c, const hdg_options* opt) {
   free_problem(c);
   c->opt = o;
   c->k = o.k;
-  mg_order_choices(o.k, c->mg);
   c->nu = tab.lay.nu;
   c->nq = 2 * c->nu;
   c->m = 3 * c->nu;

@@ -38,12 +38,11 @@ struct Inst {
   int64_t node0 = 0, cell0 = 0, face0 = 0, row0 = 0;
   MgData plan;                        // level sizes and tail (host plan)
   int64_t lev_off[kMaxLevels] = {0};  // offset of its nodes in the group's level-l buffer
-  int64_t tail_off = 0;               // offset of its LDS image in the group's tailpack
 };
 
 struct LevelBuf {
   int64_t n = 0;  // nodes of every instance at this level
-  double *a = nullptr, *dinv = nullptr, *r = nullptr, *e = nullptr, *t = nullptr;
+  double *a = nullptr, *dinv = nullptr, *r = nullptr, *e = nullptr;
   unsigned char* mask = nullptr;
 };
 
@@ -314,6 +313,10 @@ int build_quad_group(hdg_batch* b, Group& g) {
   q.Ate = g.Ate;
   q.bte = g.bte;
   q.P = g.pat;
+  for (int j = 0; j < n; ++j) {
+    g.Mi[j].part = q.part + 3 * (size_t)q.nbt + inst[j].pM;
+    g.Mi[j].npart = inst[j].nbM;
+  }
   QuadLaunch& L = g.ql;
   QuadInst* di;
   BlockMap *dM, *dE, *dQ;
@@ -516,26 +519,15 @@ int build_group(hdg_batch* b, Group& g) {
     BTRY(galloc(b, g, &B.mask, off));
     BTRY(galloc(b, g, &B.r, off));
     BTRY(galloc(b, g, &B.e, off));
-    BTRY(galloc(b, g, &B.t, off));
   }
-  int64_t tailn = 0;
-  for (Inst& I : g.in) {
-    I.tail_off = tailn;
-    for (int t = I.plan.tail; t < I.plan.nlev; ++t) tailn += (kStencil + 1) * I.plan.lev[t].n;
-  }
-  double *cinv, *tailpack;
+  double* cinv;
   BTRY(galloc(b, g, &cinv, (size_t)n * kCoarseDirect * kCoarseDirect));
-  BTRY(galloc(b, g, &tailpack, tailn));
-  MgData choice;
-  mg_order_choices(g.k, choice);  // as hdg_setup chooses for a single problem
   g.Mi.assign(n, MgData{});
   for (int j = 0; j < n; ++j) {
     const Inst& I = g.in[j];
     MgData& M = g.Mi[j];
     M = I.plan;
-    M.vsweeps = choice.vsweeps;
     M.cinv = cinv + (size_t)j * kCoarseDirect * kCoarseDirect;
-    M.tailpack = tailpack + I.tail_off;
     for (int l = 1; l < M.nlev; ++l) {
       MgLevel& V = M.lev[l];
       const LevelBuf& B = g.lev[l];
@@ -545,16 +537,15 @@ int build_group(hdg_batch* b, Group& g) {
       V.mask = B.mask + o;
       V.r = B.r + o;
       V.e = B.e + o;
-      V.t = B.t + o;
     }
   }
+  BTRY(build_quad_group(b, g));
   BTRY(upload(b, g, &g.dMi, g.Mi));
   MgGroup& G = g.G;
   G.ninst = n;
   G.dM = g.dMi;
   G.st = g.st;
   G.ndepth = ndepth;
-  G.vsweeps = choice.vsweeps;
   G.omega_v = g.Mi[0].omega_v;
   for (int d = 1; d < ndepth; ++d) {
     std::vector<VRec> rec;
@@ -563,8 +554,8 @@ int build_group(hdg_batch* b, Group& g) {
       const MgData& M = g.Mi[j];
       if (d >= M.tail) continue;
       const int p = (int)rec.size();
-      rec.push_back(VRec{M.lev[d], M.lev[d + 1], g.st + j});
-      const int64_t bn = (M.lev[d].n + 255) / 256, br = (8 * M.lev[d + 1].n + 255) / 256;
+      rec.push_back(VRec{M.lev[d], M.lev[d + 1], g.st + j, M.part, M.npart});
+      const int64_t bn = v_post_blocks(M.lev[d]), br = v_restrict_blocks(M.lev[d + 1]);
       for (int64_t u = 0; u < bn; ++u) node.push_back(BlockMap{p, (int)u});
       for (int64_t u = 0; u < br; ++u) res.push_back(BlockMap{p, (int)u});
     }
@@ -578,33 +569,28 @@ int build_group(hdg_batch* b, Group& g) {
     G.gnode[d] = (int)node.size();
     G.gres[d] = (int)res.size();
   }
-  BTRY(build_quad_group(b, g));
   BTRY(tune_group(b, g));
-  // set-up tables: cmask / RAP for every level pair
+  // set-up tables: RAP for every level pair down to the tails
   MgSetupGroup& S = g.S;
   S.ninst = n;
   S.dM = g.dMi;
-  S.ndepth = maxlev - 1;
+  S.ndepth = ndepth;
   for (int d = 1; d < S.ndepth; ++d) {
     std::vector<VRec> rec;
-    std::vector<BlockMap> cm, rp;
+    std::vector<BlockMap> rp;
     for (int j = 0; j < n; ++j) {
       const MgData& M = g.Mi[j];
-      if (d + 1 >= M.nlev) continue;
+      if (d >= M.tail) continue;
       const int p = (int)rec.size();
-      rec.push_back(VRec{M.lev[d], M.lev[d + 1], nullptr});
-      const int64_t bc = (M.lev[d + 1].n + 255) / 256, br = (8 * M.lev[d + 1].n + 255) / 256;
-      for (int64_t u = 0; u < bc; ++u) cm.push_back(BlockMap{p, (int)u});
+      rec.push_back(VRec{M.lev[d], M.lev[d + 1], nullptr, nullptr, 0});
+      const int64_t br = (8 * M.lev[d + 1].n + 255) / 256;
       for (int64_t u = 0; u < br; ++u) rp.push_back(BlockMap{p, (int)u});
     }
     VRec* drec;
-    BlockMap *dcm, *drp;
+    BlockMap* drp;
     BTRY(upload(b, g, &drec, rec));
-    BTRY(upload(b, g, &dcm, cm));
     BTRY(upload(b, g, &drp, rp));
-    S.cmask[d] = VGroup{drec, dcm};
     S.rap[d] = VGroup{drec, drp};
-    S.gcmask[d] = (int)cm.size();
     S.grap[d] = (int)rp.size();
   }
   BHIP(b, hipStreamSynchronize(g.s));  // the host arrays go out of scope
@@ -644,7 +630,7 @@ int enqueue_setup(hdg_batch* b, Group& g) {
   BLAUNCH(b, launch_quad_omega(g.qs, g.ql, quad_omega_factor(g.k), kQuadLanczos, g.s));
   BLAUNCH(b, launch_quad_init(g.qs, g.ql, g.s));
   BLAUNCH(b, launch_quad_residual(g.qs, g.ql, g.mixed, g.s));
-  BLAUNCH(b, launch_vcycle_group(g.G, g.s));
+  BLAUNCH(b, launch_vcycle_group(g.G, 0.0, -1, g.s));
   BLAUNCH(b, launch_quad_smooth(g.qs, g.ql, g.mixed, g.s));
   return HDG_OK;
 }
@@ -659,8 +645,7 @@ int enqueue_chunk(hdg_batch* b, Group& g) {
     if (g.mg) {
       BLAUNCH(b, launch_quad_product(g.qs, g.ql, rtol2_of(g), maxit_of(g), g.s));
       BLAUNCH(b, launch_quad_residual(g.qs, g.ql, g.mixed, g.s));
-      BLAUNCH(b, launch_quad_check(g.qs, g.ql, rtol2_of(g), maxit_of(g), g.s));
-      BLAUNCH(b, launch_vcycle_group(g.G, g.s));
+      BLAUNCH(b, launch_vcycle_group(g.G, rtol2_of(g), maxit_of(g), g.s));
       BLAUNCH(b, launch_quad_smooth(g.qs, g.ql, g.mixed, g.s));
     } else {
       BLAUNCH(b, launch_cg_spmv_t(g.pat, op64(g), kv(g), gr, g.nbt, 0, rtol2_of(g), maxit_of(g), 0, g.s));
@@ -846,7 +831,7 @@ int run_group(hdg_batch* b, Group& g, std::chrono::steady_clock::time_point t0) 
     const int nxt = slot ^ 1;
     behind = nread < 2;
     for (size_t j = 0; j < n && !behind; ++j)
-      behind = !chunk_converges(prev[j], last[j], chunk_iters(g) + (g.mg ? 1 : 0), rtol2_of(g));
+      behind = !chunk_converges(prev[j], last[j], chunk_iters(g), rtol2_of(g));
     if (behind) BTRY(launch_chunk(b, g, nxt));
     BHIP(b, hipEventSynchronize(g.ev[slot]));
     prev.swap(last);

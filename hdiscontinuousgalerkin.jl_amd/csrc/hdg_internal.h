@@ -153,9 +153,8 @@ struct CgState {
 // behind the one whose read-back they wait for.  From two read-backs of an
 // instance's state (prev, then last) the per-iteration log-rate of (r, r)
 // forecasts whether the chunk now running reaches (r, r) <= rtol2 (b, b) at
-// its last test, n iterations past last.it: the chunk's length, plus one
-// where a convergence test follows each multigrid update (the read-back
-// holds the product's test of the iteration before).  When it should, the
+// its last test, n iterations past last.it (the chunk's length).  When it
+// should, the
 // loop queues nothing behind it (a chunk there would only run launches that
 // return at once).  A wrong forecast costs one read-back round trip; the
 // launches that do work and their results are the same either way.
@@ -392,47 +391,37 @@ struct MgLevel {
   double* a = nullptr;           // stencils, a[s*n + v], s < kStencil
   double* dinv = nullptr;        // 1 / a[0], 0 on fixed nodes
   unsigned char* mask = nullptr; // fixed (Dirichlet) nodes
-  double *r = nullptr, *e = nullptr, *t = nullptr;
+  double *r = nullptr, *e = nullptr;
 };
-constexpr int kMaxLevels = 16;
+constexpr int kMaxLevels = 28;
 // points of the vertex-level stencils (slots listed in hdg_mg.hip)
 constexpr int kStencil = 9;
-// node budget of the levels solved inside one workgroup: their stencils,
-// diagonal inverses and three vectors live in LDS (13 doubles per node,
-// 156 KB of the CU's 160 KB), so that the 33 x 33 grid of a 1024- or
-// 512-cell side runs there instead of in 2-4 launches of its own (1024^2
-// P3 step -0.45 ms, 512^2 P2 -0.26 ms against 512 nodes, 53 KB); 1024
-// threads, one workgroup per CU
+// node budget of the levels solved inside one workgroup (two nodes per
+// thread), so that the 33 x 33 grid of a 1024- or 512-cell side runs there
+// instead of in launches of its own
 constexpr int kTailNodes = 1536;
 constexpr int kTailThreads = 1024;
-// coarsest grids up to this many nodes are solved exactly (inverse at set-up)
-constexpr int kCoarseDirect = 16;
+// coarsening stops at this many nodes, solved exactly (inverse at set-up)
+constexpr int kCoarseDirect = 96;
 struct MgData {
   int nlev = 0;                  // levels 1..nlev-1 are vertex grids
   int nx = 0, ny = 0;
   MgLevel lev[kMaxLevels];
   int tail = kMaxLevels;         // levels tail..nlev-1 run in one workgroup (LDS)
   double* cinv = nullptr;        // [kCoarseDirect^2] inverse of the coarsest operator (row-major)
-  double* tailpack = nullptr;    // stencils (9 n) and dinv (n) of levels tail.. back to back,
-                                 // the LDS image the tail kernel loads
+  const double* part = nullptr;  // the update's (r, r) partial sums, for the convergence test
+  int npart = 0;
   double omega_v = 0.7;          // vertex-level Jacobi weight
-  int coarse_sweeps = 20;
-  int vsweeps = 2;               // pre- and post-smoothing sweeps on the vertex levels (1 or 2)
 };
-// per-order choices of the V-cycle, shared by single problems and batches:
-// V(1,1) on the vertex levels for k <= 3, V(2,2) at k = 4 (fewest CG
-// iterations x cost per iteration measured on 256..1536 meshes: at k = 3
-// V(1,1) takes one iteration more and two launches fewer per level, 256^2
-// 6.40 -> 5.90 ms, 512^2 16.8 -> 16.0, 1024^2 58.6 -> 57.9, 1536^2 even;
-// at k = 4 1024^2 loses 147 -> 150 ms)
-inline void mg_order_choices(int k, MgData& M) { M.vsweeps = k <= 3 ? 1 : 2; }
 
 // A fine level, the next coarser one and the CG state of one instance: the
 // unit of a vertex-level kernel.  VOne launches one instance over the whole
 // grid; VGroup maps each block to (instance, block of that instance).
 struct VRec {
   MgLevel F, C;
-  const CgState* st;
+  CgState* st;
+  const double* part;  // MgData::part
+  int npart;
 };
 struct BlockMap {
   int inst, lb;
@@ -555,7 +544,7 @@ int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s);
 
 // Launch tables of the multigrid preconditioner of a group of instances:
 // per vertex depth d (1 <= d < ndepth), the instances whose level d lies
-// above their one-workgroup tail, with block maps for the fine-node kernels
+// above their one-workgroup tail, with block maps for the post-smoothing
 // (node, gnode blocks) and the restriction (res, gres blocks); then one
 // tail workgroup per instance.
 struct MgGroup {
@@ -567,18 +556,18 @@ struct MgGroup {
   int gnode[kMaxLevels];
   VGroup res[kMaxLevels];
   int gres[kMaxLevels];
-  int vsweeps = 2;
   double omega_v = 0.7;
 };
-// Set-up tables of a group's vertex hierarchies: per depth d, the instances
-// with a level d+1, with block maps over the coarse nodes (cmask) and 8 lanes
-// per coarse node (RAP).
+// blocks of the level kernels over one instance's level
+int v_restrict_blocks(const MgLevel& C);
+int v_post_blocks(const MgLevel& F);
+// Set-up tables of a group's vertex hierarchies: per depth d below their
+// tails, the instances with a level d+1, with block maps over 8 lanes per
+// coarse node (RAP).
 struct MgSetupGroup {
   int ninst = 0;
   const MgData* dM = nullptr;
   int ndepth = 1;
-  VGroup cmask[kMaxLevels];
-  int gcmask[kMaxLevels];
   VGroup rap[kMaxLevels];
   int grap[kMaxLevels];
 };

@@ -105,11 +105,10 @@ int launch_quad_l1(const QuadSys& S, const QuadLaunch& L, hipStream_t s);
 int launch_quad_omega(const QuadSys& S, const QuadLaunch& L, double factor, int steps, hipStream_t s);
 int launch_quad_init(const QuadSys& S, const QuadLaunch& L, hipStream_t s);
 // CG product with the convergence test; update and level-0 residual with the
-// restriction to the vertices; convergence test; post-smoothing.  W selects
-// the preconditioner's storage.
+// restriction to the vertices; post-smoothing.  mixed selects the
+// preconditioner's storage.
 int launch_quad_product(const QuadSys& S, const QuadLaunch& L, double rtol2, int maxit, hipStream_t s);
 int launch_quad_residual(const QuadSys& S, const QuadLaunch& L, bool mixed, hipStream_t s);
-int launch_quad_check(const QuadSys& S, const QuadLaunch& L, double rtol2, int maxit, hipStream_t s);
 int launch_quad_smooth(const QuadSys& S, const QuadLaunch& L, bool mixed, hipStream_t s);
 // uhat (natural numbering) with the diagonals' solution; with out, also
 // ||K uhat - rhs||^2 over the free dofs of every instance
@@ -122,8 +121,9 @@ int launch_quad_time(const QuadSys& S, const QuadLaunch& L, int which, hipStream
 double quad_omega_factor(int k);
 constexpr int kQuadLanczos = 4;
 
-// V-cycle on the vertex levels
-int launch_vcycle(const MgData& M, const MgData* dM, const CgState* st, hipStream_t s);
-int launch_vcycle_group(const MgGroup& G, hipStream_t s);
+// V-cycle on the vertex levels, the next product's convergence test first
+// (maxit < 0: none)
+int launch_vcycle(const MgData& M, const MgData* dM, CgState* st, double rtol2, int maxit, hipStream_t s);
+int launch_vcycle_group(const MgGroup& G, double rtol2, int maxit, hipStream_t s);
 
 }  // namespace hdg

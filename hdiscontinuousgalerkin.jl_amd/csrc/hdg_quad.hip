@@ -875,23 +875,22 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
       st->lz[it] = rz;
     }
   } else if (!force) {
-    const double rr = psum(S.part + nbt * 3 + I.pM, I.nbM, sh);
-    const double bb = it == 1 ? psum(S.part + nbt * 4 + I.pE, I.nbE, sh) : st->bb;
-    const bool conv = rr <= rtol2 * bb;
-    if (conv || it - 1 >= maxit) {
+    // the first vertex kernel takes the convergence test after every update;
+    // the initial residual is tested here
+    if (it == 1) {
+      const double rr = psum(S.part + nbt * 3 + I.pM, I.nbM, sh);
+      const double bb = psum(S.part + nbt * 4 + I.pE, I.nbE, sh);
+      const bool conv = rr <= rtol2 * bb;
       if (lead) {
-        st->done = conv ? 1 : 2;
-        st->it = it - 1;
+        st->it = 0;
         st->rr = rr;
         st->bb = bb;
+        if (conv || maxit < 1) st->done = conv ? 1 : 2;
       }
-      return;
+      if (conv || maxit < 1) return;
     }
     if (lead) {
       st->rz[it & 1] = rz;
-      st->it = it - 1;
-      st->rr = rr;
-      if (it == 1) st->bb = bb;
       st->i_upd = it;
     }
   }
@@ -1246,25 +1245,6 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
   if (threadIdx.x == 0) S.part[nbt * 3 + I.pM + lb] = t;
 }
 
-// the next product's convergence test right after the update, so that a
-// converged solve skips its last V-cycle
-template <class Sel>
-__global__ __launch_bounds__(kQuadThreads) void q_check_kernel(QuadSys S, Sel sel, double rtol2, int maxit) {
-  __shared__ double sh[kNW];
-  const QuadInst& I = inst_block(sel);
-  CgState* st = I.st;
-  if (st->done) return;
-  const int it = st->i_pre + 1;
-  const double rr = psum(S.part + (size_t)S.nbt * 3 + I.pM, I.nbM, sh);
-  const double bb = st->bb;
-  const bool conv = rr <= rtol2 * bb;
-  if ((conv || it - 1 >= maxit) && threadIdx.x == 0) {
-    st->done = conv ? 1 : 2;
-    st->it = it - 1;
-    st->rr = rr;
-  }
-}
-
 // z = P e1 + omega Dinv (r + res - (T P) e1), pointwise (hdg_quad.h)
 template <int NT, class W, class Sel>
 __global__ __launch_bounds__(kQuadThreads) void q_smooth_kernel(QuadSys S, Sel sel, const W* __restrict__ tp,
@@ -1607,10 +1587,6 @@ int launch_quad_residual(const QuadSys& S, const QuadLaunch& L, bool mixed, hipS
 int launch_quad_smooth(const QuadSys& S, const QuadLaunch& L, bool mixed, hipStream_t s) {
   return mixed ? smooth_t<float>(S, S.ftp, S.fDinv, L, s) : smooth_t<double>(S, S.tp, S.Dinv, L, s);
 }
-int launch_quad_check(const QuadSys& S, const QuadLaunch& L, double rtol2, int maxit, hipStream_t s) {
-  return go(L, nullptr, L.ninst, s, q_check_kernel<SelGroup>, q_check_kernel<SelOne>, S, rtol2, maxit);
-}
-
 int launch_quad_finish(const QuadSys& S, const QuadLaunch& L, double* uhat, double* out, hipStream_t s) {
   const int resid = out && !S.from_k ? 1 : 0;
 #define FIN(NT) QTRY(GO1(Q, q_finish_kernel, NT, uhat, resid));

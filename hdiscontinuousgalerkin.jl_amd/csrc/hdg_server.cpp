@@ -332,9 +332,9 @@ size_t hdg_server_footprint(const hdg_request* q) {
     // assembled trace matrix (face-ELL at most) and rhs, Jacobi blocks, CG vectors
     b += N * (8 * 5 * nt + 8 + 8 * nt + 6 * 8);
   }
-  // vertex hierarchy over ~4/3 nn nodes: 9-point stencil, inverse, three
-  // vectors (13 doubles) and a mask byte per node
-  b += (13.0 * 8 + 1) * nn * 4.0 / 3.0;
+  // vertex hierarchy over ~4/3 nn nodes: 9-point stencil, inverse, two
+  // vectors (12 doubles) and a mask byte per node
+  b += (12.0 * 8 + 1) * nn * 4.0 / 3.0;
   if (q->opt.precond != HDG_PC_BLOCK_JACOBI) {
     // the reduced trace system per grid point (hdg_quad.h)
     b += nn * (8 * (8.0 * nt * nt + 37 * nt + 10) + 2);
