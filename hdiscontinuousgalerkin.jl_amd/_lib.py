@@ -39,7 +39,7 @@ EXPORTS = (
     "hdg_batch_create", "hdg_batch_run", "hdg_batch_trace", "hdg_batch_info", "hdg_batch_destroy",
     "hdg_batch_last_error", "hdg_autotune", "hdg_set_schedule", "hdg_set_rectangle_mesh",
     "hdg_set_dirichlet_boundary", "hdg_errornorm_noalloc", "hdg_set_dirichlet_function",
-    "hdg_get_applied_system", "hdg_refine_probe",
+    "hdg_get_applied_system", "hdg_refine_probe", "hdg_get_system32", "hdg_recover_rows",
 )
 
 
@@ -109,7 +109,7 @@ class ServerSummary(C.Structure):
 
 _lib = None
 _P = C.POINTER
-_d, _i64, _i8 = _P(C.c_double), _P(C.c_int64), _P(C.c_int8)
+_d, _i64, _i32, _i8 = _P(C.c_double), _P(C.c_int64), _P(C.c_int32), _P(C.c_int8)
 _ctx = C.c_void_p
 
 
@@ -142,12 +142,14 @@ def _declare(L):
         "hdg_query_sizes": (C.c_int, [_ctx, _P(Sizes)]),
         "hdg_assemble_condense": (C.c_int, [_ctx]),
         "hdg_get_system": (C.c_int, [_ctx, _i64, _i64, _d, _d]),
+        "hdg_get_system32": (C.c_int, [_ctx, _i32, _i32, _d, _d]),
         "hdg_get_local_ops": (C.c_int, [_ctx, _d, _d]),
         "hdg_get_condensed": (C.c_int, [_ctx, _d, _d]),
         "hdg_get_element_blocks": (C.c_int, [_ctx, C.c_int64, C.c_int64] + [_d] * 7),
         "hdg_solve": (C.c_int, [_ctx, _d, _P(SolveInfo)]),
         "hdg_set_trace": (C.c_int, [_ctx, _d]),
         "hdg_recover": (C.c_int, [_ctx, _d, _d, _d]),
+        "hdg_recover_rows": (C.c_int, [_ctx, _d, _d, _d]),
         "hdg_errornorm": (C.c_int, [_ctx, C.c_int, _d, _d]),
         "hdg_errornorm_noalloc": (C.c_int, [C.c_int, C.c_int, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p,
                                             C.c_int, _d, C.c_void_p, C.c_void_p]),

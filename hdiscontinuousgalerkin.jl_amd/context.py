@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib as L
-from ._lib import check, lib, ptr, _i64
+from ._lib import check, lib, ptr, _i32, _i64
 
 
 class Context:
@@ -104,10 +104,10 @@ class Context:
         """apply!(K, b, dbc) on the device: (colptr, rowval, nzval, rhs,
         meandiag) of the applied system, Julia's CSC, 1-based."""
         s = self.sizes
-        colptr = np.zeros(s.n_dofs + 1, dtype=np.int64)
-        rowval = np.zeros(s.nnz, dtype=np.int64)
-        nzval = np.zeros(s.nnz)
-        rhs = np.zeros(s.n_dofs)
+        colptr = np.empty(s.n_dofs + 1, dtype=np.int64)
+        rowval = np.empty(s.nnz, dtype=np.int64)
+        nzval = np.empty(s.nnz)
+        rhs = np.empty(s.n_dofs)
         md = np.zeros(1)
         self._chk(lib().hdg_get_applied_system(self._h, ptr(colptr, _i64), ptr(rowval, _i64), ptr(nzval),
                                                ptr(rhs), ptr(md)))
@@ -125,26 +125,36 @@ class Context:
     def get_system(self):
         """(colptr, rowval, nzval, rhs): Julia's CSC of K, 1-based."""
         s = self.sizes
-        colptr = np.zeros(s.n_dofs + 1, dtype=np.int64)
-        rowval = np.zeros(s.nnz, dtype=np.int64)
-        nzval = np.zeros(s.nnz)
-        rhs = np.zeros(s.n_dofs)
+        colptr = np.empty(s.n_dofs + 1, dtype=np.int64)
+        rowval = np.empty(s.nnz, dtype=np.int64)
+        nzval = np.empty(s.nnz)
+        rhs = np.empty(s.n_dofs)
         self._chk(lib().hdg_get_system(self._h, ptr(colptr, _i64), ptr(rowval, _i64), ptr(nzval),
                                        ptr(rhs)))
         return colptr, rowval, nzval, rhs
 
     def get_system_scipy(self):
         import scipy.sparse as sp
-        colptr, rowval, nzval, rhs = self.get_system()
-        n = self.sizes.n_dofs
-        return sp.csc_matrix((nzval, rowval - 1, colptr - 1), shape=(n, n)), rhs
+        s = self.sizes
+        n = s.n_dofs
+        if max(n, s.nnz) < 2 ** 31 - 1:  # scipy's own choice of index type
+            indptr = np.empty(n + 1, dtype=np.int32)
+            indices = np.empty(s.nnz, dtype=np.int32)
+            data = np.empty(s.nnz)
+            rhs = np.empty(n)
+            self._chk(lib().hdg_get_system32(self._h, ptr(indptr, _i32), ptr(indices, _i32), ptr(data), ptr(rhs)))
+        else:
+            indptr, indices, data, rhs = self.get_system()
+            indptr -= 1
+            indices -= 1
+        return sp.csc_matrix((data, indices, indptr), shape=(n, n)), rhs
 
     def get_local_ops(self):
         """K_element (nc, m, ntr) and b_element (nc, m)."""
         s = self.sizes
         nc = s.n_cells
-        Ke = np.zeros((nc, s.ntr, s.m))
-        be = np.zeros((nc, s.m))
+        Ke = np.empty((nc, s.ntr, s.m))
+        be = np.empty((nc, s.m))
         self._chk(lib().hdg_get_local_ops(self._h, ptr(Ke), ptr(be)))
         return Ke.transpose(0, 2, 1), be
 
@@ -152,8 +162,8 @@ class Context:
         """Ate (nc, ntr, ntr) and bte (nc, ntr)."""
         s = self.sizes
         nc = s.n_cells
-        At = np.zeros((nc, s.ntr, s.ntr))
-        bt = np.zeros((nc, s.ntr))
+        At = np.empty((nc, s.ntr, s.ntr))
+        bt = np.empty((nc, s.ntr))
         self._chk(lib().hdg_get_condensed(self._h, ptr(At), ptr(bt)))
         return At.transpose(0, 2, 1), bt
 
@@ -169,13 +179,13 @@ class Context:
 
     def solve(self, return_uhat=True):
         info = L.SolveInfo()
-        uh = np.zeros(self.sizes.n_dofs) if return_uhat else None
+        uh = np.empty(self.sizes.n_dofs) if return_uhat else None
         self._chk(lib().hdg_solve(self._h, ptr(uh), C.byref(info)))
         return uh, info
 
     def trace(self):
         """The trace solution of the last solve / run (hdg_get_trace)."""
-        u = np.zeros(self.sizes.n_dofs)
+        u = np.empty(self.sizes.n_dofs)
         self._chk(lib().hdg_get_trace(self._h, ptr(u)))
         return u
 
@@ -187,11 +197,23 @@ class Context:
         """q (nc, nq), u (nc, nu), uhat_cell (nc, nt, 3), as m_values."""
         s = self.sizes
         nc = s.n_cells
-        q = np.zeros((s.nq, nc))
-        u = np.zeros((s.nu, nc))
-        uc = np.zeros((3, s.nt, nc))
+        q = np.empty((s.nq, nc))
+        u = np.empty((s.nu, nc))
+        uc = np.empty((3, s.nt, nc))
         self._chk(lib().hdg_recover(self._h, ptr(q), ptr(u), ptr(uc)))
         return q.T, u.T, uc.transpose(2, 1, 0)
+
+    def recover_into(self, q, u, uhat_cell):
+        """recover() into the caller's m_values arrays."""
+        s = self.sizes
+        nc = s.n_cells
+        out = (q, (nc, s.nq)), (u, (nc, s.nu)), (uhat_cell, (nc, s.nt, 3))
+        if all(type(a) is np.ndarray and a.dtype == np.float64 and a.shape == shp and a.flags.carray
+               for a, shp in out):
+            self._chk(lib().hdg_recover_rows(self._h, ptr(q), ptr(u), ptr(uhat_cell)))
+        else:
+            for (a, _), v in zip(out, self.recover()):
+                a[:] = v
 
     def errornorm(self, kind=L.UEX_SINSIN, par=None):
         out = np.zeros(1)

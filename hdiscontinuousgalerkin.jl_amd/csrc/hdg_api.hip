@@ -41,7 +41,6 @@ struct hdg_ctx {
   // mesh
   bool has_mesh = false;
   DevMesh mesh;
-  std::vector<int> h_cf;  // face ids per cell, 0-based
   int64_t nblock_cols = 0;  // stored nt x nt blocks of K
   DevPattern pat;
   bool structured = false;  // cells follow rectangle_mesh's (nx, ny) numbering
@@ -99,6 +98,9 @@ struct hdg_ctx {
   CondenseSched csched;
   bool tuned = false;
   double tuned_us = 0.0, default_us = 0.0;
+
+  // pinned memory of results on their way to the caller
+  HostStage stage;
 
   bool assembled = false, solved = false, recovered = false;
 };
@@ -716,6 +718,41 @@ int recover_impl(hdg_ctx* c) {
   return HDG_OK;
 }
 
+int recover_out(hdg_ctx* c, bool rows, double* q, double* u, double* uhat_cell) {
+  if (!c) return HDG_ERR_ARG;
+  TRY(select_device(c));
+  if (!c->recovered) TRY(recover_impl(c));
+  LAUNCHCHK(c, staged_values(c->stage, c->stream, c->k, c->mesh, c->d_qu, c->d_uhat, rows, q, u, uhat_cell));
+  return HDG_OK;
+}
+
+// CSC of K from a face-ELL value array, with an rhs in device memory
+template <class I>
+int export_csc(hdg_ctx* c, const double* d_vals, const double* d_rhs, int base, I* colptr, I* rowval, double* nzval,
+               double* rhs) {
+  LAUNCHCHK(c, staged_csc(c->stage, c->stream, c->pat, c->nt, c->mesh.nf, d_vals, base, colptr, rowval, nzval));
+  if (rhs) LAUNCHCHK(c, staged_copy(c->stage, c->stream, rhs, d_rhs, c->T.N));
+  return HDG_OK;
+}
+
+template <class I>
+int system_out(hdg_ctx* c, int base, I* colptr, I* rowval, double* nzval, double* rhs) {
+  if (!c) return HDG_ERR_ARG;
+  if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
+  TRY(select_device(c));
+  TRY(ensure_system(c));
+  if (!c->T.blk || !nzval) return export_csc(c, c->T.vals, c->T.rhs, base, colptr, rowval, nzval, rhs);
+  double* vals = nullptr;
+  TRY(dalloc(c, &vals, (size_t)kSlots * c->nt * c->T.N));
+  int r = HDG_OK;
+  const int e = launch_expand_ell(c->pat, c->T, vals, c->stream);
+  if (e) r = fail(c, HDG_ERR_HIP, "expanding the trace blocks: %s", hipGetErrorString((hipError_t)e));
+  if (r == HDG_OK) r = export_csc(c, vals, c->T.rhs, base, colptr, rowval, nzval, rhs);
+  (void)hipStreamSynchronize(c->stream);
+  dfree(c, vals);
+  return r;
+}
+
 }  // namespace
 
 extern "C" {
@@ -773,6 +810,7 @@ void hdg_destroy(hdg_ctx* c) {
     dfree(c, p);
   }
   if (c->h_st) (void)hipHostFree(c->h_st);
+  stage_free(c->stage);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->aux) {
@@ -853,7 +891,6 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
   TRY(dalloc(c, &c->pat.nbr, 4 * nf));
   LAUNCHCHK(c, launch_pattern(c->mesh, c->pat, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  c->h_cf.swap(cf);
   c->nblock_cols = nblk;
   int nx = 0, ny = 0;
   c->structured = detect_structured(nn, nc, cells, &nx, &ny);
@@ -921,7 +958,6 @@ int hdg_set_rectangle_mesh(hdg_ctx* c, int64_t nx, int64_t ny, double x0, double
     free_mesh(c);
     return fail(c, HDG_ERR_BOUNDARY, "a boundary face lies on no side of the box (generate_mesh.jl:80)");
   }
-  c->h_cf.clear();  // downloaded when an export needs it
   const int64_t nbdry = 2 * nx + 2 * ny;
   c->nblock_cols = 5 * (nf - nbdry) + 3 * nbdry;
   c->structured = true;
@@ -1138,8 +1174,7 @@ int hdg_solve(hdg_ctx* c, double* uhat_out, hdg_solve_info* info) {
   int r = solve_impl(c, info);
   if (r != HDG_OK && r != HDG_ERR_NOT_CONVERGED) return r;
   if (uhat_out) {
-    HIPCHK(c, hipMemcpyAsync(uhat_out, c->d_uhat, sizeof(double) * c->T.N, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    LAUNCHCHK(c, staged_copy(c->stage, c->stream, uhat_out, c->d_uhat, c->T.N));
   }
   return r;
 }
@@ -1159,41 +1194,16 @@ int hdg_get_trace(hdg_ctx* c, double* uhat) {
   if (!c || !uhat) return HDG_ERR_ARG;
   if (!c->solved) return fail(c, HDG_ERR_STATE, "no trace solution: call hdg_solve or hdg_run");
   TRY(select_device(c));
-  HIPCHK(c, hipMemcpyAsync(uhat, c->d_uhat, sizeof(double) * c->T.N, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  LAUNCHCHK(c, staged_copy(c->stage, c->stream, uhat, c->d_uhat, c->T.N));
   return HDG_OK;
 }
 
 int hdg_recover(hdg_ctx* c, double* q, double* u, double* uhat_cell) {
-  if (!c) return HDG_ERR_ARG;
-  TRY(select_device(c));
-  if (!c->recovered) TRY(recover_impl(c));
-  const int64_t nc = c->mesh.nc;
-  const int M = c->m, nq = c->nq, nu = c->nu, nt = c->nt;
-  if (q || u) {
-    std::vector<double> qu((size_t)nc * M);
-    HIPCHK(c, hipMemcpyAsync(qu.data(), c->d_qu, sizeof(double) * qu.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int64_t e = 0; e < nc; ++e) {
-      if (q)
-        for (int i = 0; i < nq; ++i) q[e + nc * i] = qu[e * M + i];
-      if (u)
-        for (int i = 0; i < nu; ++i) u[e + nc * i] = qu[e * M + nq + i];
-    }
-  }
-  if (uhat_cell) {
-    if ((int64_t)c->h_cf.size() != 3 * nc) {
-      c->h_cf.resize(3 * nc);
-      HIPCHK(c, hipMemcpyAsync(c->h_cf.data(), c->mesh.cf, sizeof(int) * 3 * nc, hipMemcpyDeviceToHost, c->stream));
-    }
-    std::vector<double> uh(c->T.N);
-    HIPCHK(c, hipMemcpyAsync(uh.data(), c->d_uhat, sizeof(double) * uh.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int64_t e = 0; e < nc; ++e)
-      for (int lf = 0; lf < 3; ++lf)
-        for (int t = 0; t < nt; ++t) uhat_cell[e + nc * (t + nt * lf)] = uh[(int64_t)c->h_cf[3 * e + lf] * nt + t];
-  }
-  return HDG_OK;
+  return recover_out(c, false, q, u, uhat_cell);
+}
+
+int hdg_recover_rows(hdg_ctx* c, double* q, double* u, double* uhat_cell) {
+  return recover_out(c, true, q, u, uhat_cell);
 }
 
 int hdg_errornorm(hdg_ctx* c, int kind, const double* par, double* sq) {
@@ -1227,62 +1237,15 @@ int hdg_run(hdg_ctx* c, hdg_solve_info* info) {
   return r;
 }
 
-namespace {
-
-// Julia's CSC of K (the CSR of K^T: column (g, b) holds rows (f, a) for the
-// faces f of row g's pattern, which is structurally symmetric, ascending)
-// from a face-ELL value array and an rhs in device memory.
-int export_csc(hdg_ctx* c, const double* d_vals, const double* d_rhs, int64_t* colptr, int64_t* rowval,
-               double* nzval, double* rhs) {
-  const int64_t nf = c->mesh.nf, N = c->T.N;
-  const int nt = c->nt;
-  std::vector<int> bcol(kSlots * nf);
-  std::vector<unsigned char> nslot(nf), tslot(kSlots * nf);
-  HIPCHK(c, hipMemcpyAsync(bcol.data(), c->pat.bcol, sizeof(int) * bcol.size(), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(nslot.data(), c->pat.nslot, nf, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(tslot.data(), c->pat.tslot, tslot.size(), hipMemcpyDeviceToHost, c->stream));
-  std::vector<double> vals;
-  if (nzval) {
-    vals.resize((size_t)kSlots * nt * N);
-    HIPCHK(c, hipMemcpyAsync(vals.data(), d_vals, sizeof(double) * vals.size(), hipMemcpyDeviceToHost, c->stream));
-  }
-  if (rhs) HIPCHK(c, hipMemcpyAsync(rhs, d_rhs, sizeof(double) * N, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  int64_t w = 0;
-  if (colptr) colptr[0] = 1;
-  for (int64_t g = 0; g < nf; ++g)
-    for (int b = 0; b < nt; ++b) {
-      for (int s = 0; s < nslot[g]; ++s) {
-        const int64_t f = bcol[kSlots * g + s];
-        const int ts = tslot[kSlots * g + s];
-        for (int a = 0; a < nt; ++a) {
-          if (rowval) rowval[w] = f * nt + a + 1;
-          if (nzval) nzval[w] = vals[(size_t)(ts * nt + b) * N + f * nt + a];
-          ++w;
-        }
-      }
-      if (colptr) colptr[g * nt + b + 1] = w + 1;
-    }
-  return HDG_OK;
+int hdg_get_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double* nzval, double* rhs) {
+  return system_out<int64_t>(c, 1, colptr, rowval, nzval, rhs);
 }
 
-}  // namespace
-
-int hdg_get_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double* nzval, double* rhs) {
-  if (!c) return HDG_ERR_ARG;
-  if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
-  TRY(select_device(c));
-  TRY(ensure_system(c));
-  if (!c->T.blk || !nzval) return export_csc(c, c->T.vals, c->T.rhs, colptr, rowval, nzval, rhs);
-  double* vals = nullptr;
-  TRY(dalloc(c, &vals, (size_t)kSlots * c->nt * c->T.N));
-  int r = HDG_OK;
-  const int e = launch_expand_ell(c->pat, c->T, vals, c->stream);
-  if (e) r = fail(c, HDG_ERR_HIP, "expanding the trace blocks: %s", hipGetErrorString((hipError_t)e));
-  if (r == HDG_OK) r = export_csc(c, vals, c->T.rhs, colptr, rowval, nzval, rhs);
-  (void)hipStreamSynchronize(c->stream);
-  dfree(c, vals);
-  return r;
+int hdg_get_system32(hdg_ctx* c, int32_t* indptr, int32_t* indices, double* data, double* rhs) {
+  if (c && c->assembled &&
+      (c->nblock_cols * (int64_t)c->nt * c->nt > INT32_MAX || c->T.N >= INT32_MAX))
+    return fail(c, HDG_ERR_UNSUPPORTED, "the system's indices exceed 32 bits");
+  return system_out<int32_t>(c, 0, indptr, indices, data, rhs);
 }
 
 int hdg_get_applied_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double* nzval, double* rhs,
@@ -1311,7 +1274,7 @@ int hdg_get_applied_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double*
     const hipError_t e = hipMemcpyAsync(meandiag_out, part + 1024, sizeof(double), hipMemcpyDeviceToHost, c->stream);
     if (e != hipSuccess) r = fail(c, HDG_ERR_HIP, "hipMemcpyAsync: %s", hipGetErrorString(e));
   }
-  if (r == HDG_OK) r = export_csc(c, vals, b, colptr, rowval, nzval, rhs);
+  if (r == HDG_OK) r = export_csc<int64_t>(c, vals, b, 1, colptr, rowval, nzval, rhs);
   (void)hipStreamSynchronize(c->stream);
   dfree(c, part);
   dfree(c, b);
@@ -1328,9 +1291,9 @@ int hdg_get_local_ops(hdg_ctx* c, double* Ke, double* be) {
     LAUNCHCHK(c, launch_expand_ke_spd(c->k, c->mesh, c->d_spd, c->d_Ke, c->d_be, c->stream));
     c->ke_full = true;
   }
-  if (Ke) HIPCHK(c, hipMemcpyAsync(Ke, c->d_Ke, sizeof(double) * nc * c->m * c->ntr, hipMemcpyDeviceToHost, c->stream));
-  if (be) HIPCHK(c, hipMemcpyAsync(be, c->d_be, sizeof(double) * nc * c->m, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (Ke) LAUNCHCHK(c, staged_copy(c->stage, c->stream, Ke, c->d_Ke, nc * c->m * c->ntr));
+  if (be) LAUNCHCHK(c, staged_copy(c->stage, c->stream, be, c->d_be, nc * c->m));
+  if (!Ke && !be) HIPCHK(c, hipStreamSynchronize(c->stream));
   return HDG_OK;
 }
 
@@ -1339,19 +1302,8 @@ int hdg_get_condensed(hdg_ctx* c, double* Ate, double* bte) {
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
   TRY(select_device(c));
   const int64_t nc = c->mesh.nc;
-  const int ntr = c->ntr;
-  if (Ate) {
-    std::vector<double> a((size_t)nc * ntr * ntr);
-    HIPCHK(c, hipMemcpyAsync(a.data(), c->d_Ate, sizeof(double) * a.size(), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int64_t e = 0; e < nc; ++e)
-      for (int i = 0; i < ntr; ++i)
-        for (int j = 0; j < ntr; ++j) Ate[e * ntr * ntr + i + ntr * j] = a[e * ntr * ntr + i * ntr + j];
-  }
-  if (bte) {
-    HIPCHK(c, hipMemcpyAsync(bte, c->d_bte, sizeof(double) * nc * ntr, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  }
+  if (Ate) LAUNCHCHK(c, staged_transposes(c->stage, c->stream, c->k, Ate, c->d_Ate, nc));
+  if (bte) LAUNCHCHK(c, staged_copy(c->stage, c->stream, bte, c->d_bte, nc * c->ntr));
   return HDG_OK;
 }
 

@@ -109,6 +109,7 @@ struct hdg_batch {
   bool ran = false;
   std::mutex mu;  // guards err (groups run in host threads of their own)
   std::string err;
+  HostStage stage;  // pinned memory of traces on their way to the caller
 };
 
 namespace {
@@ -919,8 +920,7 @@ int hdg_batch_trace(hdg_batch* b, int i, double* uhat, int64_t cap) {
   if (cap < I.N)
     return fail(b, HDG_ERR_ARG, "the trace of instance %d has %lld doubles, more than the buffer's %lld", i,
                 (long long)I.N, (long long)cap);
-  BHIP(b, hipMemcpyAsync(uhat, g.uhat + I.row0, sizeof(double) * I.N, hipMemcpyDeviceToHost, g.s));
-  BHIP(b, hipStreamSynchronize(g.s));
+  BHIP(b, (hipError_t)staged_copy(b->stage, g.s, uhat, g.uhat + I.row0, I.N));
   return HDG_OK;
 }
 
@@ -935,6 +935,7 @@ void hdg_batch_destroy(hdg_batch* b) {
   if (!b) return;
   (void)hipSetDevice(b->device);
   for (Group& g : b->groups) free_group(b, g);
+  stage_free(b->stage);
   delete b;
 }
 

@@ -96,17 +96,16 @@ def get_usigma(sigma_h, u_h, uhat_h, uhat, K_e, b_e, mesh, ctx=None):
     nt = uhat_h.fs.nbase
     if ctx is not None and ctx.mesh is mesh:
         ctx.set_trace(uhat)
-        q, u, uc = ctx.recover()
+        ctx.recover_into(sigma_h.m_values, u_h.m_values, uhat_h.m_values)
     else:
         idx = (mesh.cells[:, 3:][:, :, None] - 1) * nt + np.arange(nt)[None, None, :]
         ue = np.asarray(uhat)[idx.reshape(len(mesh.cells), -1)]
         dof = np.einsum("cij,cj->ci", K_e, ue) + b_e
         nq = sigma_h.fs.nbase
         q, u = dof[:, :nq], dof[:, nq:]
-        uc = np.asarray(uhat)[idx].transpose(0, 2, 1)
-    sigma_h.m_values[:] = q
-    u_h.m_values[:] = u
-    uhat_h.m_values[:] = uc
+        sigma_h.m_values[:] = q
+        u_h.m_values[:] = u
+        uhat_h.m_values[:] = np.asarray(uhat)[idx].transpose(0, 2, 1)
 
 
 def errornorm(u_h, u_ex, ctx=None):
@@ -151,10 +150,7 @@ def hdg_solve(sigma_h, u_h, uhat_h, mesh, dbc=None, f=None, tau=1.0, precision=L
     if dbc is not None:
         ctx.set_dirichlet(dbc.prescribed_dofs, dbc.values)
     info = ctx.run()
-    q, u, uc = ctx.recover()
-    sigma_h.m_values[:] = q
-    u_h.m_values[:] = u
-    uhat_h.m_values[:] = uc
+    ctx.recover_into(sigma_h.m_values, u_h.m_values, uhat_h.m_values)
     return info
 
 

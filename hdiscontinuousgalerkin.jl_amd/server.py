@@ -90,7 +90,7 @@ class Server:
         n = self._ndofs.get(int(rid))
         if n is None:
             raise L.HDGError(8, f"request {rid} has not been waited for")
-        out = np.zeros(n)
+        out = np.empty(n)
         self._chk(lib().hdg_server_trace(self._h, int(rid), out.ctypes.data_as(C.POINTER(C.c_double)), n))
         del self._ndofs[int(rid)]
         return out
@@ -156,7 +156,7 @@ class Batch:
     def trace(self, i):
         if self._ndofs[i] is None:
             raise L.HDGError(8, "run the batch first")
-        out = np.zeros(int(self._ndofs[i]))
+        out = np.empty(int(self._ndofs[i]))
         self._chk(lib().hdg_batch_trace(self._h, int(i), out.ctypes.data_as(C.POINTER(C.c_double)), out.size))
         return out
 

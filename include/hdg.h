@@ -200,6 +200,10 @@ int hdg_assemble_condense(hdg_ctx* ctx);
    NULL. */
 int hdg_get_system(hdg_ctx* ctx, int64_t* colptr, int64_t* rowval,
                    double* nzval, double* rhs);
+/* The same with 0-based 32-bit indices (scipy's layout); HDG_ERR_UNSUPPORTED
+   for systems that need more. */
+int hdg_get_system32(hdg_ctx* ctx, int32_t* indptr, int32_t* indices,
+                     double* data, double* rhs);
 /* apply!(K, b, dbc) with APPLY_TRANSPOSE (src/boundary.jl:121-175) on the
    device, exported as hdg_get_system exports K and b: the rhs lifted by the
    prescribed values (b_i -= v_d K(i, d) over the prescribed dofs d in
@@ -235,6 +239,8 @@ int hdg_get_trace(hdg_ctx* ctx, double* uhat);
 /* get_uσ! (poisson2D_HDG.jl:197-212): q (ncells x nq), u (ncells x nu),
    uhat_cell (ncells x nt x 3), all column-major; any may be NULL. */
 int hdg_recover(hdg_ctx* ctx, double* q, double* u, double* uhat_cell);
+/* The same, row-major. */
+int hdg_recover_rows(hdg_ctx* ctx, double* q, double* u, double* uhat_cell);
 /* errornorm(u_h, u_ex) (DiscreteFunctions.jl:97-120): squared L2 error of
    the recovered u against HDG_UEX_SINSIN or HDG_UEX_LINEAR (par c0,c1,c2). */
 int hdg_errornorm(hdg_ctx* ctx, int uex_kind, const double* uex_par,
