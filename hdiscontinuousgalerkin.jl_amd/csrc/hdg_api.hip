@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/hdg.h"
+#include "hdg_amg.h"
 #include "hdg_arena.h"
 #include "hdg_host.h"
 #include "hdg_quad.h"
@@ -46,6 +47,15 @@ struct hdg_ctx {
   bool structured = false;  // cells follow rectangle_mesh's (nx, ny) numbering
   MgData mg;                // vertex hierarchy (structured meshes)
   MgData* d_mg = nullptr;   // its device copy (read by the one-workgroup tail kernel)
+  // other meshes: connectivity on the host and, from the first solve with the
+  // automatic preconditioner, the aggregation hierarchy (1 there, 0 not
+  // yet, -1 not to be had) with its arrays' memory
+  std::vector<int> h_cn, h_cf, h_fcell;
+  int amg_state = 0;
+  AmgData amg;
+  AmgData* d_amg = nullptr;
+  int* amg_ints = nullptr;
+  double* amg_vals = nullptr;
 
   // discretisation
   bool has_setup = false;
@@ -237,10 +247,25 @@ void free_problem(hdg_ctx* c) {
   dfree(c, c->d_plain);
   q = QuadSys{};
   c->filled = false;
+  dfree(c, c->amg.top.g);
+  dfree(c, c->amg.top.t);
+  if (c->amg_state < 0) c->amg_state = 0;
   dfree(c, c->d_mg);
   c->has_setup = c->assembled = c->solved = c->recovered = false;
   c->csched = CondenseSched{};
   c->tuned = false;
+}
+
+// the aggregation hierarchy (top.g and top.t belong to the set-up)
+void free_amg(hdg_ctx* c) {
+  dfree(c, c->amg_ints);
+  dfree(c, c->amg_vals);
+  dfree(c, c->amg.top.vfix);
+  dfree(c, c->d_amg);
+  dfree(c, c->amg.top.g);
+  dfree(c, c->amg.top.t);
+  c->amg = AmgData{};
+  c->amg_state = 0;
 }
 
 void free_mesh(hdg_ctx* c) {
@@ -265,6 +290,10 @@ void free_mesh(hdg_ctx* c) {
     dfree(c, L.e);
   }
   c->mg = MgData{};
+  free_amg(c);
+  c->h_cn.clear();
+  c->h_cf.clear();
+  c->h_fcell.clear();
   c->structured = false;
   c->has_mesh = false;
   c->mesh = DevMesh{};
@@ -416,6 +445,9 @@ int autotune_impl(hdg_ctx* c) {
 bool use_mg(const hdg_ctx* c);
 bool mixed(const hdg_ctx* c);
 
+// the preconditioner of a solve
+enum class Pc { kJacobi, kQuad, kAmg };
+
 // The context's second stream and its events, created on first use.
 int ensure_aux(hdg_ctx* c) {
   if (c->aux) return HDG_OK;
@@ -469,6 +501,93 @@ int assemble_impl(hdg_ctx* c, bool run = false) {
 
 bool use_mg(const hdg_ctx* c) {
   return c->structured && c->opt.precond != HDG_PC_BLOCK_JACOBI;
+}
+
+// The aggregation hierarchy of a mesh without rectangle structure, built from
+// the mesh at the first solve that wants it.  1: there; 0: block-Jacobi it is
+// (asked for, a mesh the plan refuses, or no memory within the budget: what
+// fitted before fits).
+int ensure_amg(hdg_ctx* c) {
+  if (c->structured || c->opt.precond != HDG_PC_AUTO || c->amg_state < 0) return 0;
+  AmgData& A = c->amg;
+  if (c->amg_state == 0) {
+    free_amg(c);
+    AmgPlan P;
+    bool ok = false;
+    try {
+      ok = amg_plan(c->mesh.nn, c->mesh.nc, c->mesh.nf, c->h_cn.data(), c->h_cf.data(), c->h_fcell.data(), P);
+    } catch (const std::bad_alloc&) {
+    }
+    size_t nd = (size_t)kAmgDirect * kAmgDirect;
+    if (ok && P.tail < P.nlev) nd += (size_t)P.lev[P.tail].n * P.lev[P.tail].n;
+    for (int l = 0; l < P.nlev; ++l) nd += P.lev[l].nnz + 3 * ((size_t)P.lev[l].gnnz + P.lev[l].n);
+    if (!ok || dalloc(c, &c->amg_ints, P.ints.size()) || dalloc(c, &c->amg_vals, nd) ||
+        dalloc(c, &A.top.vfix, c->mesh.nn) || dalloc(c, &c->d_amg, 1) ||
+        hipMemcpyAsync(c->amg_ints, P.ints.data(), sizeof(int) * P.ints.size(), hipMemcpyHostToDevice, c->stream) !=
+            hipSuccess) {
+      (void)hipStreamSynchronize(c->stream);
+      free_amg(c);
+      c->amg_state = -1;
+      return 0;
+    }
+    const int* ints = c->amg_ints;
+    double* v = c->amg_vals;
+    const auto take = [&](size_t n) {
+      double* p = v;
+      v += n;
+      return p;
+    };
+    A.nlev = P.nlev;
+    A.tail = P.tail;
+    A.direct = P.direct;
+    A.cinv = take((size_t)kAmgDirect * kAmgDirect);
+    if (A.tail < A.nlev) A.dense = take((size_t)P.lev[A.tail].n * P.lev[A.tail].n);
+    for (int l = 0; l < P.nlev; ++l) {
+      const AmgPlan::Level& Q = P.lev[l];
+      AmgLevel& L = A.lev[l];
+      L.n = Q.n;
+      L.ap = ints + Q.ap;
+      L.ai = ints + Q.ai;
+      L.av = take(Q.nnz);
+      L.dinv = take(Q.n);
+      L.r = take(Q.n);
+      L.e = take(Q.n);
+      if (!Q.gnnz) continue;
+      L.agg = ints + Q.agg;
+      L.gp = ints + Q.gp;
+      L.gi = ints + Q.gi;
+      L.tp = ints + Q.tp;
+      L.ti = ints + Q.ti;
+      L.tx = ints + Q.tx;
+      L.gv = take(Q.gnnz);
+      L.pv = take(Q.gnnz);
+      L.apv = take(Q.gnnz);
+    }
+    AmgTop& t = A.top;
+    t.n = A.lev[0].n;
+    t.fv = ints + P.fv;
+    t.vp = ints + P.vp;
+    t.vi = ints + P.vi;
+    t.af = ints + P.af;
+    t.r = A.lev[0].r;
+    t.e = A.lev[0].e;
+    const bool up = hipMemcpyAsync(c->d_amg, &A, sizeof(AmgData), hipMemcpyHostToDevice, c->stream) == hipSuccess;
+    // the uploads read P and A: finish them here
+    if (hipStreamSynchronize(c->stream) != hipSuccess || !up) {
+      free_amg(c);
+      c->amg_state = -1;
+      return 0;
+    }
+    c->amg_state = 1;
+  }
+  if (!A.top.g && (dalloc(c, &A.top.g, 4 * c->T.N) || dalloc(c, &A.top.t, c->T.N))) {
+    dfree(c, A.top.g);
+    dfree(c, A.top.t);
+    free_amg(c);
+    c->amg_state = -1;
+    return 0;
+  }
+  return 1;
 }
 bool mixed(const hdg_ctx* c) { return use_mg(c) && c->opt.precision == HDG_MIXED; }
 
@@ -533,14 +652,14 @@ int setup_quad(hdg_ctx* c) {
 }
 
 // PCG iterations enqueued between convergence checks
-int chunk_of(const hdg_ctx* c) { return use_mg(c) ? 4 : 64; }
+int chunk_of(Pc pc) { return pc == Pc::kJacobi ? 64 : 4; }
 
 // one chunk of CG iterations; the kernels take the iteration number from the
 // device state, so the same launches serve every chunk (and a graph of them)
-int enqueue_chunk(hdg_ctx* c, double rtol2, int maxit) {
-  const int n = chunk_of(c);
+int enqueue_chunk(hdg_ctx* c, Pc pc, double rtol2, int maxit) {
+  const int n = chunk_of(pc);
   for (int it = 0; it < n; ++it) {
-    if (use_mg(c)) {
+    if (pc == Pc::kQuad) {
       LAUNCHCHK(c, launch_quad_product(c->qs, c->ql, rtol2, maxit, c->stream));
       LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));
       LAUNCHCHK(c, launch_vcycle(c->mg, c->d_mg, c->cg.st, rtol2, maxit, c->stream));
@@ -548,6 +667,8 @@ int enqueue_chunk(hdg_ctx* c, double rtol2, int maxit) {
     } else {
       LAUNCHCHK(c, launch_cg_spmv(c->pat, op64(c), kv64(c), 0, rtol2, maxit, 0, c->stream));
       LAUNCHCHK(c, launch_cg_update(c->T, c->cg, 0, 0, c->stream));
+      if (pc == Pc::kAmg)
+        LAUNCHCHK(c, launch_amg_cycle(c->pat, c->T, c->cg, c->amg, rtol2, maxit, c->stream));
     }
   }
   return HDG_OK;
@@ -559,13 +680,12 @@ int enqueue_chunk(hdg_ctx* c, double rtol2, int maxit) {
 // first solve after a set-up runs eagerly: capturing and instantiating the
 // graphs costs more than one solve's launches saves, and many contexts
 // capturing at once (the serving loop) serialise in the runtime.
-int launch_chunk(hdg_ctx* c, int slot, double rtol2, int maxit) {
-  const bool eager = (c->opt.schedule & HDG_SCHEDULE_EAGER) != 0 || c->solves == 0;
+int launch_chunk(hdg_ctx* c, Pc pc, bool eager, int slot, double rtol2, int maxit) {
   if (!eager && !c->gexec[slot]) {
     std::lock_guard<std::mutex> lk(graph_mutex());
     hipGraph_t g = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int r = enqueue_chunk(c, rtol2, maxit);
+    int r = enqueue_chunk(c, pc, rtol2, maxit);
     hipError_t e = hipMemcpyAsync(&c->h_st[slot], c->cg.st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
     if (r != HDG_OK) return r;
@@ -580,8 +700,47 @@ int launch_chunk(hdg_ctx* c, int slot, double rtol2, int maxit) {
     HIPCHK(c, hipGraphLaunch(c->gexec[slot], c->stream));
     return HDG_OK;
   }
-  TRY(enqueue_chunk(c, rtol2, maxit));
+  TRY(enqueue_chunk(c, pc, rtol2, maxit));
   HIPCHK(c, hipMemcpyAsync(&c->h_st[slot], c->cg.st, sizeof(CgState), hipMemcpyDeviceToHost, c->stream));
+  return HDG_OK;
+}
+
+// The CG iterations of a solve up to the state that ends it.  One chunk stays
+// queued behind the one whose state is read back, unless that one is forecast
+// to converge (chunk_converges); launches after convergence return at once.
+int iterate(hdg_ctx* c, Pc pc, bool eager, double rtol2, int maxit, CgState& last) {
+  hipEvent_t evs[2];
+  HIPCHK(c, hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
+  HIPCHK(c, hipEventCreateWithFlags(&evs[1], hipEventDisableTiming));
+  int slot = 0;
+  TRY(launch_chunk(c, pc, eager, slot, rtol2, maxit));
+  HIPCHK(c, hipEventRecord(evs[slot], c->stream));
+  CgState prev{};
+  last = CgState{};
+  int nread = 0;
+  bool behind = false;
+  for (;;) {
+    const int nxt = slot ^ 1;
+    behind = nread < 2 || !chunk_converges(prev, last, chunk_of(pc), rtol2);
+    if (behind) {
+      TRY(launch_chunk(c, pc, eager, nxt, rtol2, maxit));
+      HIPCHK(c, hipEventRecord(evs[nxt], c->stream));
+    }
+    HIPCHK(c, hipEventSynchronize(evs[slot]));
+    prev = last;
+    last = c->h_st[slot];
+    ++nread;
+    if (last.done) break;
+    if (!behind) {  // the forecast missed
+      TRY(launch_chunk(c, pc, eager, nxt, rtol2, maxit));
+      HIPCHK(c, hipEventRecord(evs[nxt], c->stream));
+      behind = true;
+    }
+    slot = nxt;
+  }
+  if (behind) HIPCHK(c, hipEventSynchronize(evs[slot ^ 1]));
+  (void)hipEventDestroy(evs[0]);
+  (void)hipEventDestroy(evs[1]);
   return HDG_OK;
 }
 
@@ -601,6 +760,7 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
   }
   const double rtol = c->opt.rtol > 0 ? c->opt.rtol : 1e-12;
   const int maxit = c->opt.maxit > 0 ? c->opt.maxit : 200000;
+  const Pc pc = use_mg(c) ? Pc::kQuad : (ensure_amg(c) ? Pc::kAmg : Pc::kJacobi);
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   if (use_mg(c)) {
     c->qs.uD = c->T.uD;
@@ -632,42 +792,21 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
     LAUNCHCHK(c, launch_quad_smooth(c->qs, c->ql, mixed(c), c->stream));
   } else {
     LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
+    if (pc == Pc::kAmg) {
+      LAUNCHCHK(c, launch_amg_setup(c->mesh, c->T, c->d_Ate, c->amg, c->d_amg, c->stream));
+      LAUNCHCHK(c, launch_amg_cycle(c->pat, c->T, c->cg, c->amg, 0.0, -1, c->stream));
+    }
   }
-  // one chunk stays queued behind the one whose state is read back, unless
-  // that one is forecast to converge (chunk_converges); launches after
-  // convergence return at once
-  hipEvent_t evs[2];
-  HIPCHK(c, hipEventCreateWithFlags(&evs[0], hipEventDisableTiming));
-  HIPCHK(c, hipEventCreateWithFlags(&evs[1], hipEventDisableTiming));
   const double rtol2 = rtol * rtol;
-  int slot = 0;
-  TRY(launch_chunk(c, slot, rtol2, maxit));
-  HIPCHK(c, hipEventRecord(evs[slot], c->stream));
-  CgState prev{}, last{};
-  int nread = 0;
-  bool behind = false;
-  for (;;) {
-    const int nxt = slot ^ 1;
-    behind = nread < 2 || !chunk_converges(prev, last, chunk_of(c), rtol2);
-    if (behind) {
-      TRY(launch_chunk(c, nxt, rtol2, maxit));
-      HIPCHK(c, hipEventRecord(evs[nxt], c->stream));
-    }
-    HIPCHK(c, hipEventSynchronize(evs[slot]));
-    prev = last;
-    last = c->h_st[slot];
-    ++nread;
-    if (last.done) break;
-    if (!behind) {  // the forecast missed
-      TRY(launch_chunk(c, nxt, rtol2, maxit));
-      HIPCHK(c, hipEventRecord(evs[nxt], c->stream));
-      behind = true;
-    }
-    slot = nxt;
+  const bool eager = (c->opt.schedule & HDG_SCHEDULE_EAGER) != 0 || c->solves == 0;
+  CgState last;
+  TRY(iterate(c, pc, eager, rtol2, maxit, last));
+  if (pc == Pc::kAmg && last.done == 3) {
+    // the cycle is definite only where the cells' trace blocks are
+    // semidefinite (not for every tau > 1): without it
+    LAUNCHCHK(c, launch_cg_init(c->pat, c->T, c->cg, c->stream));
+    TRY(iterate(c, Pc::kJacobi, true, rtol2, maxit, last));
   }
-  if (behind) HIPCHK(c, hipEventSynchronize(evs[slot ^ 1]));
-  (void)hipEventDestroy(evs[0]);
-  (void)hipEventDestroy(evs[1]);
   ++c->solves;
   return finish_solve(c, info, maxit, err_flag);
 }
@@ -894,7 +1033,13 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
   c->nblock_cols = nblk;
   int nx = 0, ny = 0;
   c->structured = detect_structured(nn, nc, cells, &nx, &ny);
-  if (c->structured) TRY(build_vertex_levels(c, nx, ny));
+  if (c->structured) {
+    TRY(build_vertex_levels(c, nx, ny));
+  } else {
+    c->h_cn.swap(cn);
+    c->h_cf.swap(cf);
+    c->h_fcell.swap(fcell);
+  }
   c->has_mesh = true;
   return HDG_OK;
 }

@@ -97,8 +97,12 @@ typedef struct {
   int32_t maxit;       /* trace solve iteration cap (0 -> 200000) */
   int32_t schedule;    /* HDG_SCHEDULE_* flags, 0 = default */
   int32_t precond;     /* HDG_PC_*: block-Jacobi per face, or a V-cycle of
-                          block-Jacobi on the traces + geometric multigrid on
-                          the P1 vertex space of a structured mesh */
+                          vertex grids (structured meshes).  HDG_PC_AUTO takes
+                          the V-cycle on structured meshes and, on others, one
+                          over the mesh's vertices and aggregates of them,
+                          set up at the first solve on a mesh; block-Jacobi
+                          where hbm_budget leaves no room for it or its solve
+                          breaks down */
 } hdg_options;
 
 typedef struct {
