@@ -215,7 +215,8 @@ __global__ __launch_bounds__(256) void amg_rap_kernel(AmgLevel L, AmgLevel C) {
 
 // Inverse of the last operator (n <= kAmgDirect; SPD on the rows with a
 // positive diagonal, identity rows elsewhere): Gauss-Jordan without pivoting,
-// 6 x 6 entries per thread in registers.
+// 6 x 6 entries per thread in registers, the pivot's row and column updated by
+// the same fma as the rest (factors p - 1 and 1 + 1/p, p the pivot).
 __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __restrict__ cinv) {
   constexpr int T = 16, E = kAmgDirect / T;
   __shared__ double full[kAmgDirect * kAmgDirect];
@@ -237,38 +238,35 @@ __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __
       const int r = tr + T * a, c = tc + T * b;
       m[a][b] = r < n && c < n ? full[r * n + c] : 0.0;
     }
-  for (int k = 0; k < n; ++k) {
-    const int p = k & 1, kt = k % T, ka = k / T;
-    if (tr == kt) {
+  // k = ka T + kt with ka unrolled, so that the pivot's registers are known
+#pragma unroll
+  for (int ka = 0; ka < E; ++ka)
+    for (int kt = 0; kt < T && ka * T + kt < n; ++kt) {
+      const int k = ka * T + kt, p = kt & 1;
+      if (tr == kt)
+#pragma unroll
+        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[ka][b];
+      if (tc == kt)
+#pragma unroll
+        for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][ka];
+      __syncthreads();
+      const double piv = rowb[p][k];
+      double rk[E], ck[E];
+#pragma unroll
+      for (int a = 0; a < E; ++a) {
+        rk[a] = rowb[p][tc + T * a];
+        ck[a] = colb[p][tr + T * a];
+      }
+      const double ip = 1.0 / piv;
+#pragma unroll
+      for (int a = 0; a < E; ++a) rk[a] *= ip;
+      rk[ka] = tc == kt ? 1.0 + ip : rk[ka];
+      ck[ka] = tr == kt ? piv - 1.0 : ck[ka];
 #pragma unroll
       for (int a = 0; a < E; ++a)
-        if (a == ka)
 #pragma unroll
-          for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[a][b];
+        for (int b = 0; b < E; ++b) m[a][b] = fma(-ck[a], rk[b], m[a][b]);
     }
-    if (tc == kt) {
-#pragma unroll
-      for (int b = 0; b < E; ++b)
-        if (b == ka)
-#pragma unroll
-          for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][b];
-    }
-    __syncthreads();
-    const double ip = 1.0 / rowb[p][k];
-    double rk[E], ck[E];
-#pragma unroll
-    for (int a = 0; a < E; ++a) {
-      rk[a] = rowb[p][tc + T * a] * ip;
-      ck[a] = colb[p][tr + T * a];
-    }
-#pragma unroll
-    for (int a = 0; a < E; ++a)
-#pragma unroll
-      for (int b = 0; b < E; ++b) {
-        const bool ir = tr + T * a == k, ic = tc + T * b == k;
-        m[a][b] = ir ? (ic ? ip : rk[b]) : (ic ? -ck[a] * ip : fma(-ck[a], rk[b], m[a][b]));
-      }
-  }
 #pragma unroll
   for (int a = 0; a < E; ++a)
 #pragma unroll

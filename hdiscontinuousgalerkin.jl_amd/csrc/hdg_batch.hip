@@ -571,20 +571,21 @@ int build_group(hdg_batch* b, Group& g) {
     G.gres[d] = (int)res.size();
   }
   BTRY(tune_group(b, g));
-  // set-up tables: RAP for every level pair down to the tails
+  // set-up tables: RAP for every level pair
   MgSetupGroup& S = g.S;
   S.ninst = n;
   S.dM = g.dMi;
-  S.ndepth = ndepth;
+  S.ndepth = 1;
+  for (const MgData& M : g.Mi) S.ndepth = std::max(S.ndepth, M.nlev - 1);
   for (int d = 1; d < S.ndepth; ++d) {
     std::vector<VRec> rec;
     std::vector<BlockMap> rp;
     for (int j = 0; j < n; ++j) {
       const MgData& M = g.Mi[j];
-      if (d >= M.tail) continue;
+      if (d + 1 >= M.nlev) continue;
       const int p = (int)rec.size();
       rec.push_back(VRec{M.lev[d], M.lev[d + 1], nullptr, nullptr, 0});
-      const int64_t br = (8 * M.lev[d + 1].n + 255) / 256;
+      const int64_t br = v_rap_blocks(M.lev[d + 1]);
       for (int64_t u = 0; u < br; ++u) rp.push_back(BlockMap{p, (int)u});
     }
     VRec* drec;

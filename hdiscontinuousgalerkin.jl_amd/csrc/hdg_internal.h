@@ -560,6 +560,7 @@ struct MgGroup {
 };
 // blocks of the level kernels over one instance's level
 int v_restrict_blocks(const MgLevel& C);
+int v_rap_blocks(const MgLevel& C);
 int v_post_blocks(const MgLevel& F);
 // Set-up tables of a group's vertex hierarchies: per depth d below their
 // tails, the instances with a level d+1, with block maps over 8 lanes per

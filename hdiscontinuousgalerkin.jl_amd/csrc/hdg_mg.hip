@@ -81,9 +81,12 @@ __device__ __forceinline__ bool converged(CgState* st, double rtol2, int maxit, 
 }
 
 // ------------------------------------------------------------ set-up
-// Galerkin stencil R A P, R = P^T, of coarse node C by eight lanes: lane t
-// takes the fine node at support offset t (lane 0 the ninth too), and a fixed
-// shuffle tree sums the lanes.  Every lane of a group of eight calls it.
+// Galerkin stencil R A P, R = P^T, of coarse node C by 16 lanes: lane t takes
+// the fine node at support offset t (seven lanes only help to sum), and a
+// fixed shuffle tree sums the lanes.  Bound by two dependent loads and the
+// weights' arithmetic on the small levels, by the fine stencils on the large
+// ones.  Eight lanes with two nodes on one of them, the small levels in one
+// workgroup: 41 us for 33 x 33 down to 9 x 9.
 __device__ __forceinline__ void rap_node(const MgLevel& F, const MgLevel& Cc, int64_t C, int t) {
   const int cnx = Cc.nx, cny = Cc.ny, fnx = F.nx, fny = F.ny;
   const bool live = C < Cc.n;
@@ -93,7 +96,8 @@ __device__ __forceinline__ void rap_node(const MgLevel& F, const MgLevel& Cc, in
   double st[kStencil];
 #pragma unroll
   for (int k = 0; k < kStencil; ++k) st[k] = 0.0;
-  for (int o = t; !cm && o < kStencil; o += 8) {
+  if (!cm && t < kStencil) {
+    const int o = t;
     const int fx = fine_of(I, fnx) + kOffX[o], fy = fine_of(J, fny) + kOffY[o], row = fnx + 1;
     const bool in = fx >= 0 && fx <= fnx && fy >= 0 && fy <= fny;
     const int64_t fi = in ? (int64_t)fy * row + fx : 0;
@@ -110,7 +114,6 @@ __device__ __forceinline__ void rap_node(const MgLevel& F, const MgLevel& Cc, in
       if (!on) gm[s] = 1;
     }
     const double w1 = in && !F.mask[fi] ? pw1(fx, fnx, I) * pw1(fy, fny, J) : 0.0;
-    if (w1 == 0.0) continue;
     double wx[3][3], wy[3][3];  // weight of coarse offset d at fine offset s
 #pragma unroll
     for (int s = -1; s <= 1; ++s)
@@ -133,9 +136,8 @@ __device__ __forceinline__ void rap_node(const MgLevel& F, const MgLevel& Cc, in
   }
 #pragma unroll
   for (int u = 0; u < kStencil; ++u) {
-    st[u] += __shfl_xor(st[u], 1, 8);
-    st[u] += __shfl_xor(st[u], 2, 8);
-    st[u] += __shfl_xor(st[u], 4, 8);
+#pragma unroll
+    for (int k = 1; k < 16; k <<= 1) st[u] += __shfl_xor(st[u], k, 16);
   }
   if (t != 0 || !live) return;
 #pragma unroll
@@ -156,26 +158,18 @@ __global__ __launch_bounds__(256) void mg_rap_kernel(VS sel) {
   int lb;
   const VRec& R = vrec_of(sel, lb);
   const int64_t gid = (int64_t)lb * blockDim.x + threadIdx.x;
-  rap_node(R.F, R.C, gid >> 3, (int)(gid & 7));
-}
-
-// The levels below `tail` in one workgroup per hierarchy.
-__global__ __launch_bounds__(1024) void mg_tail_rap_kernel(const MgData* __restrict__ Ms) {
-  const MgData& M = Ms[blockIdx.x];
-  for (int l = M.tail; l + 1 < M.nlev; ++l) {
-    const int64_t n8 = (8 * M.lev[l + 1].n + 1023) & ~(int64_t)1023;
-    for (int64_t u = threadIdx.x; u < n8; u += 1024) rap_node(M.lev[l], M.lev[l + 1], u >> 3, (int)(u & 7));
-    __syncthreads();
-  }
+  rap_node(R.F, R.C, gid >> 4, (int)(gid & 15));
 }
 
 // Inverse of the coarsest operator (at most kCoarseDirect nodes), one
 // workgroup per hierarchy: in-place Gauss-Jordan without pivoting (the
 // operator is SPD, fixed nodes have identity rows), the matrix in registers
 // (6 x 6 entries per thread), the pivot row and column through alternating
-// LDS buffers, one barrier of four wavefronts per step.  Bound by that chain:
-// 1.1 us per step, 88 us at 81 nodes (together with the tail's products, in
-// one workgroup of 1024 with an LDS matrix: 187 us for both; now 129).
+// LDS buffers, one barrier of four wavefronts per step.  With the pivot p, the
+// row and column k take the same fma(-c, r, m) as the rest: the row's factor c
+// is p - 1, the column's r is 1 + 1/p (m - (p - 1) m/p = m/p, c - c (1 + 1/p)
+// = -c/p).  Bound by the chain of barrier, division and LDS.  With the pivot's
+// registers chosen at run time a step took 1.1 us (88 us at 81 nodes).
 __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restrict__ Ms) {
   constexpr int T = 16, E = kCoarseDirect / T;
   __shared__ double rowb[2][kCoarseDirect], colb[2][kCoarseDirect];
@@ -195,38 +189,35 @@ __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restric
       }
       m[a][b] = v;
     }
-  for (int k = 0; k < n; ++k) {
-    const int p = k & 1, kt = k % T, ka = k / T;
-    if (tr == kt) {
+  // k = ka T + kt with ka unrolled, so that the pivot's registers are known
+#pragma unroll
+  for (int ka = 0; ka < E; ++ka)
+    for (int kt = 0; kt < T && ka * T + kt < n; ++kt) {
+      const int k = ka * T + kt, p = kt & 1;
+      if (tr == kt)
+#pragma unroll
+        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[ka][b];
+      if (tc == kt)
+#pragma unroll
+        for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][ka];
+      __syncthreads();
+      const double piv = rowb[p][k];
+      double rk[E], ck[E];
+#pragma unroll
+      for (int a = 0; a < E; ++a) {
+        rk[a] = rowb[p][tc + T * a];
+        ck[a] = colb[p][tr + T * a];
+      }
+      const double ip = 1.0 / piv;
+#pragma unroll
+      for (int a = 0; a < E; ++a) rk[a] *= ip;
+      rk[ka] = tc == kt ? 1.0 + ip : rk[ka];
+      ck[ka] = tr == kt ? piv - 1.0 : ck[ka];
 #pragma unroll
       for (int a = 0; a < E; ++a)
-        if (a == ka)
 #pragma unroll
-          for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[a][b];
+        for (int b = 0; b < E; ++b) m[a][b] = fma(-ck[a], rk[b], m[a][b]);
     }
-    if (tc == kt) {
-#pragma unroll
-      for (int b = 0; b < E; ++b)
-        if (b == ka)
-#pragma unroll
-          for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][b];
-    }
-    __syncthreads();
-    const double ip = 1.0 / rowb[p][k];
-    double rk[E], ck[E];
-#pragma unroll
-    for (int a = 0; a < E; ++a) {
-      rk[a] = rowb[p][tc + T * a] * ip;
-      ck[a] = colb[p][tr + T * a];
-    }
-#pragma unroll
-    for (int a = 0; a < E; ++a)
-#pragma unroll
-      for (int b = 0; b < E; ++b) {
-        const bool ir = tr + T * a == k, ic = tc + T * b == k;
-        m[a][b] = ir ? (ic ? ip : rk[b]) : (ic ? -ck[a] * ip : fma(-ck[a], rk[b], m[a][b]));
-      }
-  }
 #pragma unroll
   for (int a = 0; a < E; ++a)
 #pragma unroll
@@ -365,11 +356,13 @@ __global__ __launch_bounds__(256) void v_post_kernel(VS sel, double om) {
 // Levels tail .. nlev-1 of the V-cycle in one workgroup per hierarchy (Ms[b]
 // with CG state sts[b]): reads lev[tail].r, writes lev[tail].e.  The levels'
 // nodes (at most kTailNodes) are laid end to end, two per thread, whose
-// stencils, inverse diagonals and positions stay in registers; the vectors
-// that neighbours read are in LDS.  Bound by its chain of barriers: two
-// phases per level down (the residual, the restriction), one for the coarsest
-// grid, two per level up; every load comes before the first.  17 us at a 33 x
-// 33 tail (22 us with V(2,2) down to 25 nodes and stencils read from memory).
+// stencils, inverse diagonals and the LDS positions of what they read stay in
+// registers; the vectors that neighbours read are in LDS.  A neighbour off the
+// grid is read at the nearest node on it, with a zero coefficient.  Bound by
+// its chain of phases: two per level down (the residual, the restriction), one
+// for the coarsest grid, two per level up; every load comes before the first.
+// With the positions and weights worked out in every phase a 33 x 33 tail took
+// 17.4 us.
 __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __restrict__ Ms, CgState* sts, double rtol2,
                                                               int maxit) {
   constexpr int Q = (kTailNodes + kTailThreads - 1) / kTailThreads, NI = kCoarseDirect / 8;
@@ -381,29 +374,58 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
   if (st->done) return;
   const double om = M.omega_v;
   const int lt = M.tail, last = M.nlev - 1, tid = threadIdx.x;
-  // own nodes: level, offset of the level's first node, position
-  int lev[Q], off[Q], px[Q], py[Q];
+  // own nodes: level; position in the vectors (v), of the fine node under it
+  // (f) and of the coarse node at its lower left (pa); flags: neighbours on
+  // the grid (kL ..), restriction weights that are 1/2 (kFl ..), whether it
+  // lies between coarse columns (kPx) or rows (kPy)
+  enum { kL = 1, kR = 2, kD = 4, kU = 8, kFl = 16, kFr = 32, kFd = 64, kFu = 128, kPx = 256, kPy = 512 };
+  int lev[Q], v[Q], f[Q], pa[Q], fg[Q];
   double a[Q][kStencil], di[Q], r[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    int u = tid + q * kTailThreads, o = 0, l = lt;
-    while (l <= last && u >= (int)M.lev[l].n) {
-      u -= (int)M.lev[l].n;
-      o += (int)M.lev[l].n;
-      ++l;
-    }
-    const bool on = l <= last;
-    lev[q] = on ? l : -1;
-    off[q] = o;
-    const MgLevel& L = M.lev[on ? l : lt];
-    if (!on) u = 0;
-    px[q] = u % (L.nx + 1);
-    py[q] = u / (L.nx + 1);
-    const int n = (int)L.n;
+    lev[q] = -1;
+    v[q] = f[q] = pa[q] = fg[q] = 0;
+    di[q] = r[q] = 0.0;
 #pragma unroll
-    for (int k = 0; k < kStencil; ++k) a[q][k] = L.a[k * n + u];
-    di[q] = L.dinv[u];
-    r[q] = l == lt ? L.r[u] : 0.0;
+    for (int k = 0; k < kStencil; ++k) a[q][k] = 0.0;
+  }
+  // level by level, so that sizes and pointers are the wavefront's
+  for (int l = lt, o = 0, op = 0; l <= last; ++l) {
+    const MgLevel& L = M.lev[l];
+    const int nx = L.nx, ny = L.ny, row = nx + 1, n = (int)L.n;
+    const int fnx = l > lt ? M.lev[l - 1].nx : 0, fny = l > lt ? M.lev[l - 1].ny : 0;
+    const int cs = l < last ? M.lev[l + 1].nx + 1 : 0;
+    const double *La = L.a, *Ld = L.dinv, *Lr = L.r;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int u = tid + q * kTailThreads - o;
+      if (u < 0 || u >= n) continue;
+#pragma unroll
+      for (int k = 0; k < kStencil; ++k) a[q][k] = La[k * n + u];
+      di[q] = om * Ld[u];
+      if (l == lt) r[q] = Lr[u];
+      const int x = u % row, y = u / row;
+      lev[q] = l;
+      v[q] = o + u;
+      int g = (x > 0 ? kL : 0) | (x < nx ? kR : 0) | (y > 0 ? kD : 0) | (y < ny ? kU : 0);
+      if (l > lt) {
+        const int fx = fine_of(x, fnx), fy = fine_of(y, fny);
+        f[q] = op + fy * (fnx + 1) + fx;
+        if (fx > 0 && pw1(fx - 1, fnx, x) != 0.0) g |= kFl;
+        if (fx < fnx && pw1(fx + 1, fnx, x) != 0.0) g |= kFr;
+        if (fy > 0 && pw1(fy - 1, fny, y) != 0.0) g |= kFd;
+        if (fy < fny && pw1(fy + 1, fny, y) != 0.0) g |= kFu;
+      }
+      if (l < last) {
+        const int xa = x == nx ? (nx + 1) >> 1 : x >> 1, ya = y == ny ? (ny + 1) >> 1 : y >> 1;
+        pa[q] = o + n + ya * cs + xa;
+        if ((x & 1) && x != nx) g |= kPx;
+        if ((y & 1) && y != ny) g |= kPy;
+      }
+      fg[q] = g;
+    }
+    op = o;
+    o += n;
   }
   double ci[NI];
   const int nc = (int)M.lev[last].n, cv = tid >> 3, ct = tid & 7;
@@ -413,51 +435,66 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
     ci[k] = cv < nc && u < nc ? M.cinv[cv * nc + u] : 0.0;
   }
   if (lt == 1) rr_part(M.part, M.npart, maxit, sh);
+  // slots with a neighbour off the grid: to the right 1, 5, 7, left 2, 6, 8,
+  // above 3, 6, 7, below 4, 5, 8
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const bool xl = fg[q] & kL, xr = fg[q] & kR, yd = fg[q] & kD, yu = fg[q] & kU;
+    a[q][1] = xr ? a[q][1] : 0.0;
+    a[q][2] = xl ? a[q][2] : 0.0;
+    a[q][3] = yu ? a[q][3] : 0.0;
+    a[q][4] = yd ? a[q][4] : 0.0;
+    a[q][5] = xr && yd ? a[q][5] : 0.0;
+    a[q][6] = xl && yu ? a[q][6] : 0.0;
+    a[q][7] = xr && yu ? a[q][7] : 0.0;
+    a[q][8] = xl && yd ? a[q][8] : 0.0;
+  }
+  const auto stencil = [&](int q, const double* W, int row) {
+    const int c = v[q], m = c - (fg[q] & kD ? row : 0), p = c + (fg[q] & kU ? row : 0);
+    const int lft = fg[q] & kL ? -1 : 0, rgt = fg[q] & kR ? 1 : 0;
+    double s = a[q][0] * W[c];
+    s = fma(a[q][1], W[c + rgt], s);
+    s = fma(a[q][2], W[c + lft], s);
+    s = fma(a[q][3], W[p], s);
+    s = fma(a[q][4], W[m], s);
+    s = fma(a[q][5], W[m + rgt], s);
+    s = fma(a[q][6], W[p + lft], s);
+    s = fma(a[q][7], W[p + rgt], s);
+    return fma(a[q][8], W[m + lft], s);
+  };
   int o = 0;
   for (int l = lt; l < last; ++l) {
-    const int nx = M.lev[l].nx, ny = M.lev[l].ny, n = (int)M.lev[l].n, row = nx + 1;
-    // the right-hand side and the sweep from zero
+    const int row = M.lev[l].nx + 1;
+    // the sweep from zero
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      if (lev[q] == l) Z[o + py[q] * row + px[q]] = om * di[q] * r[q];
+      if (lev[q] == l) Z[v[q]] = di[q] * r[q];
     __syncthreads();
     if (l == 1 && converged<kTailThreads / 64>(st, rtol2, maxit, true, sh)) return;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      if (lev[q] == l) {
-        const int v = o + py[q] * row + px[q];
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < kStencil; ++k) {
-          const int x = px[q] + kOffX[k], y = py[q] + kOffY[k];
-          const bool on = x >= 0 && x <= nx && y >= 0 && y <= ny;
-          s = fma(on ? a[q][k] : 0.0, Z[on ? v + kOffY[k] * row + kOffX[k] : v], s);
-        }
-        Y[v] = di[q] == 0.0 ? 0.0 : r[q] - s;
-      }
+      if (lev[q] == l) Y[v[q]] = di[q] == 0.0 ? 0.0 : r[q] - stencil(q, Z, row);
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < Q; ++q)
       if (lev[q] == l + 1) {
-        const int I = px[q], J = py[q], fx = fine_of(I, nx), fy = fine_of(J, ny);
-        double s = 0.0;
-#pragma unroll
-        for (int dy = -1; dy <= 1; ++dy)
-#pragma unroll
-          for (int dx = -1; dx <= 1; ++dx) {
-            const int x = fx + dx, y = fy + dy;
-            const bool on = x >= 0 && x <= nx && y >= 0 && y <= ny;
-            s = fma(on ? pw1(x, nx, I) * pw1(y, ny, J) : 0.0, Y[on ? o + y * row + x : o], s);
-          }
+        // a fine neighbour of weight zero is read at the node itself
+        const int g = fg[q], c = f[q], m = c - (g & kFd ? row : 0), p = c + (g & kFu ? row : 0);
+        const int lft = g & kFl ? -1 : 0, rgt = g & kFr ? 1 : 0;
+        const double wl = g & kFl ? 0.5 : 0.0, wr = g & kFr ? 0.5 : 0.0;
+        const double s0 = fma(wl, Y[c + lft], fma(wr, Y[c + rgt], Y[c]));
+        const double sm = fma(wl, Y[m + lft], fma(wr, Y[m + rgt], Y[m]));
+        const double sp = fma(wl, Y[p + lft], fma(wr, Y[p + rgt], Y[p]));
+        const double s = fma(g & kFd ? 0.5 : 0.0, sm, fma(g & kFu ? 0.5 : 0.0, sp, s0));
         r[q] = di[q] == 0.0 ? 0.0 : s;
-        if (l + 1 == last) Z[off[q] + J * (M.lev[last].nx + 1) + I] = r[q];
+        if (l + 1 == last) Z[v[q]] = r[q];
       }
-    o += n;
+    o += (int)M.lev[l].n;
   }
   if (lt == last) {
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      if (lev[q] == last) Z[py[q] * (M.lev[last].nx + 1) + px[q]] = r[q];
+      if (lev[q] == last) Z[v[q]] = r[q];
   }
   __syncthreads();
   if (lt == last && lt == 1 && converged<kTailThreads / 64>(st, rtol2, maxit, true, sh)) return;
@@ -476,48 +513,39 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
     __syncthreads();
   }
   for (int l = last - 1; l >= lt; --l) {
-    const int nx = M.lev[l].nx, ny = M.lev[l].ny, row = nx + 1, cnx = M.lev[l + 1].nx;
-    const double* ec = X + o;
-    o -= (int)M.lev[l].n;
+    const int row = M.lev[l].nx + 1, cs = M.lev[l + 1].nx + 1;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-      if (lev[q] == l)
-        Y[o + py[q] * row + px[q]] =
-            di[q] == 0.0 ? 0.0 : fma(om * di[q], r[q], prolong_at(nx, ny, cnx, ec, px[q], py[q]));
+      if (lev[q] == l) {
+        const double* e = X + pa[q];
+        const int dx = fg[q] & kPx ? 1 : 0, dy = fg[q] & kPy ? cs : 0;
+        const double p = 0.25 * ((e[0] + e[dx]) + (e[dy] + e[dy + dx]));
+        Y[v[q]] = di[q] == 0.0 ? 0.0 : fma(di[q], r[q], p);
+      }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < Q; ++q)
       if (lev[q] == l) {
-        const int v = o + py[q] * row + px[q];
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < kStencil; ++k) {
-          const int x = px[q] + kOffX[k], y = py[q] + kOffY[k];
-          const bool on = x >= 0 && x <= nx && y >= 0 && y <= ny;
-          s = fma(on ? a[q][k] : 0.0, Y[on ? v + kOffY[k] * row + kOffX[k] : v], s);
-        }
-        const double ev = fma(om * di[q], r[q] - s, Y[v]);
-        X[v] = ev;
-        if (l == lt) M.lev[lt].e[v] = ev;
+        const double ev = fma(di[q], r[q] - stencil(q, Y, row), Y[v[q]]);
+        X[v[q]] = ev;
+        if (l == lt) M.lev[lt].e[v[q]] = ev;
       }
     if (l > lt) __syncthreads();
   }
   if (lt == last && cv < nc && ct == 0) M.lev[lt].e[cv] = X[cv];
 }
 
-int blocks_of(int64_t n) { return (int)((n + 255) / 256); }
-
 }  // namespace
 
+int v_rap_blocks(const MgLevel& C) { return (int)((16 * C.n + 255) / 256); }
 int v_restrict_blocks(const MgLevel& C) { return (C.nx / kRX + 1) * (C.ny / kRY + 1); }
 int v_post_blocks(const MgLevel& F) { return (F.nx / kPX + 1) * (F.ny / kPY + 1); }
 
 int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
-  for (int l = 1; l < M.tail; ++l) {
+  for (int l = 1; l + 1 < M.nlev; ++l) {
     const VOne rec{VRec{M.lev[l], M.lev[l + 1], nullptr, nullptr, 0}};
-    hipLaunchKernelGGL(mg_rap_kernel<VOne>, dim3(blocks_of(8 * M.lev[l + 1].n)), dim3(256), 0, s, rec);
+    hipLaunchKernelGGL(mg_rap_kernel<VOne>, dim3(v_rap_blocks(M.lev[l + 1])), dim3(256), 0, s, rec);
   }
-  hipLaunchKernelGGL(mg_tail_rap_kernel, dim3(1), dim3(1024), 0, s, dM);
   hipLaunchKernelGGL(mg_inverse_kernel, dim3(1), dim3(256), 0, s, dM);
   return (int)hipGetLastError();
 }
@@ -525,7 +553,6 @@ int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
 int mg_setup_levels_group(const MgSetupGroup& S, hipStream_t s) {
   for (int d = 1; d < S.ndepth; ++d)
     hipLaunchKernelGGL(mg_rap_kernel<VGroup>, dim3(S.grap[d]), dim3(256), 0, s, S.rap[d]);
-  hipLaunchKernelGGL(mg_tail_rap_kernel, dim3(S.ninst), dim3(1024), 0, s, S.dM);
   hipLaunchKernelGGL(mg_inverse_kernel, dim3(S.ninst), dim3(256), 0, s, S.dM);
   return (int)hipGetLastError();
 }
