@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, double om, doub
   constexpr int NE = (EX * EY + 255) / 256, ND = (WX * WY + 255) / 256;
   int lb;
   const VRec& R = vrec_of(sel, lb);
-  if (R.st->done) return;
+  const int done = R.st->done;
   const MgLevel& F = R.F;
   const MgLevel& Cc = R.C;
   const int ntx = Cc.nx / kRX + 1;
@@ -275,6 +275,7 @@ __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, double om, doub
     rv[k] = F.r[g];
     fr[k] = on && F.dinv[g] != 0.0;
   }
+  if (done) return;
   rr_part(R.part, R.npart, maxit, sh);
 #pragma unroll
   for (int k = 0; k < NE; ++k) {
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(256) void v_post_kernel(VS sel, double om) {
   __shared__ double e[EY * EX];
   int lb;
   const VRec& R = vrec_of(sel, lb);
-  if (R.st->done) return;
+  const int done = R.st->done;
   const MgLevel& F = R.F;
   const MgLevel& Cc = R.C;
   const int ntx = F.nx / kPX + 1;
@@ -334,15 +335,23 @@ __global__ __launch_bounds__(256) void v_post_kernel(VS sel, double om) {
 #pragma unroll
   for (int q = 0; q < kStencil; ++q) av[q] = F.a[q * F.n + g];
   const double rv = F.r[g], di = F.dinv[g];
-  for (int u = threadIdx.x; u < EX * EY; u += 256) {
-    const int x = x0 - 1 + u % EX, y = y0 - 1 + u / EX;
-    double v = 0.0;
-    if (x >= 0 && x <= F.nx && y >= 0 && y <= F.ny) {
-      const int64_t gg = (int64_t)y * row + x;
-      const double dd = F.dinv[gg], p = prolong_at(F.nx, F.ny, Cc.nx, Cc.e, x, y);
-      v = dd != 0.0 ? fma(om * dd, F.r[gg], p) : 0.0;
-    }
-    e[u] = v;
+  // the tile and its border, loaded with the stencils ahead of the branch
+  constexpr int NE = (EX * EY + 255) / 256;
+  double ev[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int u = threadIdx.x + 256 * k, x = x0 - 1 + u % EX, y = y0 - 1 + u / EX;
+    const bool on = u < EX * EY && x >= 0 && x <= F.nx && y >= 0 && y <= F.ny;
+    const int xc = on ? x : 0, yc = on ? y : 0;
+    const int64_t gg = (int64_t)yc * row + xc;
+    const double dd = F.dinv[gg], p = prolong_at(F.nx, F.ny, Cc.nx, Cc.e, xc, yc);
+    ev[k] = on && dd != 0.0 ? fma(om * dd, F.r[gg], p) : 0.0;
+  }
+  if (done) return;
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int u = threadIdx.x + 256 * k;
+    if (u < EX * EY) e[u] = ev[k];
   }
   __syncthreads();
   if (!own) return;
@@ -371,7 +380,7 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
   __shared__ double sh[kTailThreads / 64];
   const MgData& M = Ms[blockIdx.x];
   CgState* st = sts + blockIdx.x;
-  if (st->done) return;
+  const int done = st->done;
   const double om = M.omega_v;
   const int lt = M.tail, last = M.nlev - 1, tid = threadIdx.x;
   // own nodes: level; position in the vectors (v), of the fine node under it
@@ -434,6 +443,7 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
     const int u = ct + 8 * k;
     ci[k] = cv < nc && u < nc ? M.cinv[cv * nc + u] : 0.0;
   }
+  if (done) return;
   if (lt == 1) rr_part(M.part, M.npart, maxit, sh);
   // slots with a neighbour off the grid: to the right 1, 5, 7, left 2, 6, 8,
   // above 3, 6, 7, below 4, 5, 8

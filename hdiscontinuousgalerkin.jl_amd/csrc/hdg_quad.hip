@@ -73,6 +73,17 @@ __device__ __forceinline__ double psum(const double* p, int n, double* sh) {
   for (int i = threadIdx.x; i < n; i += kQuadThreads) s += p[i];
   return bsum(s, sh);
 }
+// A thread's share of n partials, loaded ahead of whatever follows: the CG
+// kernels read the solve's state and the partials of the kernel before them
+// in one flight and branch on `done` afterwards (each read is a trip to memory
+// past the XCD's own L2, most of a small problem's kernel time: 32^2 P1
+// product 6.5 -> see the product, residual 8.3).
+__device__ __forceinline__ double pshare(const double* p, int n) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += kQuadThreads) s += p[i];
+  asm volatile("" : "+v"(s));
+  return s;
+}
 
 // entry (a, b) of a triangle
 __device__ __forceinline__ constexpr int tri(int nt, int a, int b) { return dinv_slot(nt, a, b); }
@@ -687,7 +698,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_init_kernel(QuadSys S, Sel sel
   }
   if (RAND) {
     const double s = bsum(prz, sh);
-    if (threadIdx.x == 0) S.part[(size_t)S.nbt * 2 + I.pE + lb] = s;
+    if (threadIdx.x == 0) S.part[(size_t)S.nbt + I.pE + lb] = s;
   } else {
     const double s = bsum(pbb, sh);
     if (threadIdx.x == 0) S.part[(size_t)S.nbt * 4 + I.pE + lb] = s;
@@ -710,10 +721,12 @@ __global__ __launch_bounds__(kQuadThreads) void q_lupd_kernel(QuadSys S, Sel sel
   int lb;
   const QuadInst& I = inst_of(sel, lb);
   CgState* st = I.st;
-  if (st->done) return;
-  const int it = st->i_upd;
+  const int done = st->done, it = st->i_upd;
+  const double rz2[2] = {st->rz[0], st->rz[1]};
+  const double ps = pshare(S.part + I.pM, I.nbM);
+  if (done) return;
   if (lb == 0 && threadIdx.x == 0) st->i_spmv = it + 1;
-  const double pq = psum(S.part + I.pM, I.nbM, sh);
+  const double pq = bsum(ps, sh);
   if (!(pq > 0.0)) {
     if (lb == 0 && threadIdx.x == 0) {
       st->done = 3;
@@ -722,7 +735,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_lupd_kernel(QuadSys S, Sel sel
     return;
   }
   if (lb == 0 && threadIdx.x == 0) st->lpq[it] = pq;
-  const double alpha = st->rz[it & 1] / pq;
+  const double alpha = (it & 1 ? rz2[1] : rz2[0]) / pq;
   double prz = 0.0;
   for (int g = lb * kQuadThreads + threadIdx.x; g < I.G; g += I.nbE * kQuadThreads) {
     const int64_t o = at<NV>(I, g);
@@ -742,7 +755,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_lupd_kernel(QuadSys S, Sel sel
     }
   }
   const double s = bsum(prz, sh);
-  if (threadIdx.x == 0) S.part[(size_t)S.nbt * (1 + ((it + 1) & 1)) + I.pE + lb] = s;
+  if (threadIdx.x == 0) S.part[(size_t)S.nbt + I.pE + lb] = s;
 }
 
 // omega = factor / (largest eigenvalue of the Lanczos tridiagonal matrix of
@@ -754,23 +767,36 @@ __global__ __launch_bounds__(kQuadThreads) void q_omega_kernel(QuadSys S, Sel se
   __shared__ double sh[kNW];
   const QuadInst& I = inst_block(sel);
   CgState* st = I.st;
-  const double pq = psum(S.part + I.pM, I.nbM, sh);
+  const int done = st->done, its = st->it;
+  double lz[kQuadLanczos + 2], lpq[kQuadLanczos + 1];
+#pragma unroll
+  for (int j = 1; j <= kQuadLanczos; ++j) {
+    lz[j] = st->lz[j];
+    lpq[j] = st->lpq[j];
+  }
+  lz[kQuadLanczos + 1] = 0.0;
+  const double pq = bsum(pshare(S.part + I.pM, I.nbM), sh);
   if (threadIdx.x != 0) return;
-  if (st->done)
-    m = min(m, st->it);
-  else
+  if (done) {
+    m = min(m, its);
+  } else {
     st->lpq[m] = pq;
+#pragma unroll
+    for (int j = 1; j <= kQuadLanczos; ++j) lpq[j] = j == m ? pq : lpq[j];
+  }
   double d[kQuadLanczos], e2[kQuadLanczos];
   int n = 0;
-  for (int j = 1; j <= m; ++j) {
-    const double a = st->lz[j] / st->lpq[j];
+#pragma unroll
+  for (int j = 1; j <= kQuadLanczos; ++j) {
+    if (j > m || n != j - 1) continue;
+    const double a = lz[j] / lpq[j];
     double dj = 1.0 / a;
-    if (j > 1) dj += (st->lz[j] / st->lz[j - 1]) / (st->lz[j - 1] / st->lpq[j - 1]);
-    if (!(dj > 0.0) || !isfinite(dj)) break;
-    d[n] = dj;
-    e2[n] = j < m ? (st->lz[j + 1] / st->lz[j]) / (a * a) : 0.0;
-    if (!isfinite(e2[n])) break;
-    ++n;
+    if (j > 1) dj += (lz[j] / lz[j - 1]) / (lz[j - 1] / lpq[j - 1]);
+    if (!(dj > 0.0) || !isfinite(dj)) continue;
+    d[j - 1] = dj;
+    e2[j - 1] = j < m ? (lz[j + 1] / lz[j]) / (a * a) : 0.0;
+    if (!isfinite(e2[j - 1])) continue;
+    n = j;
   }
   if (n == 0) {
     st->omega = 0.5;
@@ -855,10 +881,26 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
   int lb;
   const QuadInst& I = inst_of(sel, lb);
   CgState* st = I.st;
-  if (!force && st->done) return;
-  const int it = force ? 2 : st->i_spmv;
   const size_t nbt = (size_t)S.nbt;
-  const double rz = psum(S.part + nbt * (1 + (it & 1)) + I.pE, I.nbE, sh);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ncol = I.W * I.NG;
+  const int done = st->done, it = force ? 2 : st->i_spmv, plain = *I.plain;
+  const double rz2[2] = {st->rz[0], st->rz[1]};
+  // z of the row a task starts on, loaded ahead of it
+  double zB[NT];
+  const auto start_row = [&](int task) {
+    const int c = task * kQuadOwn - 1 + lane;
+    const bool valid = c >= 0 && c < ncol;
+    const int grp = valid ? c / I.W : 0, i = valid ? c - grp * I.W : 0;
+    const int j = (grp * kNW + wave) * I.R + (wave == 0 ? -1 : 0);
+    const double* zp = S.z + at<NV>(I, valid && j >= 0 && j <= I.ny ? j * I.W + i : I.nx);
+#pragma unroll
+    for (int a = 0; a < NT; ++a) zB[a] = zp[a * 64];
+  };
+  start_row(lb);
+  const double ps = pshare(S.part + nbt + I.pE, I.nbE);
+  if (!force && done) return;
+  const double rz = bsum(ps, sh);
   const bool lead = lb == 0 && threadIdx.x == 0;
   if constexpr (LANCZOS) {
     if (!(rz > 0.0)) {
@@ -894,10 +936,8 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
       st->i_upd = it;
     }
   }
-  const double beta = it == 1 ? 0.0 : (force ? 0.5 : rz / st->rz[(it - 1) & 1]);
-  const double sf = S.shift && !*I.plain ? 1.0 : 0.0;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ncol = I.W * I.NG;
+  const double beta = it == 1 ? 0.0 : (force ? 0.5 : rz / (it & 1 ? rz2[0] : rz2[1]));
+  const double sf = S.shift && !plain ? 1.0 : 0.0;
   double part = 0.0;
   for (int task = lb; task < I.tasks; task += I.nbM) {
     const int c = task * kQuadOwn - 1 + lane;
@@ -905,16 +945,10 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
     const int grp = valid ? c / I.W : 0, i = valid ? c - grp * I.W : 0, j0 = (grp * kNW + wave) * I.R;
     const bool own = valid && lane >= 1 && lane < 63;
     const int first = wave == 0 ? -1 : 0;
-    double carry[NT], zB[NT], y0[NT];
-    {
-      const int j = j0 + first;
-      const double* zp = S.z + at<NV>(I, valid && j >= 0 && j <= I.ny ? j * I.W + i : I.nx);
+    double carry[NT], y0[NT];
 #pragma unroll
-      for (int a = 0; a < NT; ++a) {
-        carry[a] = y0[a] = 0.0;
-        zB[a] = zp[a * 64];
-      }
-    }
+    for (int a = 0; a < NT; ++a) carry[a] = y0[a] = 0.0;
+    if (task != lb) start_row(task);
     for (int s = first; s < I.R; ++s) {
       const int j = j0 + s;
       const bool ok = valid && j >= 0 && j <= I.ny, up = valid && j + 1 <= I.ny;
@@ -1056,14 +1090,16 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
   int lb;
   const QuadInst& I = inst_of(sel, lb);
   CgState* st = I.st;
-  if (!force && st->done) return;
   // the initial residual (0, nothing to update) or iteration i_upd
-  const int it = force ? 2 : st->i_upd;
+  const int done = st->done, it = force ? 2 : st->i_upd;
+  const double rz2[2] = {st->rz[0], st->rz[1]}, om = st->omega;
   const size_t nbt = (size_t)S.nbt;
+  const double ps = pshare(S.part + I.pM, I.nbM);
+  if (!force && done) return;
   double alpha = 0.0;
   if (!force) {
     if (it > 0) {
-      const double pq = psum(S.part + I.pM, I.nbM, sh);
+      const double pq = bsum(ps, sh);
       if (!(pq > 0.0)) {
         if (lb == 0 && threadIdx.x == 0) {
           st->done = 3;
@@ -1071,11 +1107,10 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
         }
         return;
       }
-      alpha = st->rz[it & 1] / pq;
+      alpha = (it & 1 ? rz2[1] : rz2[0]) / pq;
     }
     if (lb == 0 && threadIdx.x == 0) st->i_pre = it;
   }
-  const double om = st->omega;
   const double* __restrict__ rin = it & 1 ? S.r1 : S.r0;
   double* __restrict__ rout = it & 1 ? S.r0 : S.r1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1254,10 +1289,10 @@ __global__ __launch_bounds__(kQuadThreads) void q_smooth_kernel(QuadSys S, Sel s
   int lb;
   const QuadInst& I = inst_of(sel, lb);
   CgState* st = I.st;
-  if (st->done) return;
-  const int it = st->i_pre;
-  if (lb == 0 && threadIdx.x == 0) st->i_spmv = it + 1;
+  const int done = st->done, it = st->i_pre;
   const double om = st->omega;
+  if (done) return;
+  if (lb == 0 && threadIdx.x == 0) st->i_spmv = it + 1;
   const double* __restrict__ r = it & 1 ? S.r0 : S.r1;
   const double* __restrict__ e1 = I.e1;
   double prz = 0.0;
@@ -1298,7 +1333,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_smooth_kernel(QuadSys S, Sel s
     }
   }
   const double b = bsum(prz, sh);
-  if (threadIdx.x == 0) S.part[(size_t)S.nbt * (1 + ((it + 1) & 1)) + I.pE + lb] = b;
+  if (threadIdx.x == 0) S.part[(size_t)S.nbt + I.pE + lb] = b;
 }
 
 // ----------------------------------------------------------------- finish
