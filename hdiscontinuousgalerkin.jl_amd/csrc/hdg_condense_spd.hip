@@ -16,10 +16,10 @@
 // Cholesky factorisation (k = 3) and small matrix-vector products instead of
 // the elimination of its 30 x 30 local matrix.
 //
-// Mapping: 16 lanes per element (4 per wavefront); lane t < ntr carries
-// trace column t of R, U and K_e, lane ntr the rhs column (be, b_e); every
-// lane forms S and factors it, row by row, with the factor kept in LDS.  The
-// columns L^-1 R meet in LDS for the products of Ate.
+// Mapping: four lanes per element (16 per wavefront), a DPP quad.  Every lane
+// forms S and factors it in registers; lanes 0..2 carry the nt trace columns
+// of their face, one after another, lane 3 the rhs column.  The columns
+// Y = L^-1 R meet in LDS for the products of Ate.
 #include <hip/hip_runtime.h>
 
 #include "hdg_device.h"
@@ -33,97 +33,87 @@ template <int K>
 struct SpdDims {
   static constexpr int NU = (K + 1) * (K + 2) / 2, NQ = 2 * NU, M = 3 * NU, NT = K + 1, NTR = 3 * NT;
   static constexpr int NL = NU * (NU + 1) / 2;  // packed lower triangle
-  static constexpr int YS = NU * (NTR + 1);     // the L^-1 [R be] columns of one element
+  static constexpr int YS = NU * (NTR + 1) + NTR;  // LDS of one element: L^-1 [R be], Ate c
+  // tables staged in LDS: Gam, Z, then Om to the end
+  static constexpr int T1 = 18 * NU * NT;
   // table offsets (SpdLayout; the quadrature tables Nw, Mg follow at Nw)
   static constexpr int R = 0, C = 3 * NU * NU, Gam = 6 * NU * NU, Z = Gam + 6 * NU * NT, V = Z + 12 * NU * NT,
                        P = V + 6 * NU * NT, Om = P + 2 * NU * NU, H = Om + 36 * NT * NT, Nw = H + NT * NT;
 };
 
-constexpr int kSeg = 16;  // lanes per element
-constexpr int kEpw = 64 / kSeg;
+constexpr int kSeg = 16;  // lanes per element of the recovery
+constexpr int kCells = 64;  // elements per block of the condensation
 
 __host__ __device__ constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j; }  // i >= j
 
-// Entry ((fl,tl),(gs,us)) of Y'Y - E'A^-1 E - H for the lane's column y:
-// ys is column (gs,us) of Y in LDS, cg* the factors |e_f| |e_g| (n_f.n_g) /
-// detJ of the three faces g.
-template <int K>
-__device__ __forceinline__ double ate_entry(const double* T, const double* ys, const double (&y)[SpdDims<K>::NU],
-                                            int gs, int us, int fo, int fl, int tl, double el, double cg0,
-                                            double cg1, double cg2, const int (&ori)[3]) {
-  using D = SpdDims<K>;
-  constexpr int NU = D::NU, NT = D::NT;
-  double dot = 0.0;
-#pragma unroll
-  for (int i = 0; i < NU; ++i) dot += ys[i] * y[i];
-  const double cgs = gs == 0 ? cg0 : (gs == 1 ? cg1 : cg2);
-  const int og = gs == 0 ? ori[0] : (gs == 1 ? ori[1] : ori[2]);
-  const double om = T[D::Om + ((fo * 6 + gs * 2 + og) * NT + tl) * NT + us];
-  const double h = gs == fl ? el * T[D::H + tl * NT + us] : 0.0;
-  return dot - cgs * om - h;
-}
+// Tables read at compile-time offsets by every lane alike: through the scalar
+// cache, as operands that cost no vector register and no LDS.
+typedef const double __attribute__((address_space(4))) * ScalarTab;
 
-// WPE: waves per SIMD the register budget is cut for (2: 256 VGPRs, no
-// spills at k <= 2 and 60 B per lane at k = 3; 3: 168 VGPRs, 12-40 B of
-// spills per lane); the autotuner picks one, 2 by default.  GROUPED:
-// several instances packed into one mesh, the source of cell c is
+// WPE: waves per SIMD the register budget is cut for (2: none spilled at k <=
+// 2, 80 B per lane at k = 3; 3: 440 B at k = 3, 5.5 ms at 1024^2); the
+// autotuner picks one, 2 by default.
+// GROUPED: several instances packed into one mesh, the source of cell c is
 // srcs[cell_inst[c]].
+//
+// Bound by its stores (Ate, the u rows, 2.3 KB per cell at k = 3: 0.95 ms for
+// 1024^2 grid cells at the rate of a copy) and the issue of the products
+// beside them, at two waves per SIMD: 2.9 ms there, 0.29 at 768^2, k = 1.
+// With 16 lanes per element, one column each, the factor in LDS and every
+// table read from LDS by every element: 5.9 and 0.58 ms.
 template <int K, int WPE, bool GROUPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))
 void condense_spd_kernel(CondenseArgs a) {
   using D = SpdDims<K>;
   constexpr int NU = D::NU, M = D::M, NT = D::NT, NTR = D::NTR, NL = D::NL;
-  static_assert(NTR + 1 <= kSeg, "segment too small");
-  extern __shared__ double sh[];
+  extern __shared__ __align__(16) double sh[];
   const SpdLayoutDev L = a.spd;
-  for (int i = threadIdx.x; i < L.total; i += blockDim.x) sh[i] = __ldg(a.spd_tables + i);
+  const int tail = L.total - D::Om;
+  for (int i = threadIdx.x; i < D::T1; i += 256) sh[i] = a.spd_tables[D::Gam + i];
+  for (int i = threadIdx.x; i < tail; i += 256) sh[D::T1 + i] = a.spd_tables[D::Om + i];
   __syncthreads();
-  const double* T = sh;
+  const double* const TG = sh;                       // Gam
+  const double* const TZ = sh + 6 * NU * NT;         // Z
+  const double* const TO = sh + D::T1;               // Om
+  const double* const TH = TO + 36 * NT * NT;        // H
+  const double* const TN = TO + (D::Nw - D::Om);     // Nw, Mg
 
-  const int lane = threadIdx.x & 63;
-  const int seg = lane / kSeg, ls = lane - seg * kSeg, sbase = seg * kSeg;
-  // per element: the columns L^-1 [R be] (YS doubles), then L (NL)
-  double* Y = sh + L.total + ((threadIdx.x >> 6) * kEpw + seg) * (D::YS + NL);
-  double* Lb = Y + D::YS;
-  const int64_t wid = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
+  const int l = threadIdx.x & 3, slot = threadIdx.x >> 2;
+  double* const Y = sh + ((D::T1 + tail + 1) & ~1) + slot * D::YS;
+  double* const Rv = Y + NU * (NTR + 1);
   const int64_t count = a.mesh.nc;
   const int nqp = L.nqp;
   const double tau = a.tau;
-  // this lane's trace column: face fl, mode tl
-  const int fl = ls < NTR ? ls / NT : 0, tl = ls < NTR ? ls - fl * NT : 0;
+  const int fl = l < 3 ? l : 0;
 
-  for (int64_t base = wid * kEpw; base < count; base += nw * kEpw) {
-    const bool valid = base + seg < count;
-    const int64_t cell = valid ? base + seg : count - 1;
+  for (int64_t base = (int64_t)blockIdx.x * kCells; base < count; base += (int64_t)gridDim.x * kCells) {
+    const bool valid = base + slot < count;
+    const int64_t cell = valid ? base + slot : count - 1;
     Geo g;
     cell_geometry(a.mesh, cell, g);
     const SrcParams& S = GROUPED ? a.srcs[a.cell_inst[cell]] : a.src;
 
-    // be_i = sum_q w_q N_i(q) detJ f(x_q): lane q evaluates the source at
-    // point q, every lane sums over the points
-    double rc[NU];
+    // be_i = sum_q w_q N_i(q) detJ f(x_q): the lanes share the points
+    double rb[NU];
 #pragma unroll
-    for (int i = 0; i < NU; ++i) rc[i] = 0.0;
-    for (int q0 = 0; q0 < nqp; q0 += kSeg) {
-      const int q = q0 + ls;
-      double fv = 0.0;
-      if (q < nqp) {
-        double xq = 0.0, yq = 0.0;
+    for (int i = 0; i < NU; ++i) rb[i] = 0.0;
+    for (int q = l; q < nqp; q += 4) {
+      double xq = 0.0, yq = 0.0;
 #pragma unroll
-        for (int v = 0; v < 3; ++v) {
-          xq += T[L.Mg + v * nqp + q] * g.x[2 * v];
-          yq += T[L.Mg + v * nqp + q] * g.x[2 * v + 1];
-        }
-        fv = g.detJ * (S.kind == 3 ? __ldg(S.f_qp + cell + a.mesh.nc * (int64_t)q) : Src::f(S, xq, yq));
+      for (int v = 0; v < 3; ++v) {
+        xq += TN[NU * nqp + v * nqp + q] * g.x[2 * v];
+        yq += TN[NU * nqp + v * nqp + q] * g.x[2 * v + 1];
       }
-      const int qn = min(kSeg, nqp - q0);
-      for (int qq = 0; qq < qn; ++qq) {
-        const double fq = __shfl(fv, sbase + qq, 64);
+      const double fv = g.detJ * (S.kind == 3 ? __ldg(S.f_qp + cell + a.mesh.nc * (int64_t)q) : Src::f(S, xq, yq));
 #pragma unroll
-        for (int i = 0; i < NU; ++i) rc[i] += T[L.Nw + i * nqp + q0 + qq] * fq;
-      }
+      for (int i = 0; i < NU; ++i) rb[i] = fma(TN[i * nqp + q], fv, rb[i]);
     }
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      rb[i] += dpp_quad<0xB1>(rb[i]);
+      rb[i] += dpp_quad<0x4E>(rb[i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 
     // the lane's face: length, unit normal, orientation (blended, so that
     // the lane-dependent choice does not index the geometry)
@@ -133,154 +123,185 @@ void condense_spd_kernel(CondenseArgs a) {
     const double ny = w0 * g.nrm[1] + w1 * g.nrm[3] + w2 * g.nrm[5];
     const int of = (fl == 0) * g.ori[0] + (fl == 1) * g.ori[1] + (fl == 2) * g.ori[2];
     const int fo = fl * 2 + of;
-    // trace column: R = tau |e_f| Gam_fo + s0 Z_0fo + s1 Z_1fo with
-    // s_d = |e_f| (J^-1 n_f)_d
-    if (ls < NTR) {
-      const double s0 = el * (g.Ji[0] * nx + g.Ji[2] * ny), s1 = el * (g.Ji[1] * nx + g.Ji[3] * ny);
-      const double tf = tau * el;
-#pragma unroll
-      for (int i = 0; i < NU; ++i) {
-        rc[i] = tf * T[D::Gam + (fo * NU + i) * NT + tl] + s0 * T[D::Z + (fo * NU + i) * NT + tl] +
-                s1 * T[D::Z + ((6 + fo) * NU + i) * NT + tl];
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else if (ls > NTR) {
-#pragma unroll
-      for (int i = 0; i < NU; ++i) rc[i] = 0.0;
-    }
 
     // S = tau sum_f |e_f| Cref_f + detJ (G00 R00 + G01 R01 + G11 R11),
-    // G = J^-1 J^-T: lane i forms row i in the element's LDS buffer (in the
-    // space of the Y columns, which are written after the factorisation)
+    // G = J^-1 J^-T, and S = L L' in place (1 / L_ii on the diagonal)
+    double Lr[NL];
+    bool bad = !(g.detJ > 0.0);
     {
       const double c0 = tau * g.len[0], c1 = tau * g.len[1], c2 = tau * g.len[2];
       const double r0 = g.detJ * (g.Ji[0] * g.Ji[0] + g.Ji[2] * g.Ji[2]);
       const double r1 = g.detJ * (g.Ji[0] * g.Ji[1] + g.Ji[2] * g.Ji[3]);
       const double r2 = g.detJ * (g.Ji[1] * g.Ji[1] + g.Ji[3] * g.Ji[3]);
-      if (ls < NU) {
+      double dmax = 0.0;
+      // the tables' address is renewed row by row: loop-invariant to the
+      // compiler, all of their values would be kept (in spilled registers)
+      uintptr_t tab = (uintptr_t)a.spd_tables;
 #pragma unroll
-        for (int j = 0; j < NU; ++j) {
-          const int x = ls * NU + j;
-          Y[x] = c0 * T[D::C + x] + c1 * T[D::C + NU * NU + x] + c2 * T[D::C + 2 * NU * NU + x] +
-                 r0 * T[D::R + x] + r1 * T[D::R + NU * NU + x] + r2 * T[D::R + 2 * NU * NU + x];
-          __builtin_amdgcn_sched_barrier(0);
+      for (int i = 0; i < NU; ++i) {
+        asm volatile("" : "+s"(tab));
+        const ScalarTab TS = (ScalarTab)tab;
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+          const int x = i * NU + j;
+          Lr[tri(i, j)] = c0 * TS[D::C + x] + c1 * TS[D::C + NU * NU + x] + c2 * TS[D::C + 2 * NU * NU + x] +
+                          r0 * TS[D::R + x] + r1 * TS[D::R + NU * NU + x] + r2 * TS[D::R + 2 * NU * NU + x];
+          if (j % 2) __builtin_amdgcn_sched_barrier(0);
         }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // S = L L', row by row (left-looking): every lane of the element
-    // computes the same rows, lane 0 keeps them in LDS (row i packed,
-    // 1 / L_ii in place of L_ii); the forward solve rc <- L^-1 rc follows
-    // each row, in place
-    double dmax = 0.0;
-#pragma unroll
-    for (int i = 0; i < NU; ++i) dmax = fmax(dmax, Y[i * NU + i]);
-    bool bad = !(g.detJ > 0.0);
-#pragma unroll
-    for (int i = 0; i < NU; ++i) {
-      double li[NU];
-      double d = Y[i * NU + i];
-#pragma unroll
-      for (int j = 0; j < i; ++j) {
-        double v = Y[i * NU + j];
-#pragma unroll
-        for (int t = 0; t < j; ++t) v -= li[t] * Lb[tri(j, t)];
-        li[j] = v * Lb[tri(j, j)];
-        d -= li[j] * li[j];
+        dmax = fmax(dmax, Lr[tri(i, i)]);
         __builtin_amdgcn_sched_barrier(0);
       }
-      bad |= !(d > 1e-10 * dmax);
-      const double il = 1.0 / (d > 0.0 ? sqrt(d) : 1.0);
-      double v = rc[i];
 #pragma unroll
-      for (int t = 0; t < i; ++t) v -= li[t] * rc[t];
-      rc[i] = v * il;
-      if (ls == 0) {
+      for (int i = 0; i < NU; ++i) {
+        double d = Lr[tri(i, i)];
 #pragma unroll
-        for (int t = 0; t < i; ++t) Lb[tri(i, t)] = li[t];
-        Lb[tri(i, i)] = il;
+        for (int j = 0; j < i; ++j) {
+          double v = Lr[tri(i, j)];
+#pragma unroll
+          for (int t = 0; t < j; ++t) v -= Lr[tri(i, t)] * Lr[tri(j, t)];
+          v *= Lr[tri(j, j)];
+          Lr[tri(i, j)] = v;
+          d -= v * v;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        bad |= !(d > 1e-10 * dmax);
+        Lr[tri(i, i)] = 1.0 / (d > 0.0 ? sqrt(d) : 1.0);
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
 
-    // Ate = Y'Y - E'A^-1 E - H and bte = -Y' y_b, Y = L^-1 R: the columns
-    // meet in the element's LDS buffer (a wavefront's LDS instructions run
-    // in order, so the reads below see the writes)
-    if (ls <= NTR) {
+    // the columns Y = L^-1 R into LDS; trace column: R = tau |e_f| Gam_fo +
+    // s0 Z_0fo + s1 Z_1fo with s_d = |e_f| (J^-1 n_f)_d
+    {
+      const double s0 = el * (g.Ji[0] * nx + g.Ji[2] * ny), s1 = el * (g.Ji[1] * nx + g.Ji[3] * ny);
+      const double tf = tau * el;
+#pragma unroll 1
+      for (int t = 0; t < NT; ++t) {
+        double rc[NU];
 #pragma unroll
-      for (int i = 0; i < NU; ++i) Y[ls * NU + i] = rc[i];
+        for (int i = 0; i < NU; ++i) {
+          const double v = tf * TG[(fo * NU + i) * NT + t] + s0 * TZ[(fo * NU + i) * NT + t] +
+                           s1 * TZ[((6 + fo) * NU + i) * NT + t];
+          rc[i] = l < 3 ? v : rb[i];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < NU; ++i) {
+          double v = rc[i];
+#pragma unroll
+          for (int u = 0; u < i; ++u) v -= Lr[tri(i, u)] * rc[u];
+          rc[i] = v * Lr[tri(i, i)];
+        }
+        double* const y = Y + (l < 3 ? l * NT + t : NTR) * NU;
+#pragma unroll
+        for (int i = 0; i < NU; ++i) y[i] = rc[i];
+        // U = L^-T Y: the u rows of K_e (trace columns) and of b_e (rhs
+        // column), compact at the start of the cell's K_e and b_e blocks (U
+        // column-major nu x ntr); the q rows Q = A^-1 (B U - E) follow from
+        // them and the cell's geometry, and are formed where they are needed
+        // (recover_spd_kernel for the recovered q, expand_ke_spd_kernel for
+        // hdg_get_local_ops, which also restores the layout of K_e)
+#pragma unroll
+        for (int i = NU - 1; i >= 0; --i) {
+          double v = rc[i];
+#pragma unroll
+          for (int u = i + 1; u < NU; ++u) v -= Lr[tri(u, i)] * rc[u];
+          rc[i] = v * Lr[tri(i, i)];
+        }
+        if (valid && (l < 3 || t == 0)) {
+          double* out = l < 3 ? a.Ke + cell * (int64_t)(M * NTR) + (l * NT + t) * NU : a.be + cell * (int64_t)M;
+          if constexpr (NU % 2 == 0) {
+#pragma unroll
+            for (int i = 0; i < NU; i += 2) *reinterpret_cast<double2*>(out + i) = make_double2(rc[i], rc[i + 1]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < NU; ++i) out[i] = rc[i];
+          }
+        }
+      }
     }
+    // an element's lanes are of one wavefront, whose LDS instructions run in order
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    {
-      // E'A^-1 E entry ((f,t),(g,s)) = |e_f| |e_g| (n_f . n_g) / detJ Om_fo,gp(t,s)
-      const double sc = el / g.detJ;
-      const double cg0 = sc * g.len[0] * (nx * g.nrm[0] + ny * g.nrm[1]);
-      const double cg1 = sc * g.len[1] * (nx * g.nrm[2] + ny * g.nrm[3]);
-      const double cg2 = sc * g.len[2] * (nx * g.nrm[4] + ny * g.nrm[5]);
-      // Constant traces: for c = 1 on mode 0 of every face the local
-      // problem is solved by u = const, q = 0, so in exact arithmetic
-      // Ate c = F'u - H c = (tau - 1) H c (H carries no tau,
-      // poisson2D_HDG.jl:149).  The rounding of the shared tables breaks
-      // this the same way in every cell, an error the trace solve amplifies
-      // by cond(K) ~ h^-2 (1024^2 cells, P3: an L2 error of 6e-10 instead of
-      // 5e-13).  Ate is projected onto it, with d = Ate c - (tau - 1) H c:
-      //   Ate - (d c' + c d') / 3 + (c'd) c c' / 9,
-      // a symmetric change of the order of the rounding (~1e-15 relative).
-      double r_own = -(tau - 1.0) * el * T[D::H + tl * NT];
-#pragma unroll
-      for (int gs = 0; gs < 3; ++gs)
-        r_own += ate_entry<K>(T, Y + gs * NT * NU, rc, gs, 0, fo, fl, tl, el, cg0, cg1, cg2, g.ori);
-      const double r0 = __shfl(r_own, sbase + 0 * NT, 64), r1 = __shfl(r_own, sbase + 1 * NT, 64);
-      const double r2 = __shfl(r_own, sbase + 2 * NT, 64);
-      const double rsum = r0 + r1 + r2;
-      const double ct = tl == 0 ? 1.0 : 0.0;
-      if (valid && ls < NTR) {
-        double* at = a.Ate + cell * (int64_t)(NTR * NTR) + ls * NTR;
+
+    // Ate = Y'Y - E'A^-1 E - H and bte = -Y' y_b, column by column (Ate is
+    // symmetric: column s is stored as row s).  E'A^-1 E entry ((f,t),(g,s)) =
+    // |e_f| |e_g| (n_f . n_g) / detJ Om_fo,gp(t,s).
+    //
+    // Constant traces: for c = 1 on mode 0 of every face the local problem is
+    // solved by u = const, q = 0, so in exact arithmetic Ate c = F'u - H c =
+    // (tau - 1) H c (H carries no tau, poisson2D_HDG.jl:149).  The rounding of
+    // the shared tables breaks this the same way in every cell, an error the
+    // trace solve amplifies by cond(K) ~ h^-2 (1024^2 cells, P3: an L2 error
+    // of 6e-10 instead of 5e-13).  Ate is projected onto it, with d = Ate c -
+    // (tau - 1) H c:
+    //   Ate - (d c' + c d') / 3 + (c'd) c c' / 9,
+    // a symmetric change of the order of the rounding (~1e-15 relative).  The
+    // columns of modes t > 0 need their own d only, those of mode 0 all of it:
+    // t runs down, d through LDS.
+    const double sc = el / g.detJ;
+    const double cg[3] = {sc * g.len[0] * (nx * g.nrm[0] + ny * g.nrm[1]),
+                          sc * g.len[1] * (nx * g.nrm[2] + ny * g.nrm[3]),
+                          sc * g.len[2] * (nx * g.nrm[4] + ny * g.nrm[5])};
 #pragma unroll 1
-        for (int s = 0; s < NTR; ++s) {
-          const int gs = s / NT, us = s - gs * NT;
-          const double cs = us == 0 ? 1.0 : 0.0;
-          const double rs = gs == 0 ? r0 : (gs == 1 ? r1 : r2);
-          at[s] = ate_entry<K>(T, Y + s * NU, rc, gs, us, fo, fl, tl, el, cg0, cg1, cg2, g.ori) -
-                  (r_own * cs + ct * rs) * (1.0 / 3.0) + rsum * ct * cs * (1.0 / 9.0);
-        }
-        double bt = 0.0;
+    for (int t = NT - 1; t >= 0; --t) {
+      double y[NU], row[NTR];
+      // an offset the compiler takes as new from column to column: it would
+      // load all columns ahead, and hold them across the loop, otherwise
+      int o = 0;
+      asm volatile("" : "+v"(o));
+      const double* yo = Y + o + (l < 3 ? l * NT + t : NTR) * NU;
 #pragma unroll
-        for (int i = 0; i < NU; ++i) bt += Y[NTR * NU + i] * rc[i];
-        a.bte[cell * NTR + ls] = -bt;
+      for (int i = 0; i < NU; ++i) y[i] = yo[i];
+#pragma unroll
+      for (int gs = 0; gs < 3; ++gs) {
+        const double* om = TO + ((fo * 6 + gs * 2 + g.ori[gs]) * NT + t) * NT;
+        const double hl = gs == fl ? el : 0.0;
+#pragma unroll
+        for (int us = 0; us < NT; ++us) {
+          const double* ys = Y + o + (gs * NT + us) * NU;
+          double dot = 0.0;
+#pragma unroll
+          for (int i = 0; i < NU; ++i) dot = fma(ys[i], y[i], dot);
+          if ((gs * NT + us) % 2) asm volatile("" : "+v"(o), "+v"(dot));
+          row[gs * NT + us] = dot - cg[gs] * om[us] - hl * TH[t * NT + us];
+        }
+      }
+      double bt = 0.0;
+#pragma unroll
+      for (int i = 0; i < NU; ++i) bt = fma(Y[o + NTR * NU + i], y[i], bt);
+      const double d = ((row[0] + row[NT]) + row[2 * NT]) - (tau - 1.0) * el * TH[t * NT];
+      if (t > 0) {
+        if (l < 3) Rv[l * NT + t] = d;
+#pragma unroll
+        for (int gs = 0; gs < 3; ++gs) row[gs * NT] -= d * (1.0 / 3.0);
+      } else {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const double d0[3] = {dpp_quad<0x00>(d), dpp_quad<0x55>(d), dpp_quad<0xAA>(d)};
+        const double ds = (d0[0] + d0[1] + d0[2]) * (1.0 / 9.0);
+#pragma unroll
+        for (int gs = 0; gs < 3; ++gs) {
+          row[gs * NT] += ds - (d + d0[gs]) * (1.0 / 3.0);
+#pragma unroll
+          for (int us = 1; us < NT; ++us) row[gs * NT + us] -= Rv[gs * NT + us] * (1.0 / 3.0);
+        }
+      }
+      if (valid && l < 3) {
+        double* at = a.Ate + cell * (int64_t)(NTR * NTR) + (l * NT + t) * NTR;
+        if constexpr (NTR % 2 == 0) {
+#pragma unroll
+          for (int s = 0; s < NTR; s += 2) *reinterpret_cast<double2*>(at + s) = make_double2(row[s], row[s + 1]);
+        } else {
+#pragma unroll
+          for (int s = 0; s < NTR; ++s) at[s] = row[s];
+        }
+        a.bte[cell * NTR + l * NT + t] = -bt;
       }
     }
-    // rc <- L^-T rc (U, Ub), in place
-#pragma unroll
-    for (int i = NU - 1; i >= 0; --i) {
-      double v = rc[i];
-#pragma unroll
-      for (int t = i + 1; t < NU; ++t) v -= Lb[tri(t, i)] * rc[t];
-      rc[i] = v * Lb[tri(i, i)];
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    if (valid && bad && l == 0) atomicOr(a.err + (GROUPED ? a.cell_inst[cell] : 0), g.detJ > 0.0 ? 2 : 1);
     __builtin_amdgcn_wave_barrier();
-
-    // the u rows of K_e (U, trace columns) and of b_e (Ub, rhs column),
-    // compact at the start of the cell's K_e and b_e blocks (U column-major
-    // nu x ntr); the q rows Q = A^-1 (B U - E) follow from them and the
-    // cell's geometry, and are formed where they are needed
-    // (recover_spd_kernel for the recovered q, expand_ke_spd_kernel for
-    // hdg_get_local_ops, which also restores the layout of K_e): applied to
-    // one trace vector at recovery they cost an eighth of forming them here
-    // for every column, and their stores were a fifth of this kernel's time
-    if (valid && ls <= NTR) {
-      double* out = ls < NTR ? a.Ke + cell * (int64_t)(M * NTR) + ls * NU : a.be + cell * (int64_t)M;
-#pragma unroll
-      for (int i = 0; i < NU; ++i) out[i] = rc[i];
-    }
-    if (valid && bad && ls == 0) atomicOr(a.err + (GROUPED ? a.cell_inst[cell] : 0), g.detJ > 0.0 ? 2 : 1);
   }
 }
 
@@ -416,12 +437,11 @@ int spd_launch(const CondenseArgs& a, int wpe, int grid_cap, hipStream_t s) {
       L.Mg != D::Nw + D::NU * L.nqp || L.total != L.Mg + 3 * L.nqp)
     return (int)hipErrorInvalidValue;
   const int64_t n = a.mesh.nc;
-  const int64_t per_block = 4 * kEpw;
-  int64_t grid = (n + per_block - 1) / per_block;
+  int64_t grid = (n + kCells - 1) / kCells;
   const int64_t cap = grid_cap > 0 ? grid_cap : 16384;
   if (grid < 1) grid = 1;
   if (grid > cap) grid = cap;
-  const size_t lds = sizeof(double) * (a.spd.total + 4 * kEpw * (SpdDims<K>::YS + SpdDims<K>::NL));
+  const size_t lds = sizeof(double) * (((D::T1 + L.total - D::Om + 1) & ~1) + kCells * D::YS);
   if (wpe != 3) wpe = 2;
   if (a.srcs) {
     if (wpe == 2)
