@@ -258,7 +258,7 @@ int tune_group(hdg_batch* b, Group& g) {
 // and the block maps of their launches: instance j gets the blocks it would
 // get alone.
 int build_quad_group(hdg_batch* b, Group& g) {
-  const int n = (int)g.in.size(), nt = g.nt, qb = quad_build_quads(nt);
+  const int n = (int)g.in.size(), nt = g.nt;
   QuadSys& q = g.qs;
   std::vector<QuadInst> inst(n);
   std::vector<BlockMap> mM, mE, mQ;
@@ -285,8 +285,7 @@ int build_quad_group(hdg_batch* b, Group& g) {
     I.vmask = L.mask;
     for (int u = 0; u < I.nbM; ++u) mM.push_back(BlockMap{j, u});
     for (int u = 0; u < I.nbE; ++u) mE.push_back(BlockMap{j, u});
-    const int64_t nq = ((int64_t)I.nx * I.ny + qb - 1) / qb;
-    for (int64_t u = 0; u < nq; ++u) mQ.push_back(BlockMap{j, (int)u});
+    for (int u = 0; u < I.nbQ; ++u) mQ.push_back(BlockMap{j, u});
   }
   const size_t pts = (size_t)tiles * 64;
   BTRY(galloc(b, g, &q.blk, pts * quad_blk_vals(nt)));

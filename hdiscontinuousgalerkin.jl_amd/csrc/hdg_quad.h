@@ -38,6 +38,7 @@ struct QuadInst {
   // blocks of the marching and of the pointwise kernels; their first
   // partial sums
   int nbM = 0, nbE = 0, pM = 0, pE = 0;
+  int nbQ = 0;  // blocks of the set-up and finish kernels
   CgState* st = nullptr;
   int* plain = nullptr;  // != 0: a diagonal face has prescribed dofs (no constant shift)
   // vertex level 1
@@ -48,8 +49,6 @@ struct QuadInst {
 constexpr int kQuadOwn = 62;     // columns a wavefront of a marching kernel owns (64 less two halo lanes)
 constexpr int kQuadThreads = 256;
 void quad_plan(int nx, int ny, int nt, QuadInst& I);
-// quads per block of the set-up and finish kernels
-int quad_build_quads(int nt);
 
 // the arrays of one or several (packed) problems
 struct QuadSys {

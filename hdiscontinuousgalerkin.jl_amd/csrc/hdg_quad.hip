@@ -147,6 +147,14 @@ __global__ __launch_bounds__(kQuadThreads) void q_mask_kernel(QuadSys S, Sel sel
 // axis dofs) and quads per block.
 constexpr int lanes_per_quad(int nt) { return nt == 2 ? 8 : (nt <= 4 ? 16 : 32); }
 constexpr int quads_per_block(int nt) { return kQuadThreads / lanes_per_quad(nt); }
+// Stride of a quad's two staged cell blocks: the lanes of a quad read
+// neighbouring columns, so the quads of a wavefront are set 8 (two modes) or
+// 16 doubles apart modulo the 32 of an LDS row (unpadded, 288 doubles at four
+// modes put them all in the same banks).
+constexpr int quad_stride(int nt) {
+  const int n = 18 * nt * nt, want = nt == 2 ? 8 : 16;
+  return n + ((want - n) % 32 + 32) % 32;
+}
 
 // entry K[(f, a), (g, b)] of the assembled matrix
 template <int NT>
@@ -173,27 +181,55 @@ __device__ double k_entry(const QuadSys& S, int64_t f, int a, int64_t g, int b) 
 // From the assembled matrix: K_DD, the couplings and the loads split between
 // the two cells, the axis faces' own blocks left zero (q_diag_kernel adds
 // them).
+// The cells' blocks and loads of a block's quads on their way to LDS: every
+// load (and the kernel's own) is issued before the first is stored.  With a
+// loop of loads and stores the set-up was bound by that latency (1024^2 P3 2.4
+// ms, now 1.5; 768^2 P1 0.31, now 0.21; finish 1.06, now 0.80); several groups
+// per block, the next fetched ahead, took more registers than it hid (2.9 ms).
 template <int NT>
-__device__ __forceinline__ void stage_cells(const QuadSys& S, const QuadInst& I, int q0, int nq, double* A, double* b) {
-  constexpr int NTR = 3 * NT, CA = NTR * NTR;
-  if (!S.from_k) {
-    const double* src = S.Ate + (I.cell0 + 2 * (int64_t)q0) * CA;
-    if constexpr ((2 * CA) % 2 == 0) {
-      const double2* s2 = reinterpret_cast<const double2*>(src);
-      double2* d2 = reinterpret_cast<double2*>(A);
-      for (int e = threadIdx.x; e < nq * CA; e += kQuadThreads) d2[e] = s2[e];
-    }
+struct CellFetch {
+  static constexpr int CA = 9 * NT * NT, NTR = 3 * NT, QB = quads_per_block(NT);
+  static constexpr int NA = (QB * CA + kQuadThreads - 1) / kQuadThreads;
+  static constexpr int NL = (QB * 2 * NTR + kQuadThreads - 1) / kQuadThreads;
+  typedef double V2 __attribute__((ext_vector_type(2)));
+  V2 va[NA];
+  double vb[NL];
+  __device__ __forceinline__ void fetch(const QuadSys& S, const QuadInst& I, int q0, int nq) {
+    const V2* s2 = reinterpret_cast<const V2*>(S.Ate + (I.cell0 + 2 * (int64_t)q0) * CA);
     const double* sb = S.bte + (I.cell0 + 2 * (int64_t)q0) * NTR;
-    for (int e = threadIdx.x; e < nq * 2 * NTR; e += kQuadThreads) b[e] = sb[e];
-    return;
+#pragma unroll
+    for (int k = 0; k < NA; ++k) va[k] = s2[min((int)threadIdx.x + kQuadThreads * k, nq * CA - 1)];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) vb[k] = sb[min((int)threadIdx.x + kQuadThreads * k, nq * 2 * NTR - 1)];
   }
+  __device__ __forceinline__ void stage(double* A, double* b, int nq) const {
+    constexpr int QS = quad_stride(NT);
+    V2* d2 = reinterpret_cast<V2*>(A);
+#pragma unroll
+    for (int k = 0; k < NA; ++k) {
+      const int e = threadIdx.x + kQuadThreads * k;
+      if (e < nq * CA) d2[(e / CA) * (QS / 2) + e % CA] = va[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int e = threadIdx.x + kQuadThreads * k;
+      if (e < nq * 2 * NTR) b[e] = vb[k];
+    }
+  }
+};
+
+// The same from the assembled matrix (S.from_k).
+template <int NT>
+__device__ __forceinline__ void stage_assembled(const QuadSys& S, const QuadInst& I, int q0, int nq, double* A,
+                                                double* b) {
+  constexpr int NTR = 3 * NT, CA = NTR * NTR, QS = quad_stride(NT);
   for (int e = threadIdx.x; e < nq * 2 * CA; e += kQuadThreads) {
     const int q = q0 + e / (2 * CA), cell = (e / CA) & 1, r = (e % CA) / NTR, c = e % NTR;
     const int lr = r / NT, lc = c / NT, ld = cell;  // local face of D: 0 below, 1 above
     const int64_t c3 = 3 * (I.cell0 + 2 * (int64_t)q + cell);
     double v = 0.0;
     if (lr != lc || (lr == ld && cell == 0)) v = k_entry<NT>(S, S.cf[c3 + lr], r % NT, S.cf[c3 + lc], c % NT);
-    A[e] = v;
+    A[(e / (2 * CA)) * QS + e % (2 * CA)] = v;
   }
   for (int e = threadIdx.x; e < nq * 2 * NTR; e += kQuadThreads) {
     const int q = q0 + e / (2 * NTR), cell = (e / NTR) & 1, r = e % NTR, lr = r / NT;
@@ -245,29 +281,50 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
   constexpr int NTR = 3 * NT, CA = NTR * NTR, LPQ = lanes_per_quad(NT), QB = quads_per_block(NT);
   constexpr int NB = NT * NT, NS = NT * (NT + 1) / 2, NC = 4 * NT;
   constexpr int kOut = 6 * NB + 4 * NS + 9 * NT + kQuadCq;
-  static_assert(kOut <= 2 * CA, "the output staging reuses the cells' blocks");
-  __shared__ double A[QB * 2 * CA];
+  constexpr int QS = quad_stride(NT), WS = NT * NC + 2, OS = QB + 1;
+  static_assert(kOut * OS <= QB * QS, "the output staging reuses the cells' blocks");
+  __shared__ double A[QB * QS];
   __shared__ double bs[QB * 2 * NTR], us[QB * 2 * NTR];
-  __shared__ double Ws[QB * NT * NC];
+  __shared__ double Ws[QB * WS];
+  __shared__ int gq[QB];
   __shared__ double Ps[QB * 8 * 4];
   __shared__ unsigned char ms[QB * 2 * NTR];
   __shared__ int lift[QB];
   int lb;
   const QuadInst& I = inst_of(sel, lb);
   const int nquads = I.nx * I.ny;
-  const int q0 = lb * QB;
-  const int nq = min(QB, nquads - q0);
-  if (threadIdx.x < QB) lift[threadIdx.x] = 0;
+  const int q0 = lb * QB, nq = min(QB, nquads - q0);
+  // dofs of the quads' faces and their masks, fetched beside the cells' blocks
+  constexpr int NM = (QB * 2 * NTR + kQuadThreads - 1) / kQuadThreads;
+  CellFetch<NT> cells;
+  int64_t fd[NM];
+  unsigned char md[NM];
+#pragma unroll
+  for (int k = 0; k < NM; ++k) {
+    const int e = min((int)threadIdx.x + kQuadThreads * k, nq * 2 * NTR - 1), r = e % NTR;
+    fd[k] = (int64_t)S.cf[3 * (I.cell0 + 2 * (int64_t)q0 + e / NTR) + r / NT] * NT + r % NT;
+  }
+#pragma unroll
+  for (int k = 0; k < NM; ++k) md[k] = S.dmask[fd[k]];
+  if (!S.from_k) cells.fetch(S, I, q0, nq);
+  if (threadIdx.x < QB) {
+    const int q = q0 + min((int)threadIdx.x, nq - 1);
+    lift[threadIdx.x] = 0;
+    gq[threadIdx.x] = (q / I.nx) * I.W + q % I.nx;
+  }
+  if (S.from_k)
+    stage_assembled<NT>(S, I, q0, nq, A, bs);
+  else
+    cells.stage(A, bs, nq);
   __syncthreads();
-  stage_cells<NT>(S, I, q0, nq, A, bs);
-  for (int e = threadIdx.x; e < nq * 2 * NTR; e += kQuadThreads) {
-    const int q = e / (2 * NTR), r = e % NTR;
-    const int64_t f = S.cf[3 * (I.cell0 + 2 * (int64_t)q0 + e / NTR) + r / NT];
-    const unsigned char m = S.dmask[f * NT + r % NT];
-    const double u = m ? S.uD[f * NT + r % NT] : 0.0;
-    ms[e] = m;
+#pragma unroll
+  for (int k = 0; k < NM; ++k) {
+    const int e = threadIdx.x + kQuadThreads * k;
+    const double u = md[k] ? S.uD[fd[k]] : 0.0;
+    if (e >= nq * 2 * NTR) continue;
+    ms[e] = md[k];
     us[e] = u;
-    if (u != 0.0) lift[q] = 1;
+    if (u != 0.0) lift[e / (2 * NTR)] = 1;
   }
   __syncthreads();
   const int ql = threadIdx.x / LPQ, c = threadIdx.x % LPQ;
@@ -275,7 +332,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
   const int f = c / NT, b = c - f * NT;
   // cell and local face of B, T, L, R
   const int cell = f & 1, lf = f == 0 ? 2 : (f == 1 ? 0 : (f == 2 ? 1 : 2));
-  const double* Al = A + ql * 2 * CA;
+  const double* Al = A + ql * QS;
   const double* Au = Al + CA;
   double Tc[NC], w[NT], bD[NT], bred = 0.0, braw = 0.0, tpq[4] = {0, 0, 0, 0};
   if (live) {
@@ -317,7 +374,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
 #pragma unroll
     for (int a = 0; a < NT; ++a) {
       bred = fma(-w[a], y[a] * F.di[a], bred);
-      Ws[(ql * NT + a) * NC + c] = w[a];
+      Ws[ql * WS + a * NC + c] = w[a];
       w[a] *= F.di[a];
     }
     // the cell's own part of the column: rows of the faces of the same cell
@@ -333,13 +390,13 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
     for (int r = 0; r < NC; ++r) {
       double t = Tc[r];
 #pragma unroll
-      for (int a = 0; a < NT; ++a) t = fma(-Ws[(ql * NT + a) * NC + r], w[a], t);
+      for (int a = 0; a < NT; ++a) t = fma(-Ws[ql * WS + a * NC + r], w[a], t);
       Tc[r] = t;
     }
     // row c of T P on the quad's vertices (i,j), (i+1,j), (i,j+1), (i+1,j+1),
     // prescribed dofs and fixed vertices left out
     if (b < 2) {
-      const int q = q0 + ql, i = q % I.nx, j = q / I.nx, v0 = j * I.W + i;
+      const int v0 = gq[ql];
       const double keep[4] = {I.vmask[v0] ? 0.0 : 1.0, I.vmask[v0 + 1] ? 0.0 : 1.0, I.vmask[v0 + I.W] ? 0.0 : 1.0,
                               I.vmask[v0 + I.W + 1] ? 0.0 : 1.0};
       const unsigned char* mq = ms + ql * 2 * NTR;
@@ -360,7 +417,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
   __syncthreads();
   // outputs, value-major over the block's quads, in the LDS of the blocks
   double* const O = A;
-  auto put = [&](int s, double v) { O[s * QB + ql] = v; };
+  auto put = [&](int s, double v) { O[s * OS + ql] = v; };
   if (live) {
     // couplings (row face, column face) BT LR BL BR TL TR
 #pragma unroll
@@ -388,7 +445,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
   for (int e = threadIdx.x; e < nq * kQuadCq; e += kQuadThreads) {
     const int qe = e / kQuadCq, t = e % kQuadCq;
     const int u = t < 4 ? 0 : (t < 7 ? 1 : (t < 9 ? 2 : 3)), v = t < 4 ? t : (t < 7 ? t - 3 : (t < 9 ? t - 5 : 3));
-    const int q = q0 + qe, i = q % I.nx, j = q / I.nx, vx = (j + (u >> 1)) * I.W + i + (u & 1);
+    const int vx = gq[qe] + (u >> 1) * I.W + (u & 1);
     double s = 0.0;
     for (int fr = 0; fr < 4; ++fr) {
       const int lr = fr == 0 ? 2 : (fr == 1 ? 0 : (fr == 2 ? 1 : 2));
@@ -399,14 +456,14 @@ __global__ __launch_bounds__(kQuadThreads) void q_build_kernel(QuadSys S, Sel se
       if (!mf[0]) s = fma(0.5, pr[v], s);
       if (!mf[1]) s = fma(u == hi ? kS3 : -kS3, pr[4 + v], s);
     }
-    O[(6 * NB + 4 * NS + 9 * NT + t) * QB + qe] = I.vmask[vx] ? 0.0 : s;
+    O[(6 * NB + 4 * NS + 9 * NT + t) * OS + qe] = I.vmask[vx] ? 0.0 : s;
   }
   __syncthreads();
   for (int e = threadIdx.x; e < kOut * QB; e += kQuadThreads) {
     const int s = e / QB, qe = e % QB;
     if (qe >= nq) continue;
-    const int q = q0 + qe, g = (q / I.nx) * I.W + q % I.nx;
-    const double v = O[e];
+    const int g = gq[qe];
+    const double v = O[s * OS + qe];
     if (s < 6 * NB)
       S.blk[at<6 * NB>(I, g) + s * 64] = v;
     else if (s < 6 * NB + 4 * NS)
@@ -1346,7 +1403,8 @@ __global__ __launch_bounds__(kQuadThreads) void q_finish_kernel(QuadSys S, Sel s
                                                                int resid) {
   constexpr int NTR = 3 * NT, CA = NTR * NTR, LPQ = lanes_per_quad(NT), QB = quads_per_block(NT);
   constexpr int NV = 2 * NT, NC = 4 * NT;
-  __shared__ double A[QB * 2 * CA];
+  constexpr int QS = quad_stride(NT);
+  __shared__ double A[QB * QS];
   __shared__ double bs[QB * 2 * NTR], us[QB * 2 * NTR];
   __shared__ double ts[QB * NT];
   __shared__ unsigned char ms[QB * NT];
@@ -1354,7 +1412,12 @@ __global__ __launch_bounds__(kQuadThreads) void q_finish_kernel(QuadSys S, Sel s
   const QuadInst& I = inst_of(sel, lb);
   const int nquads = I.nx * I.ny;
   const int q0 = lb * QB, nq = min(QB, nquads - q0);
-  stage_cells<NT>(S, I, q0, nq, A, bs);
+  CellFetch<NT> cells;
+  if (!S.from_k) cells.fetch(S, I, q0, nq);
+  if (S.from_k)
+    stage_assembled<NT>(S, I, q0, nq, A, bs);
+  else
+    cells.stage(A, bs, nq);
   // the cells' trace values (D: the prescribed ones, zero on its free dofs)
   for (int e = threadIdx.x; e < nq * 2 * NTR; e += kQuadThreads) {
     const int ql = e / (2 * NTR), cell = (e / NTR) & 1, r = e % NTR, lr = r / NT, a = r % NT;
@@ -1379,7 +1442,7 @@ __global__ __launch_bounds__(kQuadThreads) void q_finish_kernel(QuadSys S, Sel s
   __syncthreads();
   const int ql = threadIdx.x / LPQ, c = threadIdx.x % LPQ;
   const bool live = ql < nq;
-  const double* Al = A + ql * 2 * CA;
+  const double* Al = A + ql * QS;
   const double* Au = Al + CA;
   const double* ul = us + ql * 2 * NTR;
   const double* bl = bs + ql * 2 * NTR;
@@ -1419,23 +1482,23 @@ __global__ __launch_bounds__(kQuadThreads) void q_finish_kernel(QuadSys S, Sel s
       uw[NTR + NT + a] = v;
     }
   }
-  if (!resid) return;
   __syncthreads();
-  if (!live || c >= NC) return;
-  const int q = q0 + ql, g = (q / I.nx) * I.W + q % I.nx;
-  double* out = S.bq + at<9 * NT>(I, g);
-  {
-    const int f = c / NT, b = c - f * NT, cell = f & 1, lf = f == 0 ? 2 : (f == 1 ? 0 : (f == 2 ? 1 : 2));
-    const double* row = (cell ? Au : Al) + (lf * NT + b) * NTR;
-    double t = -bl[cell * NTR + lf * NT + b];
-    for (int k = 0; k < NTR; ++k) t = fma(row[k], ul[cell * NTR + k], t);
-    out[c * 64] = t;
-  }
-  if (c < NT) {
-    double t = -(bl[c] + bl[NTR + NT + c]);
-    for (int k = 0; k < NTR; ++k) t = fma(Al[c * NTR + k], ul[k], t);
-    for (int k = 0; k < NTR; ++k) t = fma(Au[(NT + c) * NTR + k], ul[NTR + k], t);
-    out[(2 * NC + c) * 64] = ms[ql * NT + c] ? 0.0 : t;
+  if (resid && live && c < NC) {
+    const int q = q0 + ql, g = (q / I.nx) * I.W + q % I.nx;
+    double* out = S.bq + at<9 * NT>(I, g);
+    {
+      const int f = c / NT, b = c - f * NT, cell = f & 1, lf = f == 0 ? 2 : (f == 1 ? 0 : (f == 2 ? 1 : 2));
+      const double* row = (cell ? Au : Al) + (lf * NT + b) * NTR;
+      double t = -bl[cell * NTR + lf * NT + b];
+      for (int k = 0; k < NTR; ++k) t = fma(row[k], ul[cell * NTR + k], t);
+      out[c * 64] = t;
+    }
+    if (c < NT) {
+      double t = -(bl[c] + bl[NTR + NT + c]);
+      for (int k = 0; k < NTR; ++k) t = fma(Al[c * NTR + k], ul[k], t);
+      for (int k = 0; k < NTR; ++k) t = fma(Au[(NT + c) * NTR + k], ul[NTR + k], t);
+      out[(2 * NC + c) * 64] = ms[ql * NT + c] ? 0.0 : t;
+    }
   }
 }
 
@@ -1516,16 +1579,15 @@ void quad_plan(int nx, int ny, int nt, QuadInst& I) {
   }
   I.nbM = (int)std::min<int64_t>(I.tasks, 2048);
   I.nbE = std::min((I.ntiles + kNW - 1) / kNW, 1024);
+  I.nbQ = (int)(((int64_t)nx * ny + quads_per_block(nt) - 1) / quads_per_block(nt));
 }
-
-int quad_build_quads(int nt) { return quads_per_block(nt); }
 
 QuadLaunch quad_launch_one(const QuadInst& I, int nt) {
   QuadLaunch L;
   L.one = I;
   L.gM = I.nbM;
   L.gE = I.nbE;
-  L.gQ = (int)(((int64_t)I.nx * I.ny + quads_per_block(nt) - 1) / quads_per_block(nt));
+  L.gQ = I.nbQ;
   return L;
 }
 
