@@ -52,8 +52,18 @@ WORKLOADS = {
 STREAM_WORKLOADS = ("batched", "serving")
 
 
+def product_bytes(ctx, n):
+    """Algorithmic bytes of one CG product of the reduced trace system on n x
+    n grid cells (FP64), per grid point: the quad's six couplings and the two
+    faces' diagonal triangles (6 nt^2 + nt (nt + 1) doubles), z, p_old and
+    q_old read, p_new and q written (2 nt doubles each), the mask (2 bytes)."""
+    nt = ctx.sizes.nt
+    return (n + 1) ** 2 * (8 * (6 * nt * nt + nt * (nt + 1) + 10 * nt) + 2)
+
+
 def spmv_bytes(ctx):
-    """Algorithmic bytes of one trace-SpMV launch (FP64): the matrix values
+    """Algorithmic bytes of one trace-SpMV launch (FP64) of the block-Jacobi
+    preconditioned CG: the matrix values
     once, z (gathered), p_old and q_old read once (24 N), p_new and q
     written (16 N), the Dirichlet mask (N bytes).  Values: with
     symmetric face blocks (k = 3) the upper triangle of K_ff and the two
@@ -99,10 +109,10 @@ def condense_work(ctx, form):
 
 
 def measured_traffic(workload):
-    """HBM bytes per SpMV launch from the committed rocprofv3 counter
-    summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel
+    """HBM bytes per CG product (multigrid) from the committed rocprofv3
+    counter summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel
     calibration), or None if that summary is absent."""
-    path = os.path.join(REPO, "profiles", f"cg_spmv_{workload}_traffic.json")
+    path = os.path.join(REPO, "profiles", f"q_product_{workload}_traffic.json")
     if not os.path.exists(path):
         return None
     with open(path) as fh:
@@ -505,17 +515,18 @@ def main():
     l2sq = ctx.errornorm()
     iters = infos[-1].iters
 
-    # dominant kernel: one CG trace-SpMV launch, HIP events on ctx's stream
+    # dominant kernel: one CG product, HIP events on ctx's stream
+    bj = args.precond == "bj"
     spmv_us = ctx.time_kernel(0, reps=200)
     cond_us = ctx.time_kernel(2, reps=5)
     form = int(sched.get("condense_form", 0))
     cond_bytes, cond_flops = condense_work(ctx, form)
     cond_kernel = (f"condense_spd_kernel<{k}, {sched.get('condense_waves') or 2}>" if form == 1
                    else f"condense_kernel<{k}>")
-    ab = spmv_bytes(ctx)
+    ab = spmv_bytes(ctx) if bj else product_bytes(ctx, n)
     achieved = ab / (spmv_us * 1e-6) / 1e9
     copy_us = ctx.time_kernel(3, reps=3) if args.calibrate else None
-    traffic = measured_traffic(args.workload)
+    traffic = None if bj else measured_traffic(args.workload)
     nnz, ndofs = int(ctx.sizes.nnz), int(ctx.sizes.n_dofs)
 
     out = {
@@ -543,7 +554,7 @@ def main():
         "errornorm_sq": float(l2sq),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": f"cg_spmv_kernel<{nt}>", "avg_us": spmv_us, "bytes_per_launch": int(ab)},
+                     "kernel": f"cg_spmv_kernel<{nt}>" if bj else f"q_product_kernel<{nt}>", "avg_us": spmv_us, "bytes_per_launch": int(ab)},
         # the condensation kernel against both ceilings (FP64 dense MFMA peaks at the FP64
         # vector rate); it reaches neither
         "condense_roofline": {"kernel": cond_kernel,

@@ -59,8 +59,10 @@ typedef struct hdg_ctx hdg_ctx;
    only: HDG_ERR_UNSUPPORTED otherwise). */
 enum { HDG_FP64 = 0, HDG_MIXED = 1 };
 
-/* Preconditioners of the trace solve.  HDG_PC_AUTO picks multigrid when the
-   mesh is a structured rectangle_mesh and block-Jacobi otherwise. */
+/* Preconditioners of the trace solve.  HDG_PC_AUTO picks the geometric
+   multigrid of HDG_PC_MULTIGRID when the mesh is a structured rectangle_mesh
+   and, on other meshes, an aggregation multigrid over the mesh's vertices (or
+   block-Jacobi, see hdg_options). */
 enum { HDG_PC_AUTO = 0, HDG_PC_BLOCK_JACOBI = 1, HDG_PC_MULTIGRID = 2 };
 
 /* Schedule flags.  By default the first solve after hdg_setup launches its
@@ -289,7 +291,7 @@ int hdg_quadrature(int dim, int order, int cap, double* pts, double* w);
    HDG_CONDENSE_ELIMINATION, the elimination of the bordered local system
    with one element per segment of 16, 32 or 64 lanes (any width that holds
    the element's rows), or, where it applies (see HDG_SCHEDULE_LU),
-   HDG_CONDENSE_SCHUR, one element per 16 lanes with a register budget cut
+   HDG_CONDENSE_SCHUR, one element per 4 lanes with a register budget cut
    for 2 or 3 waves per SIMD.  Both stride a grid of blocks over the cells.
    hdg_autotune times every (width or register budget, grid cap) pair of the
    form the current problem takes, with HIP events, and keeps the fastest for
@@ -300,7 +302,8 @@ int hdg_quadrature(int dim, int order, int cap, double* pts, double* w);
    overwrites the assembled operators (assemble again before solving). */
 enum { HDG_CONDENSE_ELIMINATION = 0, HDG_CONDENSE_SCHUR = 1 };
 typedef struct {
-  int32_t condense_seg;   /* lanes per element (16 for the Schur form) */
+  int32_t condense_seg;   /* lanes per element (the Schur form has one width and
+                             reports 16) */
   int32_t condense_grid;  /* grid cap, blocks of 256 threads */
   double condense_us;     /* measured duration of the chosen schedule */
   double default_us;      /* of the default schedule: the narrowest width and
@@ -323,8 +326,10 @@ int hdg_set_schedule(hdg_ctx* ctx, const hdg_schedule* sched);
 /* ---- measurement --------------------------------------------------------- */
 /* Average device duration (microseconds) of one launch of an internal
    kernel, timed with HIP events around `reps` back-to-back launches on the
-   context stream with the data currently resident.  which: 0 = trace SpMV
-   (the dominant PCG kernel), 1 = PCG update, 2 = condensation, 3 = a plain
+   context stream with the data currently resident.  which: 0 = the CG
+   product (with the multigrid preconditioner on a structured mesh, that of
+   the reduced trace system), 1 = the CG update (there with the level-0
+   residual), 2 = condensation, 3 = a plain
    copy of the trace-matrix values (5 nt^2 doubles per face), the reference
    point for hardware traffic counters.  Timing runs overwrite the solver
    state; solve again before reading results. */
