@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void mg_rap_kernel(VS sel) {
 // row and column k take the same fma(-c, r, m) as the rest: the row's factor c
 // is p - 1, the column's r is 1 + 1/p (m - (p - 1) m/p = m/p, c - c (1 + 1/p)
 // = -c/p).  Bound by the chain of barrier, division and LDS.  With the pivot's
-// registers chosen at run time a step took 1.1 us (88 us at 81 nodes).
+// registers chosen at run time a step took 1.1 us (81 nodes: 88 us, now 52).
 __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restrict__ Ms) {
   constexpr int T = 16, E = kCoarseDirect / T;
   __shared__ double rowb[2][kCoarseDirect], colb[2][kCoarseDirect];
@@ -370,8 +370,8 @@ __global__ __launch_bounds__(256) void v_post_kernel(VS sel, double om) {
 // grid is read at the nearest node on it, with a zero coefficient.  Bound by
 // its chain of phases: two per level down (the residual, the restriction), one
 // for the coarsest grid, two per level up; every load comes before the first.
-// With the positions and weights worked out in every phase a 33 x 33 tail took
-// 17.4 us.
+// 33 x 33: 11.9 us, 17.4 with the positions and weights worked out in every
+// phase.
 __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __restrict__ Ms, CgState* sts, double rtol2,
                                                               int maxit) {
   constexpr int Q = (kTailNodes + kTailThreads - 1) / kTailThreads, NI = kCoarseDirect / 8;

@@ -76,8 +76,8 @@ __device__ __forceinline__ double psum(const double* p, int n, double* sh) {
 // A thread's share of n partials, loaded ahead of whatever follows: the CG
 // kernels read the solve's state and the partials of the kernel before them
 // in one flight and branch on `done` afterwards (each read is a trip to memory
-// past the XCD's own L2, most of a small problem's kernel time: 32^2 P1
-// product 6.5 -> see the product, residual 8.3).
+// past the XCD's own L2 and most of a small problem's kernel time: 32^2 P1
+// product 6.5 -> 6.4 us, residual 8.3 -> 7.9).
 __device__ __forceinline__ double pshare(const double* p, int n) {
   double s = 0.0;
   for (int i = threadIdx.x; i < n; i += kQuadThreads) s += p[i];
@@ -176,12 +176,8 @@ __device__ double k_entry(const QuadSys& S, int64_t f, int a, int64_t g, int b) 
   }
 }
 
-// The two cells' condensed blocks and loads of the block's quads into LDS,
-// A[quad][cell][row][column], b[quad][cell][row]; quads q0 .. q0 + nq - 1.
-// From the assembled matrix: K_DD, the couplings and the loads split between
-// the two cells, the axis faces' own blocks left zero (q_diag_kernel adds
-// them).
-// The cells' blocks and loads of a block's quads on their way to LDS: every
+// The two cells' condensed blocks and loads of the block's quads on their way
+// to LDS, A[quad][cell][row][column], b[quad][cell][row] (quads q0 .. q0 + nq - 1): every
 // load (and the kernel's own) is issued before the first is stored.  With a
 // loop of loads and stores the set-up was bound by that latency (1024^2 P3 2.4
 // ms, now 1.5; 768^2 P1 0.31, now 0.21; finish 1.06, now 0.80); several groups
@@ -218,7 +214,9 @@ struct CellFetch {
   }
 };
 
-// The same from the assembled matrix (S.from_k).
+// The same from the assembled matrix (S.from_k): K_DD, the couplings and the
+// loads split between the two cells, the axis faces' own blocks left zero
+// (q_diag_kernel adds them).
 template <int NT>
 __device__ __forceinline__ void stage_assembled(const QuadSys& S, const QuadInst& I, int q0, int nq, double* A,
                                                 double* b) {
@@ -929,6 +927,9 @@ __device__ __forceinline__ double shift_down(double v) { return __shfl_down(v, 1
 // to R handed to the next lane.  Row groups are laid end to end, so a
 // wavefront may run over the end of one group into the next.  HBM-bound:
 // 6 nt^2 + nt (nt+1) values of the matrix, 6 nt in and 4 nt out per point.
+// A window's 63 columns touch 4.9 cache lines on average where 62 doubles fill
+// 3.9; the rest is the next window's, so consecutive windows run on one XCD
+// (xcd_task).
 template <int NT, bool LANCZOS, class Sel>
 __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void q_product_kernel(QuadSys S, Sel sel, double rtol2, int maxit,
                                                                    int force) {
@@ -937,6 +938,7 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
   __shared__ double cs[(kNW + 1) * NT * 64];
   int lb;
   const QuadInst& I = inst_of(sel, lb);
+  lb = xcd_task(lb, I.nbM);
   CgState* st = I.st;
   const size_t nbt = (size_t)S.nbt;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1146,6 +1148,7 @@ __global__ __launch_bounds__(kQuadThreads, NT == 2 ? 4 : (NT == 3 ? 3 : 2)) void
   __shared__ double cs[(kNW + 1) * NT * 64], hs[(kNW + 1) * 64];
   int lb;
   const QuadInst& I = inst_of(sel, lb);
+  lb = xcd_task(lb, I.nbM);
   CgState* st = I.st;
   // the initial residual (0, nothing to update) or iteration i_upd
   const int done = st->done, it = force ? 2 : st->i_upd;
