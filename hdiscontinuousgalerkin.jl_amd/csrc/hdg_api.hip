@@ -36,6 +36,8 @@ struct hdg_ctx {
   bool recycling = false;
   std::unordered_multimap<size_t, void*> bin;
   size_t binned = 0;
+  // inside an export (Exporting): the solver's arrays may make room
+  bool exporting = false;
   hdg_arena* arena = nullptr;  // serving loop's arena, or null
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -177,9 +179,22 @@ struct Recycle {
   }
 };
 
+// In scope, an allocation beyond the budget first takes back the arrays that
+// only a solve needs (release_solver; the next solve makes them again), so that
+// an export fits wherever the solve does: the assembled matrix is allocated on
+// demand, beside the reduced system or in its place.
+struct Exporting {
+  hdg_ctx* c;
+  bool outer;
+  explicit Exporting(hdg_ctx* ctx, bool on = true) : c(ctx), outer(ctx->exporting) { c->exporting = on; }
+  ~Exporting() { c->exporting = outer; }
+};
+void release_solver(hdg_ctx* c);
+
 template <class T>
 int dalloc(hdg_ctx* c, T** p, size_t count) {
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+  if (c->budget && c->used + bytes > c->budget && c->exporting) release_solver(c);
   if (c->budget && c->used + bytes > c->budget)
     return fail(c, HDG_ERR_HBM_BUDGET, "device allocation of %zu bytes exceeds the budget (%zu of %zu used)",
                 bytes, c->used, c->budget);
@@ -256,6 +271,32 @@ void drop_graphs(hdg_ctx* c) {
   c->solves = 0;
 }
 
+// the reduced system of a multigrid context
+void free_quad(hdg_ctx* c) {
+  QuadSys& q = c->qs;
+  dfree(c, q.blk);
+  dfree(c, q.D);
+  dfree(c, q.Dinv);
+  dfree(c, q.tp);
+  dfree(c, q.bq);
+  dfree(c, q.cq);
+  dfree(c, q.fblk);
+  dfree(c, q.fDinv);
+  dfree(c, q.ftp);
+  dfree(c, q.mask);
+  dfree(c, q.x);
+  dfree(c, q.r0);
+  dfree(c, q.r1);
+  dfree(c, q.z);
+  dfree(c, q.p);
+  dfree(c, q.q);
+  dfree(c, q.res);
+  dfree(c, q.part);
+  dfree(c, c->d_plain);
+  dfree(c, c->d_mg);
+  q = QuadSys{};
+}
+
 void free_problem(hdg_ctx* c) {
   drop_graphs(c);
   dfree(c, c->d_tab);
@@ -281,32 +322,11 @@ void free_problem(hdg_ctx* c) {
   dfree(c, c->cg.part);
   dfree(c, c->d_uhat);
   dfree(c, c->d_part2);
-  QuadSys& q = c->qs;
-  dfree(c, q.blk);
-  dfree(c, q.D);
-  dfree(c, q.Dinv);
-  dfree(c, q.tp);
-  dfree(c, q.bq);
-  dfree(c, q.cq);
-  dfree(c, q.fblk);
-  dfree(c, q.fDinv);
-  dfree(c, q.ftp);
-  dfree(c, q.mask);
-  dfree(c, q.x);
-  dfree(c, q.r0);
-  dfree(c, q.r1);
-  dfree(c, q.z);
-  dfree(c, q.p);
-  dfree(c, q.q);
-  dfree(c, q.res);
-  dfree(c, q.part);
-  dfree(c, c->d_plain);
-  q = QuadSys{};
+  free_quad(c);
   c->filled = false;
   dfree(c, c->amg.top.g);
   dfree(c, c->amg.top.t);
   if (c->amg_state < 0) c->amg_state = 0;
-  dfree(c, c->d_mg);
   c->has_setup = c->assembled = c->solved = c->recovered = false;
   c->csched = CondenseSched{};
   c->tuned = false;
@@ -322,6 +342,13 @@ void free_amg(hdg_ctx* c) {
   dfree(c, c->amg.top.t);
   c->amg = AmgData{};
   c->amg_state = 0;
+}
+
+void release_solver(hdg_ctx* c) {
+  drop_graphs(c);
+  (void)hipStreamSynchronize(c->stream);
+  free_quad(c);
+  if (c->amg_state == 1) free_amg(c);
 }
 
 void free_mesh(hdg_ctx* c) {
@@ -529,6 +556,7 @@ int alloc_system(hdg_ctx* c) {
 // The assembled trace matrix and rhs of the current condensed blocks.
 int ensure_system(hdg_ctx* c) {
   if (c->filled) return HDG_OK;
+  Exporting room(c);
   TRY(alloc_system(c));
   LAUNCHCHK(c, launch_fill(c->mesh, c->pat, c->d_Ate, c->d_bte, c->T, c->stream));
   c->filled = true;
@@ -707,6 +735,27 @@ int setup_quad(hdg_ctx* c) {
   return HDG_OK;
 }
 
+// The reduced system for a solve: where an export took its place, that of the
+// assembled matrix.
+int ensure_quad(hdg_ctx* c) {
+  if (c->qs.part) return HDG_OK;
+  int r = setup_quad(c);
+  if (r == HDG_ERR_HBM_BUDGET) {
+    (void)hipStreamSynchronize(c->stream);
+    free_quad(c);
+    dfree(c, c->T.vals);
+    dfree(c, c->T.blk);
+    dfree(c, c->T.rhs);
+    c->filled = false;
+    r = setup_quad(c);
+  }
+  if (r != HDG_OK) {
+    (void)hipStreamSynchronize(c->stream);
+    free_quad(c);
+  }
+  return r;
+}
+
 // PCG iterations enqueued between convergence checks
 int chunk_of(Pc pc) { return pc == Pc::kJacobi ? 64 : 4; }
 
@@ -813,6 +862,8 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
       LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
       c->jacobi_dirty = false;
     }
+  } else {
+    TRY(ensure_quad(c));
   }
   const double rtol = c->opt.rtol > 0 ? c->opt.rtol : 1e-12;
   const int maxit = c->opt.maxit > 0 ? c->opt.maxit : 200000;
@@ -938,6 +989,7 @@ int system_out(hdg_ctx* c, int base, I* colptr, I* rowval, double* nzval, double
   TRY(ensure_system(c));
   if (!c->T.blk || !nzval) return export_csc(c, c->T.vals, c->T.rhs, base, colptr, rowval, nzval, rhs);
   double* vals = nullptr;
+  Exporting room(c);
   TRY(dalloc(c, &vals, (size_t)kSlots * c->nt * c->T.N));
   int r = HDG_OK;
   const int e = launch_expand_ell(c->pat, c->T, vals, c->stream);
@@ -1273,6 +1325,7 @@ int hdg_set_source(hdg_ctx* c, const hdg_source* s) {
   if (s->kind == 3) {
     if (!s->f_qp) return fail(c, HDG_ERR_ARG, "HDG_SRC_VALUES needs f_qp");
     const size_t n = (size_t)c->mesh.nc * c->nqp;
+    Exporting room(c);
     TRY(dalloc(c, &c->d_fqp, n));
     HIPCHK(c, hipMemcpyAsync(c->d_fqp, s->f_qp, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1462,6 +1515,7 @@ int hdg_get_applied_system(hdg_ctx* c, int64_t* colptr, int64_t* rowval, double*
   TRY(ensure_system(c));
   const int64_t N = c->T.N;
   double *vals = nullptr, *b = nullptr, *part = nullptr;
+  Exporting room(c);
   int r = dalloc(c, &vals, (size_t)kSlots * c->nt * N);
   if (r == HDG_OK) r = dalloc(c, &b, N);
   if (r == HDG_OK) r = dalloc(c, &part, 1024 + 1);
@@ -1524,6 +1578,7 @@ int hdg_get_element_blocks(hdg_ctx* c, int64_t first, int64_t count, double* A, 
                         (size_t)nu * ntr, (size_t)ntr * ntr, (size_t)nu};
   double* host[7] = {A, B, C, E, F, H, be};
   double* dev[7] = {nullptr};
+  Exporting room(c);
   int rc = HDG_OK;
   for (int i = 0; i < 7 && rc == HDG_OK; ++i)
     if (host[i]) rc = dalloc(c, &dev[i], sz[i] * count);
@@ -1617,8 +1672,9 @@ int hdg_time_kernel(hdg_ctx* c, int which, int reps, double* avg_us) {
   TRY(select_device(c));
   // make sure the solver state exists (pq, rz) so the kernels divide by
   // finite numbers; timing runs leave x and r untouched
-  const bool mg = use_mg(c);
-  if (!c->solved) {
+  const bool mg = use_mg(c), made = mg && which < 2 && !c->qs.part;
+  if (made) TRY(ensure_quad(c));
+  if ((!c->solved || made) && (!mg || c->qs.part)) {
     if (mg) {
       HIPCHK(c, hipMemsetAsync(c->d_plain, 0, sizeof(int), c->stream));
       LAUNCHCHK(c, launch_quad_build(c->qs, c->ql, c->stream));
@@ -1634,6 +1690,7 @@ int hdg_time_kernel(hdg_ctx* c, int which, int reps, double* avg_us) {
   // source: the face-ELL values, or (symmetric blocks) a second scratch half
   const double* csrc = c->T.vals;
   if (which == 3) {
+    Exporting room(c);
     TRY(dalloc(c, &scratch, c->T.vals ? ncopy : 2 * ncopy));
     if (!csrc) {
       csrc = scratch + ncopy;
@@ -1666,8 +1723,13 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   if (!c || !relres || outer < 0 || outer > 64 || !(inner_rtol >= 0.0)) return HDG_ERR_ARG;
   if (!c->assembled) return fail(c, HDG_ERR_STATE, "hdg_assemble_condense has not been called");
   TRY(select_device(c));
-  TRY(ensure_system(c));
   const bool mg = use_mg(c);
+  if (mg) TRY(ensure_quad(c));
+  TRY(ensure_system(c));
+  // both at once here
+  if (mg && !c->qs.part)
+    return fail(c, HDG_ERR_HBM_BUDGET, "the assembled matrix and the reduced system exceed the budget (%zu of %zu used)",
+                c->used, c->budget);
   for (int j = 0; j <= outer; ++j) relres[j] = std::nan("");
   if (inner_iters)
     for (int j = 0; j < outer; ++j) inner_iters[j] = 0;
@@ -1675,9 +1737,13 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   const int64_t nb = c->T.blk ? (int64_t)sym_blk_count(c->nt, c->mesh.nf) : 0;
   double *vr = nullptr, *vb = nullptr, *u = nullptr, *res = nullptr, *zero = nullptr, *part = nullptr;
   int rc = HDG_OK;
-  if ((!nv || (rc = dalloc(c, &vr, nv)) == HDG_OK) && (rc = dalloc(c, &u, N)) == HDG_OK && (rc = dalloc(c, &res, N)) == HDG_OK &&
-      (rc = dalloc(c, &zero, N)) == HDG_OK && (!nb || (rc = dalloc(c, &vb, nb)) == HDG_OK))
-    rc = dalloc(c, &part, refine_partials() + 1);
+  {
+    Exporting room(c, !mg);
+    if ((!nv || (rc = dalloc(c, &vr, nv)) == HDG_OK) && (rc = dalloc(c, &u, N)) == HDG_OK &&
+        (rc = dalloc(c, &res, N)) == HDG_OK &&
+        (rc = dalloc(c, &zero, N)) == HDG_OK && (!nb || (rc = dalloc(c, &vb, nb)) == HDG_OK))
+      rc = dalloc(c, &part, refine_partials() + 1);
+  }
   // graphs hold the operator's pointers: none is replayed or kept across the swap
   drop_graphs(c);
   const TraceSystem saved = c->T;
