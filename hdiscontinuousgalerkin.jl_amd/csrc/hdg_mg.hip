@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restric
 // zero: a block owns kRX x kRY coarse nodes and forms the residuals of their
 // (2 kRX + 1) x (2 kRY + 1) fine nodes once.  (Eight lanes per coarse node,
 // each forming the residuals it needs, 2.25 per fine node: 1024^2 P3 75 us
-// per V-cycle over all levels; now 70, at 512^2 29.)
+// per V-cycle over all levels; now 64, at 512^2 26.)
 constexpr int kRX = 16, kRY = 8;
 template <class VS>
 __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, double om, double rtol2, int maxit) {
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) void v_restrict_kernel(VS sel, double om, doub
 
 // e = e' + om dinv (r - A e'), e' = om dinv r + P ec on free nodes: the
 // prolongation and the post-smoothing sweep, a block owning kPX x kPY nodes
-// (47 us per V-cycle over all levels at 1024^2; 64 us with the prolongation
+// (37 us per V-cycle over all levels at 1024^2; 64 us with the prolongation
 // repeated at every neighbour that reads it).
 constexpr int kPX = 32, kPY = 8;
 template <class VS>
