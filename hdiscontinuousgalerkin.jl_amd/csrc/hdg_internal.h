@@ -575,8 +575,8 @@ int v_restrict_blocks(const MgLevel& C);
 int v_rap_blocks(const MgLevel& C);
 int v_post_blocks(const MgLevel& F);
 // Set-up tables of a group's vertex hierarchies: per depth d below their
-// tails, the instances with a level d+1, with block maps over 8 lanes per
-// coarse node (RAP).
+// tails, the instances with a level d+1, with block maps over the coarse
+// nodes (RAP).
 struct MgSetupGroup {
   int ninst = 0;
   const MgData* dM = nullptr;

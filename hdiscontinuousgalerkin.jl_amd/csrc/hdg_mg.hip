@@ -28,6 +28,7 @@ __constant__ int kOffX[kStencil] = {0, 1, -1, 0, 0, 1, -1, 1, -1};
 __constant__ int kOffY[kStencil] = {0, 0, 0, 1, -1, -1, 1, 1, -1};
 // slot of offset (dx, dy) at (dy + 1) 3 + dx + 1
 __device__ constexpr int kSlotOf[9] = {8, 4, 5, 2, 0, 1, 6, 3, 7};
+constexpr int kRapThreads = 64;  // a wavefront per block: the small levels spread over the CUs
 
 // fine index of coarse index I on a side of n fine cells
 __device__ __forceinline__ int fine_of(int I, int n) { return min(2 * I, n); }
@@ -81,84 +82,95 @@ __device__ __forceinline__ bool converged(CgState* st, double rtol2, int maxit, 
 }
 
 // ------------------------------------------------------------ set-up
-// Galerkin stencil R A P, R = P^T, of coarse node C by 16 lanes: lane t takes
-// the fine node at support offset t (seven lanes only help to sum), and a
-// fixed shuffle tree sums the lanes.  Bound by two dependent loads and the
-// weights' arithmetic on the small levels, by the fine stencils on the large
-// ones.  Eight lanes with two nodes on one of them, the small levels in one
-// workgroup: 41 us for 33 x 33 down to 9 x 9.
-__device__ __forceinline__ void rap_node(const MgLevel& F, const MgLevel& Cc, int64_t C, int t) {
-  const int cnx = Cc.nx, cny = Cc.ny, fnx = F.nx, fny = F.ny;
-  const bool live = C < Cc.n;
-  const int I = live ? (int)(C % (cnx + 1)) : 0, J = live ? (int)(C / (cnx + 1)) : 0;
-  auto fixed = [&](int i, int j) { return F.mask[(int64_t)fine_of(j, fny) * (fnx + 1) + fine_of(i, fnx)] != 0; };
-  const bool cm = !live || fixed(I, J);
+// Galerkin stencils R A P, R = P^T, a thread per coarse node C: the stencils of
+// its support's fine nodes, three at a time, weighted and summed by the node
+// they meet, then interpolated, first in x, then in y.  Consecutive threads
+// read every other column of a row, so the fine stencils leave HBM once; the
+// small levels are bound by two dependent loads.  With 16 lanes per coarse
+// node, each spreading one fine node's stencil, and a shuffle tree over the
+// lanes: all levels of 1024^2 980 us, now 417 (beside the Lanczos steps), of
+// 768^2 288, now 132, a 17 x 17 level 10, now 6.
+template <class VS>
+__global__ __launch_bounds__(kRapThreads) void mg_rap_kernel(VS sel) {
+  int lb;
+  const VRec& R = vrec_of(sel, lb);
+  const MgLevel& F = R.F;
+  const MgLevel& Cc = R.C;
+  const int64_t C = (int64_t)lb * kRapThreads + threadIdx.x;
+  if (C >= Cc.n) return;
+  constexpr int ox[kStencil] = {0, 1, -1, 0, 0, 1, -1, 1, -1}, oy[kStencil] = {0, 0, 0, 1, -1, -1, 1, 1, -1};
+  const int cnx = Cc.nx, cny = Cc.ny, fnx = F.nx, fny = F.ny, row = fnx + 1;
+  const int I = (int)(C % (cnx + 1)), J = (int)(C / (cnx + 1)), fx = fine_of(I, fnx), fy = fine_of(J, fny);
+  const int64_t f0 = (int64_t)fy * row + fx;
+  // fine nodes that are fixed or off the grid
+  unsigned off = 0;
+#pragma unroll
+  for (int p = 0; p < 25; ++p) {
+    const int x = fx + p % 5 - 2, y = fy + p / 5 - 2;
+    const bool on = x >= 0 && x <= fnx && y >= 0 && y <= fny;
+    const unsigned char m = F.mask[on ? (int64_t)y * row + x : f0];
+    if (!on || m) off |= 1u << p;
+  }
+  // own weight at the fine nodes beside C's, per side; their other parent has
+  // the rest (an odd side's last node is a parent of its own)
+  const double lx = fx & 1 ? 0.0 : 0.5, rx = fx + 1 == fnx ? 0.0 : 0.5;
+  const double ly = fy & 1 ? 0.0 : 0.5, ry = fy + 1 == fny ? 0.0 : 0.5;
   double st[kStencil];
 #pragma unroll
   for (int k = 0; k < kStencil; ++k) st[k] = 0.0;
-  if (!cm && t < kStencil) {
-    const int o = t;
-    const int fx = fine_of(I, fnx) + kOffX[o], fy = fine_of(J, fny) + kOffY[o], row = fnx + 1;
-    const bool in = fx >= 0 && fx <= fnx && fy >= 0 && fy <= fny;
-    const int64_t fi = in ? (int64_t)fy * row + fx : 0;
-    // the stencil and the masks it meets in one go; points off the grid read
-    // the fine node itself
-    double av[kStencil];
-    unsigned char gm[kStencil];
+  // byte offset of the support's centre (a level has fewer than 2^29 nodes)
+  unsigned f1 = 8u * (unsigned)f0;
 #pragma unroll
-    for (int s = 0; s < kStencil; ++s) {
-      const int gx = fx + kOffX[s], gy = fy + kOffY[s];
-      const bool on = in && gx >= 0 && gx <= fnx && gy >= 0 && gy <= fny;
-      av[s] = F.a[s * F.n + fi];
-      gm[s] = F.mask[on ? fi + kOffY[s] * row + kOffX[s] : fi];
-      if (!on) gm[s] = 1;
-    }
-    const double w1 = in && !F.mask[fi] ? pw1(fx, fnx, I) * pw1(fy, fny, J) : 0.0;
-    double wx[3][3], wy[3][3];  // weight of coarse offset d at fine offset s
+  for (int y = -1; y <= 1; ++y) {
+    // the next row's loads wait for this one's sums (all at once take 254
+    // registers, and the blocks then wait for room beside the kernels of other
+    // streams: up to 440 us in a batch)
+    if (y >= 0) asm("" : "+v"(f1), "+v"(st[0]));
+    double t[3][5];
 #pragma unroll
-    for (int s = -1; s <= 1; ++s)
+    for (int k = 0; k < 15; ++k) t[k / 5][k % 5] = 0.0;
 #pragma unroll
-      for (int d = -1; d <= 1; ++d) {
-        wx[s + 1][d + 1] = pw1(fx + s, fnx, I + d);
-        wy[s + 1][d + 1] = w1 * pw1(fy + s, fny, J + d);
+    for (int x = -1; x <= 1; ++x) {
+      const bool use = !((off >> ((y + 2) * 5 + x + 2)) & 1);
+      const unsigned fi = use ? f1 + 8u * (unsigned)(y * row + x) : f1;
+      const double w = use ? (x == 0 ? 1.0 : (x < 0 ? lx : rx)) * (y == 0 ? 1.0 : (y < 0 ? ly : ry)) : 0.0;
+#pragma unroll
+      for (int s = 0; s < kStencil; ++s) {
+        double& v = t[oy[s] + 1][x + ox[s] + 2];
+        v = fma(w, *reinterpret_cast<const double*>(reinterpret_cast<const char*>(F.a + s * F.n) + fi), v);
       }
-    constexpr int ox[kStencil] = {0, 1, -1, 0, 0, 1, -1, 1, -1}, oy[kStencil] = {0, 0, 0, 1, -1, -1, 1, 1, -1};
+    }
 #pragma unroll
-    for (int s = 0; s < kStencil; ++s) {
-      const double v = gm[s] ? 0.0 : av[s];
+    for (int q = 0; q < 3; ++q) {
+      const int py = y + q + 1;
+      double v[5];
+#pragma unroll
+      for (int px = 0; px < 5; ++px) v[px] = (off >> (py * 5 + px)) & 1 ? 0.0 : t[q][px];
+      const double u[3] = {fma(1.0 - lx, v[1], v[0]), fma(lx, v[1], fma(rx, v[3], v[2])), fma(1.0 - rx, v[3], v[4])};
+      // parents in y: below C's row, C's, above
+      const double wy[3] = {py == 0 ? 1.0 : (py == 1 ? 1.0 - ly : 0.0), py == 1 ? ly : (py == 2 ? 1.0 : ry),
+                            py == 4 ? 1.0 : (py == 3 ? 1.0 - ry : 0.0)};
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy) {
-        const double ay = v * wy[oy[s] + 1][dy];
+        if ((dy == 0 && py > 1) || (dy == 1 && (py == 0 || py == 4)) || (dy == 2 && py < 3)) continue;
 #pragma unroll
-        for (int dx = 0; dx < 3; ++dx) st[kSlotOf[dy * 3 + dx]] = fma(ay, wx[ox[s] + 1][dx], st[kSlotOf[dy * 3 + dx]]);
+        for (int dx = 0; dx < 3; ++dx) st[kSlotOf[dy * 3 + dx]] = fma(wy[dy], u[dx], st[kSlotOf[dy * 3 + dx]]);
       }
     }
   }
-#pragma unroll
-  for (int u = 0; u < kStencil; ++u) {
-#pragma unroll
-    for (int k = 1; k < 16; k <<= 1) st[u] += __shfl_xor(st[u], k, 16);
-  }
-  if (t != 0 || !live) return;
+  const bool cm = (off >> 12) & 1;
 #pragma unroll
   for (int dy = -1; dy <= 1; ++dy)
 #pragma unroll
     for (int dx = -1; dx <= 1; ++dx) {
       const int u = kSlotOf[(dy + 1) * 3 + dx + 1], i = I + dx, j = J + dy;
       // columns of fixed coarse nodes are zero; fixed rows are the identity
-      const bool off = i < 0 || i > cnx || j < 0 || j > cny || cm || fixed(i, j);
-      Cc.a[u * Cc.n + C] = cm ? (u == 0 ? 1.0 : 0.0) : (off ? 0.0 : st[u]);
+      const bool in = i >= 0 && i <= cnx && j >= 0 && j <= cny;
+      const int p = in ? (fine_of(j, fny) - fy + 2) * 5 + fine_of(i, fnx) - fx + 2 : 12;
+      Cc.a[u * Cc.n + C] = cm ? (u == 0 ? 1.0 : 0.0) : (!in || ((off >> p) & 1) ? 0.0 : st[u]);
     }
   Cc.dinv[C] = cm ? 0.0 : 1.0 / st[0];
   Cc.mask[C] = cm ? 1 : 0;
-}
-
-template <class VS>
-__global__ __launch_bounds__(256) void mg_rap_kernel(VS sel) {
-  int lb;
-  const VRec& R = vrec_of(sel, lb);
-  const int64_t gid = (int64_t)lb * blockDim.x + threadIdx.x;
-  rap_node(R.F, R.C, gid >> 4, (int)(gid & 15));
 }
 
 // Inverse of the coarsest operator (at most kCoarseDirect nodes), one
@@ -547,14 +559,14 @@ __global__ __launch_bounds__(kTailThreads) void v_tail_kernel(const MgData* __re
 
 }  // namespace
 
-int v_rap_blocks(const MgLevel& C) { return (int)((16 * C.n + 255) / 256); }
+int v_rap_blocks(const MgLevel& C) { return (int)((C.n + kRapThreads - 1) / kRapThreads); }
 int v_restrict_blocks(const MgLevel& C) { return (C.nx / kRX + 1) * (C.ny / kRY + 1); }
 int v_post_blocks(const MgLevel& F) { return (F.nx / kPX + 1) * (F.ny / kPY + 1); }
 
 int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
   for (int l = 1; l + 1 < M.nlev; ++l) {
     const VOne rec{VRec{M.lev[l], M.lev[l + 1], nullptr, nullptr, 0}};
-    hipLaunchKernelGGL(mg_rap_kernel<VOne>, dim3(v_rap_blocks(M.lev[l + 1])), dim3(256), 0, s, rec);
+    hipLaunchKernelGGL(mg_rap_kernel<VOne>, dim3(v_rap_blocks(M.lev[l + 1])), dim3(kRapThreads), 0, s, rec);
   }
   hipLaunchKernelGGL(mg_inverse_kernel, dim3(1), dim3(256), 0, s, dM);
   return (int)hipGetLastError();
@@ -562,7 +574,7 @@ int mg_setup_levels(const MgData& M, const MgData* dM, hipStream_t s) {
 
 int mg_setup_levels_group(const MgSetupGroup& S, hipStream_t s) {
   for (int d = 1; d < S.ndepth; ++d)
-    hipLaunchKernelGGL(mg_rap_kernel<VGroup>, dim3(S.grap[d]), dim3(256), 0, s, S.rap[d]);
+    hipLaunchKernelGGL(mg_rap_kernel<VGroup>, dim3(S.grap[d]), dim3(kRapThreads), 0, s, S.rap[d]);
   hipLaunchKernelGGL(mg_inverse_kernel, dim3(S.ninst), dim3(256), 0, s, S.dM);
   return (int)hipGetLastError();
 }
