@@ -44,9 +44,12 @@ struct AmgLevel {
 // The trace space beside level 0: fv[4f + j] = the ends of face f (lower id,
 // higher id) and the vertices opposite to it in its cells (or -1); per vertex
 // the codes 4f + j that name it; af = the face between the two vertices of an
-// entry of level 0's operator (-1 on the diagonal).
+// entry of level 0's operator (-1 on the diagonal; two entries where the mesh is
+// cut open along an edge).  cv = the cells' vertices: their nodes, or, where a
+// face joins two edges of the mesh, one node for those it brings together.
 struct AmgTop {
   int n = 0;
+  const int* cv = nullptr;
   const int *fv = nullptr, *vp = nullptr, *vi = nullptr, *af = nullptr;
   unsigned char* vfix = nullptr;  // vertex of a face with prescribed dofs
   double* g = nullptr;            // G: row r of vertex j at g[j N + r]
@@ -72,7 +75,8 @@ struct AmgPlan {
     int n = 0, nnz = 0, gnnz = 0;
     size_t ap, ai, agg, gp, gi, tp, ti, tx;
   } lev[kAmgLevels];
-  size_t fv, vp, vi, af;
+  size_t fv, vp, vi, af, cv = 0;
+  bool joined = false;  // cv is there
   std::vector<int> ints;
 };
 // false: the mesh's lists do not fit 32-bit indices

@@ -36,18 +36,19 @@ __global__ __launch_bounds__(256) void amg_fix_kernel(AmgTop A, TraceSystem T) {
 }
 
 // Local index of vertex v in cell c (-1: not there), and the weight of mode 1
-// of v's hat function on the cell's face lf (v an end of it).
-__device__ __forceinline__ int local_of(const int* __restrict__ cn, int64_t c, int v) {
-  return cn[3 * c] == v ? 0 : (cn[3 * c + 1] == v ? 1 : (cn[3 * c + 2] == v ? 2 : -1));
+// of v's hat function on the cell's face lf (v an end of it; the face runs from
+// its lower node id to the higher in either cell).
+__device__ __forceinline__ int local_of(const int* __restrict__ cv, int64_t c, int v) {
+  return cv[3 * c] == v ? 0 : (cv[3 * c + 1] == v ? 1 : (cv[3 * c + 2] == v ? 2 : -1));
 }
 __device__ __forceinline__ double mode1(const int* __restrict__ cn, int64_t c, int lv, int lf) {
   return cn[3 * c + lv] > cn[3 * c + 3 - lv - lf] ? kQ : -kQ;
 }
 
 // (hat v)^T (-Ate_c) (hat w)
-__device__ double cell_stiffness(const int* __restrict__ cn, const double* __restrict__ Ate, int nt, int64_t c, int v,
-                                 int w) {
-  const int lv = local_of(cn, c, v), lw = local_of(cn, c, w), ntr = 3 * nt;
+__device__ double cell_stiffness(const int* __restrict__ cn, const int* __restrict__ cv,
+                                 const double* __restrict__ Ate, int nt, int64_t c, int v, int w) {
+  const int lv = local_of(cv, c, v), lw = local_of(cv, c, w), ntr = 3 * nt;
   if (lv < 0 || lw < 0) return 0.0;
   const double* K = Ate + c * ntr * ntr;
   double s = 0.0;
@@ -75,11 +76,12 @@ __global__ __launch_bounds__(256) void amg_vertex_kernel(DevMesh m, int nt, cons
       if (w != v) {
         const int64_t f = A.af[e];
         for (int k = 0; k < 2; ++k)
-          if (m.fcell[2 * f + k] >= 0) s += cell_stiffness(m.cn, Ate, nt, m.fcell[2 * f + k], v, w);
+          if (m.fcell[2 * f + k] >= 0) s += cell_stiffness(m.cn, A.cv, Ate, nt, m.fcell[2 * f + k], v, w);
       } else {
         for (int u = A.vp[v]; u < A.vp[v + 1]; ++u) {  // the cells around v, by the faces opposite to it
           const int code = A.vi[u];
-          if ((code & 3) >= 2) s += cell_stiffness(m.cn, Ate, nt, m.fcell[2 * (code >> 2) + (code & 3) - 2], v, v);
+          if ((code & 3) >= 2)
+            s += cell_stiffness(m.cn, A.cv, Ate, nt, m.fcell[2 * (code >> 2) + (code & 3) - 2], v, v);
         }
       }
     }
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(64 * NT) void amg_g_kernel(DevMesh m, TraceSystem T
       for (int k = 0; k < 2; ++k) {
         const int64_t c = m.fcell[2 * f + k];
         if (c < 0) continue;
-        const int lv = local_of(m.cn, c, v);
+        const int lv = local_of(A.cv, c, v);
         const int l = m.cf[3 * c] == f ? 0 : (m.cf[3 * c + 1] == f ? 1 : (m.cf[3 * c + 2] == f ? 2 : -1));
         if (lv < 0 || l < 0) continue;
         const double* K = Ate + c * (NTR * NTR) + (l * NT + a) * NTR;
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __
   for (int i = threadIdx.x; i < n * n; i += 256) full[i] = 0.0;
   __syncthreads();
   for (int v = threadIdx.x; v < n; v += 256)
-    for (int e = L.ap[v]; e < L.ap[v + 1]; ++e) full[v * n + L.ai[e]] = L.av[e];
+    for (int e = L.ap[v]; e < L.ap[v + 1]; ++e) full[v * n + L.ai[e]] += L.av[e];  // a vertex pair may have two entries
   __syncthreads();
   for (int v = threadIdx.x; v < n; v += 256)
     if (!(full[v * n + v] > 0.0)) full[v * n + v] = 1.0;
@@ -554,23 +556,44 @@ bool amg_plan(int64_t nn, int64_t nc, int64_t nf, const int* cn, const int* cf, 
     plan.ints.insert(plan.ints.end(), v.begin(), v.end());
     return at;
   };
-  // the vertices of every face, and the faces of every vertex
-  Ints fv(4 * nf, -1);
+  // the vertices of every face; where a face's two cells name different nodes,
+  // it joins them, lower end to lower end and higher to higher
+  Ints fv(4 * nf, -1), to(n);
+  for (int v = 0; v < n; ++v) to[v] = v;
+  const auto vertex = [&](int v) {
+    while (to[v] != v) v = to[v] = to[to[v]];
+    return v;
+  };
   for (int64_t f = 0; f < nf; ++f)
     for (int k = 0; k < 2; ++k) {
       const int64_t c = fcell[2 * f + k];
       if (c < 0) continue;
       const int l = cf[3 * c] == f ? 0 : (cf[3 * c + 1] == f ? 1 : (cf[3 * c + 2] == f ? 2 : -1));
       if (l < 0) return false;
-      const int a = cn[3 * c + (l + 1) % 3], b = cn[3 * c + (l + 2) % 3];
+      const int a = cn[3 * c + (l + 1) % 3], b = cn[3 * c + (l + 2) % 3], lo = std::min(a, b), hi = std::max(a, b);
       if (k == 0) {
-        fv[4 * f] = std::min(a, b);
-        fv[4 * f + 1] = std::max(a, b);
-      } else if (fv[4 * f] != std::min(a, b) || fv[4 * f + 1] != std::max(a, b)) {
-        return false;  // the cells disagree on the face
+        fv[4 * f] = lo;
+        fv[4 * f + 1] = hi;
+      } else if (fv[4 * f] != lo || fv[4 * f + 1] != hi) {
+        to[vertex(lo)] = vertex(fv[4 * f]);
+        to[vertex(hi)] = vertex(fv[4 * f + 1]);
+        plan.joined = true;
       }
       fv[4 * f + 2 + k] = cn[3 * c + l];
     }
+  if (plan.joined) {
+    Ints cv(3 * nc);
+    for (int64_t i = 0; i < 3 * nc; ++i) cv[i] = vertex(cn[i]);
+    for (int64_t c = 0; c < nc; ++c)  // a cell across the whole mesh
+      if (cv[3 * c] == cv[3 * c + 1] || cv[3 * c + 1] == cv[3 * c + 2] || cv[3 * c + 2] == cv[3 * c]) return false;
+    for (int64_t f = 0; f < nf; ++f) {
+      for (int j = 0; j < 4; ++j)
+        if (fv[4 * f + j] >= 0) fv[4 * f + j] = vertex(fv[4 * f + j]);
+      if (fv[4 * f + 2] == fv[4 * f + 3]) return false;  // two cells across it
+    }
+    plan.cv = put(cv);
+  }
+  // the faces of every vertex
   Ints vp(n + 1, 0), vi;
   for (int v : fv)
     if (v >= 0) ++vp[v + 1];
@@ -589,10 +612,9 @@ bool amg_plan(int64_t nn, int64_t nc, int64_t nf, const int* cn, const int* cf, 
     for (int e = vp[v]; e < vp[v + 1]; ++e)
       if ((vi[e] & 3) < 2) row.push_back({fv[vi[e] ^ 1], vi[e] >> 2});
     std::sort(row.begin(), row.end());
-    for (size_t i = 0; i < row.size(); ++i) {
-      if (i && row[i].first == row[i - 1].first) return false;  // two faces between the same vertices
-      ai.push_back(row[i].first);
-      af.push_back(row[i].second);
+    for (const auto& [w, f] : row) {
+      ai.push_back(w);
+      af.push_back(f);
     }
     ap[v + 1] = (int)ai.size();
   }

@@ -51,7 +51,8 @@ struct hdg_ctx {
   DevMesh mesh;
   int64_t nblock_cols = 0;  // stored nt x nt blocks of K
   DevPattern pat;
-  bool structured = false;  // cells follow rectangle_mesh's (nx, ny) numbering
+  bool numbered = false;    // cells follow rectangle_mesh's (nx, ny) numbering
+  bool structured = false;  // and meet in its faces: the reduced system stands for the mesh's
   MgData mg;                // vertex hierarchy (structured meshes)
   MgData* d_mg = nullptr;   // its device copy (read by the one-workgroup tail kernel)
   // other meshes: connectivity on the host and, from the first solve with the
@@ -377,7 +378,7 @@ void free_mesh(hdg_ctx* c) {
   c->h_cn.clear();
   c->h_cf.clear();
   c->h_fcell.clear();
-  c->structured = false;
+  c->numbered = c->structured = false;
   c->has_mesh = false;
   c->mesh = DevMesh{};
 }
@@ -385,7 +386,7 @@ void free_mesh(hdg_ctx* c) {
 // Cells numbered as rectangle_mesh(TriangleCell, (nx, ny)) numbers them
 // (generate_mesh.jl:130-138): lower triangle (n(i,j), n(i+1,j), n(i,j+1)),
 // then upper (n(i+1,j), n(i+1,j+1), n(i,j+1)), n(i,j) = i + (j-1)(nx+1).
-bool detect_structured(int64_t nn, int64_t nc, const int64_t* cells, int* nx_out, int* ny_out) {
+bool detect_numbering(int64_t nn, int64_t nc, const int64_t* cells, int* nx_out, int* ny_out) {
   const int64_t nx = cells[2] - 2;
   if (nx < 1 || nc % (2 * nx) != 0) return false;
   const int64_t ny = nc / (2 * nx);
@@ -400,6 +401,35 @@ bool detect_structured(int64_t nn, int64_t nc, const int64_t* cells, int* nx_out
     }
   *nx_out = (int)nx;
   *ny_out = (int)ny;
+  return true;
+}
+
+// Whether the faces of a mesh so numbered are the grid's: one face on every
+// edge, between the edge's own cells.  The reduced system takes this for
+// granted; a mesh cut open along an edge (two faces there, of one cell each)
+// or joined at its sides (one face on two edges) is not the grid it is
+// numbered like.  cf, fcell 0-based.
+bool grid_faces(int nx, int ny, int64_t nf, const std::vector<int>& cf, const std::vector<int>& fcell) {
+  if (nf != 3 * (int64_t)nx * ny + nx + ny) return false;
+  std::vector<char> seen(nf, 0);
+  // face f of cell a and, across the edge, face g of cell b (b < 0: none)
+  const auto edge = [&](int64_t a, int la, int64_t b, int lb) {
+    const int64_t f = cf[3 * a + la];
+    if (seen[f]) return false;
+    seen[f] = 1;
+    if (b >= 0 && cf[3 * b + lb] != f) return false;
+    const int64_t p = fcell[2 * f], q = fcell[2 * f + 1];
+    return (p == a && q == b) || (p == b && q == a);
+  };
+  for (int64_t j = 0; j < ny; ++j)
+    for (int64_t i = 0; i < nx; ++i) {
+      // faces of the lower cell: diagonal, left, bottom; of the upper: top,
+      // diagonal, right
+      const int64_t lo = 2 * (j * nx + i), up = lo + 1;
+      if (!edge(lo, 0, up, 1) || !edge(lo, 1, i > 0 ? lo - 1 : -1, 2) || !edge(lo, 2, j > 0 ? up - 2 * nx : -1, 0) ||
+          (i + 1 == nx && !edge(up, 2, -1, 0)) || (j + 1 == ny && !edge(up, 0, -1, 0)))
+        return false;
+    }
   return true;
 }
 
@@ -592,7 +622,7 @@ bool use_mg(const hdg_ctx* c) {
 // (asked for, a mesh the plan refuses, or no memory within the budget: what
 // fitted before fits).
 int ensure_amg(hdg_ctx* c) {
-  if (c->structured || c->opt.precond != HDG_PC_AUTO || c->amg_state < 0) return 0;
+  if (c->structured || c->opt.precond == HDG_PC_BLOCK_JACOBI || c->amg_state < 0) return 0;
   AmgData& A = c->amg;
   if (c->amg_state == 0) {
     free_amg(c);
@@ -653,6 +683,7 @@ int ensure_amg(hdg_ctx* c) {
     t.vp = ints + P.vp;
     t.vi = ints + P.vi;
     t.af = ints + P.af;
+    t.cv = P.joined ? ints + P.cv : c->mesh.cn;
     t.r = A.lev[0].r;
     t.e = A.lev[0].e;
     const bool up = hipMemcpyAsync(c->d_amg, &A, sizeof(AmgData), hipMemcpyHostToDevice, c->stream) == hipSuccess;
@@ -1143,7 +1174,8 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->nblock_cols = nblk;
   int nx = 0, ny = 0;
-  c->structured = detect_structured(nn, nc, cells, &nx, &ny);
+  c->numbered = detect_numbering(nn, nc, cells, &nx, &ny);
+  c->structured = c->numbered && grid_faces(nx, ny, nf, cf, fcell);
   if (c->structured) {
     TRY(build_vertex_levels(c, nx, ny));
   } else {
@@ -1217,7 +1249,7 @@ int hdg_set_rectangle_mesh(hdg_ctx* c, int64_t nx, int64_t ny, double x0, double
   }
   const int64_t nbdry = 2 * nx + 2 * ny;
   c->nblock_cols = 5 * (nf - nbdry) + 3 * nbdry;
-  c->structured = true;
+  c->numbered = c->structured = true;
   TRY(build_vertex_levels(c, (int)nx, (int)ny));
   c->has_mesh = true;
   return HDG_OK;
@@ -1231,9 +1263,9 @@ int hdg_setup(hdg_ctx* c, const hdg_options* opt) {
     return fail(c, HDG_ERR_ARG, "unknown precision mode %d", opt->precision);
   if (opt->precond < HDG_PC_AUTO || opt->precond > HDG_PC_MULTIGRID)
     return fail(c, HDG_ERR_ARG, "unknown preconditioner %d", opt->precond);
-  if (opt->precond == HDG_PC_MULTIGRID && !c->structured)
+  if (opt->precond == HDG_PC_MULTIGRID && !c->numbered)
     return fail(c, HDG_ERR_UNSUPPORTED, "the multigrid preconditioner needs a structured rectangle_mesh");
-  if (opt->precision == HDG_MIXED && (!c->structured || opt->precond == HDG_PC_BLOCK_JACOBI))
+  if (opt->precision == HDG_MIXED && (!c->numbered || opt->precond == HDG_PC_BLOCK_JACOBI))
     return fail(c, HDG_ERR_UNSUPPORTED,
                 "mixed precision runs on the multigrid path: it needs a structured rectangle_mesh");
   TRY(select_device(c));

@@ -55,14 +55,18 @@ typedef struct hdg_ctx hdg_ctx;
 
 /* Precision modes of the trace solve.  HDG_MIXED keeps condensation, the
    trace matrix, the CG recurrences and the iterate in FP64 and runs the
-   multigrid preconditioner's trace-level data in float (structured meshes
-   only: HDG_ERR_UNSUPPORTED otherwise). */
+   multigrid preconditioner's trace-level data in float (meshes numbered like
+   rectangle_mesh only: HDG_ERR_UNSUPPORTED otherwise; where the faces are not
+   the grid's, see below, the preconditioner stays FP64). */
 enum { HDG_FP64 = 0, HDG_MIXED = 1 };
 
 /* Preconditioners of the trace solve.  HDG_PC_AUTO picks the geometric
    multigrid of HDG_PC_MULTIGRID when the mesh is a structured rectangle_mesh
    and, on other meshes, an aggregation multigrid over the mesh's vertices (or
-   block-Jacobi, see hdg_options). */
+   block-Jacobi, see hdg_options).  HDG_PC_MULTIGRID takes every mesh whose
+   cells are numbered like rectangle_mesh's; where its faces are not the grid's
+   (a mesh cut open along edges, or with its sides joined) it is
+   HDG_PC_AUTO's choice for other meshes. */
 enum { HDG_PC_AUTO = 0, HDG_PC_BLOCK_JACOBI = 1, HDG_PC_MULTIGRID = 2 };
 
 /* Schedule flags.  By default the first solve after hdg_setup launches its
