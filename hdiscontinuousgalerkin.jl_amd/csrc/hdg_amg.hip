@@ -216,23 +216,30 @@ __global__ __launch_bounds__(256) void amg_rap_kernel(AmgLevel L, AmgLevel C) {
 }
 
 // Inverse of the last operator (n <= kAmgDirect; SPD on the rows with a
-// positive diagonal, identity rows elsewhere): Gauss-Jordan without pivoting,
+// positive diagonal, identity rows elsewhere; singular without any fixed
+// vertex, see kNoPivot): Gauss-Jordan without pivoting,
 // 6 x 6 entries per thread in registers, the pivot's row and column updated by
 // the same fma as the rest (factors p - 1 and 1 + 1/p, p the pivot).
 __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __restrict__ cinv) {
   constexpr int T = 16, E = kAmgDirect / T;
   __shared__ double full[kAmgDirect * kAmgDirect];
-  __shared__ double rowb[2][kAmgDirect], colb[2][kAmgDirect];
+  __shared__ double rowb[2][kAmgDirect], colb[2][kAmgDirect], mean[kAmgDirect + 1];
+  __shared__ int fixed, dropped;
   const int n = L.n, tr = threadIdx.x / T, tc = threadIdx.x % T;
+  if (threadIdx.x == 0) fixed = dropped = 0;
   for (int i = threadIdx.x; i < n * n; i += 256) full[i] = 0.0;
   __syncthreads();
   for (int v = threadIdx.x; v < n; v += 256)
     for (int e = L.ap[v]; e < L.ap[v + 1]; ++e) full[v * n + L.ai[e]] += L.av[e];  // a vertex pair may have two entries
   __syncthreads();
-  for (int v = threadIdx.x; v < n; v += 256)
-    if (!(full[v * n + v] > 0.0)) full[v * n + v] = 1.0;
+  for (int v = threadIdx.x; v < n; v += 256) {
+    if (!(full[v * n + v] > 0.0)) {
+      full[v * n + v] = 1.0;
+      fixed = 1;
+    }
+  }
   __syncthreads();
-  double m[E][E];
+  double m[E][E], least[E];  // the entries, and the least pivots of those on the diagonal
 #pragma unroll
   for (int a = 0; a < E; ++a)
 #pragma unroll
@@ -240,14 +247,18 @@ __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __
       const int r = tr + T * a, c = tc + T * b;
       m[a][b] = r < n && c < n ? full[r * n + c] : 0.0;
     }
+#pragma unroll
+  for (int a = 0; a < E; ++a) least[a] = tr == tc ? kNoPivot * m[a][a] : -1.0;
   // k = ka T + kt with ka unrolled, so that the pivot's registers are known
 #pragma unroll
   for (int ka = 0; ka < E; ++ka)
     for (int kt = 0; kt < T && ka * T + kt < n; ++kt) {
       const int k = ka * T + kt, p = kt & 1;
+      const bool none = tc == kt && fabs(m[ka][ka]) <= least[ka];
+      if (none) dropped = 1;
       if (tr == kt)
 #pragma unroll
-        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[ka][b];
+        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = b == ka && none ? kLeftOut : m[ka][b];
       if (tc == kt)
 #pragma unroll
         for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][ka];
@@ -268,6 +279,7 @@ __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __
       for (int a = 0; a < E; ++a)
 #pragma unroll
         for (int b = 0; b < E; ++b) m[a][b] = fma(-ck[a], rk[b], m[a][b]);
+      m[ka][ka] = none ? 0.0 : m[ka][ka];
     }
 #pragma unroll
   for (int a = 0; a < E; ++a)
@@ -276,6 +288,7 @@ __global__ __launch_bounds__(256) void amg_inverse_kernel(AmgLevel L, double* __
       const int r = tr + T * a, c = tc + T * b;
       if (r < n && c < n) cinv[r * n + c] = m[a][b];
     }
+  if (dropped && !fixed) project_constants(cinv, n, mean);
 }
 
 // ------------------------------------------------------------------- cycle

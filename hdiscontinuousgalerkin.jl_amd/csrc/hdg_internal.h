@@ -403,6 +403,40 @@ constexpr int kTailNodes = 1536;
 constexpr int kTailThreads = 1024;
 // coarsening stops at this many nodes, solved exactly (inverse at set-up)
 constexpr int kCoarseDirect = 96;
+// Where nothing prescribes mode 0 anywhere (a pure Neumann problem) constants
+// are in the null space of the trace system and of every level, and the last
+// pivot of the coarsest operator's inverse is rounding: below this part of its
+// diagonal entry it is left out, row and column zero, which gives a semidefinite
+// inverse on the rest (taken as it came, it put multiples of 1e6 of the constant
+// into the solution).  Of the pivots of a problem with prescribed values the
+// smallest is the square of its cells' aspect below 1; one left out by mistake
+// would cost CG an iteration or two, no accuracy.
+constexpr double kNoPivot = 1e-9;
+// The Gauss-Jordan step with this in the pivot's place leaves the other entries
+// alone and zeroes the pivot's row and column (p - 1 = p, p (1 / p) = 1 exactly;
+// the pivot's own entry is set to zero afterwards).
+constexpr double kLeftOut = 0x1p900;
+// Constants taken out of such an inverse: A <- (I - 1 1^T / n) A (I - 1 1^T / n),
+// A symmetric n x n in global memory, by the block that wrote it (mean: n + 1
+// doubles of LDS).  Pinned at the node left out, it adds to every correction a
+// constant of its own size, whose rounding in the CG product ends the
+// convergence at 1e-11 of the load and turns it round.
+__device__ inline void project_constants(double* A, int n, double* mean) {
+  __syncthreads();
+  for (int r = threadIdx.x; r < n; r += blockDim.x) {
+    double s = 0.0;
+    for (int c = 0; c < n; ++c) s += A[c * n + r];
+    mean[r] = s / n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int r = 0; r < n; ++r) s += mean[r];
+    mean[n] = s / n;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n * n; e += blockDim.x) A[e] -= mean[e / n] + mean[e % n] - mean[n];
+}
 struct MgData {
   int nlev = 0;                  // levels 1..nlev-1 are vertex grids
   int nx = 0, ny = 0;

@@ -175,20 +175,25 @@ __global__ __launch_bounds__(kRapThreads) void mg_rap_kernel(VS sel) {
 
 // Inverse of the coarsest operator (at most kCoarseDirect nodes), one
 // workgroup per hierarchy: in-place Gauss-Jordan without pivoting (the
-// operator is SPD, fixed nodes have identity rows), the matrix in registers
+// operator is SPD, fixed nodes have identity rows; without any fixed node it is
+// singular, see kNoPivot), the matrix in registers
 // (6 x 6 entries per thread), the pivot row and column through alternating
 // LDS buffers, one barrier of four wavefronts per step.  With the pivot p, the
 // row and column k take the same fma(-c, r, m) as the rest: the row's factor c
 // is p - 1, the column's r is 1 + 1/p (m - (p - 1) m/p = m/p, c - c (1 + 1/p)
 // = -c/p).  Bound by the chain of barrier, division and LDS.  With the pivot's
-// registers chosen at run time a step took 1.1 us (81 nodes: 88 us, now 52).
+// registers chosen at run time a step took 1.1 us (81 nodes: 88 us, now 42).
 __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restrict__ Ms) {
   constexpr int T = 16, E = kCoarseDirect / T;
-  __shared__ double rowb[2][kCoarseDirect], colb[2][kCoarseDirect];
+  __shared__ double rowb[2][kCoarseDirect], colb[2][kCoarseDirect], mean[kCoarseDirect + 1];
+  __shared__ int fixed, dropped;
   const MgData& M = Ms[blockIdx.x];
   const MgLevel& L = M.lev[M.nlev - 1];
   const int n = (int)L.n, tr = threadIdx.x / T, tc = threadIdx.x % T, row = L.nx + 1;
-  double m[E][E];
+  if (threadIdx.x == 0) fixed = dropped = 0;
+  __syncthreads();
+  if ((int)threadIdx.x < n && L.mask[threadIdx.x]) fixed = 1;
+  double m[E][E], least[E];  // the entries, and the least pivots of those on the diagonal
 #pragma unroll
   for (int a = 0; a < E; ++a)
 #pragma unroll
@@ -201,14 +206,18 @@ __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restric
       }
       m[a][b] = v;
     }
+#pragma unroll
+  for (int a = 0; a < E; ++a) least[a] = tr == tc ? kNoPivot * m[a][a] : -1.0;
   // k = ka T + kt with ka unrolled, so that the pivot's registers are known
 #pragma unroll
   for (int ka = 0; ka < E; ++ka)
     for (int kt = 0; kt < T && ka * T + kt < n; ++kt) {
       const int k = ka * T + kt, p = kt & 1;
+      const bool none = tc == kt && fabs(m[ka][ka]) <= least[ka];
+      if (none) dropped = 1;
       if (tr == kt)
 #pragma unroll
-        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = m[ka][b];
+        for (int b = 0; b < E; ++b) rowb[p][tc + T * b] = b == ka && none ? kLeftOut : m[ka][b];
       if (tc == kt)
 #pragma unroll
         for (int a = 0; a < E; ++a) colb[p][tr + T * a] = m[a][ka];
@@ -229,6 +238,7 @@ __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restric
       for (int a = 0; a < E; ++a)
 #pragma unroll
         for (int b = 0; b < E; ++b) m[a][b] = fma(-ck[a], rk[b], m[a][b]);
+      m[ka][ka] = none ? 0.0 : m[ka][ka];
     }
 #pragma unroll
   for (int a = 0; a < E; ++a)
@@ -237,6 +247,7 @@ __global__ __launch_bounds__(256) void mg_inverse_kernel(const MgData* __restric
       const int r = tr + T * a, c = tc + T * b;
       if (r < n && c < n) M.cinv[r * n + c] = m[a][b];
     }
+  if (dropped && !fixed) project_constants(M.cinv, n, mean);
 }
 
 // ------------------------------------------------------- vertex levels
