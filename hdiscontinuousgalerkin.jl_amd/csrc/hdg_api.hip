@@ -1346,6 +1346,7 @@ int hdg_set_source(hdg_ctx* c, const hdg_source* s) {
   if (!c || !s) return HDG_ERR_ARG;
   if (!c->has_setup) return fail(c, HDG_ERR_STATE, "hdg_setup has not been called");
   if (s->kind < 0 || s->kind > 3) return fail(c, HDG_ERR_ARG, "unknown source kind %d", s->kind);
+  if (s->kind == 3 && !s->f_qp) return fail(c, HDG_ERR_ARG, "HDG_SRC_VALUES needs f_qp");
   TRY(select_device(c));
   SrcParams p;
   p.kind = s->kind;
@@ -1353,17 +1354,22 @@ int hdg_set_source(hdg_ctx* c, const hdg_source* s) {
   p.ka = s->ka;
   p.kb = s->kb;
   for (int i = 0; i < 16; ++i) p.coef[i] = s->coef[i];
-  dfree(c, c->d_fqp);
+  // the old source stands until the new one is there, so that a call that
+  // fails leaves a context whose source has its values (their number is the
+  // set-up's: old values are written over in place)
   if (s->kind == 3) {
-    if (!s->f_qp) return fail(c, HDG_ERR_ARG, "HDG_SRC_VALUES needs f_qp");
     const size_t n = (size_t)c->mesh.nc * c->nqp;
     Exporting room(c);
-    TRY(dalloc(c, &c->d_fqp, n));
+    if (!c->d_fqp) TRY(dalloc(c, &c->d_fqp, n));
+    c->src = p;
+    c->assembled = c->solved = c->recovered = false;
     HIPCHK(c, hipMemcpyAsync(c->d_fqp, s->f_qp, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+  } else {
+    dfree(c, c->d_fqp);
+    c->src = p;
+    c->assembled = c->solved = c->recovered = false;
   }
-  c->src = p;
-  c->assembled = c->solved = c->recovered = false;
   return HDG_OK;
 }
 
