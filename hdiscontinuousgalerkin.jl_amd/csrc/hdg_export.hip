@@ -168,10 +168,11 @@ struct StagePieces {
 // Launches on the stream the kernels that write chunk k to buf and lists its
 // pieces; a hipError_t.
 using StageFill = int (*)(void* arg, int64_t k, char* buf, StagePieces& out);
-void copy_share(const char* buf, const StagePieces& p, int t, int nthr) {
+// Share t of nshares of a chunk.
+void copy_share(const char* buf, const StagePieces& p, int t, int nshares) {
   size_t total = 0;
   for (int i = 0; i < p.n; ++i) total += p.bytes[i];
-  size_t lo = total / nthr * t, hi = t + 1 == nthr ? total : total / nthr * (t + 1), at = 0;
+  size_t lo = total / nshares * t, hi = t + 1 == nshares ? total : total / nshares * (t + 1), at = 0;
   for (int i = 0; i < p.n && at < hi; at += p.bytes[i++]) {
     const size_t a = std::max(lo, at), b = std::min(hi, at + p.bytes[i]);
     if (a < b) std::memcpy(p.dst[i] + (a - at), buf + p.off[i] + (a - at), b - a);
@@ -210,37 +211,57 @@ int stage_reserve(HostStage& st, size_t total, size_t head) {
   return 0;
 }
 
+// A wait of some microseconds: spins, and lets go of the core only when it has
+// lasted long.  (Where other threads spin on every core, as a BLAS library's do
+// for tens of milliseconds after a product, a thread that yields or sleeps gets
+// its core back 3 ms later: with a sleep per chunk and yields between the
+// chunks, 54 MB took 45 ms beside such threads; now 3 to 5, and 1.2 without them.)
+struct Patience {
+  int n = 0;
+  void wait() {
+    if (++n < 20000)
+      __builtin_ia32_pause();
+    else
+      std::this_thread::yield();
+  }
+};
+
 // Writes nchunks chunks (total bytes in all) and copies each out while the
-// next ones are written; returns when everything has arrived.
+// next ones are written; returns when everything has arrived.  A chunk is
+// copied in shares, taken by the caller's thread and by those of a crew
+// as each is free: nothing waits for a thread that has no core, except to the
+// end of a share it has begun.
 int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, StageFill fill, void* arg) {
   StagePieces pieces[kStageBufs];
-  std::atomic<int64_t> ready{0};
-  std::atomic<int64_t> copied{0};  // shares finished over all chunks
+  std::atomic<int64_t> ready{0};  // chunks that have arrived in their buffers
+  std::atomic<int64_t> taken{0};  // shares taken, over all chunks
+  std::atomic<int64_t> done[kStageBufs] = {};  // shares copied from each buffer
   std::atomic<bool> stop{false};
   std::thread crew[kCrew];
-  int nthr = 1;
   const int nb = (int)st.bufs;
   char* const buf0 = st.mem + st.head;
-  std::atomic<int> team{0};  // set once the crew is complete
   const int want = (int)std::min<size_t>({(size_t)kCrew, total / kPerThread,
                                           (size_t)std::max(1u, std::thread::hardware_concurrency() / 2)});
-  const auto work = [&](int t) {
-    int n;
-    while (!(n = team.load(std::memory_order_acquire)))
-      if (stop.load())
-        return;
-      else
-        std::this_thread::yield();
-    for (int64_t k = 0; k < nchunks; ++k) {
-      while (ready.load(std::memory_order_acquire) <= k) {
-        if (stop.load()) return;
-        std::this_thread::yield();
-      }
-      copy_share(buf0 + (k % nb) * st.chunk, pieces[k % nb], t, n);
-      copied.fetch_add(1, std::memory_order_release);
-    }
+  const int shares = want > 1 ? 2 * kCrew : 1;
+  // takes and copies one share of what has arrived
+  const auto copy_one = [&]() -> bool {
+    int64_t i = taken.load(std::memory_order_relaxed);
+    do {
+      if (i >= ready.load(std::memory_order_acquire) * shares) return false;
+    } while (!taken.compare_exchange_weak(i, i + 1, std::memory_order_relaxed));
+    const int b = (int)(i / shares % nb);
+    copy_share(buf0 + b * st.chunk, pieces[b], (int)(i % shares), shares);
+    done[b].fetch_add(1, std::memory_order_release);
+    return true;
   };
-  int e = 0;
+  const auto work = [&]() {
+    Patience p;
+    while (!stop.load(std::memory_order_acquire) && taken.load(std::memory_order_relaxed) < nchunks * shares)
+      if (copy_one())
+        p = Patience{};
+      else
+        p.wait();
+  };
   const auto launch = [&](int64_t k) {
     StagePieces& p = pieces[k % nb];
     p.n = 0;
@@ -248,25 +269,45 @@ int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, Stag
     if (!r) r = (int)hipEventRecord(st.ev[k % nb], s);
     return r;
   };
-  for (int64_t k = 0; k < nchunks && k < nb && !e; ++k) e = launch(k);
+  int e = 0;
+  int64_t launched = 0, arrived = 0, copied = 0;
+  while (launched < nchunks && launched < nb && !e)
+    if (!(e = launch(launched))) ++launched;
   // the crew starts beside the first chunks
   try {
-    for (int t = 1; !e && t < want; ++t) {
-      crew[t] = std::thread(work, t);
-      ++nthr;
+    for (int t = 1; !e && t < want; ++t) crew[t] = std::thread(work);
+  } catch (...) {  // fewer, then
+  }
+  Patience p;
+  while (copied < nchunks && !e) {
+    bool moved = false;
+    if (arrived < launched) {
+      hipError_t q = hipEventQuery(st.ev[arrived % nb]);
+      if (q == hipErrorNotReady) {
+        (void)hipGetLastError();
+        // long work ahead of the export on the stream
+        if (p.n > 4000 && copied == arrived) q = hipEventSynchronize(st.ev[arrived % nb]);
+      }
+      if (q == hipSuccess) {
+        ready.store(++arrived, std::memory_order_release);
+        moved = true;
+      } else if (q != hipErrorNotReady) {
+        e = (int)q;
+        break;
+      }
     }
-  } catch (...) {
+    if (copy_one()) moved = true;
+    if (copied < arrived && done[copied % nb].load(std::memory_order_acquire) == (copied / nb + 1) * shares) {
+      ++copied;
+      moved = true;
+      if (launched < nchunks && !(e = launch(launched))) ++launched;
+    }
+    if (moved)
+      p = Patience{};
+    else
+      p.wait();
   }
-  team.store(nthr, std::memory_order_release);
-  for (int64_t k = 0; k < nchunks && !e; ++k) {
-    e = (int)hipEventSynchronize(st.ev[k % nb]);
-    if (e) break;
-    ready.store(k + 1, std::memory_order_release);
-    copy_share(buf0 + (k % nb) * st.chunk, pieces[k % nb], 0, nthr);
-    while (copied.load(std::memory_order_acquire) < (k + 1) * (nthr - 1)) std::this_thread::yield();
-    if (k + nb < nchunks) e = launch(k + nb);
-  }
-  stop.store(true);
+  stop.store(true, std::memory_order_release);
   for (std::thread& t : crew)
     if (t.joinable()) t.join();
   if (e) (void)hipStreamSynchronize(s);
