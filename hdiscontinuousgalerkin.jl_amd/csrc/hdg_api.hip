@@ -593,18 +593,17 @@ int ensure_system(hdg_ctx* c) {
   return HDG_OK;
 }
 
-// Condensation and trace matrix; on a block-Jacobi context its Jacobi blocks.
-// run: the solve follows at once, and a multigrid context builds its reduced
-// system from the condensed blocks, so the assembled matrix is left to the
-// exports (ensure_system).
-int assemble_impl(hdg_ctx* c, bool run = false) {
+// Condensation, and the trace matrix with its Jacobi blocks where the solve
+// uses them; a multigrid context builds its reduced system from the condensed
+// blocks and leaves the assembled matrix to the exports (ensure_system).
+int assemble_impl(hdg_ctx* c) {
   if (!c->has_setup) return fail(c, HDG_ERR_STATE, "hdg_setup has not been called");
   if ((c->opt.schedule & HDG_SCHEDULE_AUTOTUNE) && !c->tuned) TRY(autotune_impl(c));
   c->filled = false;
   HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
   LAUNCHCHK(c, launch_condense_cells(c, condense_args(c)));
-  if (!use_mg(c) || !run) TRY(ensure_system(c));
   if (!use_mg(c)) {
+    TRY(ensure_system(c));
     LAUNCHCHK(c, launch_jacobi(c->pat, c->T, c->stream));
     c->jacobi_dirty = false;
   }
@@ -1520,7 +1519,7 @@ int hdg_errornorm(hdg_ctx* c, int kind, const double* par, double* sq) {
 int hdg_run(hdg_ctx* c, hdg_solve_info* info) {
   if (!c) return HDG_ERR_ARG;
   TRY(select_device(c));
-  TRY(assemble_impl(c, true));
+  TRY(assemble_impl(c));
   int flag = 0;
   const int r = solve_impl(c, info, &flag);
   // a singular local matrix or a negative Jacobian is reported as such, not
