@@ -1770,8 +1770,11 @@ int hdg_refine_probe(hdg_ctx* c, int outer, double inner_rtol, double* relres, i
   for (int j = 0; j <= outer; ++j) relres[j] = std::nan("");
   if (inner_iters)
     for (int j = 0; j < outer; ++j) inner_iters[j] = 0;
-  const int64_t N = c->T.N, nv = c->T.vals ? (int64_t)kSlots * c->nt * N : 0;
-  const int64_t nb = c->T.blk ? (int64_t)sym_blk_count(c->nt, c->mesh.nf) : 0;
+  // the rounded matrix: a copy for the CG on it; the reduced system of a
+  // multigrid context rounds as it reads (with both systems held, a copy as
+  // well would need more memory than the probe's callers ever had to have)
+  const int64_t N = c->T.N, nv = c->T.vals && !mg ? (int64_t)kSlots * c->nt * N : 0;
+  const int64_t nb = c->T.blk && !mg ? (int64_t)sym_blk_count(c->nt, c->mesh.nf) : 0;
   double *vr = nullptr, *vb = nullptr, *u = nullptr, *res = nullptr, *zero = nullptr, *part = nullptr;
   int rc = HDG_OK;
   {

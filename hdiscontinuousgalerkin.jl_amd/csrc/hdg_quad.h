@@ -69,7 +69,8 @@ struct QuadSys {
   const unsigned char* dmask = nullptr;
   const double* uD = nullptr;
   const double *Ate = nullptr, *bte = nullptr;
-  // the assembled matrix instead of the cells' blocks (hdg_refine_probe)
+  // the assembled matrix, its entries rounded to float as they are read,
+  // instead of the cells' blocks (hdg_refine_probe)
   int from_k = 0;
   DevPattern P;
   TraceSystem K;

@@ -156,22 +156,22 @@ constexpr int quad_stride(int nt) {
   return n + ((want - n) % 32 + 32) % 32;
 }
 
-// entry K[(f, a), (g, b)] of the assembled matrix
+// entry K[(f, a), (g, b)] of the assembled matrix, rounded to float
 template <int NT>
 __device__ double k_entry(const QuadSys& S, int64_t f, int a, int64_t g, int b) {
   if constexpr (kSymBlocks<NT>) {
     const int64_t nf = S.K.nf;
-    if (f == g) return S.K.blk[(int64_t)dinv_slot(NT, a, b) * nf + f];
+    if (f == g) return (double)(float)S.K.blk[(int64_t)dinv_slot(NT, a, b) * nf + f];
     const double* own = S.K.blk + (int64_t)(NT * (NT + 1) / 2) * nf;
     for (int k = 0; k < 2; ++k) {
-      if (S.P.nbr[4 * f + k] == g) return own[((2 * f + k) * NT + a) * NT + b];
+      if (S.P.nbr[4 * f + k] == g) return (double)(float)own[((2 * f + k) * NT + a) * NT + b];
       const int code = S.P.nbr[4 * f + 2 + k];
-      if ((code >> 1) == g) return own[((2 * g + (code & 1)) * NT + b) * NT + a];
+      if ((code >> 1) == g) return (double)(float)own[((2 * g + (code & 1)) * NT + b) * NT + a];
     }
     return 0.0;
   } else {
     for (int s = 0; s < S.P.nslot[f]; ++s)
-      if (S.P.bcol[f * kSlots + s] == g) return S.K.vals[(int64_t)(s * NT + b) * S.K.N + f * NT + a];
+      if (S.P.bcol[f * kSlots + s] == g) return (double)(float)S.K.vals[(int64_t)(s * NT + b) * S.K.N + f * NT + a];
     return 0.0;
   }
 }

@@ -351,7 +351,9 @@ int hdg_time_kernel(hdg_ctx* ctx, int which, int reps, double* avg_us);
    (outer + 1 values, outer <= 64); inner_iters[j] (may be null) the CG
    iterations of step j.  Leaves u_outer as the trace (hdg_recover and
    hdg_errornorm then measure it) and the assembled system as it was.
-   Allocates a second copy of the trace-matrix values while it runs.
+   Allocates a second copy of the trace-matrix values while it runs (none on
+   a rectangle_mesh with the multigrid, which holds the matrix beside its own
+   system).
    HDG_ERR_NOT_CONVERGED if an inner solve fails (entries after it are
    NaN). */
 int hdg_refine_probe(hdg_ctx* ctx, int outer, double inner_rtol, double* relres, int32_t* inner_iters);

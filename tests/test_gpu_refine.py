@@ -88,3 +88,27 @@ def test_refine_probe_one_step_is_the_rounded_solution(hdg, O):
     # and it is not the FP64 solution: the rounding shows
     assert np.abs(x32 - x64).max() > 1e-8 * scale
     assert rel[1] > 1e-7
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_refine_probe_budget(hdg, k):
+    """On a rectangle mesh the probe holds the solve's arrays, the assembled
+    matrix (face-ELL, or symmetric blocks at four modes) and rhs, and three
+    vectors of its own, no second copy of the matrix (0.7 MB here at least):
+    with a budget of that plus 0.3 MB, the same figures as without one."""
+    out, budget = [], 0
+    for _ in range(2):
+        with hdg.Context(0, hbm_budget=budget) as ctx:
+            ctx.set_rectangle_mesh(40, 37, jitter=0.2, seed=k)
+            ctx.setup(k, quad_degree={1: 2, 2: 3, 3: 6, 4: 6}[k])
+            ctx.set_source()
+            ctx.set_dirichlet_boundary(0.0)
+            ctx.run()
+            s = ctx.sizes
+            vals = 42 * s.n_faces if k == 3 else 5 * s.nt * s.n_dofs
+            assert 8 * vals > 0.7e6
+            budget = ctx.memory_used() + 8 * (vals + 4 * s.n_dofs) + 300000
+            rel, its = ctx.refine_probe(2, inner_rtol=1e-12)
+            out.append((rel, its, ctx.trace()))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
