@@ -79,7 +79,11 @@ struct AmgPlan {
   bool joined = false;  // cv is there
   std::vector<int> ints;
 };
-// false: the mesh's lists do not fit 32-bit indices
+// The aspect that a quarter of the cells exceed: the square of the longest
+// edge over four times the area, 1 for half a square, s / 2 for half a
+// rectangle of s by 1.
+double amg_aspect(int64_t nc, const int* cn, const double* xy);
+// false: the mesh's lists do not fit 32-bit indices, or do not fit together
 bool amg_plan(int64_t nn, int64_t nc, int64_t nf, const int* cn, const int* cf, const int* fcell, AmgPlan& plan);
 
 // operators and transfers of the current matrix (T with its Jacobi blocks)

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <utility>
 
 #include "hdg_amg.h"
@@ -558,6 +559,25 @@ void transpose(int n, int ncol, const Ints& ap, const Ints& ai, Ints& tp, Ints& 
 }
 
 }  // namespace
+
+double amg_aspect(int64_t nc, const int* cn, const double* xy) {
+  std::vector<double> a(nc);
+  for (int64_t c = 0; c < nc; ++c) {
+    double x[3], y[3], l2 = 0.0;
+    for (int v = 0; v < 3; ++v) {
+      const double *p = xy + 2 * (size_t)cn[3 * c + v], *q = xy + 2 * (size_t)cn[3 * c + (v + 1) % 3];
+      x[v] = q[0] - p[0];
+      y[v] = q[1] - p[1];
+      l2 = std::max(l2, x[v] * x[v] + y[v] * y[v]);
+    }
+    const double twice = std::fabs(x[0] * y[1] - x[1] * y[0]);
+    a[c] = l2 / (2.0 * twice);
+    if (!(a[c] < HUGE_VAL)) a[c] = HUGE_VAL;  // no area, or no numbers
+  }
+  const int64_t q = nc * 3 / 4;
+  std::nth_element(a.begin(), a.begin() + q, a.end());
+  return a[q];
+}
 
 bool amg_plan(int64_t nn, int64_t nc, int64_t nf, const int* cn, const int* cf, const int* fcell, AmgPlan& plan) {
   plan = AmgPlan{};

@@ -107,8 +107,9 @@ typedef struct {
                           the V-cycle on structured meshes and, on others, one
                           over the mesh's vertices and aggregates of them,
                           set up at the first solve on a mesh; block-Jacobi
-                          where hbm_budget leaves no room for it or its solve
-                          breaks down */
+                          where hbm_budget leaves no room for it, its solve
+                          breaks down, or (odd k) the cells are so stretched
+                          that it is the faster one */
 } hdg_options;
 
 typedef struct {
