@@ -51,14 +51,17 @@ __host__ __device__ constexpr int tri(int i, int j) { return i * (i + 1) / 2 + j
 typedef const double __attribute__((address_space(4))) * ScalarTab;
 
 // WPE: waves per SIMD the register budget is cut for (2: none spilled at k <=
-// 2, 80 B per lane at k = 3; 3: 440 B at k = 3, 5.5 ms at 1024^2); the
-// autotuner picks one, 2 by default.
+// 2, 80 B per lane at k = 3; 3: 440 B at k = 3, 5.5 ms at 1024^2); 2 by
+// default, or the autotuner's choice.  The LDS of a block (spd_lds) decides how
+// many waves there are: 84,448 B at k = 3 and degree 6, one block of the CU's
+// 163,840 B and one wave per SIMD.
 // GROUPED: several instances packed into one mesh, the source of cell c is
 // srcs[cell_inst[c]].
 //
 // Bound by its stores (Ate, the u rows, 2.3 KB per cell at k = 3: 0.95 ms for
 // 1024^2 grid cells at the rate of a copy) and the issue of the products
-// beside them, at two waves per SIMD: 2.9 ms there, 0.29 at 768^2, k = 1.
+// beside them, at k = 3 from one wave per SIMD: 2.9 ms there, 0.29 at 768^2,
+// k = 1.
 // With 16 lanes per element, one column each, the factor in LDS and every
 // table read from LDS by every element: 5.9 and 0.58 ms.
 template <int K, int WPE, bool GROUPED>
@@ -427,6 +430,18 @@ __global__ __launch_bounds__(256) void recover_spd_kernel(DevMesh m, const doubl
   }
 }
 
+// LDS bytes of a block of the condensation
+template <int K>
+size_t spd_lds(const SpdLayoutDev& L) {
+  using D = SpdDims<K>;
+  return sizeof(double) * (((D::T1 + L.total - D::Om + 1) & ~1) + kCells * D::YS);
+}
+// blocks on a CU by their LDS, a wave per SIMD each
+constexpr size_t kLdsPerCu = 160u << 10;
+int spd_waves(int k, const SpdLayoutDev& L) {
+  return (int)(kLdsPerCu / (k == 1 ? spd_lds<1>(L) : (k == 2 ? spd_lds<2>(L) : spd_lds<3>(L))));
+}
+
 template <int K>
 int spd_launch(const CondenseArgs& a, int wpe, int grid_cap, hipStream_t s) {
   using D = SpdDims<K>;
@@ -441,7 +456,7 @@ int spd_launch(const CondenseArgs& a, int wpe, int grid_cap, hipStream_t s) {
   const int64_t cap = grid_cap > 0 ? grid_cap : 16384;
   if (grid < 1) grid = 1;
   if (grid > cap) grid = cap;
-  const size_t lds = sizeof(double) * (((D::T1 + L.total - D::Om + 1) & ~1) + kCells * D::YS);
+  const size_t lds = spd_lds<K>(L);
   if (wpe != 3) wpe = 2;
   if (a.srcs) {
     if (wpe == 2)
@@ -509,7 +524,8 @@ int tune_condense_spd(int k, const CondenseArgs& a, hipStream_t s, CondenseSched
   double bt = 1e300, dt = 0.0;
   CondenseSched bs = *best;
   int rc = 0;
-  for (int wpe = 3; wpe >= 2 && rc == 0; --wpe)
+  // the narrow register budget only where three blocks fit on a CU
+  for (int wpe = spd_waves(k, a.spd) >= 3 ? 3 : 2; wpe >= 2 && rc == 0; --wpe)
     for (int g : grids) {
       CondenseSched sc = *best;
       sc.spd_wpe = wpe;

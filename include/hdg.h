@@ -297,7 +297,9 @@ int hdg_quadrature(int dim, int order, int cap, double* pts, double* w);
    with one element per segment of 16, 32 or 64 lanes (any width that holds
    the element's rows), or, where it applies (see HDG_SCHEDULE_LU),
    HDG_CONDENSE_SCHUR, one element per 4 lanes with a register budget cut
-   for 2 or 3 waves per SIMD.  Both stride a grid of blocks over the cells.
+   for 2 or 3 waves per SIMD (3 is timed only where the blocks' shared memory
+   leaves room for three waves, k <= 2).  Both stride a grid of blocks over the
+   cells.
    hdg_autotune times every (width or register budget, grid cap) pair of the
    form the current problem takes, with HIP events, and keeps the fastest for
    this context until the next hdg_setup (HDG_SCHEDULE_AUTOTUNE in
@@ -307,8 +309,9 @@ int hdg_quadrature(int dim, int order, int cap, double* pts, double* w);
    overwrites the assembled operators (assemble again before solving). */
 enum { HDG_CONDENSE_ELIMINATION = 0, HDG_CONDENSE_SCHUR = 1 };
 typedef struct {
-  int32_t condense_seg;   /* lanes per element (the Schur form has one width and
-                             reports 16) */
+  int32_t condense_seg;   /* lanes per element (the Schur form has one width, 4
+                             lanes, and reports 16, its width when this field
+                             was made) */
   int32_t condense_grid;  /* grid cap, blocks of 256 threads */
   double condense_us;     /* measured duration of the chosen schedule */
   double default_us;      /* of the default schedule: the narrowest width and
