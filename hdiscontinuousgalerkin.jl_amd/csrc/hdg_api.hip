@@ -944,7 +944,7 @@ int solve_impl(hdg_ctx* c, hdg_solve_info* info, int* err_flag = nullptr) {
     LAUNCHCHK(c, launch_quad_tp(c->qs, c->ql, ss));
     if (mixed(c)) LAUNCHCHK(c, launch_quad_float(c->qs, ss));
     if (fork) HIPCHK(c, hipEventRecord(c->ev_join, c->aux));
-    LAUNCHCHK(c, launch_quad_omega(c->qs, c->ql, quad_omega_factor(c->k), kQuadLanczos, c->stream));
+    LAUNCHCHK(c, launch_quad_omega(c->qs, c->ql, quad_omega_factor(c->k), kLanczos, c->stream));
     LAUNCHCHK(c, launch_quad_init(c->qs, c->ql, c->stream));
     if (fork) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
     LAUNCHCHK(c, launch_quad_residual(c->qs, c->ql, mixed(c), c->stream));

@@ -628,7 +628,7 @@ int enqueue_setup(hdg_batch* b, Group& g) {
   BLAUNCH(b, launch_quad_tp(g.qs, g.ql, g.s));
   if (g.mixed) BLAUNCH(b, launch_quad_float(g.qs, g.s));
   // the CG vectors serve as scratch before the solve initialises them
-  BLAUNCH(b, launch_quad_omega(g.qs, g.ql, quad_omega_factor(g.k), kQuadLanczos, g.s));
+  BLAUNCH(b, launch_quad_omega(g.qs, g.ql, quad_omega_factor(g.k), kLanczos, g.s));
   BLAUNCH(b, launch_quad_init(g.qs, g.ql, g.s));
   BLAUNCH(b, launch_quad_residual(g.qs, g.ql, g.mixed, g.s));
   BLAUNCH(b, launch_vcycle_group(g.G, 0.0, -1, g.s));

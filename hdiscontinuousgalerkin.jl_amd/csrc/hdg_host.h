@@ -8,7 +8,7 @@
 namespace hdg {
 
 // Sizes of the vertex hierarchy of an nx x ny rectangle mesh: fills nlev,
-// lev[1..nlev-1].nx, ny, n, npts and tail (no device arrays).
+// lev[1..nlev-1].nx, ny, n and tail (no device arrays).
 void mg_plan_levels(int nx, int ny, MgData& M);
 
 // Pinned memory through which results leave for host arrays: a head for

@@ -121,8 +121,9 @@ struct DirichletRule {
   double leg[5 * kMaxFacePoints];
 };
 
-// PCG coefficients kept for the Lanczos estimate of lambda_max(Dinv S)
-constexpr int kLanczos = 16;
+// Lanczos steps behind the smoothing weight of the reduced trace system, an
+// estimate of lambda_max(Dinv T)
+constexpr int kLanczos = 4;
 
 // PCG scalar state, resident on the device; written by block 0 of the
 // kernels that own each field, read by later launches.
@@ -131,7 +132,7 @@ struct CgState {
   double pq;
   double rr;     // (r, r) at the last convergence test
   double bb;     // (b~, b~)
-  double omega;  // block-Jacobi smoothing weight of the multigrid preconditioner
+  double omega;  // block-Jacobi smoothing weight on the reduced trace system
   int it;        // completed iterations when the solve stopped
   int maxit;
   int done;      // 0 running, 1 converged, 2 iteration cap, 3 breakdown
@@ -142,9 +143,9 @@ struct CgState {
   int i_spmv;    // for the next CG product (written by the update / smoother)
   int i_upd;     // for the update (written by the product)
   int i_pre;     // for the smoother (written by the multigrid update)
-  // iteration i <= kLanczos of a run: (r, z) at its product and (p, S p) at
-  // its update; block-Jacobi PCG's coefficients are those of the Lanczos
-  // process of Dinv S
+  // step i of the Lanczos run: (r, z) at its product and (p, T p) at its
+  // update; block-Jacobi PCG's coefficients are those of the Lanczos process
+  // of Dinv T
   double lz[kLanczos + 1];
   double lpq[kLanczos + 1];
 };

@@ -117,9 +117,8 @@ int launch_quad_finish(const QuadSys& S, const QuadLaunch& L, double* uhat, doub
 int launch_quad_time(const QuadSys& S, const QuadLaunch& L, int which, hipStream_t s);
 
 // the smoothing weight over the Lanczos estimate of lambda_max(Dinv T), by
-// order, and the number of steps behind the estimate
+// order
 double quad_omega_factor(int k);
-constexpr int kQuadLanczos = 4;
 
 // V-cycle on the vertex levels, the next product's convergence test first
 // (maxit < 0: none)

@@ -823,13 +823,13 @@ __global__ __launch_bounds__(kQuadThreads) void q_omega_kernel(QuadSys S, Sel se
   const QuadInst& I = inst_block(sel);
   CgState* st = I.st;
   const int done = st->done, its = st->it;
-  double lz[kQuadLanczos + 2], lpq[kQuadLanczos + 1];
+  double lz[kLanczos + 2], lpq[kLanczos + 1];
 #pragma unroll
-  for (int j = 1; j <= kQuadLanczos; ++j) {
+  for (int j = 1; j <= kLanczos; ++j) {
     lz[j] = st->lz[j];
     lpq[j] = st->lpq[j];
   }
-  lz[kQuadLanczos + 1] = 0.0;
+  lz[kLanczos + 1] = 0.0;
   const double pq = bsum(pshare(S.part + I.pM, I.nbM), sh);
   if (threadIdx.x != 0) return;
   if (done) {
@@ -837,12 +837,12 @@ __global__ __launch_bounds__(kQuadThreads) void q_omega_kernel(QuadSys S, Sel se
   } else {
     st->lpq[m] = pq;
 #pragma unroll
-    for (int j = 1; j <= kQuadLanczos; ++j) lpq[j] = j == m ? pq : lpq[j];
+    for (int j = 1; j <= kLanczos; ++j) lpq[j] = j == m ? pq : lpq[j];
   }
-  double d[kQuadLanczos], e2[kQuadLanczos];
+  double d[kLanczos], e2[kLanczos];
   int n = 0;
 #pragma unroll
-  for (int j = 1; j <= kQuadLanczos; ++j) {
+  for (int j = 1; j <= kLanczos; ++j) {
     if (j > m || n != j - 1) continue;
     const double a = lz[j] / lpq[j];
     double dj = 1.0 / a;
@@ -1633,7 +1633,7 @@ int launch_quad_tp(const QuadSys& S, const QuadLaunch& L, hipStream_t s) {
 int launch_quad_l1(const QuadSys& S, const QuadLaunch& L, hipStream_t s) { return GO(E, q_l1_kernel); }
 
 int launch_quad_omega(const QuadSys& S, const QuadLaunch& L, double factor, int steps, hipStream_t s) {
-  steps = std::min(std::max(steps, 1), kQuadLanczos);
+  steps = std::min(std::max(steps, 1), kLanczos);
 #define INIT(NT) QTRY(GO2(E, q_init_kernel, NT, true));
 #define PROD(NT) QTRY(GO2(M, q_product_kernel, NT, true, 0.0, steps, 0));
 #define UPD(NT) QTRY(GO1(E, q_lupd_kernel, NT));
