@@ -179,37 +179,91 @@ void copy_share(const char* buf, const StagePieces& p, int t, int nshares) {
   }
 }
 
-void stage_free_buffer(HostStage& st) {
-  if (st.mem) (void)hipHostFree(st.mem);
-  st.mem = nullptr;
-  st.head = st.chunk = st.bufs = 0;
+// The process's pinned memory for exports, in pieces of two sizes (one chunk,
+// or kStageBufs of them, and a head) that are lent to one export each, on any stream or thread.  Pinning costs 0.25-0.3 ms a
+// piece whatever its size (30 us where nothing was unpinned before it), more
+// than a small export: with pieces of its own, grown twice, a new context's
+// first export of 12 x 9 P1 cells took 1.2 ms, now 0.4.  Up to kIdle of each
+// size wait for the next export; when the last context and batch go, all but
+// one small piece are given back.
+constexpr size_t kSmallPiece = kChunk + (64u << 10), kLargePiece = kStageBufs * kChunk + (1u << 20);
+constexpr int kIdle = 8;
+struct StagePiece {
+  char* mem = nullptr;
+  size_t bytes = 0;
+  int device = -1;
+  bool small() const { return bytes <= kSmallPiece; }
+};
+struct StagePool {
+  std::mutex m;
+  int owners = 0, n = 0;
+  StagePiece idle[2 * kIdle];
+};
+StagePool& stage_pool() {
+  static StagePool* p = new StagePool;  // outlives every owner, static ones too
+  return *p;
 }
 
-// Memory and events for a result of `total` bytes and a head of `head` bytes.
-int stage_reserve(HostStage& st, size_t total, size_t head) {
-  head = (head + kHeadAlign - 1) / kHeadAlign * kHeadAlign;
-  // one buffer for what fits, else kStageBufs chunks
-  const size_t one = std::max<size_t>(65536, (total + 4095) / 4096 * 4096);
-  const size_t chunk = std::min(one, kChunk), bufs = total <= chunk ? 1 : kStageBufs;
-  for (hipEvent_t& e : st.ev)
-    if (!e) {
-      const hipError_t r = hipEventCreateWithFlags(&e, hipEventDisableTiming);
-      if (r != hipSuccess) return (int)r;
+// Memory for a result of `total` bytes and a head of `head` bytes: bufs chunks
+// behind the head; 0 or a hipError_t in err.
+struct StageLease {
+  HostStage& st;
+  StagePiece p;
+  int err = 0;
+  size_t head, chunk, bufs;
+  StageLease(HostStage& owner, size_t total, size_t head_bytes) : st(owner) {
+    head = (head_bytes + kHeadAlign - 1) / kHeadAlign * kHeadAlign;
+    // one buffer for what fits, else kStageBufs chunks
+    const size_t one = std::max<size_t>(65536, (total + 4095) / 4096 * 4096);
+    chunk = std::min(one, kChunk);
+    bufs = total <= chunk ? 1 : kStageBufs;
+    hipError_t e = hipSuccess;
+    for (hipEvent_t& ev : st.ev)
+      if (!ev && e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    const size_t need = head + bufs * chunk;
+    int device = 0;
+    if (e == hipSuccess) e = hipGetDevice(&device);
+    if (e == hipSuccess) {
+      StagePool& pool = stage_pool();
+      std::lock_guard<std::mutex> lk(pool.m);
+      int best = -1;
+      for (int i = 0; i < pool.n; ++i)
+        if (pool.idle[i].device == device && pool.idle[i].bytes >= need &&
+            (best < 0 || pool.idle[i].bytes < pool.idle[best].bytes))
+          best = i;
+      if (best >= 0) {
+        p = pool.idle[best];
+        pool.idle[best] = pool.idle[--pool.n];
+      }
     }
-  if (head > st.head || chunk > st.chunk || bufs > st.bufs) {
-    const size_t h = std::max(head, st.head), ch = std::max(chunk, st.chunk), nb = std::max(bufs, st.bufs);
-    stage_free_buffer(st);
-    const hipError_t r = hipHostMalloc((void**)&st.mem, h + nb * ch, hipHostMallocDefault);
-    if (r != hipSuccess) {
-      st.mem = nullptr;
-      return (int)r;
+    if (e == hipSuccess && !p.mem) {
+      const size_t mb = 1u << 20, bytes = need <= kSmallPiece ? kSmallPiece : std::max(kLargePiece, (need + mb - 1) / mb * mb);
+      e = hipHostMalloc((void**)&p.mem, bytes, hipHostMallocDefault);
+      if (e != hipSuccess) p.mem = nullptr;
+      p.bytes = bytes;
+      p.device = device;
     }
-    st.head = h;
-    st.chunk = ch;
-    st.bufs = nb;
+    err = (int)e;
   }
-  return 0;
-}
+  // after the export: nothing on the device writes the piece any more
+  ~StageLease() {
+    if (!p.mem) return;
+    {
+      StagePool& pool = stage_pool();
+      std::lock_guard<std::mutex> lk(pool.m);
+      int same = 0;
+      for (int i = 0; i < pool.n; ++i) same += pool.idle[i].small() == p.small();
+      if (same < kIdle) {
+        pool.idle[pool.n++] = p;
+        return;
+      }
+    }
+    (void)hipHostFree(p.mem);
+  }
+  StageLease(const StageLease&) = delete;
+  StageLease& operator=(const StageLease&) = delete;
+  char* chunk_at(int64_t b) const { return p.mem + head + b * chunk; }
+};
 
 // A wait of some microseconds: spins, and lets go of the core only when it has
 // lasted long.  (Where other threads spin on every core, as a BLAS library's do
@@ -231,15 +285,15 @@ struct Patience {
 // copied in shares, taken by the caller's thread and by those of a crew
 // as each is free: nothing waits for a thread that has no core, except to the
 // end of a share it has begun.
-int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, StageFill fill, void* arg) {
+int staged_out(StageLease& L, hipStream_t s, int64_t nchunks, size_t total, StageFill fill, void* arg) {
+  HostStage& st = L.st;
   StagePieces pieces[kStageBufs];
   std::atomic<int64_t> ready{0};  // chunks that have arrived in their buffers
   std::atomic<int64_t> taken{0};  // shares taken, over all chunks
   std::atomic<int64_t> done[kStageBufs] = {};  // shares copied from each buffer
   std::atomic<bool> stop{false};
   std::thread crew[kCrew];
-  const int nb = (int)st.bufs;
-  char* const buf0 = st.mem + st.head;
+  const int nb = (int)L.bufs;
   const int want = (int)std::min<size_t>({(size_t)kCrew, total / kPerThread,
                                           (size_t)std::max(1u, std::thread::hardware_concurrency() / 2)});
   const int shares = want > 1 ? 2 * kCrew : 1;
@@ -250,7 +304,7 @@ int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, Stag
       if (i >= ready.load(std::memory_order_acquire) * shares) return false;
     } while (!taken.compare_exchange_weak(i, i + 1, std::memory_order_relaxed));
     const int b = (int)(i / shares % nb);
-    copy_share(buf0 + b * st.chunk, pieces[b], (int)(i % shares), shares);
+    copy_share(L.chunk_at(b), pieces[b], (int)(i % shares), shares);
     done[b].fetch_add(1, std::memory_order_release);
     return true;
   };
@@ -265,7 +319,7 @@ int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, Stag
   const auto launch = [&](int64_t k) {
     StagePieces& p = pieces[k % nb];
     p.n = 0;
-    int r = fill(arg, k, buf0 + (k % nb) * st.chunk, p);
+    int r = fill(arg, k, L.chunk_at(k % nb), p);
     if (!r) r = (int)hipEventRecord(st.ev[k % nb], s);
     return r;
   };
@@ -316,8 +370,31 @@ int staged_out(HostStage& st, hipStream_t s, int64_t nchunks, size_t total, Stag
 
 }  // namespace
 
+HostStage::HostStage() {
+  StagePool& pool = stage_pool();
+  std::lock_guard<std::mutex> lk(pool.m);
+  ++pool.owners;
+}
+
+HostStage::~HostStage() {
+  StagePiece out[2 * kIdle];
+  int n = 0;
+  {
+    StagePool& pool = stage_pool();
+    std::lock_guard<std::mutex> lk(pool.m);
+    if (--pool.owners > 0) return;
+    int kept = 0;
+    for (int i = 0; i < pool.n; ++i)
+      if (pool.idle[i].small() && kept == 0)
+        pool.idle[kept++] = pool.idle[i];
+      else
+        out[n++] = pool.idle[i];
+    pool.n = kept;
+  }
+  for (int i = 0; i < n; ++i) (void)hipHostFree(out[i].mem);
+}
+
 void stage_free(HostStage& st) {
-  stage_free_buffer(st);
   for (hipEvent_t& e : st.ev)
     if (e) {
       (void)hipEventDestroy(e);
@@ -327,15 +404,16 @@ void stage_free(HostStage& st) {
 
 int staged_copy(HostStage& st, hipStream_t s, double* dst, const double* src, int64_t n) {
   std::lock_guard<std::mutex> lk(st.m);
-  if (int e = stage_reserve(st, sizeof(double) * n, 0)) return e;
+  StageLease L(st, sizeof(double) * n, 0);
+  if (L.err) return L.err;
   struct Arg {
     double* dst;
     const double* src;
     int64_t n, per;
     hipStream_t s;
-  } a{dst, src, n, (int64_t)(st.chunk / sizeof(double)), s};
+  } a{dst, src, n, (int64_t)(L.chunk / sizeof(double)), s};
   return staged_out(
-      st, s, (n + a.per - 1) / a.per, sizeof(double) * n,
+      L, s, (n + a.per - 1) / a.per, sizeof(double) * n,
       [](void* p, int64_t k, char* buf, StagePieces& out) {
         const Arg& a = *static_cast<Arg*>(p);
         const int64_t i0 = k * a.per, m = std::min(a.per, a.n - i0);
@@ -353,7 +431,8 @@ int staged_values(HostStage& st, hipStream_t s, int k, const DevMesh& m, const d
   if (!per) return 0;
   const size_t total = sizeof(double) * per * m.nc;
   std::lock_guard<std::mutex> lk(st.m);
-  if (int e = stage_reserve(st, total, 0)) return e;
+  StageLease L(st, total, 0);
+  if (L.err) return L.err;
   struct Arg {
     int k, nu, nt;
     DevMesh m;
@@ -362,9 +441,9 @@ int staged_values(HostStage& st, hipStream_t s, int k, const DevMesh& m, const d
     double *q, *u, *uc;
     int64_t per;
     hipStream_t s;
-  } a{k, nu, nt, m, qu, uhat, rows, q, u, uc, (int64_t)(st.chunk / (sizeof(double) * per)), s};
+  } a{k, nu, nt, m, qu, uhat, rows, q, u, uc, (int64_t)(L.chunk / (sizeof(double) * per)), s};
   return staged_out(
-      st, s, (m.nc + a.per - 1) / a.per, total,
+      L, s, (m.nc + a.per - 1) / a.per, total,
       [](void* p, int64_t c, char* buf, StagePieces& out) {
         const Arg& a = *static_cast<Arg*>(p);
         const int64_t nc = a.m.nc, e0 = c * a.per, n = std::min(a.per, nc - e0);
@@ -405,16 +484,17 @@ int staged_transposes(HostStage& st, hipStream_t s, int k, double* dst, const do
   const int ntr = 3 * (k + 1), w = ntr * ntr;
   const size_t total = sizeof(double) * w * nc;
   std::lock_guard<std::mutex> lk(st.m);
-  if (int e = stage_reserve(st, total, 0)) return e;
+  StageLease L(st, total, 0);
+  if (L.err) return L.err;
   struct Arg {
     int k, w;
     double* dst;
     const double* src;
     int64_t nc, per;
     hipStream_t s;
-  } a{k, w, dst, src, nc, (int64_t)(st.chunk / (sizeof(double) * w)), s};
+  } a{k, w, dst, src, nc, (int64_t)(L.chunk / (sizeof(double) * w)), s};
   return staged_out(
-      st, s, (nc + a.per - 1) / a.per, total,
+      L, s, (nc + a.per - 1) / a.per, total,
       [](void* p, int64_t c, char* buf, StagePieces& out) {
         const Arg& a = *static_cast<Arg*>(p);
         const int64_t e0 = c * a.per, n = std::min(a.per, a.nc - e0);
@@ -483,8 +563,9 @@ int staged_csc(HostStage& st, hipStream_t s, const DevPattern& pat, int nt, int6
   const size_t total = face * nf;
   // at least one block of faces per chunk (524 KB at five modes)
   std::lock_guard<std::mutex> lk(st.m);
-  if (int e = stage_reserve(st, std::max<size_t>(total, face * kCscFaces), sizeof(int64_t) * (nblk + 1))) return e;
-  int64_t* pre = (int64_t*)st.mem;
+  StageLease L(st, std::max<size_t>(total, face * kCscFaces), sizeof(int64_t) * (nblk + 1));
+  if (L.err) return L.err;
+  int64_t* pre = (int64_t*)L.p.mem;
   hipLaunchKernelGGL(csc_count_kernel, dim3((unsigned)nblk), dim3(kBlock), 0, s, pat, nf, pre);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -495,9 +576,9 @@ int staged_csc(HostStage& st, hipStream_t s, const DevPattern& pat, int nt, int6
     pre[b] = sum;
     sum += n;
   }
-  const int64_t nb = (int64_t)(st.chunk / (face * kCscFaces));
+  const int64_t nb = (int64_t)(L.chunk / (face * kCscFaces));
   CscArg<I> a{pat, vals, nf, nf * nt, nblk, nb, nt, base, pre, colptr, rowval, nzval, s};
-  const int r = staged_out(st, s, (nblk + nb - 1) / nb, total, csc_chunk<I>, &a);
+  const int r = staged_out(L, s, (nblk + nb - 1) / nb, total, csc_chunk<I>, &a);
   if (!r && colptr) colptr[nf * nt] = (I)(sum * nt * nt + base);
   return r;
 }

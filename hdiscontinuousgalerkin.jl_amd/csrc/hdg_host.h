@@ -11,15 +11,17 @@ namespace hdg {
 // lev[1..nlev-1].nx, ny, n and tail (no device arrays).
 void mg_plan_levels(int nx, int ny, MgData& M);
 
-// Pinned memory through which results leave for host arrays: a head for
-// offsets and up to kStageBufs chunks of up to 4 MB, kept by its owner until
-// the owner goes; concurrent exports of one owner take turns.
+// An owner of exports, a context or a batch: the events of its chunks; its
+// concurrent exports take turns.  The pinned memory through which results leave
+// for host arrays is the process's, lent to one export at a time.
 constexpr int kStageBufs = 3;
 struct HostStage {
   std::mutex m;
-  char* mem = nullptr;
-  size_t head = 0, chunk = 0, bufs = 0;
   hipEvent_t ev[kStageBufs] = {};
+  HostStage();
+  ~HostStage();
+  HostStage(const HostStage&) = delete;
+  HostStage& operator=(const HostStage&) = delete;
 };
 void stage_free(HostStage& st);
 
