@@ -746,8 +746,6 @@ int setup_quad(hdg_ctx* c) {
   const int nt = c->nt;
   const size_t pts = (size_t)I.ntiles * 64;
   TRY(dalloc(c, &q.blk, pts * quad_blk_vals(nt)));
-  // the couplings of the quads that do not exist stay zero
-  HIPCHK(c, hipMemsetAsync(q.blk, 0, sizeof(double) * pts * quad_blk_vals(nt), c->stream));
   TRY(dalloc(c, &q.D, pts * quad_diag_vals(nt)));
   TRY(dalloc(c, &q.Dinv, pts * quad_diag_vals(nt)));
   TRY(dalloc(c, &q.tp, pts * quad_tp_vals(nt)));
@@ -785,6 +783,7 @@ int setup_quad(hdg_ctx* c) {
   I.l1dinv = L.dinv;
   I.vmask = L.mask;
   c->ql = quad_launch_one(I, nt);
+  LAUNCHCHK(c, launch_quad_clear(q, c->ql, c->stream));
   return HDG_OK;
 }
 

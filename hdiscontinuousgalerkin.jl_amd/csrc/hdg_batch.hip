@@ -289,7 +289,6 @@ int build_quad_group(hdg_batch* b, Group& g) {
   }
   const size_t pts = (size_t)tiles * 64;
   BTRY(galloc(b, g, &q.blk, pts * quad_blk_vals(nt)));
-  BHIP(b, hipMemsetAsync(q.blk, 0, sizeof(double) * pts * quad_blk_vals(nt), g.s));
   BTRY(galloc(b, g, &q.D, pts * quad_diag_vals(nt)));
   BTRY(galloc(b, g, &q.Dinv, pts * quad_diag_vals(nt)));
   BTRY(galloc(b, g, &q.tp, pts * quad_tp_vals(nt)));
@@ -332,6 +331,7 @@ int build_quad_group(hdg_batch* b, Group& g) {
   L.gE = (int)mE.size();
   L.gQ = (int)mQ.size();
   L.ninst = n;
+  BLAUNCH(b, launch_quad_clear(q, L, g.s));
   return HDG_OK;
 }
 

@@ -76,7 +76,7 @@ struct QuadSys {
   TraceSystem K;
 };
 // doubles per point of the arrays above (x .. res: 2 nt each)
-inline int quad_blk_vals(int nt) { return 6 * nt * nt; }
+__host__ __device__ inline int quad_blk_vals(int nt) { return 6 * nt * nt; }
 inline int quad_diag_vals(int nt) { return nt * (nt + 1); }
 inline int quad_tp_vals(int nt) { return 12 * nt; }
 inline int quad_bq_vals(int nt) { return 9 * nt; }
@@ -94,6 +94,8 @@ struct QuadLaunch {
 };
 QuadLaunch quad_launch_one(const QuadInst& I, int nt);
 
+// once per set-up, before the first launch_quad_build
+int launch_quad_clear(const QuadSys& S, const QuadLaunch& L, hipStream_t s);
 // masks, the reduced system and its loads from the condensed cells, D, Dinv
 int launch_quad_build(const QuadSys& S, const QuadLaunch& L, hipStream_t s);
 // float copies for HDG_MIXED (after launch_quad_tp)
