@@ -1166,6 +1166,11 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
       cn[3 * e + l] = (int)(nd - 1);
       cf[3 * e + l] = (int)(fc - 1);
     }
+  int nx = 0, ny = 0;
+  const bool numbered = detect_numbering(nn, nc, cells, &nx, &ny);
+  const bool structured = numbered && grid_faces(nx, ny, nf, cf, fcell);
+  std::vector<double> places;
+  if (!structured) places.assign(xy, xy + 2 * nn);
   Recycle reuse(c);
   free_mesh(c);
   double* dxy;
@@ -1194,16 +1199,15 @@ int hdg_set_mesh(hdg_ctx* c, int64_t nn, const double* xy, int64_t nc, const int
   LAUNCHCHK(c, launch_pattern(c->mesh, c->pat, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->nblock_cols = nblk;
-  int nx = 0, ny = 0;
-  c->numbered = detect_numbering(nn, nc, cells, &nx, &ny);
-  c->structured = c->numbered && grid_faces(nx, ny, nf, cf, fcell);
-  if (c->structured) {
+  c->numbered = numbered;
+  c->structured = structured;
+  if (structured) {
     TRY(build_vertex_levels(c, nx, ny));
   } else {
     c->h_cn.swap(cn);
     c->h_cf.swap(cf);
     c->h_fcell.swap(fcell);
-    c->h_xy.assign(xy, xy + 2 * nn);
+    c->h_xy.swap(places);
   }
   c->has_mesh = true;
   return HDG_OK;
